@@ -317,33 +317,278 @@ __device__ __forceinline__ int t2c_row_len(const int *tile_nnz, const unsigned c
     return e - s;
 }
 
-template <int PASS>
-__global__ void __launch_bounds__(256)
-k_t2c_rows(int m, const int *__restrict__ tile_ptr, const int *__restrict__ tile_colidx,
-           const int *__restrict__ tile_nnz, const unsigned char *__restrict__ csr_ptr,
-           const unsigned char *__restrict__ tcol, const double *__restrict__ tval,
-           int *__restrict__ rowcnt_or_ptr, int *__restrict__ col, double *__restrict__ val, int jbase) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    const int I = i >> 4, r = i & 15;
-    const int rowlen = min(16, m - I * 16);
-    const int t0 = tile_ptr[I], t1 = tile_ptr[I + 1];
-    if (PASS == 0) {
-        int c = 0;
-        for (int t = t0; t < t1; t++) c += t2c_row_len(tile_nnz, csr_ptr, t, r, rowlen);
-        rowcnt_or_ptr[i] = c;
-    } else {
-        int out = rowcnt_or_ptr[i];
-        for (int t = t0; t < t1; t++) {
-            const int k = t2c_row_len(tile_nnz, csr_ptr, t, r, rowlen);
-            if (k <= 0) continue;
-            const int s = tile_nnz[t] + csr_ptr[(long long)t * 16 + r];
-            const int J16 = (tile_colidx[t] - jbase) * 16;
-            for (int j = 0; j < k; j++) {
-                col[out + j] = J16 + tcol[s + j];
-                val[out + j] = tval[s + j];
+// A tile-row's entries are the same contiguous range in both formats, so the
+// conversion is a permutation inside it and needs no scan over the rows:
+// row 16I+r starts at the tile-row's first entry plus the entries of its
+// rows before r.  Work is one wave per run of at most CV_SEG tiles of a
+// tile-row (a hub tile-row's further runs go through an item list, each with
+// its 16 rows' entries before it), in batches of at most 64 tiles and CV_CAP
+// entries: the batch is loaded as one contiguous range, permuted through
+// LDS, and written as 16 row runs.  Bound by HBM: 9 bytes in (plus the tile
+// index) and 12 out per entry.  One thread per matrix row walking its tiles
+// left 8-byte accesses to 64 different lines per instruction and a hub
+// row's whole walk on one lane: 62M entries of a 27-point product (27d
+// 79x83x81, A^2) 2.31 -> 0.55 ms for the call, 2.9 TB/s in k_t2c_emit; the
+// row index of R-MAT scale 18 17.4 -> 0.48 ms (both kernels).
+#define CV_WAVES 4
+#define CV_SEG 1024
+#define CV_CAP 448
+struct T2cItem {
+    int I, seg;     // tiles [CV_SEG * seg, CV_SEG * (seg + 1)) of tile-row I
+    int carry[16];  // entries of each row in the tile-row's tiles before them
+};
+
+// A tile's row offsets with those past the matrix's rows (rowlen < 16, the
+// last tile-row) set to the tile's entry count, at most 240 there.
+__device__ __forceinline__ uint4 t2c_offsets(uint4 p, int tnnz, int rowlen) {
+    unsigned w[4] = {p.x, p.y, p.z, p.w};
+    if (rowlen < 16) {
+#pragma unroll
+        for (int q = 0; q < 16; q++)
+            if (q >= rowlen) w[q >> 2] = (w[q >> 2] & ~(0xffu << (8 * (q & 3)))) | ((unsigned)tnnz << (8 * (q & 3)));
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+// The 16 row lengths of a tile, one byte each, from those offsets: next
+// offset minus offset, byte by byte.  Offsets ascend, so no borrow crosses a
+// byte; the last byte's minuend is the entry count (mod 256).
+__device__ __forceinline__ uint4 t2c_row_lens(uint4 p, int tnnz) {
+    return make_uint4(((p.x >> 8) | (p.y << 24)) - p.x, ((p.y >> 8) | (p.z << 24)) - p.y,
+                      ((p.z >> 8) | (p.w << 24)) - p.z, ((p.w >> 8) | ((unsigned)tnnz << 24)) - p.w);
+}
+// Bytes as 16-bit pairs: v[2q] = rows 4q and 4q+2, v[2q+1] = rows 4q+1, 4q+3.
+__device__ __forceinline__ void t2c_widen(uint4 l, unsigned v[8]) {
+    const unsigned w[4] = {l.x, l.y, l.z, l.w};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        v[2 * q] = w[q] & 0x00ff00ffu;
+        v[2 * q + 1] = (w[q] >> 8) & 0x00ff00ffu;
+    }
+}
+
+// 16 bytes from an address of any alignment (one load: the target allows
+// unaligned global access).
+__device__ __forceinline__ uint4 load16(const unsigned char *p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
+// Row pointers; one wave per tile-row of up to CV_SEG tiles (four tiles at a
+// time, lane = (tile, row)), the block's four waves together for a longer
+// one (four tiles per thread and run).  *nitems (zeroed beforehand) counts
+// the further runs (the first maxitems are listed); host (pinned) gets the
+// entries and the tiles of the matrix or view.
+__global__ void __launch_bounds__(64 * CV_WAVES)
+k_t2c_rowptr(int m, int tilem, const int *__restrict__ tile_ptr, const int *__restrict__ tile_nnz,
+             const unsigned char *__restrict__ csr_ptr, int *__restrict__ rowptr, T2cItem *__restrict__ items,
+             int *__restrict__ nitems, int maxitems, long long *__restrict__ host) {
+    __shared__ int s_sum[CV_WAVES][16];
+    __shared__ int s_slot;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, ts = lane >> 4;
+    const int nb0 = tile_nnz[tile_ptr[0]];
+    const int I = blockIdx.x * CV_WAVES + wave;
+    if (I < tilem) {
+        const int t0 = tile_ptr[I], t1 = tile_ptr[I + 1];
+        if (t1 - t0 <= CV_SEG) {
+            const int rowlen = min(16, m - 16 * I);
+            int c = 0;
+#pragma unroll 4
+            for (int t = t0 + ts; t < t1; t += 4)
+                if (r < rowlen) c += t2c_row_len(tile_nnz, csr_ptr, t, r, rowlen);
+            c += __shfl_xor(c, 16, 64);
+            c += __shfl_xor(c, 32, 64);
+            const int incl = tsg_group16_incl_scan(c);
+            if (lane < rowlen) rowptr[16 * I + lane] = tile_nnz[t0] - nb0 + incl - c;
+        }
+        if (I == tilem - 1 && lane == 0) {
+            const int nnz = tile_nnz[t1] - nb0;
+            rowptr[m] = nnz;
+            host[0] = nnz;
+            host[1] = t1 - tile_ptr[0];
+        }
+    }
+    for (int w = 0; w < CV_WAVES; w++) {
+        const int Iw = blockIdx.x * CV_WAVES + w;
+        if (Iw >= tilem) break;
+        const int t0 = tile_ptr[Iw], t1 = tile_ptr[Iw + 1];
+        if (t1 - t0 <= CV_SEG) continue;  // block-uniform
+        const int rowlen = min(16, m - 16 * Iw), nseg = (t1 - t0 + CV_SEG - 1) / CV_SEG;
+        if (tid == 0) s_slot = atomicAdd(nitems, nseg - 1);
+        __syncthreads();
+        const int slot = s_slot;
+        int carry = 0;  // threads 0..15: the row's entries so far
+        for (int sg = 0; sg < nseg; sg++) {
+            if (sg > 0 && tid < 16 && slot + sg <= maxitems) {
+                items[slot + sg - 1].carry[tid] = carry;
+                if (tid == 0) {
+                    items[slot + sg - 1].I = Iw;
+                    items[slot + sg - 1].seg = sg;
+                }
             }
-            out += k;
+            unsigned v[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // at most 16 * CV_SEG per half
+#pragma unroll
+            for (int k = 0; k < CV_SEG / (64 * CV_WAVES); k++) {
+                const int t = t0 + sg * CV_SEG + k * 64 * CV_WAVES + tid;
+                if (t < t1) {
+                    unsigned x[8];
+                    const int tn = tile_nnz[t + 1] - tile_nnz[t];
+                    t2c_widen(t2c_row_lens(t2c_offsets(load16(csr_ptr + 16 * (long long)t), tn, rowlen), tn), x);
+#pragma unroll
+                    for (int q = 0; q < 8; q++) v[q] += x[q];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] = tsg_wave_sum(v[q]);
+            if (lane == 0) {
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    s_sum[wave][4 * (q >> 1) + (q & 1)] = (int)(v[q] & 0xffffu);
+                    s_sum[wave][4 * (q >> 1) + (q & 1) + 2] = (int)(v[q] >> 16);
+                }
+            }
+            __syncthreads();
+            if (tid < 16)
+                for (int w2 = 0; w2 < CV_WAVES; w2++) carry += s_sum[w2][tid];
+            __syncthreads();
+        }
+        if (tid < 16) {
+            const int incl = tsg_group16_incl_scan(carry);
+            if (tid < rowlen) rowptr[16 * Iw + tid] = tile_nnz[t0] - nb0 + incl - carry;
+        }
+        __syncthreads();  // s_slot
+    }
+}
+
+// Bytes of w that are at most j, as 0x80 bits (unsigned, per byte).
+__device__ __forceinline__ unsigned bytes_le(unsigned w, unsigned j) {
+    const unsigned H = 0x80808080u, x = j * 0x01010101u;
+    const unsigned t = (x | H) - (w & ~H);  // per byte, no borrow out
+    return ((x & ~w) | (~(x ^ w) & t)) & H;
+}
+
+// Entries: the first tilem waves take each tile-row's first run, the others
+// the item list.  One lane per entry: its tile from a mark at each tile's
+// first entry (running maximum over the lanes), its row from the tile's row
+// offsets, its place in the batch from the (tile, row)'s entries before it.
+#define CV_ROUNDS (CV_CAP / 64)
+__global__ void __launch_bounds__(64 * CV_WAVES)
+k_t2c_emit(int m, int tilem, const int *__restrict__ tile_ptr, const int *__restrict__ tile_colidx,
+           const int *__restrict__ tile_nnz, const unsigned char *__restrict__ csr_ptr,
+           const unsigned char *__restrict__ tcol, const double *__restrict__ tval, const int *__restrict__ rowptr,
+           const T2cItem *__restrict__ items, const int *__restrict__ nitems, int nblocks_rows, int jbase,
+           int *__restrict__ col, double *__restrict__ val) {
+    static_assert(CV_CAP % 64 == 0 && CV_CAP >= 256, "whole rounds; a full tile fits");
+    // per wave: the batch's values, columns and rows in output order (the
+    // row bytes first hold the tile marks), each tile's row offsets, and each
+    // (tile, row)'s first output position (row 64: the rows' ends)
+    __shared__ double s_val[CV_WAVES][CV_CAP];
+    __shared__ int s_col[CV_WAVES][CV_CAP];
+    __shared__ __align__(16) unsigned char s_row[CV_WAVES][CV_CAP];
+    __shared__ uint4 s_p16[CV_WAVES][64];
+    __shared__ __align__(16) unsigned short s_pre[CV_WAVES][65 * 16];
+    __shared__ int s_dst[CV_WAVES][16];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15;
+    double *sv = s_val[wave];
+    int *sc = s_col[wave], *sd = s_dst[wave];
+    unsigned char *sr = s_row[wave];
+    unsigned short *sp = s_pre[wave];
+    const bool listed = (int)blockIdx.x >= nblocks_rows;
+    const int nwork = listed ? *nitems : tilem;
+    const int step = listed ? (int)(gridDim.x - nblocks_rows) * CV_WAVES : tilem;
+    for (int w = (listed ? (int)blockIdx.x - nblocks_rows : (int)blockIdx.x) * CV_WAVES + wave; w < nwork; w += step) {
+        const int I = listed ? items[w].I : w, sg = listed ? items[w].seg : 0;
+        const int rowlen = min(16, m - 16 * I);
+        const int t1 = tile_ptr[I + 1], ta = tile_ptr[I] + sg * CV_SEG, te = min(t1, ta + CV_SEG);
+        // lanes r, r + 16, ...: where row r's next run starts in the output
+        int gout = r < rowlen ? rowptr[16 * I + r] : 0;
+        if (listed) gout += items[w].carry[r];
+        for (int tb = ta; tb < te;) {
+            const int t = min(tb + lane, te - 1);
+            const int n0 = tile_nnz[t], n1 = tile_nnz[t + 1];
+            const uint4 p16 = t2c_offsets(load16(csr_ptr + 16 * (long long)t), n1 - n0, rowlen);
+            const int J16 = (tile_colidx[t] - jbase) * 16;
+            const int start = __builtin_amdgcn_readfirstlane(n0);
+            // the batch: the leading tiles whose entries fit (a tile holds at most 256)
+            const int nt = __popcll(__ballot(tb + lane < te && n1 - start <= CV_CAP));
+            const int total = __builtin_amdgcn_readlane(n1, nt - 1) - start;
+            if (total == 0) {
+                tb += nt;
+                continue;
+            }
+            double v[CV_ROUNDS];
+            unsigned char c8[CV_ROUNDS];
+#pragma unroll
+            for (int i = 0; i < CV_ROUNDS; i++) {  // every lane loads in bounds
+                const int x = min(lane + 64 * i, total - 1);
+                v[i] = tval[start + x];
+                c8[i] = tcol[start + x];
+            }
+            // tile marks (k + 1 at each nonempty tile's first entry), row offsets
+            for (int i = lane; i < CV_CAP / 4; i += 64) reinterpret_cast<unsigned *>(sr)[i] = 0u;
+            s_p16[wave][lane] = p16;
+            tsg_wave_sync();
+            if (lane < nt && n1 > n0) sr[n0 - start] = (unsigned char)(lane + 1);
+            // entries of each row in the tiles before the lane's; the rows' runs
+            unsigned len[8], tot[8];
+            t2c_widen(t2c_row_lens(p16, n1 - n0), len);
+            unsigned run = 0;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                if (lane >= nt) len[q] = 0u;
+                const unsigned incl = (unsigned)tsg_wave_incl_scan_dpp((int)len[q]);
+                tot[q] = (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+                len[q] = incl - len[q];  // from here on: before the lane's tile
+            }
+            unsigned *spw = reinterpret_cast<unsigned *>(sp);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {  // rows 4q..4q+3 in order
+                const unsigned r0 = run, r1 = r0 + (tot[2 * q] & 0xffffu), r2 = r1 + (tot[2 * q + 1] & 0xffffu);
+                const unsigned r3 = r2 + (tot[2 * q] >> 16);
+                run = r3 + (tot[2 * q + 1] >> 16);
+                const unsigned e = len[2 * q] + (r0 | (r2 << 16)), o = len[2 * q + 1] + (r1 | (r3 << 16));
+                spw[lane * 8 + 2 * q] = (e & 0xffffu) | (o << 16);
+                spw[lane * 8 + 2 * q + 1] = (e >> 16) | (o & 0xffff0000u);
+                if (lane == 0) {
+                    spw[64 * 8 + 2 * q] = r1 | (r2 << 16);
+                    spw[64 * 8 + 2 * q + 1] = r3 | (run << 16);
+                }
+            }
+            tsg_wave_sync();
+            const int rend = sp[64 * 16 + r], rbeg = r ? sp[64 * 16 + r - 1] : 0;
+            if (lane < 16) sd[lane] = gout - rbeg;
+            gout += rend - rbeg;
+            int k[CV_ROUNDS], last = 0;
+#pragma unroll
+            for (int i = 0; i < CV_ROUNDS; i++) {
+                k[i] = max(last, tsg_wave_incl_max_dpp((int)sr[lane + 64 * i]));
+                last = __builtin_amdgcn_readlane(k[i], 63);
+            }
+            tsg_wave_sync();  // the marks are read; their bytes take the rows
+#pragma unroll
+            for (int i = 0; i < CV_ROUNDS; i++) {
+                const int x = lane + 64 * i;
+                const int kk = k[i] - 1;
+                const int j = x - (__shfl(n0, kk, 64) - start), Jk = __shfl(J16, kk, 64);
+                if (x < total) {
+                    const uint4 pk = s_p16[wave][kk];
+                    // the last row starting at or before entry j
+                    const int rr = __popc(bytes_le(pk.x, j)) + __popc(bytes_le(pk.y, j)) + __popc(bytes_le(pk.z, j)) +
+                             __popc(bytes_le(pk.w, j)) - 1;
+                    const int pos = sp[kk * 16 + rr] + j - reinterpret_cast<const unsigned char *>(&s_p16[wave][kk])[rr];
+                    sv[pos] = v[i];
+                    sc[pos] = Jk + c8[i];
+                    sr[pos] = (unsigned char)rr;
+                }
+            }
+            tsg_wave_sync();
+            for (int o = lane; o < total; o += 64) {
+                const int d = sd[sr[o]] + o;
+                col[d] = sc[o];
+                val[d] = sv[o];
+            }
+            tsg_wave_sync();  // the next batch rewrites the LDS arrays
+            tb += nt;
         }
     }
 }
@@ -360,23 +605,44 @@ int tsg_tile2csr_view(tsg_ctx *ctx, const tsg_dtiles *t, int jbase, tsg_dcsr *ou
     out->m = t->m;
     out->n = t->n;
     TSG_TRY(tsg_alloc_t(ctx, &out->rowptr, (size_t)t->m + 1));
-    if (t->m > 0) {
-        hipLaunchKernelGGL(k_t2c_rows<0>, dim3(tsg_div_up(t->m, 256)), dim3(256), 0, ctx->stream, t->m, t->tile_ptr,
-                           t->tile_colidx, t->tile_nnz, t->csr_ptr, t->csr_col, t->val, out->rowptr,
-                           (int *)nullptr, (double *)nullptr, jbase);
-        TSG_LAUNCH_CHECK();
+    if (t->m <= 0) {
+        TSG_HIP(hipMemsetAsync(out->rowptr, 0, 4, ctx->stream));
+        TSG_TRY(tsg_alloc_t(ctx, &out->colidx, 1));
+        TSG_TRY(tsg_alloc_t(ctx, &out->val, 1));
+        return TSG_OK;
     }
-    long long nnz = 0;
-    TSG_TRY(tsg_scan_i32(ctx, out->rowptr, out->rowptr, t->m, &nnz));
+    const int tilem = (int)tsg_div_up(t->m, 16);
+    const unsigned nb = tsg_div_up(tilem, CV_WAVES);
+    char *buf = nullptr;  // the item count, then the items
+    long long maxitems = 0, nnz = 0;
+    for (long long tiles = std::max(t->numtile, 0);;) {
+        maxitems = tiles / CV_SEG + 1;  // further runs: at most one per CV_SEG tiles
+        TSG_TRY(tsg_alloc(ctx, (void **)&buf, 64 + (size_t)maxitems * sizeof(T2cItem)));
+        TSG_HIP(hipMemsetAsync(buf, 0, 4, ctx->stream));
+        hipLaunchKernelGGL(k_t2c_rowptr, dim3(nb), dim3(64 * CV_WAVES), 0, ctx->stream, t->m, tilem, t->tile_ptr,
+                           t->tile_nnz, t->csr_ptr, out->rowptr, (T2cItem *)(buf + 64), (int *)buf, (int)maxitems,
+                           ctx->pinned);
+        TSG_LAUNCH_CHECK();
+        TSG_HIP(hipStreamSynchronize(ctx->stream));
+        nnz = ((volatile long long *)ctx->pinned)[0];
+        const long long have = ((volatile long long *)ctx->pinned)[1];
+        if (have <= tiles) break;
+        tiles = have;  // a view whose numtile is not its own: once more, with room for every run
+        tsg_free(ctx, buf);
+    }
+    const T2cItem *items = (const T2cItem *)(buf + 64);
+    const int *nitems = (const int *)buf;
     out->nnz = (int)nnz;
     TSG_TRY(tsg_alloc_t(ctx, &out->colidx, (size_t)nnz + 1));
     TSG_TRY(tsg_alloc_t(ctx, &out->val, (size_t)nnz + 1));
-    if (t->m > 0 && nnz > 0) {
-        hipLaunchKernelGGL(k_t2c_rows<1>, dim3(tsg_div_up(t->m, 256)), dim3(256), 0, ctx->stream, t->m, t->tile_ptr,
-                           t->tile_colidx, t->tile_nnz, t->csr_ptr, t->csr_col, t->val, out->rowptr,
-                           out->colidx, out->val, jbase);
+    if (nnz > 0) {
+        const unsigned extra = (unsigned)std::min<long long>(maxitems, 1024);
+        hipLaunchKernelGGL(k_t2c_emit, dim3(nb + extra), dim3(64 * CV_WAVES), 0, ctx->stream, t->m, tilem, t->tile_ptr,
+                           t->tile_colidx, t->tile_nnz, t->csr_ptr, t->csr_col, t->val, out->rowptr, items, nitems,
+                           (int)nb, jbase, out->colidx, out->val);
         TSG_LAUNCH_CHECK();
     }
+    tsg_free(ctx, buf);
     return TSG_OK;
 }
 

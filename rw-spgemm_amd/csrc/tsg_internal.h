@@ -206,6 +206,29 @@ __device__ __forceinline__ T tsg_wave_incl_scan(T v) {
     }
     return v;
 }
+// The same for 32-bit values by DPP (six VALU moves, no LDS traffic); every
+// lane of the wave must be active.  Row shifts inside the 16-lane rows, then
+// row 0's last lane into row 1 and row 2's into row 3, then lane 31 into
+// rows 2 and 3; lanes without a source take 0.
+__device__ __forceinline__ int tsg_wave_incl_scan_dpp(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+// inclusive running maximum of non-negative values, likewise
+__device__ __forceinline__ int tsg_wave_incl_max_dpp(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+    return v;
+}
 // inclusive scan inside groups of 16 lanes
 template <typename T>
 __device__ __forceinline__ T tsg_group16_incl_scan(T v) {
