@@ -6,245 +6,593 @@
 // tile-row, per-tile exclusive nnz offsets, per-row u8 offsets inside a
 // tile, MSB-first u16 row masks, values row-major inside a tile with
 // ascending columns.  The reference builds it on the host with per-thread
-// dense flag arrays of tilen entries; here each tile-row is one wave64 with a
-// windowed LDS bitmap over the tile columns it touches, followed by one
-// thread per matrix row walking its (sorted) entries against the tile list.
+// dense flag arrays of tilen entries; here one wave64 per tile-row collects
+// the tile columns it touches in a windowed LDS bitmap, and one wave per run
+// of those tiles builds their masks in LDS and permutes the entries.
 #include <string.h>
 
 #include "tsg_internal.h"
 
 #define WAVES_PER_BLOCK 4
 #define BM_WORDS 256  // LDS bitmap window per wave: 256 x 32 = 8192 tile columns
+// Tile <-> CSR work split: waves per block, tiles of a tile-row per wave, and
+// entries of a batch of at most 64 tiles that are permuted through LDS.
+#define CV_WAVES 4
+#define CV_SEG 1024
+#define CV_CAP 448
+#define CV_ROUNDS (CV_CAP / 64)
 
-// ---------------------------------------------------------------- tile-row bitmaps
-// Tile columns touched by rows [16I, 16I+16): entry e -> colidx[e] >> 4.
-// Rows are sorted, so the window range comes from first/last entries.
-template <bool FILL>
-__global__ void __launch_bounds__(64 * WAVES_PER_BLOCK)
-k_c2t_tiles(const int *__restrict__ rowptr, const int *__restrict__ colidx, int m, int tilem,
-            int *__restrict__ cnt_or_ptr, int *__restrict__ out_col, int *__restrict__ out_row) {
-    __shared__ unsigned bm_all[WAVES_PER_BLOCK][BM_WORDS];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int I = blockIdx.x * WAVES_PER_BLOCK + wave;
-    if (I >= tilem) return;
-    unsigned *bm = bm_all[wave];
-    const int r0 = I * TSG_TILE, r1 = min(r0 + TSG_TILE, m);
-    const int e0 = rowptr[r0], e1 = rowptr[r1];
-    int jmin = 0x7fffffff, jmax = -1;
-    if (lane < r1 - r0) {
-        int a = rowptr[r0 + lane], b = rowptr[r0 + lane + 1];
-        if (b > a) { jmin = colidx[a] >> 4; jmax = colidx[b - 1] >> 4; }
+// First index in [lo, hi) with list[index] >= key (list ascending; any list
+// ends in range).
+__device__ __forceinline__ int first_ge(const int *__restrict__ list, int lo, int hi, int key) {
+    while (lo < hi) {
+        const int mid = (int)(((unsigned)lo + (unsigned)hi) >> 1);
+        if (list[mid] < key) lo = mid + 1; else hi = mid;
     }
-    jmin = tsg_wave_min(jmin);
-    jmax = tsg_wave_max(jmax);
-    int total = 0;
-    int base = FILL ? cnt_or_ptr[I] : 0;
-    for (int w0 = jmin; w0 <= jmax; w0 += 32 * BM_WORDS) {
-        const int nw = min(BM_WORDS, ((jmax - w0) >> 5) + 1);
-        for (int k = lane; k < nw; k += 64) bm[k] = 0u;
-        tsg_wave_sync();
-        for (int e = e0 + lane; e < e1; e += 64) {
-            int d = (colidx[e] >> 4) - w0;
-            if (d >= 0 && d < 32 * BM_WORDS) atomicOr(&bm[d >> 5], 1u << (d & 31));
-        }
-        tsg_wave_sync();
-        if (!FILL) {
-            int c = 0;
-            for (int k = lane; k < nw; k += 64) c += __popc(bm[k]);
-            total += tsg_wave_sum(c);
-        } else {
-            const int chunk = (nw + 63) >> 6;
-            const int k0 = lane * chunk, k1 = min(nw, k0 + chunk);
-            int c = 0;
-            for (int k = k0; k < k1; k++) c += __popc(bm[k]);
-            int excl = tsg_wave_incl_scan(c) - c;
-            int pos = base + total + excl;
-            for (int k = k0; k < k1; k++) {
-                unsigned x = bm[k];
-                while (x) {
-                    int b = __ffs(x) - 1;
-                    x &= x - 1;
-                    out_col[pos] = w0 + k * 32 + b;
-                    out_row[pos] = I;
-                    pos++;
-                }
-            }
-            total += tsg_wave_sum(c);
-        }
-        tsg_wave_sync();
-    }
-    if (!FILL && lane == 0) cnt_or_ptr[I] = total;
+    return lo;
 }
 
-// One thread per matrix row: walk its sorted entries against the sorted
-// tile-column list of its tile-row.  PASS 0 writes per-(tile,row) counts and
-// masks; PASS 1 writes values and in-tile columns at their final offsets.
-template <int PASS>
-__global__ void __launch_bounds__(256)
-k_c2t_rowwalk(const int *__restrict__ rowptr, const int *__restrict__ colidx, const double *__restrict__ val,
-              int m, const int *__restrict__ tile_ptr, const int *__restrict__ tile_colidx,
-              unsigned char *__restrict__ cnt16, unsigned short *__restrict__ mask,
-              const int *__restrict__ tile_nnz, double *__restrict__ tval, unsigned char *__restrict__ tcol) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    const int I = i >> 4, r = i & 15;
-    int t = tile_ptr[I];
-    const int tend = tile_ptr[I + 1] - 1;
-    int curJ = -1, n = 0, base = 0;
-    unsigned mk = 0;
-    const int e1 = rowptr[i + 1];
-    for (int e = rowptr[i]; e < e1; e++) {
-        const int col = colidx[e];
-        const int J = col >> 4, c = col & 15;
-        if (J != curJ) {
-            if (PASS == 0 && curJ >= 0) {
-                cnt16[(long long)t * 16 + r] = (unsigned char)n;
-                mask[(long long)t * 16 + r] = (unsigned short)mk;
-            }
-            while (t < tend && tile_colidx[t] < J) t++;  // input validated sorted: always finds J
-            curJ = J;
-            n = 0;
-            mk = 0;
-            if (PASS == 1) base = tile_nnz[t] + cnt16[(long long)t * 16 + r];
-        }
-        if (PASS == 0) {
-            mk |= 0x8000u >> c;
-        } else {
-            tval[base + n] = val[e];
-            tcol[base + n] = (unsigned char)c;
-        }
-        n++;
+// The same by a whole wave: 64 probes a step.
+__device__ __forceinline__ int wave_first_ge(const int *__restrict__ list, int lo, int hi, int key) {
+    const int lane = __lane_id();
+    while (hi - lo > 64) {
+        const int step = (int)(((unsigned)(hi - lo) + 63u) / 64u);
+        const int p = min(lo + (int)min((long long)step * (lane + 1) - 1, (long long)(hi - lo - 1)), hi - 1);
+        const int k = __popcll(__ballot(list[p] < key));  // probes ascend: a prefix of the lanes
+        const int lo0 = lo;
+        if (k > 0) lo = lo0 + (int)min((long long)step * k, (long long)(hi - lo0));
+        if (k < 64) hi = lo0 + (int)min((long long)step * (k + 1) - 1, (long long)(hi - lo0 - 1));
     }
-    if (PASS == 0 && curJ >= 0) {
-        cnt16[(long long)t * 16 + r] = (unsigned char)n;
-        mask[(long long)t * 16 + r] = (unsigned short)mk;
+    const bool less = lo + lane < hi && list[lo + lane] < key;
+    return lo + __popcll(__ballot(less));
+}
+// The same for 16 searches by a wave, lane's search = lane & 15, its four
+// lanes probing a fifth apart.
+__device__ __forceinline__ int rows16_first_ge(const int *__restrict__ list, int lo, int hi, int key) {
+    const int lane = __lane_id(), g = lane >> 4, r = lane & 15;
+    while (__ballot(lo < hi)) {
+        const unsigned n = (unsigned)(hi - lo);  // 0 once done
+        const int p = lo + (int)((n * (unsigned long long)(g + 1)) / 5u);  // the four ascend, all below hi if n > 0
+        const bool less = n > 0 && list[p] < key;
+        const int k = __popcll((__ballot(less) >> r) & 0x0001000100010001ull);
+        const int lo0 = lo;
+        if (n > 0) {
+            if (k > 0) lo = lo0 + (int)((n * (unsigned long long)k) / 5u) + 1;
+            if (k < 4) hi = lo0 + (int)((n * (unsigned long long)(k + 1)) / 5u);
+        }
     }
+    return lo;
 }
 
-// One thread per tile: per-row counts -> exclusive u8 offsets, tile nnz.
-__global__ void __launch_bounds__(256)
-k_c2t_finalize(int numtile, unsigned char *__restrict__ ptr16, int *__restrict__ tnnz) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= numtile) return;
-    uint4 v = *reinterpret_cast<const uint4 *>(ptr16 + (long long)t * 16);
-    unsigned w[4] = {v.x, v.y, v.z, v.w};
-    unsigned o[4];
-    int s = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        unsigned out = 0;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            unsigned cnt = (w[q] >> (8 * b)) & 0xffu;
-            out |= (unsigned)s << (8 * b);
-            s += cnt;
-        }
-        o[q] = out;
-    }
-    *reinterpret_cast<uint4 *>(ptr16 + (long long)t * 16) = make_uint4(o[0], o[1], o[2], o[3]);
-    tnnz[t] = s;
-}
-
+// ---------------------------------------------------------------- input checks
 // Input contract of the conversion: row pointers non-decreasing from 0 to
 // nnz, columns in [0, n) and (when `sorted`) strictly increasing inside each
 // row.  Any violation sets a flag instead of letting a later kernel index
-// out of range.
+// out of range.  The first nrow blocks check the row pointers, the others
+// VAL_BLOCK entries each: a column not above its predecessor is allowed at a
+// row's first entry only (the row starts of the block as bits in LDS).
+// Entry parallel, so a hub row is not one lane's walk: R-MAT scale 18 5.07
+// -> 0.05 ms, 27p 96^3 0.30 -> 0.035 ms.
+#define VAL_BLOCK 4096
+#define VAL_MARK_ROWS 16384  // rows starting in a block that are marked; more are searched
 __global__ void __launch_bounds__(256)
 k_validate_csr(const int *__restrict__ rowptr, const int *__restrict__ colidx, int m, int n, int nnz,
-               int sorted, int *__restrict__ bad) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i > m) return;
-    const int s = rowptr[i];
-    if (i == 0 && s != 0) atomicOr(bad, 1);
-    if (i == m) {
-        if (s != nnz) atomicOr(bad, 1);
+               int sorted, int nrow, int *__restrict__ bad) {
+    if ((int)blockIdx.x < nrow) {
+        const int i = blockIdx.x * 256 + threadIdx.x;
+        if (i > m) return;
+        const int s = rowptr[i];
+        if (i == 0 && s != 0) atomicOr(bad, 1);
+        if (i == m) {
+            if (s != nnz) atomicOr(bad, 1);
+            return;
+        }
+        const int e = rowptr[i + 1];
+        if (s < 0 || e < s || e > nnz) atomicOr(bad, 1);
         return;
     }
-    const int e = rowptr[i + 1];
-    if (s < 0 || e < s || e > nnz) { atomicOr(bad, 1); return; }
-    int prev = -1;
-    for (int k = s; k < e; k++) {
-        const int c = colidx[k];
-        if ((sorted && c <= prev) || c < 0 || c >= n) { atomicOr(bad, 2); return; }
-        prev = c;
+    const int end = min(nnz, max(rowptr[m], 0));  // nothing past what the rows claim is read
+    const long long b0 = (long long)(blockIdx.x - nrow) * VAL_BLOCK;
+    if (b0 >= end) return;
+    const int e0 = (int)b0, ne = (int)min((long long)VAL_BLOCK, end - b0);
+    __shared__ int s_lo[2];
+    __shared__ unsigned s_start[VAL_BLOCK / 32];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    if (tid < VAL_BLOCK / 32) s_start[tid] = 0u;
+    if (sorted && wave < 2) {  // rows starting in [e0, e0 + ne)
+        const int i = wave_first_ge(rowptr, 0, m + 1, wave ? e0 + ne : e0);
+        if (lane == 0) s_lo[wave] = i;
     }
+    // a wave's entries: 64 consecutive ones per round
+    int c[VAL_BLOCK / 256], p[VAL_BLOCK / 256];
+#pragma unroll
+    for (int k = 0; k < VAL_BLOCK / 256; k++) {
+        const int x = (k * 4 + wave) * 64;
+        c[k] = colidx[e0 + min(x + lane, ne - 1)];
+        p[k] = colidx[max(e0 + min(x, ne - 1) - 1, 0)];  // wave-uniform
+    }
+    __syncthreads();
+    bool marked = true;
+    if (sorted) {
+        const int lo = s_lo[0], hi = s_lo[1];
+        marked = hi - lo <= VAL_MARK_ROWS;
+        if (marked)
+            for (int i = lo + tid; i < hi; i += 256) {
+                const int x = rowptr[i] - e0;
+                if (x >= 0 && x < ne) atomicOr(&s_start[x >> 5], 1u << (x & 31));
+            }
+        __syncthreads();
+    }
+    int f = 0;
+#pragma unroll
+    for (int k = 0; k < VAL_BLOCK / 256; k++) {
+        const int x = (k * 4 + wave) * 64 + lane;
+        int prev = __shfl_up(c[k], 1, 64);
+        if (lane == 0) prev = p[k];
+        if (x >= ne) continue;
+        if (c[k] < 0 || c[k] >= n) f = 2;
+        if (sorted && e0 + x > 0 && c[k] <= prev) {
+            if (marked) {
+                if (!((s_start[x >> 5] >> (x & 31)) & 1u)) f = 2;
+            } else {
+                const int i = first_ge(rowptr, s_lo[0], s_lo[1], e0 + x);
+                if (i > m || rowptr[i] != e0 + x) f = 2;
+            }
+        }
+    }
+    if (f) atomicOr(bad, f);
+}
+
+static int launch_validate(tsg_ctx *ctx, const tsg_dcsr *a, int sorted, int *bad) {
+    const unsigned nrow = tsg_div_up((long long)a->m + 1, 256), ncol = tsg_div_up(a->nnz, VAL_BLOCK);
+    hipLaunchKernelGGL(k_validate_csr, dim3(nrow + ncol), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, a->m, a->n,
+                       a->nnz, sorted, (int)nrow, bad);
+    TSG_LAUNCH_CHECK();
+    return TSG_OK;
+}
+
+static int validate_status(long long bad, int sorted) {
+    if (!bad) return TSG_OK;
+    tsg_set_error(bad & 1 ? "CSR row pointers inconsistent with nnz"
+                  : sorted ? "CSR columns out of range or not strictly increasing inside a row"
+                           : "CSR columns out of range");
+    return TSG_ERR_ARG;
 }
 
 int tsg_validate_csr_mode(tsg_ctx *ctx, const tsg_dcsr *a, int sorted) {
     void *scr;
     TSG_TRY(tsg_scratch(ctx, 64, &scr));
     TSG_HIP(hipMemsetAsync(scr, 0, 4, ctx->stream));
-    hipLaunchKernelGGL(k_validate_csr, dim3(tsg_div_up((long long)a->m + 1, 256)), dim3(256), 0, ctx->stream,
-                       a->rowptr, a->colidx, a->m, a->n, a->nnz, sorted, (int *)scr);
-    TSG_LAUNCH_CHECK();
+    TSG_TRY(launch_validate(ctx, a, sorted, (int *)scr));
     long long bad = 0;
     TSG_TRY(tsg_read_scalar_i64(ctx, scr, 0, &bad));
-    if (bad) {
-        tsg_set_error(bad & 1 ? "CSR row pointers inconsistent with nnz"
-                      : sorted ? "CSR columns out of range or not strictly increasing inside a row"
-                               : "CSR columns out of range");
-        return TSG_ERR_ARG;
-    }
-    return TSG_OK;
+    return validate_status(bad, sorted);
 }
 
 int tsg_validate_csr(tsg_ctx *ctx, const tsg_dcsr *a) { return tsg_validate_csr_mode(ctx, a, 1); }
 
+// ---------------------------------------------------------------- CSR -> tiles
+// Counters of one conversion (zeroed beforehand): a flag for bad input, the
+// tile-rows left to k_c2t_tiles_big, the runs of tiles past a tile-row's
+// first CV_SEG.
+struct C2tCount {
+    int bad, nbig, nitems, pad;
+};
+#define C2T_BIG 4096  // entries of a tile-row above which a whole block collects its tiles
+
+// Tile columns of tile-row I into list[0..), ascending, from words [0, nw)
+// of a wave's bitmap window that starts at tile column w0; returns their number.
+// A window with many tiles writes one pair of words per step, each bit a
+// lane, so that a store instruction covers consecutive entries; with few,
+// each lane writes the bits of its own word.
+__device__ __forceinline__ int emit_window(const unsigned *bm, int nw, int w0, int lane, int *__restrict__ list) {
+    int done = 0;
+    for (int k0 = 0; k0 < nw; k0 += 64) {
+        const unsigned x = k0 + lane < nw ? bm[k0 + lane] : 0u;
+        const int c = __popc(x), incl = tsg_wave_incl_scan_dpp(c);
+        const int tot = __builtin_amdgcn_readlane(incl, 63);
+        const int pos = done + incl - c;
+        if (tot > 256) {
+            unsigned long long nz = __ballot(x != 0u);
+            while (nz) {
+                const int j0 = __ffsll((long long)nz) - 1;
+                nz &= nz - 1;
+                const int j1 = nz ? __ffsll((long long)nz) - 1 : j0;
+                const bool both = nz != 0;
+                nz &= nz - 1;  // 0 stays 0
+                const int j = lane < 32 ? j0 : j1;
+                const unsigned wd = lane < 32 ? (unsigned)__builtin_amdgcn_readlane((int)x, j0)
+                                              : (unsigned)__builtin_amdgcn_readlane((int)x, j1);
+                const int p = lane < 32 ? __builtin_amdgcn_readlane(pos, j0) : __builtin_amdgcn_readlane(pos, j1);
+                const int b = lane & 31;
+                if ((lane < 32 || both) && (wd >> b) & 1u)
+                    list[p + __popc(wd & ((1u << b) - 1u))] = w0 + 32 * (k0 + j) + b;
+            }
+        } else {
+            unsigned y = x;
+            for (int q = pos; y; q++) {
+                list[q] = w0 + 32 * (k0 + lane) + __ffs(y) - 1;
+                y &= y - 1;
+            }
+        }
+        done += tot;
+    }
+    return done;
+}
+
+// Tiles of each tile-row: their number into cnt[I], their columns into
+// list[rowptr[16I]..) (a tile has an entry, so they fit).  One wave per
+// tile-row; a tile-row of more than C2T_BIG entries is put on the list of
+// k_c2t_tiles_big.  Row pointers and columns are used only as far as they
+// are in range: the input is checked in the same stream, not before.
+__global__ void __launch_bounds__(64 * WAVES_PER_BLOCK)
+k_c2t_tiles(const int *__restrict__ rowptr, const int *__restrict__ colidx, int m, int nnz, int tilem, int tilen,
+            int *__restrict__ cnt, int *__restrict__ list, C2tCount *__restrict__ count, int *__restrict__ big,
+            int maxbig, int2 *__restrict__ items, int maxitems) {
+    __shared__ unsigned bm_all[WAVES_PER_BLOCK][BM_WORDS];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int I = blockIdx.x * WAVES_PER_BLOCK + wave;
+    if (I >= tilem) return;
+    unsigned *bm = bm_all[wave];
+    const int r0 = I * TSG_TILE, rl = min(TSG_TILE, m - r0);
+    const int rp = rowptr[r0 + min(lane, rl)], rpe = rowptr[r0 + min(lane + 1, rl)];
+    if (__ballot(rp < 0 || rpe < rp || rpe > nnz)) {  // reported by the input check
+        if (lane == 0) cnt[I] = 0;
+        return;
+    }
+    const int e0 = __builtin_amdgcn_readlane(rp, 0), e1 = __builtin_amdgcn_readlane(rpe, 63);
+    if (e1 - e0 > C2T_BIG) {
+        if (lane == 0) {
+            const int s = atomicAdd(&count->nbig, 1);
+            if (s < maxbig) big[s] = I;
+            cnt[I] = 0;
+        }
+        return;
+    }
+    int jmin = 0x7fffffff, jmax = -1;
+    if (lane < rl && rpe > rp) {
+        jmin = max(colidx[rp] >> 4, 0);
+        jmax = min(colidx[rpe - 1] >> 4, tilen - 1);
+    }
+    jmin = tsg_wave_min(jmin);
+    jmax = tsg_wave_max(jmax);
+    int total = 0;
+    for (int w0 = jmin; w0 <= jmax; w0 += 32 * BM_WORDS) {
+        const int nw = min(BM_WORDS, ((jmax - w0) >> 5) + 1);
+        for (int k = lane; k < nw; k += 64) bm[k] = 0u;
+        tsg_wave_sync();
+        for (int x = lane; x < e1 - e0; x += 256) {
+            int d[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) d[v] = colidx[e0 + min(x + 64 * v, e1 - e0 - 1)];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {  // a repeated last entry sets its bit again
+                const int j = (d[v] >> 4) - w0;
+                if (j >= 0 && j < 32 * nw) atomicOr(&bm[j >> 5], 1u << (j & 31));
+            }
+        }
+        tsg_wave_sync();
+        total += emit_window(bm, nw, w0, lane, list + e0 + total);
+        tsg_wave_sync();
+    }
+    if (lane == 0) {
+        cnt[I] = total;
+        const int more = (total - 1) / CV_SEG;  // runs past the first
+        if (total > CV_SEG) {
+            const int s = atomicAdd(&count->nitems, more);
+            for (int k = 0; k < more && s + k < maxitems; k++) items[s + k] = make_int2(I, k + 1);
+        }
+    }
+}
+
+// The same by a block of 16 waves per listed tile-row, with a window of
+// 8192 words.
+#define C2T_BIG_WORDS 8192
+__global__ void __launch_bounds__(1024)
+k_c2t_tiles_big(const int *__restrict__ rowptr, const int *__restrict__ colidx, int m, int tilen,
+                int *__restrict__ cnt, int *__restrict__ list, C2tCount *__restrict__ count,
+                const int *__restrict__ big, int maxbig, int2 *__restrict__ items, int maxitems) {
+    __shared__ unsigned bm[C2T_BIG_WORDS];
+    __shared__ int s_j[2], s_w[16];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int nbig = min(count->nbig, maxbig);
+    for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
+        const int I = big[q];
+        const int r0 = I * TSG_TILE, rl = min(TSG_TILE, m - r0);
+        const int e0 = rowptr[r0], e1 = rowptr[r0 + rl];
+        if (wave == 0) {
+            int jmin = 0x7fffffff, jmax = -1;
+            if (lane < rl) {
+                const int a = rowptr[r0 + lane], b = rowptr[r0 + lane + 1];
+                if (b > a) {
+                    jmin = max(colidx[a] >> 4, 0);
+                    jmax = min(colidx[b - 1] >> 4, tilen - 1);
+                }
+            }
+            jmin = tsg_wave_min(jmin);
+            jmax = tsg_wave_max(jmax);
+            if (lane == 0) {
+                s_j[0] = jmin;
+                s_j[1] = jmax;
+            }
+        }
+        __syncthreads();
+        const int jmin = s_j[0], jmax = s_j[1];
+        int total = 0;
+        for (int w0 = jmin; w0 <= jmax; w0 += 32 * C2T_BIG_WORDS) {
+            const int nw = min(C2T_BIG_WORDS, ((jmax - w0) >> 5) + 1);
+            for (int k = tid; k < nw; k += 1024) bm[k] = 0u;
+            __syncthreads();
+            const unsigned ne = (unsigned)(e1 - e0);
+            for (unsigned x = tid; x < ne; x += 4096) {
+                int d[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) d[v] = colidx[e0 + (int)min(x + 1024u * v, ne - 1u)];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int j = (d[v] >> 4) - w0;
+                    if (j >= 0 && j < 32 * nw) {
+                        const unsigned bit = 1u << (j & 31);
+                        if (!(bm[j >> 5] & bit)) atomicOr(&bm[j >> 5], bit);
+                    }
+                }
+            }
+            __syncthreads();
+            // each wave counts, then emits, a sixteenth of the words
+            const int per = (nw + 15) / 16, k0 = min(nw, wave * per), k1 = min(nw, k0 + per);
+            int c = 0;
+            for (int k = k0 + lane; k < k1; k += 64) c += __popc(bm[k]);
+            c = tsg_wave_sum(c);
+            if (lane == 0) s_w[wave] = c;
+            __syncthreads();
+            int before = 0, all = 0;
+            for (int w = 0; w < 16; w++) {
+                before += w < wave ? s_w[w] : 0;
+                all += s_w[w];
+            }
+            emit_window(bm + k0, k1 - k0, w0 + 32 * k0, lane, list + e0 + total + before);
+            total += all;
+            __syncthreads();
+        }
+        if (tid == 0) {
+            cnt[I] = total;
+            if (total > CV_SEG) {
+                const int more = (total - 1) / CV_SEG;
+                const int s = atomicAdd(&count->nitems, more);
+                for (int k = 0; k < more && s + k < maxitems; k++) items[s + k] = make_int2(I, k + 1);
+            }
+        }
+        __syncthreads();  // s_j
+    }
+}
+
+// Masks, offsets, columns and values of the tiles, one wave per run of at
+// most CV_SEG tiles of a tile-row (the first tilem waves the first runs, the
+// others the item list), in batches of 64 tiles.  The entries of a batch are
+// one range of each of the 16 rows (the columns ascend), and the entries of
+// the tile-row before the batch are those before the ranges, so a run needs
+// nothing from the runs before it.  Masks are OR-ed in LDS; an entry's place
+// is its tile's and row's offset plus the mask bits before its own.  Batches
+// of up to CV_CAP entries keep their entries in registers between the two
+// and are permuted through LDS; denser ones are read twice and written in
+// place, in runs of up to 16.  Bound by HBM: 12 bytes in and 9 out per entry
+// plus 60 per tile.  One thread per matrix row (two walks of its entries,
+// 64 lines per instruction, a hub row on one lane): 27p 96^3 1.38 ->
+// 0.115 ms (4.4 TB/s), R-MAT scale 18 66.9 -> 0.55 ms.
+__global__ void __launch_bounds__(64 * CV_WAVES)
+k_c2t_fill(const int *__restrict__ rowptr, const int *__restrict__ colidx, const double *__restrict__ val, int m,
+           int tilem, int nnz, int numtile, const int *__restrict__ tile_ptr, const int *__restrict__ list,
+           const int2 *__restrict__ items, const C2tCount *__restrict__ count, int nblocks_rows,
+           int *__restrict__ tile_colidx, int *__restrict__ tile_rowidx, int *__restrict__ tile_nnz,
+           unsigned char *__restrict__ csr_ptr, unsigned short *__restrict__ mask, unsigned char *__restrict__ tcol,
+           double *__restrict__ tval) {
+    __shared__ double s_val[CV_WAVES][CV_CAP];
+    __shared__ __align__(16) unsigned s_mask[CV_WAVES][64 * 8];  // two rows per word, even row low
+    __shared__ uint4 s_ptr[CV_WAVES][64];
+    __shared__ int s_J[CV_WAVES][64];
+    __shared__ int s_off[CV_WAVES][16], s_src[CV_WAVES][16];
+    __shared__ unsigned short s_toff[CV_WAVES][64];
+    __shared__ unsigned char s_c8[CV_WAVES][CV_CAP];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15;
+    unsigned *sm = s_mask[wave];
+    int *sJ = s_J[wave], *so = s_off[wave], *ss = s_src[wave];
+    if (blockIdx.x == 0 && threadIdx.x < 16) {  // the arrays' tails
+        csr_ptr[16 * (long long)numtile + threadIdx.x] = 0;
+        mask[16 * (long long)numtile + threadIdx.x] = 0;
+        if (threadIdx.x == 0) tile_nnz[numtile] = nnz;
+    }
+    const bool listed = (int)blockIdx.x >= nblocks_rows;
+    const int nwork = listed ? count->nitems : tilem;
+    const int step = listed ? (int)(gridDim.x - nblocks_rows) * CV_WAVES : tilem;
+    for (int w = (listed ? (int)blockIdx.x - nblocks_rows : (int)blockIdx.x) * CV_WAVES + wave; w < nwork; w += step) {
+        const int I = listed ? items[w].x : w, sg = listed ? items[w].y : 0;
+        const int t0 = tile_ptr[I], t1 = tile_ptr[I + 1], ta = t0 + sg * CV_SEG, te = min(t1, ta + CV_SEG);
+        if (ta >= te) continue;
+        // lanes r, r + 16, ...: row r's entries [rp, rpe) and where its next range starts
+        const int rp = rowptr[min(16 * I + r, m)], rpe = rowptr[min(16 * I + r + 1, m)];
+        const int e0 = __builtin_amdgcn_readlane(rp, 0);
+        const int *tl = list + e0 - t0;  // tile columns by tile id
+        int cur = sg == 0 ? rp : rows16_first_ge(colidx, rp, rpe, tl[ta] * 16);
+        for (int tb = ta; tb < te; tb += 64) {
+            const int nt = min(64, te - tb);
+            const int J = tl[tb + min(lane, nt - 1)];
+            // rows end with the tile-row's last tile; otherwise 64 tiles hold at most 1024 of a row's entries
+            int end = rpe;
+            if (tb + nt < t1)
+                end = rows16_first_ge(colidx, cur, cur + min(rpe - cur, 1024), (__builtin_amdgcn_readlane(J, nt - 1) + 1) * 16);
+            const int len = end - cur, incl = tsg_row16_incl_scan_dpp(len);
+            const int total = __builtin_amdgcn_readlane(incl, 15);
+            const int base = e0 + __builtin_amdgcn_readlane(tsg_row16_incl_scan_dpp(cur - rp), 15);
+            if (lane < 16) {
+                so[lane] = incl - len;
+                ss[lane] = cur - (incl - len);
+            }
+            cur = end;
+            sJ[lane] = lane < nt ? J : 0x7fffffff;
+            for (int i = lane; i < 64 * 2; i += 64) reinterpret_cast<uint4 *>(sm)[i] = make_uint4(0u, 0u, 0u, 0u);
+            tsg_wave_sync();
+            // entry x of the batch: its row (the last whose range starts at or before x), then its tile
+            auto row_of = [&](int x) {
+                int q = 0;
+#pragma unroll
+                for (int st = 8; st > 0; st >>= 1)
+                    if (so[q + st] <= x) q += st;
+                return q;
+            };
+            auto tile_of = [&](int c) {
+                int k = 0;
+#pragma unroll
+                for (int st = 32; st > 0; st >>= 1)
+                    if (sJ[k + st] <= (c >> 4)) k += st;
+                return k;
+            };
+            int code[CV_ROUNDS];  // column, then tile << 8 | in-tile column << 4 | row
+            unsigned rows = 0;    // four bits per round
+            static_assert(CV_ROUNDS <= 8, "rows of a lane's entries in one word");
+            double v[CV_ROUNDS];
+            if (total <= CV_CAP) {
+#pragma unroll
+                for (int i = 0; i < CV_ROUNDS; i++) {  // every lane loads in bounds
+                    const int x = min(lane + 64 * i, total - 1), q = row_of(x), e = ss[q] + x;
+                    v[i] = val[e];
+                    code[i] = colidx[e];
+                    rows |= (unsigned)q << (4 * i);
+                }
+#pragma unroll
+                for (int i = 0; i < CV_ROUNDS; i++) {
+                    const int q = (rows >> (4 * i)) & 15, c = code[i], k = tile_of(c);
+                    code[i] = k << 8 | (c & 15) << 4 | q;
+                    if (lane + 64 * i < total) atomicOr(&sm[k * 8 + (q >> 1)], (0x8000u >> (c & 15)) << (16 * (q & 1)));
+                }
+            } else {
+                for (int x = lane; x < total; x += 64) {
+                    const int q = row_of(x), c = colidx[ss[q] + x], k = tile_of(c);
+                    atomicOr(&sm[k * 8 + (q >> 1)], (0x8000u >> (c & 15)) << (16 * (q & 1)));
+                }
+            }
+            tsg_wave_sync();
+            // lane = tile: row offsets, entries
+            const uint4 ma = reinterpret_cast<const uint4 *>(sm)[2 * lane], mb = reinterpret_cast<const uint4 *>(sm)[2 * lane + 1];
+            const unsigned mw[8] = {ma.x, ma.y, ma.z, ma.w, mb.x, mb.y, mb.z, mb.w};
+            unsigned o[4];
+            int sum = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                o[q] = 0;
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    o[q] |= (unsigned)sum << (8 * b);
+                    sum += __popc((mw[2 * q + (b >> 1)] >> (16 * (b & 1))) & 0xffffu);
+                }
+            }
+            const int toff = tsg_wave_incl_scan_dpp(sum) - sum;
+            s_ptr[wave][lane] = make_uint4(o[0], o[1], o[2], o[3]);
+            s_toff[wave][lane] = (unsigned short)toff;
+            if (lane < nt) {
+                const long long t = tb + lane;
+                tile_colidx[t] = J;
+                tile_rowidx[t] = I;
+                tile_nnz[t] = base + toff;
+                reinterpret_cast<uint4 *>(csr_ptr)[t] = make_uint4(o[0], o[1], o[2], o[3]);
+                reinterpret_cast<uint4 *>(mask)[2 * t] = ma;
+                reinterpret_cast<uint4 *>(mask)[2 * t + 1] = mb;
+            }
+            tsg_wave_sync();
+            auto place = [&](int k, int q, int c) {
+                const unsigned mr = (sm[k * 8 + (q >> 1)] >> (16 * (q & 1))) & 0xffffu;
+                return (int)s_toff[wave][k] + reinterpret_cast<const unsigned char *>(&s_ptr[wave][k])[q] +
+                       __popc(mr >> (16 - c));
+            };
+            if (total <= CV_CAP) {
+#pragma unroll
+                for (int i = 0; i < CV_ROUNDS; i++) {
+                    if (lane + 64 * i >= total) continue;
+                    const int q = code[i] & 15, c = (code[i] >> 4) & 15, pos = place(code[i] >> 8, q, c);
+                    s_val[wave][pos] = v[i];
+                    s_c8[wave][pos] = (unsigned char)c;
+                }
+                tsg_wave_sync();
+                for (int x = lane; x < total; x += 64) {
+                    tval[base + x] = s_val[wave][x];
+                    tcol[base + x] = s_c8[wave][x];
+                }
+            } else {
+                for (int x = lane; x < total; x += 64) {
+                    const int q = row_of(x), e = ss[q] + x, c = colidx[e];
+                    const int pos = base + place(tile_of(c), q, c & 15);
+                    tval[pos] = val[e];
+                    tcol[pos] = (unsigned char)(c & 15);
+                }
+            }
+            tsg_wave_sync();  // the next batch rewrites the LDS arrays
+        }
+    }
+}
+
 extern "C" int tsg_csr2tile(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dtiles *out) {
     memset(out, 0, sizeof(*out));
     if (!a || a->m < 0 || a->n < 0 || a->nnz < 0) { tsg_set_error("tsg_csr2tile: bad matrix"); return TSG_ERR_ARG; }
-    TSG_TRY(tsg_validate_csr(ctx, a));
     tsg_dtiles &T = *out;
     T.m = a->m;
     T.n = a->n;
     T.nnz = a->nnz;
     T.tilem = (a->m + 15) / 16;
-    T.tilen = (a->n + 15) / 16;
+    T.tilen = (int)(((long long)a->n + 15) / 16);
+    // counters, the tile-rows of more than C2T_BIG entries, the further runs
+    // of tiles, the tile columns
+    const int maxbig = a->nnz / C2T_BIG + 1, maxitems = a->nnz / CV_SEG + 1;
+    const size_t o_big = 64, o_items = o_big + (((size_t)maxbig * 4 + 15) & ~(size_t)15);
+    const size_t o_list = o_items + (((size_t)maxitems * 8 + 15) & ~(size_t)15);
+    char *buf = nullptr;
     TSG_TRY(tsg_alloc_t(ctx, &T.tile_ptr, (size_t)T.tilem + 1));
-    if (T.tilem > 0) {
-        hipLaunchKernelGGL(k_c2t_tiles<false>, dim3(tsg_div_up(T.tilem, WAVES_PER_BLOCK)), dim3(64 * WAVES_PER_BLOCK),
-                           0, ctx->stream, a->rowptr, a->colidx, a->m, T.tilem, T.tile_ptr, (int *)nullptr,
-                           (int *)nullptr);
-        TSG_LAUNCH_CHECK();
-    }
+    int st = tsg_alloc(ctx, (void **)&buf, o_list + ((size_t)a->nnz + 1) * 4);
     long long numtile = 0;
-    TSG_TRY(tsg_scan_i32(ctx, T.tile_ptr, T.tile_ptr, T.tilem, &numtile));
-    T.numtile = (int)numtile;
-    TSG_TRY(tsg_alloc_t(ctx, &T.tile_colidx, (size_t)numtile + 1));
-    TSG_TRY(tsg_alloc_t(ctx, &T.tile_rowidx, (size_t)numtile + 1));
-    TSG_TRY(tsg_alloc_t(ctx, &T.tile_nnz, (size_t)numtile + 1));
-    TSG_TRY(tsg_alloc_t(ctx, &T.csr_ptr, (size_t)numtile * 16 + 16));
-    TSG_TRY(tsg_alloc_t(ctx, &T.mask, (size_t)numtile * 16 + 16));
-    TSG_TRY(tsg_alloc_t(ctx, &T.csr_col, (size_t)a->nnz + 1));
-    TSG_TRY(tsg_alloc_t(ctx, &T.val, (size_t)a->nnz + 1));
-    TSG_HIP(hipMemsetAsync(T.csr_ptr, 0, (size_t)numtile * 16 + 16, ctx->stream));
-    TSG_HIP(hipMemsetAsync(T.mask, 0, ((size_t)numtile * 16 + 16) * 2, ctx->stream));
-    if (numtile > 0) {
-        hipLaunchKernelGGL(k_c2t_tiles<true>, dim3(tsg_div_up(T.tilem, WAVES_PER_BLOCK)), dim3(64 * WAVES_PER_BLOCK),
-                           0, ctx->stream, a->rowptr, a->colidx, a->m, T.tilem, T.tile_ptr, T.tile_colidx,
-                           T.tile_rowidx);
+    if (st == TSG_OK) st = [&]() -> int {
+        C2tCount *count = (C2tCount *)buf;
+        int *big = (int *)(buf + o_big), *list = (int *)(buf + o_list);
+        int2 *items = (int2 *)(buf + o_items);
+        hipStream_t s = ctx->stream;
+        TSG_HIP(hipMemsetAsync(count, 0, sizeof(C2tCount), s));
+        TSG_TRY(launch_validate(ctx, a, 1, &count->bad));
+        if (T.tilem > 0) {
+            hipLaunchKernelGGL(k_c2t_tiles, dim3(tsg_div_up(T.tilem, WAVES_PER_BLOCK)), dim3(64 * WAVES_PER_BLOCK), 0, s,
+                               a->rowptr, a->colidx, a->m, a->nnz, T.tilem, T.tilen, T.tile_ptr, list, count, big,
+                               maxbig, items, maxitems);
+            TSG_LAUNCH_CHECK();
+            if (a->nnz > C2T_BIG) {
+                hipLaunchKernelGGL(k_c2t_tiles_big, dim3((unsigned)std::min(maxbig, 512)), dim3(1024), 0, s, a->rowptr,
+                                   a->colidx, a->m, T.tilen, T.tile_ptr, list, count, big, maxbig, items, maxitems);
+                TSG_LAUNCH_CHECK();
+            }
+        }
+        const long long np = tsg_scan_partial_count(T.tilem);
+        void *part;
+        TSG_TRY(tsg_scratch(ctx, (size_t)np * sizeof(long long), &part));
+        TSG_TRY(tsg_scan_i32_enqueue(s, T.tile_ptr, T.tile_ptr, T.tilem, (long long *)part));
+        long long *pin = ctx->pinned;
+        TSG_HIP(hipMemcpyAsync(pin, (long long *)part + np - 1, 8, hipMemcpyDeviceToHost, s));
+        TSG_HIP(hipMemcpyAsync(pin + 1, &count->bad, 4, hipMemcpyDeviceToHost, s));
+        TSG_HIP(hipStreamSynchronize(s));
+        TSG_TRY(validate_status(((int *)(pin + 1))[0], 1));
+        numtile = pin[0];  // at most nnz
+        T.numtile = (int)numtile;
+        TSG_TRY(tsg_alloc_t(ctx, &T.tile_colidx, (size_t)numtile + 1));
+        TSG_TRY(tsg_alloc_t(ctx, &T.tile_rowidx, (size_t)numtile + 1));
+        TSG_TRY(tsg_alloc_t(ctx, &T.tile_nnz, (size_t)numtile + 1));
+        TSG_TRY(tsg_alloc_t(ctx, &T.csr_ptr, (size_t)numtile * 16 + 16));
+        TSG_TRY(tsg_alloc_t(ctx, &T.mask, (size_t)numtile * 16 + 16));
+        TSG_TRY(tsg_alloc_t(ctx, &T.csr_col, (size_t)a->nnz + 1));
+        TSG_TRY(tsg_alloc_t(ctx, &T.val, (size_t)a->nnz + 1));
+        const unsigned nb = tsg_div_up(T.tilem, CV_WAVES), extra = (unsigned)std::min(maxitems, 1024);
+        hipLaunchKernelGGL(k_c2t_fill, dim3(nb + extra), dim3(64 * CV_WAVES), 0, s, a->rowptr, a->colidx, a->val, a->m,
+                           T.tilem, a->nnz, T.numtile, T.tile_ptr, list, items, count, (int)nb, T.tile_colidx,
+                           T.tile_rowidx, T.tile_nnz, T.csr_ptr, T.mask, T.csr_col, T.val);
         TSG_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_c2t_rowwalk<0>, dim3(tsg_div_up(a->m, 256)), dim3(256), 0, ctx->stream, a->rowptr,
-                           a->colidx, a->val, a->m, T.tile_ptr, T.tile_colidx, T.csr_ptr, T.mask, (const int *)nullptr,
-                           (double *)nullptr, (unsigned char *)nullptr);
-        TSG_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_c2t_finalize, dim3(tsg_div_up(numtile, 256)), dim3(256), 0, ctx->stream, T.numtile,
-                           T.csr_ptr, T.tile_nnz);
-        TSG_LAUNCH_CHECK();
-    }
-    long long nnz = 0;
-    TSG_TRY(tsg_scan_i32(ctx, T.tile_nnz, T.tile_nnz, numtile, &nnz));
-    if (nnz != a->nnz) {
-        tsg_set_error("tsg_csr2tile: tile nnz %lld != csr nnz %d (rows not sorted/unique?)", nnz, a->nnz);
-        return TSG_ERR_ARG;
-    }
-    if (numtile > 0 && a->m > 0) {
-        hipLaunchKernelGGL(k_c2t_rowwalk<1>, dim3(tsg_div_up(a->m, 256)), dim3(256), 0, ctx->stream, a->rowptr,
-                           a->colidx, a->val, a->m, T.tile_ptr, T.tile_colidx, T.csr_ptr, T.mask, T.tile_nnz, T.val,
-                           T.csr_col);
-        TSG_LAUNCH_CHECK();
-    }
-    return TSG_OK;
+        return TSG_OK;
+    }();
+    tsg_free(ctx, buf);
+    if (st != TSG_OK) tsg_tiles_free(ctx, out);
+    return st;
 }
 
 // ---------------------------------------------------------------- CSC tile index
@@ -329,10 +677,7 @@ __device__ __forceinline__ int t2c_row_len(const int *tile_nnz, const unsigned c
 // left 8-byte accesses to 64 different lines per instruction and a hub
 // row's whole walk on one lane: 62M entries of a 27-point product (27d
 // 79x83x81, A^2) 2.31 -> 0.55 ms for the call, 2.9 TB/s in k_t2c_emit; the
-// row index of R-MAT scale 18 17.4 -> 0.48 ms (both kernels).
-#define CV_WAVES 4
-#define CV_SEG 1024
-#define CV_CAP 448
+// row index of R-MAT scale 18 17.4 -> 0.37 ms (both kernels).
 struct T2cItem {
     int I, seg;     // tiles [CV_SEG * seg, CV_SEG * (seg + 1)) of tile-row I
     int carry[16];  // entries of each row in the tile-row's tiles before them
@@ -374,31 +719,53 @@ __device__ __forceinline__ uint4 load16(const unsigned char *p) {
     return v;
 }
 
-// Row pointers; one wave per tile-row of up to CV_SEG tiles (four tiles at a
-// time, lane = (tile, row)), the block's four waves together for a longer
-// one (four tiles per thread and run).  *nitems (zeroed beforehand) counts
-// the further runs (the first maxitems are listed); host (pinned) gets the
-// entries and the tiles of the matrix or view.
+// Entries of each row over up to CV_SEG tiles [ta, te) by a wave starting at
+// tile ta + lane with the given stride: v[2q] = rows 4q and 4q+2, v[2q+1] =
+// rows 4q+1 and 4q+3 (at most 16 * CV_SEG per half), summed over the wave.
+__device__ __forceinline__ void t2c_row_sums(const int *__restrict__ tile_nnz, const unsigned char *__restrict__ csr_ptr,
+                                             int ta, int te, int stride, int rowlen, unsigned v[8]) {
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = 0u;
+#pragma unroll 4
+    for (int t = ta; t < te; t += stride) {
+        unsigned x[8];
+        const int tn = tile_nnz[t + 1] - tile_nnz[t];
+        t2c_widen(t2c_row_lens(t2c_offsets(load16(csr_ptr + 16 * (long long)t), tn, rowlen), tn), x);
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] += x[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = (unsigned)__builtin_amdgcn_readlane(tsg_wave_incl_scan_dpp((int)v[q]), 63);
+}
+// v's entry for row r (0..15)
+__device__ __forceinline__ int t2c_row_of(const unsigned v[8], int r) {
+    unsigned x = 0;
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+        if (2 * (r >> 2) + (r & 1) == q) x = v[q];
+    return (int)((r & 2) ? x >> 16 : x & 0xffffu);
+}
+
+// Row pointers; one wave per tile-row of up to CV_SEG tiles, a tile per lane,
+// the block's four waves together for a longer one.  *nitems (zeroed
+// beforehand) counts the further runs (the first maxitems are listed); host
+// (pinned) gets the entries and the tiles of the matrix or view.
 __global__ void __launch_bounds__(64 * CV_WAVES)
 k_t2c_rowptr(int m, int tilem, const int *__restrict__ tile_ptr, const int *__restrict__ tile_nnz,
              const unsigned char *__restrict__ csr_ptr, int *__restrict__ rowptr, T2cItem *__restrict__ items,
              int *__restrict__ nitems, int maxitems, long long *__restrict__ host) {
     __shared__ int s_sum[CV_WAVES][16];
     __shared__ int s_slot;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, ts = lane >> 4;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int nb0 = tile_nnz[tile_ptr[0]];
     const int I = blockIdx.x * CV_WAVES + wave;
+    unsigned v[8];
     if (I < tilem) {
         const int t0 = tile_ptr[I], t1 = tile_ptr[I + 1];
         if (t1 - t0 <= CV_SEG) {
             const int rowlen = min(16, m - 16 * I);
-            int c = 0;
-#pragma unroll 4
-            for (int t = t0 + ts; t < t1; t += 4)
-                if (r < rowlen) c += t2c_row_len(tile_nnz, csr_ptr, t, r, rowlen);
-            c += __shfl_xor(c, 16, 64);
-            c += __shfl_xor(c, 32, 64);
-            const int incl = tsg_group16_incl_scan(c);
+            t2c_row_sums(tile_nnz, csr_ptr, t0 + lane, t1, 64, rowlen, v);
+            const int c = t2c_row_of(v, lane & 15), incl = tsg_row16_incl_scan_dpp(c);
             if (lane < rowlen) rowptr[16 * I + lane] = tile_nnz[t0] - nb0 + incl - c;
         }
         if (I == tilem - 1 && lane == 0) {
@@ -426,27 +793,9 @@ k_t2c_rowptr(int m, int tilem, const int *__restrict__ tile_ptr, const int *__re
                     items[slot + sg - 1].seg = sg;
                 }
             }
-            unsigned v[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // at most 16 * CV_SEG per half
-#pragma unroll
-            for (int k = 0; k < CV_SEG / (64 * CV_WAVES); k++) {
-                const int t = t0 + sg * CV_SEG + k * 64 * CV_WAVES + tid;
-                if (t < t1) {
-                    unsigned x[8];
-                    const int tn = tile_nnz[t + 1] - tile_nnz[t];
-                    t2c_widen(t2c_row_lens(t2c_offsets(load16(csr_ptr + 16 * (long long)t), tn, rowlen), tn), x);
-#pragma unroll
-                    for (int q = 0; q < 8; q++) v[q] += x[q];
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 8; q++) v[q] = tsg_wave_sum(v[q]);
-            if (lane == 0) {
-#pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    s_sum[wave][4 * (q >> 1) + (q & 1)] = (int)(v[q] & 0xffffu);
-                    s_sum[wave][4 * (q >> 1) + (q & 1) + 2] = (int)(v[q] >> 16);
-                }
-            }
+            t2c_row_sums(tile_nnz, csr_ptr, t0 + sg * CV_SEG + tid, min(t1, t0 + (sg + 1) * CV_SEG), 64 * CV_WAVES,
+                         rowlen, v);
+            if (lane < 16) s_sum[wave][lane] = t2c_row_of(v, lane);
             __syncthreads();
             if (tid < 16)
                 for (int w2 = 0; w2 < CV_WAVES; w2++) carry += s_sum[w2][tid];
@@ -471,7 +820,6 @@ __device__ __forceinline__ unsigned bytes_le(unsigned w, unsigned j) {
 // the item list.  One lane per entry: its tile from a mark at each tile's
 // first entry (running maximum over the lanes), its row from the tile's row
 // offsets, its place in the batch from the (tile, row)'s entries before it.
-#define CV_ROUNDS (CV_CAP / 64)
 __global__ void __launch_bounds__(64 * CV_WAVES)
 k_t2c_emit(int m, int tilem, const int *__restrict__ tile_ptr, const int *__restrict__ tile_colidx,
            const int *__restrict__ tile_nnz, const unsigned char *__restrict__ csr_ptr,

@@ -40,6 +40,9 @@ def inputs():
     # wide rows: bitmap windows of 8192 tile columns
     yield "wide", csr(18, 600011, {r: some(600011, 3 + 50 * (r % 3)) for r in range(18)})
     yield "wide_hub", csr(18, 600011, {2: some(600011, 9000), 3: some(600011, 5), 17: [600010]})
+    # columns near the end of the int32 range
+    top = 2**31 - 32
+    yield "int32_columns", csr(3, top, {0: [0, top - 40, top - 1], 1: [5, top - 2], 2: [top - 17, top - 16, top - 1]})
     yield "one", csr(1, 1, {0: [0]})
     yield "norows", csr(0, 5, {})
 
@@ -90,6 +93,20 @@ def test_tile2csr_ignores_offsets_past_the_rows(ctx):
     p[h["tile_ptr"][1]:, 5:] = 0
     raw = np.ascontiguousarray(p).reshape(-1)
     assert ts.lib.tsg_h2d(ctx.h, t.csr_ptr, raw.ctypes.data, raw.size) == 0
+    o = ctx.tile2csr(t)
+    b = ctx.download(o)
+    assert np.array_equal(b.rowptr, a.rowptr) and np.array_equal(b.colidx, a.colidx) and np.array_equal(b.val, a.val)
+    for x in (o, t, d):
+        ctx.free(x)
+
+
+def test_check_accepts_row_starts_anywhere(ctx):
+    """Descending columns across row starts at every place of a block of 4096 entries; long runs of empty rows."""
+    n = 5000
+    rows = {0: np.arange(4095), 1: np.arange(4096), 2: [0], 3: [n - 1], 4: [0], 5: np.arange(3000), 20009: np.arange(1095), 20010: [7]}
+    a = csr(40011, n, rows)
+    d = ctx.upload(a)
+    t = ctx.csr2tile(d)
     o = ctx.tile2csr(t)
     b = ctx.download(o)
     assert np.array_equal(b.rowptr, a.rowptr) and np.array_equal(b.colidx, a.colidx) and np.array_equal(b.val, a.val)
