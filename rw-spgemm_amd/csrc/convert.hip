@@ -565,16 +565,11 @@ extern "C" int tsg_csr2tile(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dtiles *out) {
                 TSG_LAUNCH_CHECK();
             }
         }
-        const long long np = tsg_scan_partial_count(T.tilem);
-        void *part;
-        TSG_TRY(tsg_scratch(ctx, (size_t)np * sizeof(long long), &part));
-        TSG_TRY(tsg_scan_i32_enqueue(s, T.tile_ptr, T.tile_ptr, T.tilem, (long long *)part));
-        long long *pin = ctx->pinned;
-        TSG_HIP(hipMemcpyAsync(pin, (long long *)part + np - 1, 8, hipMemcpyDeviceToHost, s));
-        TSG_HIP(hipMemcpyAsync(pin + 1, &count->bad, 4, hipMemcpyDeviceToHost, s));
-        TSG_HIP(hipStreamSynchronize(s));
-        TSG_TRY(validate_status(((int *)(pin + 1))[0], 1));
-        numtile = pin[0];  // at most nnz
+        // a bad input's counts may add up to anything: its flag is looked at first
+        const int sc = tsg_scan_i32(ctx, T.tile_ptr, T.tile_ptr, T.tilem, &numtile, &count->bad, 1);
+        if (sc != TSG_OK && sc != TSG_ERR_OVERFLOW) return sc;
+        TSG_TRY(validate_status(((volatile int *)(ctx->pinned + 1))[0], 1));
+        TSG_TRY(sc);
         T.numtile = (int)numtile;
         TSG_TRY(tsg_alloc_t(ctx, &T.tile_colidx, (size_t)numtile + 1));
         TSG_TRY(tsg_alloc_t(ctx, &T.tile_rowidx, (size_t)numtile + 1));

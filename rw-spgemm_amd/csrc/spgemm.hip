@@ -2294,9 +2294,10 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
 }
 
 // out[0] = sum and out[1..6] = maxima of the nb blocks' k_row_class partials
-// (one block of 1024 threads); out[7] = 0.
+// (one block of 1024 threads); out[7] = 0.  host (may be NULL): pinned
+// memory that gets the eight words too.
 __global__ void __launch_bounds__(1024)
-k_row_class_reduce(const int *__restrict__ part, int nb, int *__restrict__ out) {
+k_row_class_reduce(const int *__restrict__ part, int nb, int *__restrict__ out, int *__restrict__ host) {
     __shared__ int s_r[16][7];
     int v[7] = {0, 0, 0, 0, 0, 0, 0};
     for (int b = threadIdx.x; b < nb; b += 1024) {
@@ -2320,6 +2321,7 @@ k_row_class_reduce(const int *__restrict__ part, int nb, int *__restrict__ out) 
             for (int w = 1; w < 16; w++) r = i == 0 ? r + s_r[w][i] : max(r, s_r[w][i]);
         }
         out[i] = r;
+        if (host) host[i] = r;
     }
 }
 
@@ -2676,12 +2678,12 @@ static int launch_step2(hipStream_t s, const TileOperands &op, const tsg_dtiles 
 }
 
 static int launch_row_class(hipStream_t s, const TileOperands &op, tsg_dtiles *C, unsigned char *rowcls,
-                            int *cls_part, int *cls_out, int none_fit) {
+                            int *cls_part, int *cls_out, int none_fit, int *host = nullptr) {
     const int nb = (int)tsg_div_up(C->tilem, 16);
     hipLaunchKernelGGL(k_row_class, dim3(nb), dim3(256), 0, s, op, C->tile_ptr, C->tile_nnz, C->tilem, rowcls,
                        cls_part, none_fit);
     TSG_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_row_class_reduce, dim3(1), dim3(1024), 0, s, (const int *)cls_part, nb, cls_out);
+    hipLaunchKernelGGL(k_row_class_reduce, dim3(1), dim3(1024), 0, s, (const int *)cls_part, nb, cls_out, host);
     TSG_LAUNCH_CHECK();
     return TSG_OK;
 }
@@ -2832,21 +2834,8 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     long long numtileC = 0;
     int smax[4] = {0, 0, 0, 0};
     {
-        const long long np1 = tsg_scan_partial_count(C->tilem);
-        void *part1v;
-        TSG_TRY(tsg_scratch(ctx, (size_t)np1 * sizeof(long long), &part1v));
-        long long *part1 = (long long *)part1v;
-        TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_ptr, C->tile_ptr, C->tilem, part1));
-        long long *pin = ctx->pinned;
-        TSG_HIP(hipMemcpyAsync(pin, part1 + np1 - 1, sizeof(long long), hipMemcpyDeviceToHost, s));
-        TSG_HIP(hipMemcpyAsync(pin + 1, st2, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
-        TSG_HIP(hipStreamSynchronize(s));
-        numtileC = pin[0];
-        if (numtileC > 0x7fffffffLL) {
-            tsg_set_error("prefix sum total %lld exceeds int32", numtileC);
-            return TSG_ERR_OVERFLOW;
-        }
-        memcpy(smax, pin + 1, sizeof(smax));
+        TSG_TRY(tsg_scan_i32(ctx, C->tile_ptr, C->tile_ptr, C->tilem, &numtileC, st2, 4));
+        memcpy(smax, ctx->pinned + 1, sizeof(smax));
     }
     tsg_free(ctx, T.span);
     T.span = nullptr;
@@ -2886,20 +2875,18 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     // device offsets); C's nonzero count and the class maxima come back in
     // one read-back
     long long nnzC = 0;
-    const long long np2 = tsg_scan_partial_count(numtileC);
     void *part2v;
-    TSG_TRY(tsg_scratch(ctx, (size_t)np2 * sizeof(long long), &part2v));
+    TSG_TRY(tsg_scratch(ctx, (size_t)tsg_scan_partial_count(numtileC) * sizeof(long long), &part2v));
     long long *part2 = (long long *)part2v;
-    TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_nnz, C->tile_nnz, numtileC, part2));
-    if (timed) TSG_HIP(hipEventRecord(ev[2], s));
     const bool classes = !P.all && numtileC > 0;
-    if (classes) {
-        TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all));
-    }
     {
         long long *pin = ctx->pinned;  // [0] the total, [1..4] the eight class words
-        TSG_HIP(hipMemcpyAsync(pin, part2 + np2 - 1, sizeof(long long), hipMemcpyDeviceToHost, s));
-        if (classes) TSG_HIP(hipMemcpyAsync(pin + 1, w.cls_out, 8 * sizeof(int), hipMemcpyDeviceToHost, s));
+        tsg_scan_publish pub;
+        pub.host = pin;
+        TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_nnz, C->tile_nnz, numtileC, part2, pub));
+        if (timed) TSG_HIP(hipEventRecord(ev[2], s));
+        if (classes)
+            TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, (int *)(pin + 1)));
         TSG_HIP(hipStreamSynchronize(s));
         nnzC = pin[0];
         if (nnzC > 0x7fffffffLL) {
@@ -2945,15 +2932,14 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                                    hflag, hcnt, hinfo);
                 TSG_LAUNCH_CHECK();
                 long long ni = 0;
-                TSG_TRY(tsg_scan_i32(ctx, hcnt, hcnt, m, &ni));
+                TSG_TRY(tsg_scan_i32(ctx, hcnt, hcnt, m, &ni, hinfo, 2));
                 if (ni > 0x7fffffffLL) {
                     tsg_set_error("spgemm: %lld heavy-row work items exceed the int32 range", ni);
                     return TSG_ERR_ARG;
                 }
                 if (ni > 0) {
-                    long long info = 0;  // {longest heavy A row, heavy rows}
-                    TSG_TRY(tsg_read_scalar_i64(ctx, hinfo, 1, &info));
-                    const long long maxdeg = info & 0xffffffffLL, nrows = info >> 32;
+                    const volatile int *info = (const volatile int *)(ctx->pinned + 1);
+                    const long long maxdeg = info[0], nrows = info[1];
                     TSG_TRY(tsg_alloc_t(ctx, &T.hitems, (size_t)ni));
                     int2 *hitems = T.hitems;
                     hipLaunchKernelGGL(k_heavy_list, dim3(tsg_div_up(m, 256)), dim3(256), 0, s, (const int *)hcnt,

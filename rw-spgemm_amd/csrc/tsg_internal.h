@@ -101,13 +101,23 @@ size_t tsg_alloc_size(const tsg_ctx *ctx, const void *p);
 // ------------------------------------------------------------------ scans
 // Exclusive scan of n non-negative int32 counts into out[0..n] (out[n] =
 // total).  `in` may alias `out`.  total (may be NULL) is read back to the
-// host; TSG_ERR_OVERFLOW when the total exceeds INT32_MAX.
-int tsg_scan_i32(tsg_ctx *ctx, const int *in, int *out, long long n, long long *total);
+// host; TSG_ERR_OVERFLOW when the total exceeds INT32_MAX.  With total,
+// nwords device ints are read back behind it (ctx->pinned + 1).
+int tsg_scan_i32(tsg_ctx *ctx, const int *in, int *out, long long n, long long *total, const int *words = nullptr,
+                 int nwords = 0);
 // Enqueue-only form (no host read-back, no memset: graph-capturable).
 // `partial` holds tsg_scan_partial_count(n) int64 values; the int64 total
-// is left in partial[tsg_scan_partial_count(n) - 1].
+// is left in partial[tsg_scan_partial_count(n) - 1].  With pub.host (pinned
+// memory) the scan's last block also writes the total there and nwords
+// device ints behind it: valid once the stream has been waited for.
+struct tsg_scan_publish {
+    long long *host = nullptr;
+    const int *words = nullptr;
+    int nwords = 0;
+};
 long long tsg_scan_partial_count(long long n);
-int tsg_scan_i32_enqueue(hipStream_t stream, const int *in, int *out, long long n, long long *partial);
+int tsg_scan_i32_enqueue(hipStream_t stream, const int *in, int *out, long long n, long long *partial,
+                         tsg_scan_publish pub = {});
 // Same for unsigned-char counts of 16-row tiles is done inside the kernels.
 // Sum of n int64 values (device) -> host.
 int tsg_reduce_u64(tsg_ctx *ctx, const unsigned long long *in, long long n,
