@@ -180,46 +180,6 @@ struct C2tCount {
 };
 #define C2T_BIG 4096  // entries of a tile-row above which a whole block collects its tiles
 
-// Tile columns of tile-row I into list[0..), ascending, from words [0, nw)
-// of a wave's bitmap window that starts at tile column w0; returns their number.
-// A window with many tiles writes one pair of words per step, each bit a
-// lane, so that a store instruction covers consecutive entries; with few,
-// each lane writes the bits of its own word.
-__device__ __forceinline__ int emit_window(const unsigned *bm, int nw, int w0, int lane, int *__restrict__ list) {
-    int done = 0;
-    for (int k0 = 0; k0 < nw; k0 += 64) {
-        const unsigned x = k0 + lane < nw ? bm[k0 + lane] : 0u;
-        const int c = __popc(x), incl = tsg_wave_incl_scan_dpp(c);
-        const int tot = __builtin_amdgcn_readlane(incl, 63);
-        const int pos = done + incl - c;
-        if (tot > 256) {
-            unsigned long long nz = __ballot(x != 0u);
-            while (nz) {
-                const int j0 = __ffsll((long long)nz) - 1;
-                nz &= nz - 1;
-                const int j1 = nz ? __ffsll((long long)nz) - 1 : j0;
-                const bool both = nz != 0;
-                nz &= nz - 1;  // 0 stays 0
-                const int j = lane < 32 ? j0 : j1;
-                const unsigned wd = lane < 32 ? (unsigned)__builtin_amdgcn_readlane((int)x, j0)
-                                              : (unsigned)__builtin_amdgcn_readlane((int)x, j1);
-                const int p = lane < 32 ? __builtin_amdgcn_readlane(pos, j0) : __builtin_amdgcn_readlane(pos, j1);
-                const int b = lane & 31;
-                if ((lane < 32 || both) && (wd >> b) & 1u)
-                    list[p + __popc(wd & ((1u << b) - 1u))] = w0 + 32 * (k0 + j) + b;
-            }
-        } else {
-            unsigned y = x;
-            for (int q = pos; y; q++) {
-                list[q] = w0 + 32 * (k0 + lane) + __ffs(y) - 1;
-                y &= y - 1;
-            }
-        }
-        done += tot;
-    }
-    return done;
-}
-
 // Tiles of each tile-row: their number into cnt[I], their columns into
 // list[rowptr[16I]..) (a tile has an entry, so they fit).  One wave per
 // tile-row; a tile-row of more than C2T_BIG entries is put on the list of

@@ -335,25 +335,12 @@ k_step1(const int *__restrict__ Aptr, const int *__restrict__ Acol, int tilem,
             for (int k = lane; k < nw; k += 64) cnt += __popc(bm[k]);
             total += tsg_wave_sum(cnt);
         } else {
-            const int chunk = (nw + 63) >> 6;
-            const int k0 = lane * chunk, k1 = min(nw, k0 + chunk);
-            int cnt = 0;
-            for (int k = k0; k < k1; k++) cnt += __popc(bm[k]);
-            int pos = base + total + tsg_wave_incl_scan(cnt) - cnt;
-            for (int k = k0; k < k1; k++) {
-                unsigned x = bm[k];
-                while (x) {
-                    const int b = __ffs(x) - 1;
-                    x &= x - 1;
-                    Ccol[pos] = w0 + k * 32 + b;
-                    Crow[pos] = I;
-                    pos++;
-                }
-            }
-            total += tsg_wave_sum(cnt);
+            total += emit_window(bm, nw, w0, lane, Ccol + base + total);
         }
         tsg_wave_sync();
     }
+    if (FILL)
+        for (int k = lane; k < total; k += 64) Crow[base + k] = I;
     if (!FILL && lane == 0) {
         Cptr_or_cnt[I] = total;
         // the candidates are exactly C's tiles, so this is the row's C tile-column span
