@@ -36,6 +36,7 @@
 #define S1_WAVES 4
 #define S23_WAVES 4
 #define TILES_PER_WAVE 4
+#define S2_KINDS 4  // step-2 kernels (step2_kind)
 
 extern "C" void tsg_tune_default(tsg_tune *t) {
     memset(t, 0, sizeof(*t));
@@ -143,6 +144,9 @@ k_step1(const int *__restrict__ Aptr, const int *__restrict__ Acol, int tilem,
         const int *__restrict__ Bptr, const int *__restrict__ Bcol, const int4 *__restrict__ Bdesc,
         const unsigned *__restrict__ Bbits, const int *__restrict__ Bany, int *__restrict__ Cptr_or_cnt,
         int *__restrict__ Ccol, int *__restrict__ Crow, unsigned *__restrict__ bmstore, int *__restrict__ rowspan) {
+    // rowspan (may be NULL): count pass, each row's C tile-column span; fill
+    // pass, S2_KINDS counters to clear for k_seg2_fill
+    if (FILL && rowspan && blockIdx.x == 0 && threadIdx.x < S2_KINDS) rowspan[threadIdx.x] = 0;
     __shared__ unsigned s_bm[S1_WAVES][BMW];
     __shared__ int s_pre[S1_WAVES][64];
     __shared__ int s_b0[S1_WAVES][64];
@@ -427,88 +431,131 @@ __device__ __forceinline__ void for_each_pair(const TileOperands &op, int I, int
 
 // ------------------------------------------------------------------ segments
 // A segment is a range [s0, s1) of the C tiles of one tile-row I, stored
-// as int4 {I, s0, s1, 0}.  Long tile-rows are cut into segments so each
-// fits a block's LDS; a segment's C tiles cover the tile columns
-// [Ccol[c0+s0], Ccol[c0+s1-1]], and only the B tiles inside that column
-// range meet them.  MODE 0 cuts by tile count; MODE 1 also keeps every
-// segment within max_nnz C nonzeros (tile nnz <= 256 <= max_nnz).  Only
-// tile-rows with rowcls == want (want < 0: all) are cut.
-template <int MODE>
-__device__ __forceinline__ int seg_walk(const int *__restrict__ Cnnz, int c0, int u, int max_tiles, int max_nnz,
-                                        int4 *out, int I, int kind = 0) {
-    if (MODE == 0) {
-        const int n = (u + max_tiles - 1) / max_tiles;
-        if (out)
-            for (int j = 0; j < n; j++) out[j] = make_int4(I, j * max_tiles, min(u, (j + 1) * max_tiles), kind);
-        return n;
-    }
-    // MODE 1: tile s belongs to segment floor(p(s) / H), p(s) = C nonzeros of
-    // the row before tile s and H = max_nnz - 255; a tile holds at most 256
-    // nonzeros, so ids grow by at most one per tile, every id up to the last
-    // is present, and a segment holds at most H + 255 = max_nnz nonzeros.
-    // Count in O(1), each boundary by one binary search (no tile walk).
-    const int H = max_nnz - 255;
-    const int base = Cnnz[c0];
-    const int n = (Cnnz[c0 + u - 1] - base) / H + 1;
-    if (out) {
-        int s0 = 0;
-        for (int j = 0; j < n; j++) {
-            int s1 = u;
-            if (j + 1 < n) {  // first tile with p >= (j+1) H
-                const int key = base + (j + 1) * H;
-                int lo = s0, hi = u - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (Cnnz[c0 + mid] < key) lo = mid + 1; else hi = mid;
-                }
-                s1 = lo;
-            }
-            out[j] = make_int4(I, s0, s1, j);  // .w: index of the segment in its tile-row
-            s0 = s1;
-        }
-    }
-    return n;
+// as int4 {I, s0, s1, index in the tile-row}; its C tiles cover the tile
+// columns [Ccol[c0+s0], Ccol[c0+s1-1]], and only the B tiles inside that
+// column range meet them.
+
+// Step-2 segments: tile-rows are cut so that a segment fits a block's LDS.
+#define G2_UMAX 512       // C tiles of one segment of the tile-pair and hash kernels
+#define G2_MAP_MAX 16384  // widest tile-row span with a direct column map (bytes of LDS)
+#define G2D_WIN 4096      // tile columns of one window of the dense kernel (128 KiB of bits)
+#define G2D_SMALL 1024    // widest tile-row span that takes it with small blocks
+
+// Step-2 kernel of a tile-row with u > 0 C tiles over `span` tile columns,
+// whose A tile-row has `ents` entries in `tiles` tiles:
+//   0  tile pairs (k_step2_rows)
+//   1  element-wise, C tiles in a hash (k_step2_elem)
+//   2  element-wise, the tile-row's columns as bits in LDS, one small block
+//      per tile-row (k_step2_dense)
+//   3  the same in windows of G2D_WIN tile columns, one large block each
+// Element-wise needs B's row index (elem), and the dense form A's too (rx).
+// Hypersparse tile-rows (at most 4 entries per A tile, or all with `all`)
+// go element-wise: one step per product instead of one per tile pair.  The
+// dense form costs its window's 32 bytes a tile column whatever is in it and
+// one LDS atomic a product, and a second window walks the A rows again with
+// two searches in every B row; the hash costs a probe chain a product and
+// such a walk per 512 tiles.  Erdos-Renyi A^2, hash against dense: 65536 rows
+// with 43 / 53 / 63% of the span filled 408 / 483 / 632 against 413 / 486 /
+// 535 us, 16384 rows with 29 / 50% 165 / 162 against 182 / 157 us; 131072
+// rows (two windows) with 39 / 54 / 67 / 86% 1138 / 1487 / 1830 / 2423
+// against 1240 / 1537 / 1820 / 2326 us.  So half of one window, three fifths
+// of several.  Tile-pair rows of more than one segment take it too (each
+// pair a loop over 16 rows, the segments a walk each): the 72 hub tile-rows
+// of R-MAT scale 16 A*A^T, 24% of its products, were 5.5 ms of step 2's 17.1;
+// all of it is 2.1 ms now.
+__device__ __forceinline__ int step2_kind(int u, int span, long long ents, int tiles, int elem, int all, int rx) {
+    if (!elem) return 0;
+    const bool el = all || ents <= 4ll * tiles;
+    if (rx && (el || u > G2_UMAX) && (span <= G2D_WIN ? 2ll * u >= span : 5ll * u >= 3ll * span))
+        return span <= G2D_SMALL ? 2 : 3;
+    return el ? 1 : 0;
+}
+// Segments of such a tile-row.  Kind 3: windows of equal width of at most
+// G2D_WIN tile columns, and one more per G2D_ENTS entries of the A tile-row
+// (a hub tile-row's products would keep one CU busy long after the others: R-MAT
+// scale 16 2.4 ms with 16384, 2.15 with 4096, 2.2 with 1024),
+// at most as many as the hash kernel would take, so that a list of one per
+// tile-row and G2_UMAX tiles holds every kind's.
+#define G2D_ENTS 4096
+__device__ __forceinline__ int step2_segments(int kind, int u, int span, long long ents) {
+    if (kind == 2) return 1;
+    const int n = (u + G2_UMAX - 1) / G2_UMAX;
+    if (kind < 2) return n;
+    return max((span + G2D_WIN - 1) / G2D_WIN, (int)min((long long)n, ents / G2D_ENTS + 1));
 }
 
-template <int MODE>
+// The step-2 segments of every kind, kind k from items[base.k] on in no
+// particular order (neighbouring tile-rows stay near each other); ctr[k]
+// (zeroed beforehand) counts them.  One atomic per wave and kind present.
 __global__ void __launch_bounds__(256)
-k_seg(const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tilem, const unsigned char *__restrict__ rowcls,
-      int want, int max_tiles, int max_nnz, int *__restrict__ cnt_or_off, int4 *__restrict__ items) {
+k_seg2_fill(const int *__restrict__ Cptr, const int *__restrict__ Ccol, const int *__restrict__ Aptr,
+            const int *__restrict__ Annz, int tilem, int elem, int all, int rx, int4 base, int *__restrict__ ctr,
+            int4 *__restrict__ items) {
+    const int I = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+    int c0 = 0, u = 0, span = 0, kind = -1, n = 0;
+    if (I < tilem) {
+        c0 = Cptr[I];
+        u = Cptr[I + 1] - c0;
+        if (u > 0) {
+            const int a0 = Aptr[I], a1 = Aptr[I + 1];
+            span = Ccol[c0 + u - 1] - Ccol[c0] + 1;
+            kind = step2_kind(u, span, (long long)Annz[a1] - Annz[a0], a1 - a0, elem, all, rx);
+            n = step2_segments(kind, u, span, (long long)Annz[a1] - Annz[a0]);
+        }
+    }
+    int pos = 0;
+#pragma unroll
+    for (int k = 0; k < S2_KINDS; k++) {
+        if (!__ballot(kind == k)) continue;
+        const int mine = kind == k ? n : 0, incl = tsg_wave_incl_scan_dpp(mine);
+        int b = 0;
+        if (lane == 63) b = atomicAdd(&ctr[k], incl);
+        b = __builtin_amdgcn_readlane(b, 63) + (k == 0 ? base.x : k == 1 ? base.y : k == 2 ? base.z : base.w);
+        if (kind == k) pos = b + incl - mine;
+    }
+    if (kind < 0) return;
+    if (kind < 2) {
+        for (int j = 0; j < n; j++)
+            items[pos + j] = make_int4(I, j * G2_UMAX, min(u, (j + 1) * G2_UMAX), j);
+    } else {
+        int s0 = 0;
+        const int jlo = Ccol[c0], win = (span + n - 1) / n;
+        for (int j = 0; j < n; j++) {  // first tile at or past each window's end
+            int lo = s0, hi = u;
+            if (j + 1 < n) {
+                const int key = jlo + (j + 1) * win;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (Ccol[c0 + mid] < key) lo = mid + 1; else hi = mid;
+                }
+            } else {
+                lo = u;
+            }
+            items[pos + j] = make_int4(I, s0, lo, j);
+            s0 = lo;
+        }
+    }
+}
+
+// Step-3 element segments: tile s belongs to segment floor(p(s) / H), p(s) =
+// C nonzeros of the row before tile s and H = max_nnz - 255; a tile holds at
+// most 256 nonzeros, so ids grow by at most one per tile, every id up to the
+// last is present, and a segment holds at most H + 255 = max_nnz nonzeros.
+// Counts of the tile-rows with rowcls == want; k_seg1_fill writes them.
+__global__ void __launch_bounds__(256)
+k_seg1_count(const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tilem,
+             const unsigned char *__restrict__ rowcls, int want, int max_nnz, int *__restrict__ cnt) {
     const int I = blockIdx.x * 256 + threadIdx.x;
     if (I >= tilem) return;
     const int c0 = Cptr[I], u = Cptr[I + 1] - c0;
-    // MODE 0 carries rowcls (the step-2 kernel kind) into each item's .w
-    const bool take = u > 0 && (want < 0 || rowcls[I] == want);
-    const int kind = (MODE == 0 && rowcls) ? rowcls[I] : 0;
-    if (!items) {
-        cnt_or_off[I] = take ? seg_walk<MODE>(Cnnz, c0, u, max_tiles, max_nnz, nullptr, I, kind) : 0;
-    } else if (take) {
-        seg_walk<MODE>(Cnnz, c0, u, max_tiles, max_nnz, items + cnt_or_off[I], I, kind);
-    }
+    cnt[I] = u > 0 && rowcls[I] == want ? (Cnnz[c0 + u - 1] - Cnnz[c0]) / (max_nnz - 255) + 1 : 0;
 }
 
-// Step-2 kernel kind of every tile-row: 1 = element-wise (B has its row
-// index and A's tile-row is hypersparse: at most 4 entries per tile on
-// average, or every row when all_elem), 0 = tile pairs.
-__global__ void __launch_bounds__(256)
-k_step2_kind(const int *__restrict__ Aptr, const int *__restrict__ Annz, int tilem, int all_elem,
-             unsigned char *__restrict__ kind) {
-    const int I = blockIdx.x * 256 + threadIdx.x;
-    if (I >= tilem) return;
-    const int a0 = Aptr[I], a1 = Aptr[I + 1];
-    const long long e = (long long)Annz[a1] - Annz[a0];
-    kind[I] = (unsigned char)((all_elem || e <= 4LL * (a1 - a0)) ? 1 : 0);
-}
-
-// Upper bound on the segments of a C with tilem tile-rows and numtile
-// tiles: one per tile-row, one per max_tiles tiles closed by count, and
-// (MODE 1) one per (max_nnz - 255) nonzeros closed by size, with at most
-// 256 nonzeros per tile.
-static long long seg_bound(long long tilem, long long numtile, int max_tiles, int max_nnz, int mode) {
-    long long b = tilem + numtile / max_tiles + 1;
-    if (mode == 1) b += 256 * numtile / (max_nnz - 255) + 1;
-    return b;
-}
+// Upper bound on the step-2 segments of a C with tilem tile-rows and numtile
+// tiles: one per tile-row and one per G2_UMAX tiles (a dense window past a
+// row's first stands for at least G2D_WIN / 2 tiles or for G2_UMAX).
+static long long seg2_bound(long long tilem, long long numtile) { return tilem + numtile / G2_UMAX + 1; }
+static_assert(G2D_WIN / 2 >= G2_UMAX, "dense windows within the segment bound");
 
 // First index in [lo, hi) with list[index] >= key (list ascending).
 __device__ __forceinline__ int lower_bound_i(const int *__restrict__ list, int lo, int hi, int key) {
@@ -519,11 +566,11 @@ __device__ __forceinline__ int lower_bound_i(const int *__restrict__ list, int l
     return lo;
 }
 
-// MODE 1 segments, one thread per segment (a hub tile-row has thousands, each
+// Step-3 element segments, one thread per segment (a hub tile-row has thousands, each
 // found by a binary search; one thread per row left the whole launch
 // waiting on the longest row): segment j's row is the last row whose first
 // segment is at or before j (off[] is the scanned per-row count, off[tilem]
-// the total), and its bounds are the same tiles seg_walk finds.
+// the total), its bounds the first tiles at or past its ends.
 __global__ void __launch_bounds__(256)
 k_seg1_fill(const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tilem, const int *__restrict__ off,
             int max_nnz, int4 *__restrict__ items) {
@@ -553,51 +600,61 @@ k_seg1_fill(const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tile
 // (r, k) contribute B row k to C row r alone; their pairs are enumerated
 // before the others' so that a wave's lanes take one kind of pair.
 #define G2_THREADS 256
-#define G2_UMAX 512    // C tiles of one segment held in LDS
 #define G2_PCHUNK 256  // A tiles per enumeration round
-#define G2_MAP_MAX 16384  // widest tile-row span with a direct column map (bytes of LDS)
 #define G2_MSTRIDE 9      // LDS words per C tile mask set / per thread B mask copy (8 used)
 
-// Most C tiles of a tile-row (capped at the step-2 segment size), the
-// widest tile-column span of a tile-row, and the widest span of at most
-// G2_MAP_MAX: out[0], out[1], out[2] (atomic maxima), from the step-1 count
-// pass's per-row tile counts and spans.
+// Sizes of steps 2 and 3 from the step-1 count pass's per-row tile counts
+// and spans (atomics on out[0..8), zeroed beforehand):
+//   [0] most C tiles of a tile-pair tile-row (capped at the segment size)
+//   [1] widest tile-column span of a tile-row
+//   [2] widest span of at most G2_MAP_MAX of a tile-pair tile-row
+//   [3 + k] step-2 segments of kind k
+//   [7] widest span of a kind-2 tile-row
 // A few large blocks stride over the rows, so that the atomics (one cache
 // line, serialised) are few.
 #define ROW_STATS_BLOCKS 64
+#define ROW_STATS 8
 __global__ void __launch_bounds__(1024)
-k_row_stats(const int *__restrict__ cnt, const int *__restrict__ span, int tilem, int *__restrict__ out) {
-    __shared__ int s_r[16][3];
-    int nu = 0, sp = 0, ms = 0;
+k_row_stats(const int *__restrict__ cnt, const int *__restrict__ span, const int *__restrict__ Aptr,
+            const int *__restrict__ Annz, int tilem, int elem, int all, int rx, int *__restrict__ out) {
+    __shared__ int s_r[16][ROW_STATS];
+    int v[ROW_STATS];
+#pragma unroll
+    for (int i = 0; i < ROW_STATS; i++) v[i] = 0;
     for (int I = blockIdx.x * 1024 + threadIdx.x; I < tilem; I += gridDim.x * 1024) {
-        if (cnt[I] > 0) {
-            const int s1 = span[I];
-            nu = max(nu, min(cnt[I], G2_UMAX));
-            sp = max(sp, s1);
-            if (s1 <= G2_MAP_MAX) ms = max(ms, s1);
+        const int u = cnt[I];
+        if (u <= 0) continue;
+        const int s1 = span[I], a0 = Aptr[I], a1 = Aptr[I + 1];
+        const long long ents = (long long)Annz[a1] - Annz[a0];
+        const int kind = step2_kind(u, s1, ents, a1 - a0, elem, all, rx);
+        v[1] = max(v[1], s1);
+        if (kind == 0) {
+            v[0] = max(v[0], min(u, G2_UMAX));
+            if (s1 <= G2_MAP_MAX) v[2] = max(v[2], s1);
         }
+#pragma unroll
+        for (int k = 0; k < S2_KINDS; k++) v[3 + k] += kind == k ? step2_segments(kind, u, s1, ents) : 0;
+        if (kind == 2) v[7] = max(v[7], s1);
     }
-    nu = tsg_wave_max(nu);
-    sp = tsg_wave_max(sp);
-    ms = tsg_wave_max(ms);
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        s_r[wave][0] = nu;
-        s_r[wave][1] = sp;
-        s_r[wave][2] = ms;
+#pragma unroll
+    for (int i = 0; i < ROW_STATS; i++) {
+        v[i] = i >= 3 && i < 7 ? tsg_wave_sum(v[i]) : tsg_wave_max(v[i]);
+        if ((threadIdx.x & 63) == 0) s_r[threadIdx.x >> 6][i] = v[i];
     }
     __syncthreads();
-    if (threadIdx.x < 3) {
-        int v = s_r[0][threadIdx.x];
-        for (int w = 1; w < 16; w++) v = max(v, s_r[w][threadIdx.x]);
-        atomicMax(&out[threadIdx.x], v);
+    if (threadIdx.x < ROW_STATS) {
+        const int i = threadIdx.x;
+        const bool sum = i >= 3 && i < 7;
+        int x = s_r[0][i];
+        for (int w = 1; w < 16; w++) x = sum ? x + s_r[w][i] : max(x, s_r[w][i]);
+        if (sum) atomicAdd(&out[i], x);
+        else atomicMax(&out[i], x);
     }
 }
 
 static_assert(G2_PCHUNK == G2_THREADS, "one A tile of a chunk per thread");
 __global__ void __launch_bounds__(G2_THREADS)
-k_step2_rows(TileOperands op, const int4 *__restrict__ segs, const int *__restrict__ nseg, const int *__restrict__ Cptr,
-             const int *__restrict__ Ccol, unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16,
+k_step2_rows(TileOperands op, const int4 *__restrict__ segs, const int *__restrict__ Cptr, const int *__restrict__ Ccol, unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16,
              int *__restrict__ Cnnz, int umax, int mapbytes) {
     // dynamic LDS, sized by the largest segment: the segment's C tile masks
     // (two 16-bit rows per word, even row high; G2_MSTRIDE words per tile so
@@ -622,13 +679,16 @@ k_step2_rows(TileOperands op, const int4 *__restrict__ segs, const int *__restri
     // and 2i+1), so that a wave's lanes read and write consecutive banks
     __shared__ unsigned s_bst[8][G2_THREADS];
     const int tid = threadIdx.x;
-    // the grid is an upper bound: the first *nseg blocks (spread evenly over
-    // the XCDs) take the segments, each XCD a contiguous range
-    const int ns = *nseg;
-    if ((int)blockIdx.x >= ns) return;  // block-uniform
-    const int w = (int)tsg_xcd_block(blockIdx.x, (unsigned)ns);
-    const int4 sg = segs[w];
-    if (sg.w) return;  // element-wise segment (k_step2_elem)
+    // one block per segment, each XCD a contiguous range; without a list
+    // (segs NULL) every tile-row is one segment
+    const int w = (int)tsg_xcd_block(blockIdx.x, gridDim.x);
+    int4 sg = make_int4(w, 0, 0, 0);
+    if (segs) {
+        sg = segs[w];
+    } else {
+        sg.z = Cptr[w + 1] - Cptr[w];
+        if (sg.z == 0) return;  // block-uniform
+    }
     const int I = sg.x;
     const int c0 = Cptr[I] + sg.y, u = sg.z - sg.y;
     const bool whole = sg.y == 0 && sg.z == Cptr[I + 1] - Cptr[I];
@@ -809,20 +869,15 @@ __device__ __forceinline__ unsigned col_hash10(int J) { return ((unsigned)J * 26
 
 __global__ void __launch_bounds__(G2_THREADS)
 k_step2_elem(TileOperands op, const int *__restrict__ Browp, const int *__restrict__ Bcolx,
-             const int4 *__restrict__ segs, const int *__restrict__ nseg, const int *__restrict__ Cptr,
-             const int *__restrict__ Ccol, unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16,
-             int *__restrict__ Cnnz) {
+             const int4 *__restrict__ segs, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
+             unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16, int *__restrict__ Cnnz) {
     __shared__ unsigned s_m[G2_UMAX * 8];  // two 16-bit rows per word, even row high
     // hash of the segment's tile columns: slot (J - jlo + 1) << 9 | C tile
     // index (J - jlo + 1 < 2^23 as B has at most 2^27 - 32 columns when this
     // kernel runs, index < G2_UMAX = 512); 0 = empty
     __shared__ unsigned s_hkey[G2E_HASH];
     const int tid = threadIdx.x;
-    const int ns = *nseg;
-    if ((int)blockIdx.x >= ns) return;  // block-uniform
-    const int w = (int)tsg_xcd_block(blockIdx.x, (unsigned)ns);
-    const int4 sg = segs[w];
-    if (!sg.w) return;  // tile-pair segment (k_step2_rows)
+    const int4 sg = segs[tsg_xcd_block(blockIdx.x, gridDim.x)];
     const int I = sg.x;
     const int c0 = Cptr[I] + sg.y, u = sg.z - sg.y;
     for (int i = tid; i < u * 8; i += G2_THREADS) s_m[i] = 0u;
@@ -939,6 +994,165 @@ k_step2_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
         cm4[1] = make_uint4(mk[4], mk[5], mk[6], mk[7]);
         *reinterpret_cast<uint4 *>(Cptr16 + t * 16) = make_uint4(pt[0], pt[1], pt[2], pt[3]);
         Cnnz[t] = sum;
+    }
+}
+
+// Row offsets, entry count and masks of a C tile from its 16 row masks.
+__device__ __forceinline__ void step2_store(const unsigned mk[8], long long t, unsigned short *__restrict__ Cmask,
+                                            unsigned char *__restrict__ Cptr16, int *__restrict__ Cnnz) {
+    unsigned pt[4];
+    int sum = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        pt[q] = 0;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            pt[q] |= (unsigned)sum << (8 * b);
+            sum += __popc((mk[2 * q + (b >> 1)] >> (16 * (b & 1))) & 0xffffu);
+        }
+    }
+    uint4 *cm4 = reinterpret_cast<uint4 *>(Cmask + t * 16);
+    cm4[0] = make_uint4(mk[0], mk[1], mk[2], mk[3]);
+    cm4[1] = make_uint4(mk[4], mk[5], mk[6], mk[7]);
+    *reinterpret_cast<uint4 *>(Cptr16 + t * 16) = make_uint4(pt[0], pt[1], pt[2], pt[3]);
+    Cnnz[t] = sum;
+}
+
+// Element-wise bitmask symbolic with the window's 16 rows as bits in LDS (a
+// u16 per row and tile column): one block per segment, at most one LDS atomic
+// OR per intermediate product and no lookup.  A wave takes up to 64 entries
+// of the tile-row's A rows at a time.  B rows of G2D_LONG or more entries in
+// the window are taken by the whole wave one after another; the products of
+// the others are numbered through and taken one per lane, the entry of each
+// found from a mark at its first product (running maximum over the lanes).
+// Bound by the block's chain of loads and its 52 bytes of output per tile
+// for short rows (one block of 131 KiB fits a CU at a time), by LDS and
+// VALU issue for hub rows.  Against the hash kernel (a probe chain per
+// product, the tile-row cut every 512 tiles) and tile pairs: ER 65521 A^2 0.53
+// -> 0.285 ms, R-MAT scale 16 A*A^T 17.1 -> 2.15 ms (580 G products/s).  Without
+// the read before the atomic, the long rows' own path and the split of hub
+// tile-rows the latter took 5.5 ms.
+#define G2D_LONG 256                      // entries of a B row that a wave takes by itself
+#define G2D_ROUNDS 8                      // products per lane and batch
+#define G2D_BATCH (64 * G2D_ROUNDS)
+#define G2D_WAVE_LDS (64 * 8 + G2D_BATCH) // bytes per wave
+// LDS of a block of `threads` for windows of up to `width` tile columns.
+static size_t g2d_lds(int width, int threads) {
+    return 32 * (size_t)((width + 2) & ~1) + (size_t)(threads / 64) * G2D_WAVE_LDS;
+}
+__global__ void __launch_bounds__(1024)
+k_step2_dense(const int *__restrict__ Arowp, const int *__restrict__ Acolx, int m, const int *__restrict__ Browp,
+              const int *__restrict__ Bcolx, const int4 *__restrict__ segs, int nseg, const int *__restrict__ Cptr,
+              const int *__restrict__ Ccol, unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16,
+              int *__restrict__ Cnnz, int width) {
+    extern __shared__ __align__(16) unsigned char g2d_smem[];
+    __shared__ int s_rp[17];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nthr = blockDim.x, nwave = nthr >> 6;
+    unsigned *bm = reinterpret_cast<unsigned *>(g2d_smem);
+    unsigned char *ws = g2d_smem + 32 * (size_t)((width + 2) & ~1) + (size_t)wave * G2D_WAVE_LDS;
+    int *s_delta = reinterpret_cast<int *>(ws), *s_row = s_delta + 64;
+    unsigned char *s_mark = ws + 64 * 8;
+    for (int w = blockIdx.x; w < nseg; w += gridDim.x) {
+        const int4 sg = segs[w];
+        const int I = sg.x, cb = Cptr[I], c0 = cb + sg.y, u = sg.z - sg.y;
+        if (u == 0) continue;  // block-uniform: a window without tiles
+        // the window starts at an even tile column, so that a word's half and
+        // bit follow from the column alone: bit (column & 31) ^ 15
+        const int j0 = Ccol[c0] & ~1, j1 = Ccol[c0 + u - 1];
+        const int stride = (j1 - j0 + 2) & ~1;  // u16 per row
+        const bool whole = cb + sg.y == cb && c0 + u == Cptr[I + 1];
+        for (int i = tid; i < 2 * stride; i += nthr) reinterpret_cast<uint4 *>(bm)[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (tid < 17) s_rp[tid] = Arowp[min(16 * I + tid, m)];
+        __syncthreads();
+        const int x0 = s_rp[0], nx = s_rp[16] - x0;
+        const int per = min(64, max(1, (nx + nwave - 1) / nwave));
+        for (int c = wave * per; c < nx; c += nwave * per) {
+            int b0 = 0, len = 0, row = 0;
+            if (lane < per && c + lane < nx) {
+                const int x = x0 + c + lane, k = Acolx[x];
+                b0 = Browp[k];
+                int b1 = Browp[k + 1];
+                if (!whole) {  // B row k's entries in the window's columns
+                    b0 = lower_bound_i(Bcolx, b0, b1, j0 * 16);
+                    b1 = lower_bound_i(Bcolx, b0, b1, j1 * 16 + 16);
+                }
+                len = b1 - b0;
+#pragma unroll
+                for (int st = 8; st > 0; st >>= 1)
+                    if (s_rp[row + st] <= x) row += st;
+            }
+            const int rw = (row * stride - j0) / 2;  // word of column 0 in the row
+            // sets the bits of a lane's columns; those already set (most, in
+            // a hub tile-row) cost a read, which lanes of one word share
+            auto set = [&](const int (&col)[G2D_ROUNDS], const int (&rwi)[G2D_ROUNDS], int n) {
+                unsigned have[G2D_ROUNDS];
+#pragma unroll
+                for (int i = 0; i < G2D_ROUNDS; i++) have[i] = bm[rwi[i] + (col[i] >> 5)];
+#pragma unroll
+                for (int i = 0; i < G2D_ROUNDS; i++) {
+                    const unsigned bit = 1u << ((col[i] & 31) ^ 15);
+                    if (64 * i + lane < n && !(have[i] & bit)) atomicOr(&bm[rwi[i] + (col[i] >> 5)], bit);
+                }
+            };
+            // long B rows one at a time by the whole wave
+            unsigned long long lm = __ballot(len >= G2D_LONG);
+            while (lm) {
+                const int j = __ffsll((long long)lm) - 1;
+                lm &= lm - 1;
+                const int n = __builtin_amdgcn_readlane(len, j), rwj = __builtin_amdgcn_readlane(rw, j);
+                const int *bc = Bcolx + __builtin_amdgcn_readlane(b0, j);
+                int rwi[G2D_ROUNDS];
+#pragma unroll
+                for (int i = 0; i < G2D_ROUNDS; i++) rwi[i] = rwj;
+                for (int e = 0; e < n; e += G2D_BATCH) {
+                    int col[G2D_ROUNDS];
+#pragma unroll
+                    for (int i = 0; i < G2D_ROUNDS; i++) col[i] = bc[min(e + 64 * i + lane, n - 1)];
+                    set(col, rwi, n - e);
+                }
+            }
+            if (len >= G2D_LONG) len = 0;
+            const int incl = tsg_wave_incl_scan_dpp(len), pre = incl - len;
+            const int total = __builtin_amdgcn_readlane(incl, 63);
+            s_delta[lane] = b0 - pre;
+            s_row[lane] = rw;
+            int last = 0;
+            for (int base = 0; base < total; base += G2D_BATCH) {
+                reinterpret_cast<uint2 *>(s_mark)[lane] = make_uint2(0u, 0u);
+                tsg_wave_sync();
+                if (len > 0 && pre >= base && pre < base + G2D_BATCH) s_mark[pre - base] = (unsigned char)(lane + 1);
+                tsg_wave_sync();
+                int rwi[G2D_ROUNDS], col[G2D_ROUNDS];
+#pragma unroll
+                for (int i = 0; i < G2D_ROUNDS; i++) {
+                    int q = s_mark[64 * i + lane];
+                    if (__ballot(q != 0)) {
+                        q = max(last, tsg_wave_incl_max_dpp(q));
+                        last = __builtin_amdgcn_readlane(q, 63);
+                    } else {  // all of one B row
+                        q = last;
+                    }
+                    col[i] = s_delta[q - 1];
+                    rwi[i] = s_row[q - 1];
+                }
+#pragma unroll
+                for (int i = 0; i < G2D_ROUNDS; i++)  // every lane loads in bounds
+                    col[i] = Bcolx[col[i] + min(base + 64 * i + lane, total - 1)];
+                set(col, rwi, total - base);
+                tsg_wave_sync();
+            }
+        }
+        __syncthreads();
+        const unsigned short *bm16 = reinterpret_cast<const unsigned short *>(bm);
+        for (int t = tid; t < u; t += nthr) {
+            const int at = Ccol[c0 + t] - j0;
+            unsigned mk[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                mk[q] = bm16[2 * q * stride + at] | (unsigned)bm16[(2 * q + 1) * stride + at] << 16;
+            step2_store(mk, c0 + t, Cmask, Cptr16, Cnnz);
+        }
+        __syncthreads();  // the next segment clears the bits
     }
 }
 
@@ -2500,7 +2714,7 @@ static int launch_brow_bits(hipStream_t s, const tsg_dtiles *B, void *buf, const
 
 static int launch_step1(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B, tsg_dtiles *C, bool fill,
                         int words, unsigned *bmstore, const int4 *bdesc, const unsigned *bbits,
-                        const int *bany, int *rowspan = nullptr) {
+                        const int *bany, int *rowspan) {
     if (C->tilem <= 0) return TSG_OK;
     const dim3 g(tsg_div_up(C->tilem, S1_WAVES)), blk(64 * S1_WAVES);
     const bool wide = words == 2048;
@@ -2512,7 +2726,7 @@ static int launch_step1(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B,
         else
             hipLaunchKernelGGL((k_step1<true, 1024>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem,
                                B->tile_ptr, B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, C->tile_colidx,
-                               C->tile_rowidx, bmstore, (int *)nullptr);
+                               C->tile_rowidx, bmstore, rowspan);
     } else if (!fill && !wide)
         hipLaunchKernelGGL((k_step1<false, 256>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
                            B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, (int *)nullptr, (int *)nullptr, bmstore, rowspan);
@@ -2522,11 +2736,11 @@ static int launch_step1(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B,
     else if (!wide)
         hipLaunchKernelGGL((k_step1<true, 256>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
                            B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, C->tile_colidx, C->tile_rowidx, bmstore,
-                           (int *)nullptr);
+                           rowspan);
     else
         hipLaunchKernelGGL((k_step1<true, 2048>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
                            B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, C->tile_colidx, C->tile_rowidx, bmstore,
-                           (int *)nullptr);
+                           rowspan);
     TSG_LAUNCH_CHECK();
     return TSG_OK;
 }
@@ -2536,7 +2750,8 @@ struct SpgemmWork {
     long long *part1;  // scan partials: C tile pointers
     long long *part2;  // scan partials: C tile nnz
     long long *part3;  // scan partials: segment counts
-    int *segcnt;       // tilem+1 segment counts -> offsets (total at [tilem])
+    int *segcnt;       // tilem+1 step-3 segment counts -> offsets (total at [tilem])
+    int *segctr;       // S2_KINDS step-2 segment counters
     unsigned char *rowcls;
     int *cls_out;
     int *cls_part;  // k_row_class partials, 8 ints per block
@@ -2544,7 +2759,7 @@ struct SpgemmWork {
     int4 *seg2;        // step-2 segments
     unsigned *bmstore; // step-1 bitmaps kept from the count pass (may be NULL)
     int4 *seg3;        // step-3 element segments
-    long long seg2_cap, seg3_cap;
+    long long seg3_cap;
     // heavy rows (synchronous pipeline only; NULL = none)
     unsigned char *hflag;  // per C row
     int2 *hitems;          // heavy-row work items
@@ -2560,17 +2775,18 @@ static size_t up16(size_t x) { return (x + 15) & ~(size_t)15; }
 // Offsets of the work arrays inside one buffer; returns its size.  The
 // step-3 segments go last (the synchronous pipeline adds them only once
 // C's nonzero count is known).
-#define WORK_NARR 11
+#define WORK_NARR 12
 
 static size_t work_layout(long long tilem, long long numtile, long long nnz, size_t off[WORK_NARR],
                           int s1w = 256, size_t bbytes = 0) {
     const size_t sz[WORK_NARR] = {
         8 * (size_t)tsg_scan_partial_count(tilem), 8 * (size_t)tsg_scan_partial_count(numtile),
         8 * (size_t)tsg_scan_partial_count(tilem), 4 * ((size_t)tilem + 1), (size_t)tilem + 1, 32,
-        16 * (size_t)seg_bound(tilem, numtile, G2_UMAX, 0, 0),
+        16 * (size_t)seg2_bound(tilem, numtile),
         keep_bytes(tilem, s1w),  // step-1 bitmaps (enqueue-only pipeline)
         32 * (size_t)((tilem + 15) / 16 + 1),  // row-class partials, 8 ints per block
         bbytes,                                // B's tile-row bitmaps (enqueue-only pipeline)
+        4 * S2_KINDS,
         16 * (size_t)(tilem + nnz / (G3E_NNZ - 255) + 2)};
     size_t o = 0;
     for (int i = 0; i < WORK_NARR; i++) {
@@ -2596,8 +2812,8 @@ static SpgemmWork work_at(void *base, long long tilem, long long numtile, long l
     w.bmstore = keep_bytes(tilem, s1w) ? (unsigned *)(b + off[7]) : nullptr;
     w.cls_part = (int *)(b + off[8]);
     w.bbits = bbytes ? (void *)(b + off[9]) : nullptr;
-    w.seg3 = (int4 *)(seg3_base ? (char *)seg3_base : b + off[10]);
-    w.seg2_cap = seg_bound(tilem, numtile, G2_UMAX, 0, 0);
+    w.segctr = (int *)(b + off[10]);
+    w.seg3 = (int4 *)(seg3_base ? (char *)seg3_base : b + off[11]);
     w.seg3_cap = tilem + nnz / (G3E_NNZ - 255) + 2;
     w.hflag = nullptr;
     w.hitems = nullptr;
@@ -2609,27 +2825,19 @@ static SpgemmWork work_at(void *base, long long tilem, long long numtile, long l
     return w;
 }
 
-// Segments of the selected tile-rows into items; the count lands in
-// w.segcnt[tilem].
-template <int MODE>
-static int launch_segments(hipStream_t s, const tsg_dtiles *C, const SpgemmWork &w, int want, int max_tiles,
-                           int max_nnz, int4 *items, const unsigned char *cls, long long cap = 0) {
-    const unsigned g = tsg_div_up(C->tilem, 256);
-    hipLaunchKernelGGL(k_seg<MODE>, dim3(g), dim3(256), 0, s, C->tile_ptr, C->tile_nnz, C->tilem, cls, want,
-                       max_tiles, max_nnz, w.segcnt, (int4 *)nullptr);
+// Step-3 element segments of the tile-rows of class `want` into w.seg3 (cap
+// = its capacity, at least the count); the count lands in w.segcnt[tilem].
+static int launch_segments(hipStream_t s, const tsg_dtiles *C, const SpgemmWork &w, int want, int max_nnz,
+                           const unsigned char *cls) {
+    hipLaunchKernelGGL(k_seg1_count, dim3(tsg_div_up(C->tilem, 256)), dim3(256), 0, s, C->tile_ptr, C->tile_nnz,
+                       C->tilem, cls, want, max_nnz, w.segcnt);
     TSG_LAUNCH_CHECK();
     TSG_TRY(tsg_scan_i32_enqueue(s, w.segcnt, w.segcnt, C->tilem, w.part3));
-    if (MODE == 1) {  // one thread per segment, cap = the segment array's capacity (>= the count)
-        if (cap > 0) {
-            hipLaunchKernelGGL(k_seg1_fill, dim3((unsigned)tsg_div_up(cap, 256)), dim3(256), 0, s, C->tile_ptr,
-                               C->tile_nnz, C->tilem, (const int *)w.segcnt, max_nnz, items);
-            TSG_LAUNCH_CHECK();
-        }
-        return TSG_OK;
+    if (w.seg3_cap > 0) {
+        hipLaunchKernelGGL(k_seg1_fill, dim3((unsigned)tsg_div_up(w.seg3_cap, 256)), dim3(256), 0, s, C->tile_ptr,
+                           C->tile_nnz, C->tilem, (const int *)w.segcnt, max_nnz, w.seg3);
+        TSG_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(k_seg<MODE>, dim3(g), dim3(256), 0, s, C->tile_ptr, C->tile_nnz, C->tilem, cls, want,
-                       max_tiles, max_nnz, w.segcnt, items);
-    TSG_LAUNCH_CHECK();
     return TSG_OK;
 }
 
@@ -2643,22 +2851,40 @@ static int launch_step2(hipStream_t s, const TileOperands &op, const tsg_dtiles 
         TSG_LAUNCH_CHECK();
         return TSG_OK;
     }
-    if (P.s3_elem) {  // B has its row index: element-wise symbolic for hypersparse tile-rows
-        hipLaunchKernelGGL(k_step2_kind, dim3(tsg_div_up(C->tilem, 256)), dim3(256), 0, s, op.Aptr, op.Annz,
-                           C->tilem, P.elem_all, w.rowcls);
+    const int *n2 = P.n2;
+    // only tile-row-long tile-pair segments: no list
+    const bool list = n2[1] || n2[2] || n2[3] || P.s2u >= G2_UMAX;
+    const int4 base = make_int4(0, n2[0], n2[0] + n2[1], n2[0] + n2[1] + n2[2]);
+    if (list) {
+        hipLaunchKernelGGL(k_seg2_fill, dim3(tsg_div_up(C->tilem, 256)), dim3(256), 0, s, C->tile_ptr, C->tile_colidx,
+                           op.Aptr, op.Annz, C->tilem, P.s3_elem, P.elem_all, op.Arowp ? 1 : 0, base, w.segctr, w.seg2);
         TSG_LAUNCH_CHECK();
     }
-    TSG_TRY(launch_segments<0>(s, C, w, -1, G2_UMAX, 0, w.seg2, P.s3_elem ? w.rowcls : nullptr));
-    const int s2u = P.s2u > 0 ? P.s2u : G2_UMAX;
-    const size_t lds2 = (4 * G2_MSTRIDE + 4) * (size_t)s2u + (((size_t)P.s2map + 15) & ~(size_t)15);
-    hipLaunchKernelGGL(k_step2_rows, dim3((unsigned)w.seg2_cap), dim3(G2_THREADS), lds2, s, op, (const int4 *)w.seg2,
-                       (const int *)(w.segcnt + C->tilem), C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
-                       C->tile_nnz, s2u, P.s2map);
-    TSG_LAUNCH_CHECK();
-    if (P.s3_elem) {
-        hipLaunchKernelGGL(k_step2_elem, dim3((unsigned)w.seg2_cap), dim3(G2_THREADS), 0, s, op, (const int *)B->rowx_ptr,
-                           (const int *)B->rowx_col, (const int4 *)w.seg2, (const int *)(w.segcnt + C->tilem),
-                           C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr, C->tile_nnz);
+    if (n2[0] > 0) {
+        const int s2u = P.s2u > 0 ? P.s2u : G2_UMAX;
+        const size_t lds2 = (4 * G2_MSTRIDE + 4) * (size_t)s2u + (((size_t)P.s2map + 15) & ~(size_t)15);
+        hipLaunchKernelGGL(k_step2_rows, dim3((unsigned)(list ? n2[0] : C->tilem)), dim3(G2_THREADS), lds2, s, op,
+                           list ? (const int4 *)w.seg2 : (const int4 *)nullptr, C->tile_ptr, C->tile_colidx, C->mask,
+                           C->csr_ptr, C->tile_nnz, s2u, P.s2map);
+        TSG_LAUNCH_CHECK();
+    }
+    if (n2[1] > 0) {
+        hipLaunchKernelGGL(k_step2_elem, dim3((unsigned)n2[1]), dim3(G2_THREADS), 0, s, op, (const int *)B->rowx_ptr,
+                           (const int *)B->rowx_col, (const int4 *)(w.seg2 + base.y), C->tile_ptr, C->tile_colidx,
+                           C->mask, C->csr_ptr, C->tile_nnz);
+        TSG_LAUNCH_CHECK();
+    }
+    for (int k = 2; k < 4; k++) {
+        if (n2[k] <= 0) continue;
+        const int width = k == 2 ? P.s2w : G2D_WIN;
+        const int threads = k == 2 ? 256 : 1024;
+        const size_t lds = g2d_lds(width, threads);
+        // kind 3: a few blocks per CU take the windows in turn (one at a time fits)
+        const unsigned grid = k == 2 ? (unsigned)n2[k] : (unsigned)std::min(n2[k], 4096);
+        hipLaunchKernelGGL(k_step2_dense, dim3(grid), dim3(threads), lds, s, op.Arowp, op.Acolx, C->m,
+                           (const int *)B->rowx_ptr, (const int *)B->rowx_col,
+                           (const int4 *)(w.seg2 + (k == 2 ? base.z : base.w)), n2[k], C->tile_ptr, C->tile_colidx,
+                           C->mask, C->csr_ptr, C->tile_nnz, width);
         TSG_LAUNCH_CHECK();
     }
     return TSG_OK;
@@ -2692,7 +2918,7 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
         if (ev) TSG_HIP(hipEventRecord(ev[1], s));
     }
     if (!P.all && P.s3_unfit && P.s3_elem) {
-        TSG_TRY(launch_segments<1>(s, C, w, 0, 0x7fffffff, G3E_NNZ, w.seg3, w.rowcls, w.seg3_cap));
+        TSG_TRY(launch_segments(s, C, w, 0, G3E_NNZ, w.rowcls));
         const bool rx = op.Arowp != nullptr;
         hipLaunchKernelGGL(P.s3pk ? (rx ? k_step3_elem<true, true> : k_step3_elem<true, false>)
                                   : (rx ? k_step3_elem<false, true> : k_step3_elem<false, false>),
@@ -2797,12 +3023,12 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     P.s1w = tsg_s1_words(B, tune);
     const size_t kb = keep_bytes(C->tilem, P.s1w);
     if (kb) TSG_TRY(tsg_alloc(ctx, (void **)&T.keep, kb));
-    TSG_TRY(tsg_alloc(ctx, &T.scr, 64));
+    TSG_TRY(tsg_alloc(ctx, &T.scr, 128));
     void *scr = T.scr;
     unsigned long long *bins = (unsigned long long *)scr;
-    int *st2 = reinterpret_cast<int *>(static_cast<char *>(scr) + 32);  // step-2 sizing maxima
-    int *bany = reinterpret_cast<int *>(static_cast<char *>(scr) + 48);  // some B tile-row bitmap kept
-    TSG_HIP(hipMemsetAsync(scr, 0, 64, s));
+    int *bany = reinterpret_cast<int *>(static_cast<char *>(scr) + 32);  // some B tile-row bitmap kept
+    int *st2 = reinterpret_cast<int *>(static_cast<char *>(scr) + 64);   // k_row_stats
+    TSG_HIP(hipMemsetAsync(scr, 0, 128, s));
     TSG_TRY(tsg_alloc_t(ctx, &T.span, (size_t)C->tilem + 1));
     const int4 *bdesc = nullptr;
     const unsigned *bbits = nullptr;
@@ -2813,15 +3039,16 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     TSG_TRY(launch_step1(s, A, B, C, false, P.s1w, T.keep, bdesc, bbits, bany, T.span));
     if (C->tilem > 0) {
         hipLaunchKernelGGL(k_row_stats, dim3(std::min<unsigned>(ROW_STATS_BLOCKS, tsg_div_up(C->tilem, 1024))),
-                           dim3(1024), 0, s, (const int *)C->tile_ptr, (const int *)T.span, C->tilem, st2);
+                           dim3(1024), 0, s, (const int *)C->tile_ptr, (const int *)T.span, A->tile_ptr, A->tile_nnz,
+                           C->tilem, P.s3_elem, P.elem_all, A->rowx_ptr ? 1 : 0, st2);
         TSG_LAUNCH_CHECK();
     }
     // C's tile-row offsets; their total and the step-2 sizing maxima come
     // back in one read-back
     long long numtileC = 0;
-    int smax[4] = {0, 0, 0, 0};
+    int smax[ROW_STATS] = {};
     {
-        TSG_TRY(tsg_scan_i32(ctx, C->tile_ptr, C->tile_ptr, C->tilem, &numtileC, st2, 4));
+        TSG_TRY(tsg_scan_i32(ctx, C->tile_ptr, C->tile_ptr, C->tilem, &numtileC, st2, ROW_STATS));
         memcpy(smax, ctx->pinned + 1, sizeof(smax));
     }
     tsg_free(ctx, T.span);
@@ -2835,7 +3062,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     (void)wbytes;
     void *wbuf = T.wbuf;
     SpgemmWork w = work_at(wbuf, C->tilem, numtileC, 0, nullptr);
-    TSG_TRY(launch_step1(s, A, B, C, true, P.s1w, T.keep, bdesc, bbits, bany));
+    TSG_TRY(launch_step1(s, A, B, C, true, P.s1w, T.keep, bdesc, bbits, bany, w.segctr));
     tsg_free(ctx, T.keep);
     T.keep = nullptr;
     tsg_free(ctx, T.bb);
@@ -2849,6 +3076,8 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         P.s2u = std::max(1, umax);
         P.s2map = umax <= 256 ? mspan : 0;
         P.s3pk = span < G3E_PK_SPAN ? 1 : 0;
+        for (int k = 0; k < S2_KINDS; k++) P.n2[k] = smax[3 + k];
+        P.s2w = smax[7];
     }
     // ---- step 2
     const TileOperands op = make_operands(A, B);
@@ -3000,9 +3229,9 @@ int tsg_spgemm_enqueue(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B, 
     const int4 *bdesc = nullptr;
     const unsigned *bbits = nullptr;
     if (C->tilem > 0) TSG_TRY(launch_brow_bits(s, B, w.bbits, &bdesc, &bbits, nullptr));
-    TSG_TRY(launch_step1(s, A, B, C, false, P.s1w, w.bmstore, bdesc, bbits, nullptr));
+    TSG_TRY(launch_step1(s, A, B, C, false, P.s1w, w.bmstore, bdesc, bbits, nullptr, nullptr));
     TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_ptr, C->tile_ptr, C->tilem, w.part1));
-    TSG_TRY(launch_step1(s, A, B, C, true, P.s1w, w.bmstore, bdesc, bbits, nullptr));
+    TSG_TRY(launch_step1(s, A, B, C, true, P.s1w, w.bmstore, bdesc, bbits, nullptr, w.segctr));
     const TileOperands op = make_operands(A, B);
     TSG_TRY(launch_step2(s, op, B, C, P, w));
     TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_nnz, C->tile_nnz, C->numtile, w.part2));

@@ -143,6 +143,8 @@ struct tsg_spgemm_plan {
     int s1w;        // step-1 bitmap window, 32-bit words per wave
     int s2u;        // most C tiles of a step-2 tile-pair segment (LDS sizing)
     int s2map;      // bytes of the step-2 column -> slot map (0: binary search)
+    int n2[4];      // step-2 segments per kernel (step2_kind)
+    int s2w;        // widest tile-row span of the dense step 2's small blocks
     int s3pk;       // element step 3 packs hash keys and positions (narrow tile-rows)
 };
 // symbolic = true runs steps 1-2 and the step-3 plan only (C's values and
