@@ -555,9 +555,28 @@ __global__ void k_iota(int *v, long long n) {
     long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i < n) v[i] = (int)i;
 }
-__global__ void k_count_keys(const int *__restrict__ k, long long n, int *__restrict__ cnt) {
-    long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) atomicAdd(&cnt[k[i]], 1);
+// keys[i] = src[i], idx[i] = i: the input of a sort by src.
+__global__ void __launch_bounds__(256)
+k_sort_input(const int *__restrict__ src, long long n, unsigned *__restrict__ keys, int *__restrict__ idx) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) {
+        keys[i] = (unsigned)src[i];
+        idx[i] = (int)i;
+    }
+}
+// ptr[j] = first position of a key >= j in the sorted keys, j = 0..ncol.  A
+// search per pointer: counting the keys instead met one atomic per entry of
+// a hub column on one address (R-MAT scale 18: 648 us against 13).
+__global__ void __launch_bounds__(256)
+k_ptr_of_sorted(const unsigned *__restrict__ keys, long long n, int ncol, int *__restrict__ ptr) {
+    const long long j = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (j > ncol) return;
+    long long lo = 0, hi = n;
+    while (lo < hi) {
+        const long long mid = (lo + hi) >> 1;
+        if (keys[mid] < (unsigned)j) lo = mid + 1; else hi = mid;
+    }
+    ptr[j] = (int)lo;
 }
 __global__ void k_gather_i32(const int *__restrict__ src, const int *__restrict__ idx, long long n, int *__restrict__ dst) {
     long long i = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -567,13 +586,14 @@ __global__ void k_scatter_i32(const int *__restrict__ src, const int *__restrict
     long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i < n) dst[idx[i]] = src[i];
 }
-__global__ void k_gather_f64(const double *__restrict__ src, const int *__restrict__ idx, long long n, double *__restrict__ dst) {
+__global__ void k_gather_entries(const int *__restrict__ src, const double *__restrict__ val, const int *__restrict__ idx,
+                                 long long n, int *__restrict__ dst, double *__restrict__ oval) {
     long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) dst[i] = src[idx[i]];
-}
-__global__ void k_u32_from_i32(const int *__restrict__ src, long long n, unsigned *__restrict__ dst) {
-    long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) dst[i] = (unsigned)src[i];
+    if (i < n) {
+        const int e = idx[i];
+        dst[i] = src[e];
+        oval[i] = val[e];
+    }
 }
 
 static int bits_for(long long v) {
@@ -588,21 +608,21 @@ extern "C" int tsg_tiles_build_csc(tsg_ctx *ctx, tsg_dtiles *t) {
     TSG_TRY(tsg_alloc_t(ctx, &t->csc_ptr, (size_t)t->tilen + 1));
     TSG_TRY(tsg_alloc_t(ctx, &t->csc_rowidx, (size_t)nt + 1));
     TSG_TRY(tsg_alloc_t(ctx, &t->csc_tileid, (size_t)nt + 1));
-    TSG_HIP(hipMemsetAsync(t->csc_ptr, 0, ((size_t)t->tilen + 1) * 4, ctx->stream));
+    unsigned *keys = nullptr;
     if (nt > 0) {
-        unsigned *keys;
         TSG_TRY(tsg_alloc_t(ctx, &keys, (size_t)nt));
-        hipLaunchKernelGGL(k_u32_from_i32, dim3(tsg_div_up(nt, 256)), dim3(256), 0, ctx->stream, t->tile_colidx, nt, keys);
-        hipLaunchKernelGGL(k_iota, dim3(tsg_div_up(nt, 256)), dim3(256), 0, ctx->stream, t->csc_tileid, nt);
-        hipLaunchKernelGGL(k_count_keys, dim3(tsg_div_up(nt, 256)), dim3(256), 0, ctx->stream, t->tile_colidx, nt, t->csc_ptr);
+        hipLaunchKernelGGL(k_sort_input, dim3(tsg_div_up(nt, 256)), dim3(256), 0, ctx->stream, t->tile_colidx, nt, keys,
+                           t->csc_tileid);
         TSG_LAUNCH_CHECK();
         TSG_TRY(tsg_sort_pairs_u32(ctx, keys, t->csc_tileid, nt, bits_for(t->tilen)));
         hipLaunchKernelGGL(k_gather_i32, dim3(tsg_div_up(nt, 256)), dim3(256), 0, ctx->stream, t->tile_rowidx,
                            t->csc_tileid, nt, t->csc_rowidx);
         TSG_LAUNCH_CHECK();
-        tsg_free(ctx, keys);
     }
-    TSG_TRY(tsg_scan_i32(ctx, t->csc_ptr, t->csc_ptr, t->tilen, nullptr));
+    hipLaunchKernelGGL(k_ptr_of_sorted, dim3(tsg_div_up((long long)t->tilen + 1, 256)), dim3(256), 0, ctx->stream,
+                       (const unsigned *)keys, nt, t->tilen, t->csc_ptr);
+    TSG_LAUNCH_CHECK();
+    tsg_free(ctx, keys);
     return TSG_OK;
 }
 
@@ -1203,10 +1223,43 @@ extern "C" void tsg_htiles_free(tsg_htiles *h) {
 }
 
 // ---------------------------------------------------------------- transpose
-__global__ void k_row_of_entry(const int *__restrict__ rowptr, int m, int *__restrict__ rowid) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    for (int e = rowptr[i]; e < rowptr[i + 1]; e++) rowid[e] = i;
+// The row of every entry, VAL_BLOCK entries per block: each row start of the
+// block marks its entry in LDS and the marks' running maximum is the row.
+// Entry parallel, so a hub row is not one lane's loop (R-MAT scale 18: 848 ->
+// 32 us).
+__global__ void __launch_bounds__(256)
+k_row_of_entry(const int *__restrict__ rowptr, int m, int nnz, int *__restrict__ rowid) {
+    __shared__ int s_row[VAL_BLOCK];  // row + 1 at a row's first entry
+    __shared__ int s_lo[2], s_max[4];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int e0 = blockIdx.x * VAL_BLOCK, ne = min(VAL_BLOCK, nnz - e0);
+    for (int i = tid; i < VAL_BLOCK; i += 256) s_row[i] = 0;
+    if (wave < 2) {
+        const int i = wave_first_ge(rowptr, 0, m + 1, wave ? e0 + ne : e0);
+        if (lane == 0) s_lo[wave] = i;
+    }
+    __syncthreads();
+    const int lo = s_lo[0], hi = s_lo[1];  // rows starting in the block
+    if (hi - lo > VAL_MARK_ROWS) {         // mostly empty rows: a search per entry
+        for (int x = tid; x < ne; x += 256) rowid[e0 + x] = first_ge(rowptr, 0, m + 1, e0 + x + 1) - 1;
+        return;  // block-uniform
+    }
+    // of rows starting at one entry the last has it
+    for (int i = lo + tid; i < hi; i += 256) atomicMax(&s_row[rowptr[i] - e0], i + 1);
+    __syncthreads();
+    int mx = 0;
+    for (int k = 0; k < VAL_BLOCK / 256; k++) mx = max(mx, s_row[wave * (VAL_BLOCK / 4) + 64 * k + lane]);
+    mx = tsg_wave_max(mx);
+    if (lane == 0) s_max[wave] = mx;
+    __syncthreads();
+    int last = lo;  // row lo - 1 holds the entries before the block's first row start
+    for (int w = 0; w < wave; w++) last = max(last, s_max[w]);
+    for (int k = 0; k < VAL_BLOCK / 256; k++) {
+        const int x = wave * (VAL_BLOCK / 4) + 64 * k + lane;
+        const int r = max(last, tsg_wave_incl_max_dpp(s_row[x]));
+        last = __builtin_amdgcn_readlane(r, 63);
+        if (x < ne) rowid[e0 + x] = r - 1;
+    }
 }
 
 // Stable CSR -> CSC (src/utils.h:158-195): a stable sort of the entries by
@@ -1221,28 +1274,28 @@ extern "C" int tsg_dcsr_transpose(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dcsr *at)
     TSG_TRY(tsg_alloc_t(ctx, &at->rowptr, (size_t)a->n + 1));
     TSG_TRY(tsg_alloc_t(ctx, &at->colidx, (size_t)nnz + 1));
     TSG_TRY(tsg_alloc_t(ctx, &at->val, (size_t)nnz + 1));
-    TSG_HIP(hipMemsetAsync(at->rowptr, 0, ((size_t)a->n + 1) * 4, ctx->stream));
+    unsigned *keys = nullptr;
     if (nnz > 0) {
-        unsigned *keys;
         int *perm, *rowid;
         TSG_TRY(tsg_alloc_t(ctx, &keys, (size_t)nnz));
         TSG_TRY(tsg_alloc_t(ctx, &perm, (size_t)nnz));
         TSG_TRY(tsg_alloc_t(ctx, &rowid, (size_t)nnz));
         const unsigned g = tsg_div_up(nnz, 256);
-        hipLaunchKernelGGL(k_u32_from_i32, dim3(g), dim3(256), 0, ctx->stream, a->colidx, nnz, keys);
-        hipLaunchKernelGGL(k_iota, dim3(g), dim3(256), 0, ctx->stream, perm, nnz);
-        hipLaunchKernelGGL(k_count_keys, dim3(g), dim3(256), 0, ctx->stream, a->colidx, nnz, at->rowptr);
-        hipLaunchKernelGGL(k_row_of_entry, dim3(tsg_div_up(a->m, 256)), dim3(256), 0, ctx->stream, a->rowptr, a->m, rowid);
+        hipLaunchKernelGGL(k_sort_input, dim3(g), dim3(256), 0, ctx->stream, a->colidx, nnz, keys, perm);
+        hipLaunchKernelGGL(k_row_of_entry, dim3(tsg_div_up(nnz, VAL_BLOCK)), dim3(256), 0, ctx->stream, a->rowptr, a->m,
+                           a->nnz, rowid);
         TSG_LAUNCH_CHECK();
         TSG_TRY(tsg_sort_pairs_u32(ctx, keys, perm, nnz, bits_for(a->n)));
-        hipLaunchKernelGGL(k_gather_i32, dim3(g), dim3(256), 0, ctx->stream, rowid, perm, nnz, at->colidx);
-        hipLaunchKernelGGL(k_gather_f64, dim3(g), dim3(256), 0, ctx->stream, a->val, perm, nnz, at->val);
+        hipLaunchKernelGGL(k_gather_entries, dim3(g), dim3(256), 0, ctx->stream, rowid, a->val, perm, nnz, at->colidx,
+                           at->val);
         TSG_LAUNCH_CHECK();
-        tsg_free(ctx, keys);
         tsg_free(ctx, perm);
         tsg_free(ctx, rowid);
     }
-    TSG_TRY(tsg_scan_i32(ctx, at->rowptr, at->rowptr, a->n, nullptr));
+    hipLaunchKernelGGL(k_ptr_of_sorted, dim3(tsg_div_up((long long)a->n + 1, 256)), dim3(256), 0, ctx->stream,
+                       (const unsigned *)keys, nnz, a->n, at->rowptr);
+    TSG_LAUNCH_CHECK();
+    tsg_free(ctx, keys);
     return TSG_OK;
 }
 

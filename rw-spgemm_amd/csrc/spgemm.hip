@@ -1654,22 +1654,30 @@ k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
 #define HEAVY_CURSOR_BYTES (512ll << 20)
 
 // Per C row of an element-wise tile-row: heavy flag and work items (runs of
-// parts); info[0] = longest heavy A row, info[1] = heavy rows.
+// parts); info[0] = longest heavy A row, info[1] = heavy rows.  16 lanes per
+// row, so that a long A row's B row lengths are not one lane's chain of
+// loads (R-MAT scale 16: 665 -> 92 us).
 __global__ void __launch_bounds__(256)
 k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const int *__restrict__ Browp,
               const unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
               int m, long long min_products, long long item_products, unsigned char *__restrict__ flag,
               int *__restrict__ cnt, int *__restrict__ info) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int i = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15;
+    if (i >= m) return;
     int h = 0, items = 0;
-    if (i < m && rowcls[i >> 4] == 0) {
+    if (rowcls[i >> 4] == 0) {  // uniform in the 16 lanes, as everything below
         const int x0 = Arowp[i], x1 = Arowp[i + 1];
         long long p = -1;  // unknown for long A rows
         if (x1 - x0 > 2048) {
             h = 1;
         } else {
             p = 0;
-            for (int x = x0; x < x1; x++) p += Browp[Acolx[x] + 1] - Browp[Acolx[x]];
+#pragma unroll 4
+            for (int x = x0 + l; x < x1; x += 16) {
+                const int k = Acolx[x];
+                p += Browp[k + 1] - Browp[k];
+            }
+            p = tsg_group16_sum(p);
             h = p > min_products;
         }
         if (h) {
@@ -1678,11 +1686,13 @@ k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
             const int nparts = (int)((span + HEAVY_PART_COLS - 1) / HEAVY_PART_COLS);
             items = p < 0 ? nparts
                           : (int)min<long long>(nparts, max<long long>(1, (p + item_products - 1) / item_products));
-            atomicMax(&info[0], x1 - x0);
-            atomicAdd(&info[1], 1);
+            if (l == 0) {
+                atomicMax(&info[0], x1 - x0);
+                atomicAdd(&info[1], 1);
+            }
         }
     }
-    if (i < m) {
+    if (l == 0) {
         flag[i] = (unsigned char)h;
         cnt[i] = items;
     }
@@ -3138,7 +3148,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                 unsigned char *hflag = T.hflag;
                 int *hcnt = T.hcnt, *hinfo = T.hinfo;
                 TSG_HIP(hipMemsetAsync(hinfo, 0, 16, s));
-                hipLaunchKernelGGL(k_heavy_flags, dim3(tsg_div_up(m, 256)), dim3(256), 0, s, op.Arowp, op.Acolx,
+                hipLaunchKernelGGL(k_heavy_flags, dim3(tsg_div_up(m, 16)), dim3(256), 0, s, op.Arowp, op.Acolx,
                                    (const int *)B->rowx_ptr, (const unsigned char *)w.rowcls, C->tile_ptr,
                                    C->tile_colidx, m,
                                    (long long)(tune.heavy_min_products > 0 ? tune.heavy_min_products
