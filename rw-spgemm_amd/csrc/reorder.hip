@@ -76,11 +76,19 @@ __global__ void k_mirror_deg(const int *__restrict__ rowptr, const int *__restri
     for (int e = rowptr[i]; e < rowptr[i + 1]; e++)
         if (col[e] != i) atomicAdd(&deg[col[e]], 1);
 }
-__global__ void k_max_i32(const int *__restrict__ v, int n, int *__restrict__ out) {
+// (few large blocks: the atomics on one address are what this costs)
+__global__ void __launch_bounds__(1024)
+k_max_i32(const int *__restrict__ v, int n, int *__restrict__ out) {
+    __shared__ int s_m[16];
     int mx = 0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) mx = max(mx, v[i]);
+    for (int i = blockIdx.x * 1024 + threadIdx.x; i < n; i += gridDim.x * 1024) mx = max(mx, v[i]);
     mx = tsg_wave_max(mx);
-    if ((threadIdx.x & 63) == 0) atomicMax(out, mx);
+    if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) mx = max(mx, s_m[w]);
+        atomicMax(out, mx);
+    }
 }
 __global__ void k_deg_key(const int *__restrict__ deg, int n, int maxdeg, int descending, unsigned *__restrict__ key) {
     int i = blockIdx.x * 256 + threadIdx.x;
@@ -92,7 +100,7 @@ static int max_of(tsg_ctx *ctx, const int *v, int n, int *out) {
     TSG_TRY(tsg_scratch(ctx, 64, &scr));
     TSG_HIP(hipMemsetAsync(scr, 0, 4, ctx->stream));
     if (n > 0) {
-        hipLaunchKernelGGL(k_max_i32, dim3(std::min<unsigned>(1024, tsg_div_up(n, 256))), dim3(256), 0, ctx->stream, v, n,
+        hipLaunchKernelGGL(k_max_i32, dim3(std::min<unsigned>(64, tsg_div_up(n, 1024))), dim3(1024), 0, ctx->stream, v, n,
                            (int *)scr);
         TSG_LAUNCH_CHECK();
     }
@@ -170,23 +178,58 @@ __global__ void k_fill_f64(double *v, long long n, double x) {
     if (i < n) v[i] = x;
 }
 
+// First index in [lo, hi) with list[index] >= key.
+__device__ __forceinline__ int lower_bound_r(const int *__restrict__ list, int lo, int hi, int key) {
+    while (lo < hi) {
+        const int mid = (int)(((unsigned)lo + (unsigned)hi) >> 1);
+        if (list[mid] < key) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+}
+
+// Union of two sorted rows, 16 lanes per row: an entry's place is its index
+// plus the other row's smaller entries, less those of both rows before it.
+// (One thread merging a row: 27-point mesh of 230k rows 357 -> 87 us.)
 template <bool FILL>
 __global__ void __launch_bounds__(256)
 k_union_rows(int m, const int *__restrict__ ap, const int *__restrict__ ac, const int *__restrict__ tp,
              const int *__restrict__ tc, int *__restrict__ cnt_or_ptr, int *__restrict__ gc) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    int a = ap[i], ae = ap[i + 1], b = tp[i], be = tp[i + 1];
-    int out = FILL ? cnt_or_ptr[i] : 0;
-    while (a < ae || b < be) {
-        int v;
-        if (b >= be || (a < ae && ac[a] < tc[b])) v = ac[a++];
-        else if (a >= ae || tc[b] < ac[a]) v = tc[b++];
-        else { v = ac[a]; a++; b++; }
-        if (FILL) gc[out] = v;
-        out++;
+    const int i = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15, gb = threadIdx.x & 48;
+    if (i >= m) return;  // whole groups
+    const int a0 = ap[i], a1 = ap[i + 1], b0 = tp[i], b1 = tp[i + 1];
+    const int out = FILL ? cnt_or_ptr[i] : 0;
+    int both = 0;  // entries of both rows so far
+    for (int e0 = a0; e0 < a1; e0 += 16) {
+        const int e = e0 + l;
+        bool dup = false;
+        int x = 0, at = 0;
+        if (e < a1) {
+            x = ac[e];
+            at = lower_bound_r(tc, b0, b1, x);
+            dup = at < b1 && tc[at] == x;
+        }
+        const unsigned d = (unsigned)(__ballot(dup) >> gb) & 0xffffu;
+        if (FILL && e < a1) gc[out + (e - a0) + (at - b0) - both - __popc(d & ((1u << l) - 1u))] = x;
+        both += __popc(d);
     }
-    if (!FILL) cnt_or_ptr[i] = out;
+    if (!FILL) {
+        if (l == 0) cnt_or_ptr[i] = (a1 - a0) + (b1 - b0) - both;
+        return;
+    }
+    both = 0;
+    for (int e0 = b0; e0 < b1; e0 += 16) {  // entries of the second row alone
+        const int e = e0 + l;
+        bool dup = false;
+        int x = 0, at = 0;
+        if (e < b1) {
+            x = tc[e];
+            at = lower_bound_r(ac, a0, a1, x);
+            dup = at < a1 && ac[at] == x;
+        }
+        const unsigned d = (unsigned)(__ballot(dup) >> gb) & 0xffffu;
+        if (e < b1 && !dup) gc[out + (e - b0) + (at - a0) - both - __popc(d & ((1u << l) - 1u))] = x;
+        both += __popc(d);
+    }
 }
 
 // pattern(A + A^T), sorted rows, self loops kept
@@ -197,7 +240,7 @@ extern "C" int tsg_dcsr_symmetrize(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dcsr *g)
     TSG_TRY(tsg_dcsr_transpose(ctx, a, &at));
     g->m = g->n = a->m;
     TSG_TRY(tsg_alloc_t(ctx, &g->rowptr, (size_t)a->m + 1));
-    const unsigned gr = tsg_div_up(a->m, 256);
+    const unsigned gr = tsg_div_up(a->m, 16);
     if (a->m > 0) {
         hipLaunchKernelGGL(k_union_rows<false>, dim3(gr), dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
                            at.rowptr, at.colidx, g->rowptr, (int *)nullptr);
@@ -223,40 +266,83 @@ extern "C" int tsg_dcsr_symmetrize(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dcsr *g)
 __global__ void k_rcm_deg(const int *__restrict__ gp, const int *__restrict__ gc, int n, int *__restrict__ deg) {
     int v = blockIdx.x * 256 + threadIdx.x;
     if (v >= n) return;
-    int d = gp[v + 1] - gp[v];
-    for (int e = gp[v]; e < gp[v + 1]; e++)
-        if (gc[e] == v) { d++; break; }
-    deg[v] = d;
+    const int e1 = gp[v + 1];
+    const int e = lower_bound_r(gc, gp[v], e1, v);
+    deg[v] = e1 - gp[v] + (e < e1 && gc[e] == v);
 }
-__global__ void k_scatter_rank(const int *__restrict__ order, int n, int *__restrict__ rank, int *__restrict__ label) {
+__global__ void k_scatter_rank(const int *__restrict__ order, int n, int *__restrict__ rank) {
     int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= n) return;
-    rank[order[r]] = r;
-    label[order[r]] = r;
+    if (r < n) rank[order[r]] = r;
 }
-// label <- min label over the closed neighbourhood, then pointer jumping
-// through the vertex that owns the label (labels only decrease).
-__global__ void k_cc_prop(const int *__restrict__ gp, const int *__restrict__ gc, int n, int *label, int *changed) {
-    int v = blockIdx.x * 256 + threadIdx.x;
+// Connected components as a forest over the ranks whose parents only ever get
+// smaller, so a component's root ends as its lowest rank whatever order the
+// edges are taken in.  CC_ROUNDS rounds hook every vertex, then every tree, to
+// the lowest rank next to it (a minimum, no retries) and flatten the forest;
+// a last pass joins what is left, root to root by compare-and-swap, and is
+// what the result rests on.  No read-back in between.  Label propagation with
+// pointer jumping took 26 rounds with a read-back each on a shuffled 27-point
+// mesh (27d 61x64x59; 1.5 ms of kernels), the last pass alone 2.9 ms (every
+// tree's root swapped at once), after 3 / 4 / 5 rounds 0.97 / 0.48 / 0.33 ms.
+#define CC_ROUNDS 5
+// Parents are read past the caches of the other XCDs; an older parent is
+// still an ancestor, and a failed swap returns the current one, so every
+// step moves down.
+__device__ __forceinline__ int cc_load(const int *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int cc_root(const int *parent, int x) {
+    int p = cc_load(&parent[x]);
+    while (p != x) {  // p < x
+        const int g = cc_load(&parent[p]);
+        x = p;
+        p = g;
+    }
+    return x;
+}
+#define VERT_LANES 16  // lanes per vertex of the kernels that walk adjacency lists
+// FIRST: parent of each vertex = the lowest rank among itself and its
+// neighbours.  Else: the parent of its tree's root, label[v], lowered to the
+// lowest label next to it.
+template <bool FIRST>
+__global__ void __launch_bounds__(256)
+k_cc_hook(const int *__restrict__ gp, const int *__restrict__ gc, int n, const int *__restrict__ id, int *parent) {
+    const int v = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VERT_LANES), l = threadIdx.x % VERT_LANES;
     if (v >= n) return;
-    int l = label[v];
-    const int l0 = l;
-    for (int e = gp[v]; e < gp[v + 1]; e++) l = min(l, label[gc[e]]);
-    if (l < l0) {
-        atomicMin(&label[v], l);
-        *changed = 1;
+    const int iv = id[v], e1 = gp[v + 1];
+    int mn = iv;
+    for (int e = gp[v] + l; e < e1; e += VERT_LANES) mn = min(mn, id[gc[e]]);
+#pragma unroll
+    for (int o = VERT_LANES / 2; o > 0; o >>= 1) mn = min(mn, __shfl_xor(mn, o, VERT_LANES));
+    if (l == 0) {
+        if (FIRST) parent[iv] = mn;
+        else if (mn < iv && mn < cc_load(&parent[iv])) atomicMin(&parent[iv], mn);  // few trees: one address for many
     }
 }
-__global__ void k_cc_jump(const int *__restrict__ order, int n, int *label) {
-    int v = blockIdx.x * 256 + threadIdx.x;
+// label[v] = root of v's tree, and v's parent set to it.
+__global__ void __launch_bounds__(256)
+k_cc_label(const int *__restrict__ rank, int n, int *parent, int *__restrict__ label) {
+    const int v = blockIdx.x * 256 + threadIdx.x;
     if (v >= n) return;
-    int l = label[v];
-    for (int it = 0; it < 64; it++) {
-        const int l2 = label[order[l]];
-        if (l2 >= l) break;
-        l = l2;
+    const int r = rank[v], t = cc_root(parent, r);
+    label[v] = t;
+    if (t != r) __hip_atomic_store(&parent[r], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__global__ void __launch_bounds__(256)
+k_cc_link(const int *__restrict__ gp, const int *__restrict__ gc, int n, const int *__restrict__ label, int *parent) {
+    const int v = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VERT_LANES), l = threadIdx.x % VERT_LANES;
+    if (v >= n) return;
+    const int lv = label[v], e1 = gp[v + 1];
+    for (int e = gp[v] + l; e < e1; e += VERT_LANES) {
+        const int lu = label[gc[e]];
+        if (lu >= lv) continue;  // one tree, or the edge's other end takes it (the pattern is symmetric)
+        int a = cc_root(parent, lv), b = cc_root(parent, lu);
+        while (a != b) {
+            if (a < b) { const int t = a; a = b; b = t; }
+            const int old = atomicCAS(&parent[a], a, b);
+            if (old == a) break;
+            a = cc_root(parent, old);
+        }
     }
-    atomicMin(&label[v], l);
 }
 // seeds (component minima) in rank order: flag, scan, compact
 __global__ void k_seed_flag(const int *__restrict__ order, const int *__restrict__ label, int n, int *__restrict__ flag) {
@@ -271,43 +357,113 @@ __global__ void k_seed_compact(const int *__restrict__ order, const int *__restr
         visited[order[r]] = 1;
     }
 }
-__global__ void k_claim(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ front, int nf,
-                        const int *__restrict__ visited, int *__restrict__ claim) {
-    int q = blockIdx.x * 256 + threadIdx.x;
+// One BFS level: every unvisited neighbour is claimed by its first parent in
+// level order (its position q), the claimed ones are counted per parent, and
+// put in (degree, id) order behind one another.  VERT_LANES lanes per parent
+// for the first two, a wave for the last, which sorts a parent's children by
+// counting the smaller keys; a level with more than RCM_KIDS children of one
+// parent (word[0] then) goes through the radix sort instead.  Against sorting
+// every level (62 of a 27-point 61x64x59 mesh, some 40 launches each, 18 ms for
+// the call): 4 launches, 1.9 ms.
+#define RCM_KIDS 64
+__global__ void __launch_bounds__(256)
+k_claim(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ front, int nf,
+        const int *__restrict__ visited, int *__restrict__ claim, int *__restrict__ word) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) word[0] = 0;
+    const int q = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VERT_LANES), l = threadIdx.x % VERT_LANES;
     if (q >= nf) return;
-    const int p = front[q];
-    for (int e = gp[p]; e < gp[p + 1]; e++) {
+    const int p = front[q], e1 = gp[p + 1];
+    for (int e = gp[p] + l; e < e1; e += VERT_LANES) {
         const int u = gc[e];
         if (!visited[u]) atomicMin(&claim[u], q);
     }
 }
-template <bool EMIT>
-__global__ void k_children(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ front, int nf,
-                           const int *__restrict__ visited, const int *__restrict__ claim, const int *__restrict__ deg,
-                           int *__restrict__ cnt_or_off, unsigned long long *__restrict__ key, int *__restrict__ par) {
-    int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= nf) return;
-    const int p = front[q];
-    int k = EMIT ? cnt_or_off[q] : 0;
-    for (int e = gp[p]; e < gp[p + 1]; e++) {
-        const int u = gc[e];
-        if (!visited[u] && claim[u] == q) {
-            if (EMIT) {
-                key[k] = ((unsigned long long)(unsigned)deg[u] << 32) | (unsigned)u;
-                par[k] = q;
-            }
-            k++;
+__global__ void __launch_bounds__(256)
+k_count_children(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ front, int nf,
+                 const int *__restrict__ visited, const int *__restrict__ claim, int *__restrict__ cnt,
+                 int *__restrict__ word) {
+    const int q = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VERT_LANES), l = threadIdx.x % VERT_LANES;
+    int c = 0;
+    if (q < nf) {
+        const int p = front[q], e1 = gp[p + 1];
+        for (int e = gp[p] + l; e < e1; e += VERT_LANES) {
+            const int u = gc[e];
+            c += !visited[u] && claim[u] == q;
         }
     }
-    if (!EMIT) cnt_or_off[q] = k;
+    c = tsg_group16_sum(c);
+    if (q < nf && l == 0) cnt[q] = c;
+    const int mx = tsg_wave_max(c);
+    if ((threadIdx.x & 63) == 0 && mx > RCM_KIDS) atomicMax(&word[0], mx);
+}
+// Children of a wave's parent q into out[off[q]..), marked visited (only q's
+// own claims are, so the other parents' tests do not change).
+__global__ void __launch_bounds__(256)
+k_emit_children(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ front, int nf,
+                int *__restrict__ visited, const int *__restrict__ claim, const int *__restrict__ deg,
+                const int *__restrict__ off, int *__restrict__ out) {
+    __shared__ unsigned long long s_key[4][RCM_KIDS];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int q = blockIdx.x * 4 + wave;
+    if (q >= nf) return;
+    const int n = off[q + 1] - off[q];  // at most RCM_KIDS
+    if (n == 0) return;
+    const int p = front[q], e1 = gp[p + 1];
+    int have = 0;
+    for (int e0 = gp[p]; e0 < e1; e0 += 64) {
+        const int e = e0 + lane;
+        int u = 0;
+        bool mine = false;
+        if (e < e1) {
+            u = gc[e];
+            mine = !visited[u] && claim[u] == q;
+        }
+        const unsigned long long b = __ballot(mine);
+        if (mine)
+            s_key[wave][have + __popcll(b & ((1ull << lane) - 1ull))] =
+                ((unsigned long long)(unsigned)deg[u] << 32) | (unsigned)u;
+        have += __popcll(b);
+    }
+    tsg_wave_sync();
+    if (lane < n) {
+        const unsigned long long key = s_key[wave][lane];
+        int r = 0;
+        for (int j = 0; j < n; j++) r += s_key[wave][j] < key;  // ids differ, so keys do
+        const int u = (int)(key & 0xffffffffu);
+        out[off[q] + r] = u;
+        visited[u] = 1;
+    }
+}
+// The children of a level as sort keys (degree, id) with their parents.
+__global__ void __launch_bounds__(256)
+k_list_children(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ front, int nf,
+                const int *__restrict__ visited, const int *__restrict__ claim, const int *__restrict__ deg,
+                const int *__restrict__ off, unsigned long long *__restrict__ key, int *__restrict__ par) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int q = blockIdx.x * 4 + wave;
+    if (q >= nf) return;
+    const int p = front[q], e1 = gp[p + 1];
+    int k = off[q];
+    for (int e0 = gp[p]; e0 < e1; e0 += 64) {
+        const int e = e0 + lane;
+        int u = 0;
+        bool mine = false;
+        if (e < e1) {
+            u = gc[e];
+            mine = !visited[u] && claim[u] == q;
+        }
+        const unsigned long long b = __ballot(mine);
+        if (mine) {
+            const int at = k + __popcll(b & ((1ull << lane) - 1ull));
+            key[at] = ((unsigned long long)(unsigned)deg[u] << 32) | (unsigned)u;
+            par[at] = q;
+        }
+        k += __popcll(b);
+    }
 }
 __global__ void k_mark_children(const unsigned long long *__restrict__ key, int nc, int *__restrict__ visited) {
     int i = blockIdx.x * 256 + threadIdx.x;
     if (i < nc) visited[(int)(key[i] & 0xffffffffu)] = 1;
-}
-__global__ void k_parent_key(const int *__restrict__ par, int nc, unsigned *__restrict__ k2) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < nc) k2[i] = (unsigned)par[i];
 }
 __global__ void k_gather_children(const unsigned long long *__restrict__ key, const int *__restrict__ idx, int nc,
                                   int *__restrict__ out) {
@@ -333,7 +489,8 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     if (n == 0) return TSG_OK;
     tsg_dcsr g;
     TSG_TRY(tsg_dcsr_symmetrize(ctx, a, &g));
-    int *deg, *order, *rank, *label, *visited, *claim, *seq, *flag, *pos;
+    int *deg, *order, *rank, *label, *visited, *claim, *seq, *flag, *pos, *word;
+    TSG_TRY(tsg_alloc_t(ctx, &word, 4));
     TSG_TRY(tsg_alloc_t(ctx, &deg, (size_t)n + 1));
     TSG_TRY(tsg_alloc_t(ctx, &order, (size_t)n + 1));
     TSG_TRY(tsg_alloc_t(ctx, &rank, (size_t)n + 1));
@@ -348,20 +505,18 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     hipLaunchKernelGGL(k_rcm_deg, dim3(gn), dim3(256), 0, s, g.rowptr, g.colidx, n, deg);
     TSG_LAUNCH_CHECK();
     TSG_TRY(sort_ids_by_degree(ctx, deg, n, 0, order));  // ascending (degree, id)
-    hipLaunchKernelGGL(k_scatter_rank, dim3(gn), dim3(256), 0, s, order, n, rank, label);
-    TSG_LAUNCH_CHECK();
-    // connected components: label = lowest rank in the component
-    void *scr;
-    TSG_TRY(tsg_scratch(ctx, 64, &scr));
-    for (int it = 0; it < 4 * n + 8; it++) {
-        TSG_HIP(hipMemsetAsync(scr, 0, 4, s));
-        hipLaunchKernelGGL(k_cc_prop, dim3(gn), dim3(256), 0, s, g.rowptr, g.colidx, n, label, (int *)scr);
-        hipLaunchKernelGGL(k_cc_jump, dim3(gn), dim3(256), 0, s, order, n, label);
-        TSG_LAUNCH_CHECK();
-        long long ch = 0;
-        TSG_TRY(tsg_read_scalar_i64(ctx, scr, 0, &ch));
-        if (!ch) break;
+    // connected components: label = lowest rank in the component (parents in
+    // claim, which is set up for the traversal below)
+    const unsigned gv = tsg_div_up((long long)n * VERT_LANES, 256);
+    hipLaunchKernelGGL(k_scatter_rank, dim3(gn), dim3(256), 0, s, order, n, rank);
+    for (int round = 0; round < CC_ROUNDS; round++) {
+        hipLaunchKernelGGL(round == 0 ? k_cc_hook<true> : k_cc_hook<false>, dim3(gv), dim3(256), 0, s, g.rowptr,
+                           g.colidx, n, (const int *)(round == 0 ? rank : label), claim);
+        hipLaunchKernelGGL(k_cc_label, dim3(gn), dim3(256), 0, s, (const int *)rank, n, claim, label);
     }
+    hipLaunchKernelGGL(k_cc_link, dim3(gv), dim3(256), 0, s, g.rowptr, g.colidx, n, (const int *)label, claim);
+    hipLaunchKernelGGL(k_cc_label, dim3(gn), dim3(256), 0, s, (const int *)rank, n, claim, label);
+    TSG_LAUNCH_CHECK();
     // level 0: all component seeds, in rank order
     TSG_HIP(hipMemsetAsync(visited, 0, (size_t)n * 4, s));
     hipLaunchKernelGGL(k_fill_i32, dim3(gn), dim3(256), 0, s, claim, (long long)n, 0x7fffffff);
@@ -384,32 +539,38 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     const int nbits = bits_of(n);
     while (nf > 0 && done < n) {
         const int *front = seq + fstart;
-        const unsigned gf = tsg_div_up(nf, 256);
-        hipLaunchKernelGGL(k_claim, dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited, claim);
-        hipLaunchKernelGGL((k_children<false>), dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
-                           claim, deg, cnt, (unsigned long long *)nullptr, (int *)nullptr);
+        const unsigned gf = tsg_div_up(nf * VERT_LANES, 256), gw = tsg_div_up(nf, 4);
+        hipLaunchKernelGGL(k_claim, dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited, claim, word);
+        hipLaunchKernelGGL(k_count_children, dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
+                           claim, cnt, word);
         TSG_LAUNCH_CHECK();
         long long nc = 0;
-        TSG_TRY(tsg_scan_i32(ctx, cnt, cnt, nf, &nc));
+        TSG_TRY(tsg_scan_i32(ctx, cnt, cnt, nf, &nc, word, 1));
         if (nc == 0) break;
-        hipLaunchKernelGGL((k_children<true>), dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
-                           claim, deg, cnt, key, par);
-        TSG_LAUNCH_CHECK();
-        const unsigned gc2 = tsg_div_up(nc, 256);
-        hipLaunchKernelGGL(k_mark_children, dim3(gc2), dim3(256), 0, s, key, (int)nc, visited);
-        // order children by (parent position, degree, id): sort by (degree,
-        // id), then stably by parent position
-        hipLaunchKernelGGL(k_iota2, dim3(gc2), dim3(256), 0, s, idx, nc);
-        TSG_LAUNCH_CHECK();
-        TSG_TRY(tsg_sort_pairs_u64(ctx, key, idx, nc, 32 + nbits));
-        // after the sort, idx[i] is the emit slot of the i-th smallest key:
-        // parent of the i-th smallest key is par[idx[i]]
-        hipLaunchKernelGGL(k_gather_i32_r, dim3(gc2), dim3(256), 0, s, par, idx, (int)nc, (int *)k2);
-        hipLaunchKernelGGL(k_iota2, dim3(gc2), dim3(256), 0, s, idx, nc);
-        TSG_LAUNCH_CHECK();
-        TSG_TRY(tsg_sort_pairs_u32(ctx, k2, idx, nc, bits_of(nf)));
-        hipLaunchKernelGGL(k_gather_children, dim3(gc2), dim3(256), 0, s, key, idx, (int)nc, seq + fstart + nf);
-        TSG_LAUNCH_CHECK();
+        if (((volatile int *)(ctx->pinned + 1))[0] <= RCM_KIDS) {
+            hipLaunchKernelGGL(k_emit_children, dim3(gw), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
+                               claim, deg, cnt, seq + fstart + nf);
+            TSG_LAUNCH_CHECK();
+        } else {
+            hipLaunchKernelGGL(k_list_children, dim3(gw), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
+                               claim, deg, cnt, key, par);
+            TSG_LAUNCH_CHECK();
+            const unsigned gc2 = tsg_div_up(nc, 256);
+            hipLaunchKernelGGL(k_mark_children, dim3(gc2), dim3(256), 0, s, key, (int)nc, visited);
+            // order children by (parent position, degree, id): sort by (degree,
+            // id), then stably by parent position
+            hipLaunchKernelGGL(k_iota2, dim3(gc2), dim3(256), 0, s, idx, nc);
+            TSG_LAUNCH_CHECK();
+            TSG_TRY(tsg_sort_pairs_u64(ctx, key, idx, nc, 32 + bits_of((long long)n + 1)));
+            // after the sort, idx[i] is the emit slot of the i-th smallest key:
+            // parent of the i-th smallest key is par[idx[i]]
+            hipLaunchKernelGGL(k_gather_i32_r, dim3(gc2), dim3(256), 0, s, par, idx, (int)nc, (int *)k2);
+            hipLaunchKernelGGL(k_iota2, dim3(gc2), dim3(256), 0, s, idx, nc);
+            TSG_LAUNCH_CHECK();
+            TSG_TRY(tsg_sort_pairs_u32(ctx, k2, idx, nc, bits_of(nf)));
+            hipLaunchKernelGGL(k_gather_children, dim3(gc2), dim3(256), 0, s, key, idx, (int)nc, seq + fstart + nf);
+            TSG_LAUNCH_CHECK();
+        }
         fstart += nf;
         nf = nc;
         done += nc;
@@ -426,27 +587,99 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     hipLaunchKernelGGL(k_reverse_gather, dim3(gn), dim3(256), 0, s, seq, idx, n, d_old_id);
     TSG_LAUNCH_CHECK();
     if (levels_out) *levels_out = levels;
-    void *ps[] = {deg, order, rank, label, visited, claim, seq, flag, pos, key, par, cnt, idx, k2, ck};
+    void *ps[] = {deg, order, rank, label, visited, claim, seq, flag, pos, word, key, par, cnt, idx, k2, ck};
     for (void *p : ps) tsg_free(ctx, p);
     tsg_dcsr_free(ctx, &g);
     return TSG_OK;
 }
 
 // ------------------------------------------------------------------ P A Q^T
-__global__ void k_perm_counts(const int *__restrict__ rowptr, const int *__restrict__ row_old, int m, int *__restrict__ cnt) {
-    int r = blockIdx.x * 256 + threadIdx.x;
-    if (r < m) cnt[r] = rowptr[row_old[r] + 1] - rowptr[row_old[r]];
+#define PERM_WAVE 64
+#define PERM_BLOCK 4096
+// Row lengths of the result; word[0] (zeroed beforehand) = the longest over
+// PERM_WAVE, if any (an atomic per wave on one address is 43 us of its own).
+__global__ void __launch_bounds__(256)
+k_perm_counts(const int *__restrict__ rowptr, const int *__restrict__ row_old, int m, int *__restrict__ cnt,
+              int *__restrict__ word) {
+    int mx = 0;
+    for (int r = blockIdx.x * 256 + threadIdx.x; r < m; r += gridDim.x * 256) {
+        const int c = rowptr[row_old[r] + 1] - rowptr[row_old[r]];
+        cnt[r] = c;
+        mx = max(mx, c);
+    }
+    mx = tsg_wave_max(mx);
+    if ((threadIdx.x & 63) == 0 && mx > PERM_WAVE) atomicMax(&word[0], mx);
+}
+// Rows of at most PERM_WAVE entries: one wave per row, each entry's place by
+// counting the smaller columns.  Up to PERM_BLOCK: one block per row, bitonic
+// sort in LDS.  A matrix with a longer row has all its entries sorted by
+// (row, column) with the radix sort (two words an entry, five passes and
+// more): 27-point 61x64x59 (5.9M entries) some 0.9 ms of kernels
+// -> 0.11.
+__global__ void __launch_bounds__(256)
+k_perm_rows(const int *__restrict__ rowptr, const int *__restrict__ col, const double *__restrict__ val,
+            const int *__restrict__ row_old, const int *__restrict__ col_new, int m, const int *__restrict__ optr,
+            int *__restrict__ ocol, double *__restrict__ oval) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = blockIdx.x * 4 + wave;
+    if (r >= m) return;
+    const int e0 = rowptr[row_old[r]], o0 = optr[r], n = optr[r + 1] - o0;
+    if (n == 0 || n > PERM_WAVE) return;  // wave-uniform
+    int c = 0x7fffffff;
+    double v = 0.0;
+    if (lane < n) {
+        c = col_new[col[e0 + lane]];
+        v = val[e0 + lane];
+    }
+    int at = 0;
+    for (int j = 0; j < n; j++) at += __builtin_amdgcn_readlane(c, j) < c;  // columns differ inside a row
+    if (lane < n) {
+        ocol[o0 + at] = c;
+        oval[o0 + at] = v;
+    }
+}
+__global__ void __launch_bounds__(256)
+k_perm_rows_block(const int *__restrict__ rowptr, const int *__restrict__ col, const double *__restrict__ val,
+                  const int *__restrict__ row_old, const int *__restrict__ col_new, const int *__restrict__ optr,
+                  int *__restrict__ ocol, double *__restrict__ oval) {
+    __shared__ unsigned long long s_key[PERM_BLOCK];
+    const int r = blockIdx.x, tid = threadIdx.x;
+    const int e0 = rowptr[row_old[r]], o0 = optr[r], n = optr[r + 1] - o0;
+    if (n <= PERM_WAVE) return;  // block-uniform
+    int p2 = 2 * PERM_WAVE;
+    while (p2 < n) p2 <<= 1;
+    for (int i = tid; i < p2; i += 256)
+        s_key[i] = i < n ? ((unsigned long long)(unsigned)col_new[col[e0 + i]] << 32) | (unsigned)i : ~0ull;
+    __syncthreads();
+    for (int k = 2; k <= p2; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int i = tid; i < p2; i += 256) {
+                const int x = i ^ j;
+                if (x > i) {
+                    const unsigned long long a = s_key[i], b = s_key[x];
+                    if ((a > b) == ((i & k) == 0)) {
+                        s_key[i] = b;
+                        s_key[x] = a;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    for (int i = tid; i < n; i += 256) {
+        const unsigned long long key = s_key[i];
+        ocol[o0 + i] = (int)(key >> 32);
+        oval[o0 + i] = val[e0 + (int)(key & 0xffffffffu)];
+    }
 }
 __global__ void k_perm_emit(const int *__restrict__ rowptr, const int *__restrict__ col, const int *__restrict__ row_old,
                             const int *__restrict__ col_new, int m, int n, const int *__restrict__ optr,
                             unsigned long long *__restrict__ key, int *__restrict__ src) {
-    int r = blockIdx.x * 256 + threadIdx.x;
+    const int r = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15;  // 16 lanes per row
     if (r >= m) return;
-    const int o = row_old[r];
-    int w = optr[r];
-    for (int e = rowptr[o]; e < rowptr[o + 1]; e++, w++) {
-        key[w] = (unsigned long long)r * (unsigned long long)n + (unsigned)col_new[col[e]];
-        src[w] = e;
+    const int e0 = rowptr[row_old[r]], w0 = optr[r], len = optr[r + 1] - w0;
+    for (int j = l; j < len; j += 16) {
+        key[w0 + j] = (unsigned long long)r * (unsigned long long)n + (unsigned)col_new[col[e0 + j]];
+        src[w0 + j] = e0 + j;
     }
 }
 __global__ void k_perm_gather(const unsigned long long *__restrict__ key, const int *__restrict__ src,
@@ -471,20 +704,33 @@ extern "C" int tsg_dcsr_permute(tsg_ctx *ctx, const tsg_dcsr *a, const int *d_ro
     TSG_TRY(tsg_alloc_t(ctx, &out->rowptr, (size_t)m + 1));
     TSG_TRY(tsg_alloc_t(ctx, &out->colidx, (size_t)nnz + 1));
     TSG_TRY(tsg_alloc_t(ctx, &out->val, (size_t)nnz + 1));
-    const unsigned gm = tsg_div_up(m, 256);
+    int *word;
+    TSG_TRY(tsg_alloc_t(ctx, &word, 4));
+    TSG_HIP(hipMemsetAsync(word, 0, 4, ctx->stream));
     if (m > 0) {
-        hipLaunchKernelGGL(k_perm_counts, dim3(gm), dim3(256), 0, ctx->stream, a->rowptr, d_row_old, m, out->rowptr);
+        hipLaunchKernelGGL(k_perm_counts, dim3(std::min<unsigned>(1024, tsg_div_up(m, 256))), dim3(256), 0, ctx->stream,
+                           a->rowptr, d_row_old, m, out->rowptr, word);
         TSG_LAUNCH_CHECK();
     }
     long long tot = 0;
-    TSG_TRY(tsg_scan_i32(ctx, out->rowptr, out->rowptr, m, &tot));
+    const int sc = tsg_scan_i32(ctx, out->rowptr, out->rowptr, m, &tot, word, 1);
+    tsg_free(ctx, word);
+    TSG_TRY(sc);
+    const int longest = ((volatile int *)(ctx->pinned + 1))[0];
     if (tot != nnz) { tsg_set_error("permute: row permutation is not a bijection"); return TSG_ERR_ARG; }
-    if (nnz > 0) {
+    if (nnz > 0 && longest <= PERM_BLOCK) {
+        hipLaunchKernelGGL(k_perm_rows, dim3(tsg_div_up(m, 4)), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, a->val,
+                           d_row_old, d_col_new, m, out->rowptr, out->colidx, out->val);
+        if (longest > PERM_WAVE)
+            hipLaunchKernelGGL(k_perm_rows_block, dim3((unsigned)m), dim3(256), 0, ctx->stream, a->rowptr, a->colidx,
+                               a->val, d_row_old, d_col_new, out->rowptr, out->colidx, out->val);
+        TSG_LAUNCH_CHECK();
+    } else if (nnz > 0) {
         unsigned long long *key;
         int *src;
         TSG_TRY(tsg_alloc_t(ctx, &key, (size_t)nnz));
         TSG_TRY(tsg_alloc_t(ctx, &src, (size_t)nnz));
-        hipLaunchKernelGGL(k_perm_emit, dim3(gm), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, d_row_old, d_col_new,
+        hipLaunchKernelGGL(k_perm_emit, dim3(tsg_div_up(m, 16)), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, d_row_old, d_col_new,
                            m, n, out->rowptr, key, src);
         TSG_LAUNCH_CHECK();
         TSG_TRY(tsg_sort_pairs_u64(ctx, key, src, nnz, bits_of((long long)m * n)));
