@@ -669,23 +669,6 @@ __device__ __forceinline__ uint4 t2c_offsets(uint4 p, int tnnz, int rowlen) {
     }
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
-// The 16 row lengths of a tile, one byte each, from those offsets: next
-// offset minus offset, byte by byte.  Offsets ascend, so no borrow crosses a
-// byte; the last byte's minuend is the entry count (mod 256).
-__device__ __forceinline__ uint4 t2c_row_lens(uint4 p, int tnnz) {
-    return make_uint4(((p.x >> 8) | (p.y << 24)) - p.x, ((p.y >> 8) | (p.z << 24)) - p.y,
-                      ((p.z >> 8) | (p.w << 24)) - p.z, ((p.w >> 8) | ((unsigned)tnnz << 24)) - p.w);
-}
-// Bytes as 16-bit pairs: v[2q] = rows 4q and 4q+2, v[2q+1] = rows 4q+1, 4q+3.
-__device__ __forceinline__ void t2c_widen(uint4 l, unsigned v[8]) {
-    const unsigned w[4] = {l.x, l.y, l.z, l.w};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        v[2 * q] = w[q] & 0x00ff00ffu;
-        v[2 * q + 1] = (w[q] >> 8) & 0x00ff00ffu;
-    }
-}
-
 // 16 bytes from an address of any alignment (one load: the target allows
 // unaligned global access).
 __device__ __forceinline__ uint4 load16(const unsigned char *p) {
@@ -705,22 +688,13 @@ __device__ __forceinline__ void t2c_row_sums(const int *__restrict__ tile_nnz, c
     for (int t = ta; t < te; t += stride) {
         unsigned x[8];
         const int tn = tile_nnz[t + 1] - tile_nnz[t];
-        t2c_widen(t2c_row_lens(t2c_offsets(load16(csr_ptr + 16 * (long long)t), tn, rowlen), tn), x);
+        tile_widen_lens(tile_row_lens(t2c_offsets(load16(csr_ptr + 16 * (long long)t), tn, rowlen), tn), x);
 #pragma unroll
         for (int q = 0; q < 8; q++) v[q] += x[q];
     }
 #pragma unroll
     for (int q = 0; q < 8; q++) v[q] = (unsigned)__builtin_amdgcn_readlane(tsg_wave_incl_scan_dpp((int)v[q]), 63);
 }
-// v's entry for row r (0..15)
-__device__ __forceinline__ int t2c_row_of(const unsigned v[8], int r) {
-    unsigned x = 0;
-#pragma unroll
-    for (int q = 0; q < 8; q++)
-        if (2 * (r >> 2) + (r & 1) == q) x = v[q];
-    return (int)((r & 2) ? x >> 16 : x & 0xffffu);
-}
-
 // Row pointers; one wave per tile-row of up to CV_SEG tiles, a tile per lane,
 // the block's four waves together for a longer one.  *nitems (zeroed
 // beforehand) counts the further runs (the first maxitems are listed); host
@@ -740,7 +714,7 @@ k_t2c_rowptr(int m, int tilem, const int *__restrict__ tile_ptr, const int *__re
         if (t1 - t0 <= CV_SEG) {
             const int rowlen = min(16, m - 16 * I);
             t2c_row_sums(tile_nnz, csr_ptr, t0 + lane, t1, 64, rowlen, v);
-            const int c = t2c_row_of(v, lane & 15), incl = tsg_row16_incl_scan_dpp(c);
+            const int c = tile_row_of(v, lane & 15), incl = tsg_row16_incl_scan_dpp(c);
             if (lane < rowlen) rowptr[16 * I + lane] = tile_nnz[t0] - nb0 + incl - c;
         }
         if (I == tilem - 1 && lane == 0) {
@@ -770,7 +744,7 @@ k_t2c_rowptr(int m, int tilem, const int *__restrict__ tile_ptr, const int *__re
             }
             t2c_row_sums(tile_nnz, csr_ptr, t0 + sg * CV_SEG + tid, min(t1, t0 + (sg + 1) * CV_SEG), 64 * CV_WAVES,
                          rowlen, v);
-            if (lane < 16) s_sum[wave][lane] = t2c_row_of(v, lane);
+            if (lane < 16) s_sum[wave][lane] = tile_row_of(v, lane);
             __syncthreads();
             if (tid < 16)
                 for (int w2 = 0; w2 < CV_WAVES; w2++) carry += s_sum[w2][tid];
@@ -782,13 +756,6 @@ k_t2c_rowptr(int m, int tilem, const int *__restrict__ tile_ptr, const int *__re
         }
         __syncthreads();  // s_slot
     }
-}
-
-// Bytes of w that are at most j, as 0x80 bits (unsigned, per byte).
-__device__ __forceinline__ unsigned bytes_le(unsigned w, unsigned j) {
-    const unsigned H = 0x80808080u, x = j * 0x01010101u;
-    const unsigned t = (x | H) - (w & ~H);  // per byte, no borrow out
-    return ((x & ~w) | (~(x ^ w) & t)) & H;
 }
 
 // Entries: the first tilem waves take each tile-row's first run, the others
@@ -854,7 +821,7 @@ k_t2c_emit(int m, int tilem, const int *__restrict__ tile_ptr, const int *__rest
             if (lane < nt && n1 > n0) sr[n0 - start] = (unsigned char)(lane + 1);
             // entries of each row in the tiles before the lane's; the rows' runs
             unsigned len[8], tot[8];
-            t2c_widen(t2c_row_lens(p16, n1 - n0), len);
+            tile_widen_lens(tile_row_lens(p16, n1 - n0), len);
             unsigned run = 0;
 #pragma unroll
             for (int q = 0; q < 8; q++) {

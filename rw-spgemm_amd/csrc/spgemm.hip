@@ -1389,13 +1389,8 @@ __device__ __forceinline__ void step3_tile_body(const TileOperands &op, const in
 // LDS hash of the segment's C entries: key (column - col_lo) * 16 + row,
 // stored + 1 (0 = empty), value = the entry's position in the segment,
 // linear probing.  2560 slots (load factor at most 0.6): six blocks per CU
-// packed (25.6 KB of LDS; 24.2 KB with A's row index, which needs no
-// per-group decode scratch), five unpacked when A is decoded from its tiles
-// (30.7 KB).  Unpacked with A's row index, 2048 slots (at most 0.75) fit
-// six blocks (26.1 KB); the packed table stays at 2560, since at seven
-// blocks per CU its higher load factor cost more than the occupancy gave.
+// packed (25.6 KB of LDS), five unpacked (30.7 KB).
 #define G3E_EHASH 2560
-#define G3E_EHASH_RXW 2048
 #define G3E_PF 4  // C tiles per thread whose metadata is loaded per round
 // home slot of a key in a table of HS slots (multiply-shift range
 // reduction) and the next slot
@@ -1412,17 +1407,17 @@ __device__ __forceinline__ unsigned ent_next(unsigned h) { return h + 1 == HS ? 
 #define G3E_PK_SPAN 8192
 static_assert(G3E_NNZ <= 2048, "positions take 11 bits of a packed hash slot");
 
-// RX: A carries its element row index (rows' entries read directly); else
-// A row r's entries are decoded from its tiles.
-template <bool PK, bool RX>
-__global__ void __launch_bounds__(256, PK || RX ? 6 : 5)
+// For an A without its row index (its rows' entries are decoded from its
+// tiles); with it, k_step3_flat takes these tile-rows.
+template <bool PK>
+__global__ void __launch_bounds__(256, PK ? 6 : 5)
 k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restrict__ Bcolx,
              const double *__restrict__ Bvalx, int m, const int4 *__restrict__ segs, const int *__restrict__ nseg,
              const int *__restrict__ Cptr, const int *__restrict__ Ccol, const unsigned short *__restrict__ Cmask,
              const unsigned char *__restrict__ Cptr16, const int *__restrict__ Cnnz, unsigned char *__restrict__ Ccol8,
-             double *__restrict__ Cval, const unsigned char *__restrict__ heavy) {
+             double *__restrict__ Cval) {
     __shared__ double s_acc[G3E_NNZ];
-    constexpr unsigned HS = RX && !PK ? G3E_EHASH_RXW : G3E_EHASH;
+    constexpr unsigned HS = G3E_EHASH;
     __shared__ unsigned s_ekey[HS];
     __shared__ unsigned short s_epos[PK ? 1 : HS];
     __shared__ unsigned char s_ecol[G3E_NNZ];  // in-tile column of each entry, final order
@@ -1490,12 +1485,9 @@ k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
     __syncthreads();
     const int r = tid >> 4, l = tid & 15;
     const int row = 16 * I + r;
-    // rows flagged heavy are computed by k_step3_heavy, which runs after
-    // this kernel and overwrites their values
-    const bool skip = heavy && row < m && heavy[row];
     const int gb = tid & 48;  // first lane of this group in its wave
-    __shared__ int s_gex[RX ? 1 : 16][16];             // per group: entries before each lane's tile
-    __shared__ unsigned short s_gam[RX ? 1 : 16][16];  // per group: each lane's tile row mask
+    __shared__ int s_gex[16][16];             // per group: entries before each lane's tile
+    __shared__ unsigned short s_gam[16][16];  // per group: each lane's tile row mask
     // adds a * b into C entry (row 16I+r, col), located through the hash
     // (the entry is in C's structure; the probe bound is not reached for a
     // consistent C)
@@ -1518,56 +1510,7 @@ k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
             }
         }
     };
-    if (RX && row < m && nseg_nnz > 0 && !skip) {
-        // A's row index: row 16I+r's entries are contiguous, ascending k.  The
-        // 16 lanes take 16 of them (sources) and find their B ranges in
-        // parallel; then the first 16 in-range B entries of all 16 sources are
-        // loaded at once (lane l holds entry l of each), so the ordered
-        // accumulation below waits on no global load for rows of up to 16
-        // entries in the segment's column range.
-        const int x1 = op.Arowp[row + 1];
-        for (int x0 = op.Arowp[row]; x0 < x1; x0 += 16) {
-            const int x = x0 + l;
-            int e0 = 0, e1 = 0;
-            double a = 0.0;
-            if (x < x1) {
-                const int k = op.Acolx[x];
-                a = op.Avalx[x];
-                e1 = Browp[k + 1];
-                // every entry of B row k is in a C tile of the tile-row, so
-                // none lies before the row's first segment
-                e0 = sg.w == 0 ? Browp[k] : lower_bound_i(Bcolx, Browp[k], e1, col_lo);
-            }
-            int pc[16];
-            double pv[16];
-#pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int qs0 = tsg_row16_bcast(e0, q), qs1 = tsg_row16_bcast(e1, q);
-                const int e = qs0 + l;
-                pc[q] = 0x7fffffff;
-                pv[q] = 0.0;
-                if (e < qs1) {
-                    pc[q] = Bcolx[e];
-                    pv[q] = Bvalx[e];
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 16; q++) {  // sources in ascending k
-                const double as = tsg_row16_bcast(a, q);
-                const int qs0 = tsg_row16_bcast(e0, q), qs1 = tsg_row16_bcast(e1, q);
-                if (pc[q] < col_hi) acc_add(pc[q], as, pv[q]);
-                // entries past the first 16 (the last prefetched one in range)
-                if (qs1 - qs0 > 16 && tsg_row16_bcast(pc[q], 15) < col_hi) {
-                    for (int e = qs0 + 16 + l; e < qs1; e += 16) {
-                        const int col = Bcolx[e];
-                        if (col >= col_hi) break;
-                        acc_add(col, as, Bvalx[e]);
-                    }
-                }
-                tsg_wave_sync();  // the next k of this row reads what lanes wrote
-            }
-        }
-    } else if (!RX && row < m && nseg_nnz > 0 && !skip) {
+    if (row < m && nseg_nnz > 0) {
         const int a0 = op.Aptr[I], a1 = op.Aptr[I + 1];
         for (int t0 = a0; t0 < a1; t0 += 16) {
             // 16 A tiles per round, one per lane: their row-r entries are
@@ -1632,22 +1575,301 @@ k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
     }
 }
 
+// ------------------------------------------------------------------ step 3, flat rows
+// [b0, b1) cut to list's entries in [lo, hi) (list ascending; an end that is
+// not to be cut keeps its place).  Both ends at once and a quarter of the
+// range left per step, six loads in flight: a lane's search is a chain of
+// round trips, so their number is what it costs.
+__device__ __forceinline__ void range_in(const int *__restrict__ list, int &b0, int &b1, bool cut_lo, int lo,
+                                         bool cut_hi, int hi) {
+    int la = b0, na = cut_lo ? b1 - b0 : 0;  // first entry >= lo is in [la, la + na]
+    int lb = b0, nb = cut_hi ? b1 - b0 : 0;  // first entry >= hi is in [lb, lb + nb]
+    if (!cut_hi) lb = b1;
+    while (na > 0 || nb > 0) {
+        int pa[3], pb[3], va[3], vb[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            pa[i] = (int)(((unsigned long long)(unsigned)na * (i + 1)) >> 2);  // < na when na > 0
+            pb[i] = (int)(((unsigned long long)(unsigned)nb * (i + 1)) >> 2);
+            va[i] = na > 0 ? list[la + pa[i]] : 0;
+            vb[i] = nb > 0 ? list[lb + pb[i]] : 0;
+        }
+        if (na > 0) {
+            const int k = (va[0] < lo) + (va[1] < lo) + (va[2] < lo);
+            const int from = k == 0 ? 0 : (k == 1 ? pa[0] : k == 2 ? pa[1] : pa[2]) + 1;
+            const int to = k == 0 ? pa[0] : k == 1 ? pa[1] : k == 2 ? pa[2] : na;
+            la += from;
+            na = to - from;
+        }
+        if (nb > 0) {
+            const int k = (vb[0] < hi) + (vb[1] < hi) + (vb[2] < hi);
+            const int from = k == 0 ? 0 : (k == 1 ? pb[0] : k == 2 ? pb[1] : pb[2]) + 1;
+            const int to = k == 0 ? pb[0] : k == 1 ? pb[1] : k == 2 ? pb[2] : nb;
+            lb += from;
+            nb = to - from;
+        }
+    }
+    b0 = la;
+    b1 = max(lb, la);
+}
+// Element-wise numeric step with A's and B's row index: one block of eight
+// waves per segment of a tile-row (k_seg1_count; at most G3F_NNZ C nonzeros,
+// summed in LDS in final order).
+//   Hash.  Each row of the segment has its own table of one and a half slots
+//   per entry: column offset (20 bits, + 1) and position (12) in one word, in
+//   two with WIDE.  Entries are inserted one per lane, their tile from marks,
+//   their row from the tile's row offsets, their column from the row mask:
+//   a lane per tile walking its masks had 6 of 64 lanes inserting (54k VALU
+//   instructions a tile-row of ER 65521, 42k now).
+//   Products.  A wave owns two rows, a long one and a short one.  It takes up
+//   to 64 of their A entries (sources) at a time, cuts their B rows to the
+//   segment's columns, numbers the products through in ascending k and takes
+//   64 at a time, one per lane.  Two of them can meet in one C entry only if
+//   they come from different sources: each lane leaves its number at its
+//   entry and reads it back, and a batch in which some lane finds another's
+//   is added source by source.  So every C entry still sums its products in
+//   ascending k, without atomics.
+// Four blocks (32 waves) fit a CU; it is bound by the latency of each block's
+// phases and half by VALU issue.  Against 16 lanes per C row taking one
+// source at a time (4.5 entries of a source in a segment of ER 65521), a
+// search per source and segment of 1536: ER 65521 A^2 0.62 -> 0.545 ms, banded
+// 39989 (half-bandwidth 20) 0.29 -> 0.167, R-MAT scale 16 A*A^T 12.9 -> 7.7.
+// Segments of 1920 / 2048 / 2496 / 3200 nonzeros: ER 573 / 533 / 545 / 579 us,
+// R-MAT 8.4 / 8.2 / 7.7 / 8.8 ms.
+#define G3F_NNZ 2496
+#define G3F_THREADS 512
+#define G3F_WAVES (G3F_THREADS / 64)
+#define G3F_SLOTS (G3F_NNZ + G3F_NNZ / 2 + 32)
+#define G3F_ROUNDS 4
+#define G3F_BATCH (64 * G3F_ROUNDS)
+#define G3F_SPAN 65535  // tile columns of a tile-row: offsets + 1 below 2^20
+__device__ __forceinline__ unsigned flat_home(unsigned key, unsigned n) {
+    return (unsigned)(((unsigned long long)(key * 2654435761u) * n) >> 32);
+}
+template <bool WIDE>
+__global__ void __launch_bounds__(G3F_THREADS)
+k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const double *__restrict__ Avalx,
+             const int *__restrict__ Browp, const int *__restrict__ Bcolx, const double *__restrict__ Bvalx, int m,
+             const int4 *__restrict__ segs, const int *__restrict__ nseg, const int *__restrict__ Cptr,
+             const int *__restrict__ Ccol, const unsigned short *__restrict__ Cmask,
+             const unsigned char *__restrict__ Cptr16, const int *__restrict__ Cnnz, unsigned char *__restrict__ Ccol8,
+             double *__restrict__ Cval, const unsigned char *__restrict__ heavy) {
+    __shared__ double s_acc[G3F_NNZ];
+    __shared__ unsigned s_key[G3F_SLOTS];
+    __shared__ unsigned short s_pos[WIDE ? G3F_SLOTS : 1];
+    __shared__ unsigned char s_tag[G3F_NNZ];
+    __shared__ unsigned s_mark[G3F_WAVES][G3F_BATCH / 4];
+    __shared__ int s_cnt[G3F_WAVES][16], s_rb[17];
+    __shared__ unsigned char s_ord[16];
+    static_assert(G3F_NNZ <= 4096, "positions take 12 bits of a slot");
+    static_assert(G3F_NNZ >= G3E_NNZ, "the segment array is sized for segments of G3E_NNZ");
+    static_assert(G3F_WAVES == 8, "two rows per wave");
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    // the grid is an upper bound: the first *nseg blocks (spread evenly over
+    // the XCDs) take the segments, each XCD a contiguous range
+    const int ns = *nseg;
+    if ((int)blockIdx.x >= ns) return;  // block-uniform
+    const int4 sg = segs[tsg_xcd_block(blockIdx.x, (unsigned)ns)];
+    const int I = sg.x, cend = Cptr[I + 1];
+    const int c0 = Cptr[I] + sg.y, u = sg.z - sg.y;
+    const int nbase = Cnnz[c0], n = Cnnz[c0 + u] - nbase;
+    if (n == 0) return;  // block-uniform
+    const int col_lo = Ccol[c0] * 16, col_hi = Ccol[c0 + u - 1] * 16 + 16;
+    const bool first = sg.w == 0, last = c0 + u == cend;
+    for (int i = tid; i < n; i += G3F_THREADS) s_acc[i] = 0.0;
+    for (int i = tid; i < n + n / 2 + 32; i += G3F_THREADS) s_key[i] = 0u;
+    // entries of each row of the segment; rows left to k_step3_heavy take no slots
+    unsigned skip = 0;
+    if (heavy) {
+        const int row = 16 * I + (lane & 15);
+        skip = (unsigned)__ballot(row < m && heavy[row]) & 0xffffu;
+    }
+    {
+        unsigned v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = 0u;
+        for (int i = tid; i < u; i += G3F_THREADS) {
+            const long long t = c0 + i;
+            unsigned x[8];
+            tile_widen_lens(tile_row_lens(reinterpret_cast<const uint4 *>(Cptr16)[t], Cnnz[t + 1] - Cnnz[t]), x);
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] += x[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = (unsigned)__builtin_amdgcn_readlane(tsg_wave_incl_scan_dpp((int)v[q]), 63);
+        if (lane < 16) s_cnt[wave][lane] = tile_row_of(v, lane);
+    }
+    __syncthreads();
+    if (tid < 16) {
+        int c = 0;
+        for (int w = 0; w < G3F_WAVES; w++) c += s_cnt[w][tid];
+        if ((skip >> tid) & 1u) c = 0;
+        const int slots = c ? c + c / 2 + 2 : 0;
+        const int incl = tsg_row16_incl_scan_dpp(slots);
+        s_rb[tid] = incl - slots;
+        if (tid == 15) s_rb[16] = incl;
+        int rank = 0;  // by entries, longest first
+        for (int j = 0; j < 16; j++) {
+            const int cj = __builtin_amdgcn_readlane(c, j);
+            rank += cj > c || (cj == c && j < tid);
+        }
+        s_ord[rank] = (unsigned char)tid;
+    }
+    __syncthreads();
+    // the segment's entries into their rows' tables, their columns to memory
+    unsigned char *mk = reinterpret_cast<unsigned char *>(s_mark[wave]);
+    const int per = min(64, (u + G3F_WAVES - 1) / G3F_WAVES);  // few, fuller tiles: every wave has some
+    for (int tg = per * wave; tg < u; tg += per * G3F_WAVES) {
+        const int te = min(u, tg + per);
+        for (int tb = tg; tb < te;) {
+            const long long tl = c0 + min(tb + lane, te - 1);
+            const int n0 = Cnnz[tl] - nbase, n1 = Cnnz[tl + 1] - nbase, Jl = Ccol[tl];
+            const int start = __builtin_amdgcn_readfirstlane(n0);
+            const int nt = __popcll(__ballot(tb + lane < te && n1 - start <= G3F_BATCH));
+            const int total = __builtin_amdgcn_readlane(n1, nt - 1) - start;
+            if (total > 0) {
+                s_mark[wave][lane] = 0u;
+                tsg_wave_sync();
+                if (lane < nt && n1 > n0) mk[n0 - start] = (unsigned char)(lane + 1);
+                tsg_wave_sync();
+                int prev = 0;
+                for (int x0 = 0; x0 < total; x0 += 64) {
+                    const int x = x0 + lane;
+                    const int k = max(prev, tsg_wave_incl_max_dpp((int)mk[x])) - 1;
+                    prev = __builtin_amdgcn_readlane(k, 63) + 1;
+                    const long long t = c0 + tb + k;
+                    const int j = x - (__shfl(n0, k, 64) - start), J = __shfl(Jl, k, 64);
+                    const uint4 p = reinterpret_cast<const uint4 *>(Cptr16)[t];
+                    const int r = __popc(bytes_le(p.x, j & 255)) + __popc(bytes_le(p.y, j & 255)) +
+                                  __popc(bytes_le(p.z, j & 255)) + __popc(bytes_le(p.w, j & 255)) - 1;
+                    unsigned mr = Cmask[t * 16 + r];
+                    const unsigned pw = (r & 8) ? ((r & 4) ? p.w : p.z) : ((r & 4) ? p.y : p.x);
+                    int skipn = j - (int)((pw >> (8 * (r & 3))) & 255u);
+                    if (x < total) {
+                        // entry j of the tile: the (j - row offset)-th column of row r
+                    for (; skipn > 0; skipn--) mr &= ~(0x80000000u >> __clz((int)mr));
+                        const int c = __clz((int)mr) - 16, pos = start + x;
+                        Ccol8[(long long)nbase + pos] = (unsigned char)c;
+                        if (!((skip >> r) & 1u)) {
+                            const int rb = s_rb[r];
+                            const unsigned rs = (unsigned)(s_rb[r + 1] - rb), key = (unsigned)(J * 16 + c - col_lo) + 1u;
+                            unsigned h = flat_home(key, rs);
+                            const unsigned ent = WIDE ? key : key << 12 | (unsigned)pos;
+                            while (atomicCAS(&s_key[rb + h], 0u, ent) != 0u) h = h + 1 == rs ? 0u : h + 1;
+                            if (WIDE) s_pos[rb + h] = (unsigned short)pos;
+                        }
+                    }
+                }
+                tsg_wave_sync();
+            }
+            tb += nt;
+        }
+    }
+    __syncthreads();
+    // two rows per wave, a long one with a short one; their A entries (row ra's
+    // first) are taken together, so products of both share a batch.  Rows
+    // without entries here, or left to k_step3_heavy, are not walked.
+    const int ra = s_ord[wave], rz = s_ord[15 - wave];
+    int xa = 0, na = 0, xz = 0, nz = 0;
+    if (s_rb[ra + 1] > s_rb[ra]) {
+        xa = Arowp[min(16 * I + ra, m)];
+        na = Arowp[min(16 * I + ra + 1, m)] - xa;
+    }
+    if (s_rb[rz + 1] > s_rb[rz]) {
+        xz = Arowp[min(16 * I + rz, m)];
+        nz = Arowp[min(16 * I + rz + 1, m)] - xz;
+    }
+    for (int xc = 0; xc < na + nz; xc += 64) {
+        int b0 = 0, len = 0, rb = 0, rs = 0;
+        double a = 0.0;
+        if (xc + lane < na + nz) {
+            const bool z = xc + lane >= na;
+            const int x = z ? xz + (xc + lane - na) : xa + xc + lane, r = z ? rz : ra;
+            const int k = Acolx[x];
+            a = Avalx[x];
+            b0 = Browp[k];
+            int b1 = Browp[k + 1];
+            rb = s_rb[r];
+            rs = s_rb[r + 1] - rb;
+            range_in(Bcolx, b0, b1, !first, col_lo, !last, col_hi);
+            len = b1 - b0;
+        }
+        const int incl = tsg_wave_incl_scan_dpp(len), pre = incl - len, delta = b0 - pre, reg = rb | rs << 16;
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        int prev = 0;
+        for (int base = 0; base < total; base += G3F_BATCH) {
+            s_mark[wave][lane] = 0u;
+            tsg_wave_sync();
+            if (len > 0 && pre >= base && pre < base + G3F_BATCH) mk[pre - base] = (unsigned char)(lane + 1);
+            tsg_wave_sync();
+            int q[G3F_ROUNDS], col[G3F_ROUNDS];
+            double b[G3F_ROUNDS];
+#pragma unroll
+            for (int i = 0; i < G3F_ROUNDS; i++) {
+                q[i] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * i + lane]));
+                prev = __builtin_amdgcn_readlane(q[i], 63);
+            }
+#pragma unroll
+            for (int i = 0; i < G3F_ROUNDS; i++) {  // every lane loads in bounds
+                const int e = __shfl(delta, q[i] - 1, 64) + min(base + 64 * i + lane, total - 1);
+                col[i] = Bcolx[e];
+                b[i] = Bvalx[e];
+            }
+#pragma unroll
+            for (int i = 0; i < G3F_ROUNDS; i++) {
+                if (base + 64 * i >= total) break;  // wave-uniform
+                const bool on = base + 64 * i + lane < total;
+                const double as = __shfl(a, q[i] - 1, 64);
+                const int rg = __shfl(reg, q[i] - 1, 64);
+                const unsigned *key0 = s_key + (rg & 0xffff);
+                const unsigned n_r = (unsigned)rg >> 16, key = (unsigned)(col[i] - col_lo) + 1u;
+                unsigned h = flat_home(key, n_r), ent;
+                unsigned probe = 0;
+                // (the entry is in C's structure: the probe bound is not reached)
+                while ((ent = key0[h], WIDE ? ent : ent >> 12) != key && ++probe < n_r) h = h + 1 == n_r ? 0u : h + 1;
+                const int pos = WIDE ? (int)s_pos[(rg & 0xffff) + h] : (int)(ent & 4095u);
+                const int q0 = __builtin_amdgcn_readlane(q[i], 0), q1 = __builtin_amdgcn_readlane(q[i], 63);
+                bool clash = false;
+                if (q0 != q1) {
+                    if (on) s_tag[pos] = (unsigned char)lane;
+                    tsg_wave_sync();
+                    clash = __ballot(on && s_tag[pos] != (unsigned char)lane) != 0;
+                }
+                if (!clash) {
+                    if (on) s_acc[pos] = __builtin_fma(as, b[i], s_acc[pos]);
+                } else {
+                    for (int s = q0; s <= q1; s++) {
+                        if (on && q[i] == s) s_acc[pos] = __builtin_fma(as, b[i], s_acc[pos]);
+                        tsg_wave_sync();
+                    }
+                }
+                tsg_wave_sync();
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += G3F_THREADS) Cval[(long long)nbase + i] = s_acc[i];
+}
+
 // ------------------------------------------------------------------ step 3, heavy rows
 // Rows with very many intermediate products (hub rows of power-law graphs)
 // would make every C segment of their tile-row re-walk the whole A row.
 // They are computed one wave at a time instead, in column parts of
 // HEAVY_PART_COLS columns whose FP64 accumulators live in the wave's own
 // LDS window: for part [lo, lo + HEAVY_PART_COLS) the wave walks A row i in
-// ascending k, its lanes adding a_ik * b_kj for the entries of B row k in
-// the part (distinct columns per k; LDS instructions of one wave complete
-// in order, so the next k reads what this one wrote), then copies the part
-// into C's final positions.  A work item is a run of consecutive parts of
-// one row; between parts the wave keeps, per A entry, the position in
-// B row k where the next part starts (a cursor in global scratch), so only
-// an item's first part searches B's rows.
+// ascending k, 64 entries (sources) at a time, and adds their products with
+// the B entries in the part as k_step3_flat does (numbered through, 64 per
+// step, source by source where two meet in one column), then copies the
+// part into C's final positions.  A work item is a run of consecutive parts
+// of one row; between parts the wave keeps, per A entry, the position in
+// B row k where the next part starts (a cursor in global scratch), so a
+// search starts there.  Against one source per step (22 of 64 lanes busy on
+// R-MAT scale 16, their first 8 entries staged through LDS): 13.6 -> 6.7 ms
+// there (120 G products/s); parts of 1024 / 2048 / 4096 columns 7.5 / 6.9 /
+// 8.4 ms, 4 / 8 rounds of loads in flight 6.9 / 6.7 ms.
 #define HEAVY_MIN_PRODUCTS 65536
 #ifndef HEAVY_PART_COLS
-#define HEAVY_PART_COLS 2048         // 16 KiB of LDS per wave, seven waves per CU
+#define HEAVY_PART_COLS 2048         // 19 KiB of LDS per wave, eight waves per CU
 #endif
 #define HEAVY_ITEM_PRODUCTS 32768    // products per work item, about
 #define HEAVY_MAX_WAVES 4096
@@ -1714,17 +1936,8 @@ k_heavy_list(const int *__restrict__ off, const unsigned char *__restrict__ flag
     }
 }
 
-#ifndef HEAVY_STAGE
-#define HEAVY_STAGE 8  // B entries per source staged in LDS per part
-#endif
-// lane q's double, read by the whole wave (q wave-uniform)
-__device__ __forceinline__ double rl_f64(double v, int q) {
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, q);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), q);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
+#define HEAVY_ROUNDS 8
+#define HEAVY_BATCH (64 * HEAVY_ROUNDS)
 __global__ void __launch_bounds__(64)
 k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const double *__restrict__ Avalx,
               const int *__restrict__ Browp, const int *__restrict__ Bcolx, const double *__restrict__ Bvalx,
@@ -1733,9 +1946,10 @@ k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
               const unsigned char *__restrict__ Cptr16, const int *__restrict__ Cnnz, double *__restrict__ Cval,
               int *__restrict__ cursor, long long cur_stride, int *__restrict__ next_item) {
     __shared__ double s_acc[HEAVY_PART_COLS];
-    __shared__ double s_sv[64 * HEAVY_STAGE];  // staged B values, source-major
-    __shared__ int s_sc[64 * HEAVY_STAGE];     // their columns
+    __shared__ unsigned char s_tag[HEAVY_PART_COLS];
+    __shared__ unsigned s_mark[HEAVY_BATCH / 4];
     const int lane = threadIdx.x;
+    unsigned char *mk = reinterpret_cast<unsigned char *>(s_mark);
     int *cur = cursor + (long long)blockIdx.x * cur_stride;
     const int ni = *nitems;
     // items are taken from a shared counter, so waves that drew short items
@@ -1755,141 +1969,66 @@ k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
             const int lo = colbase + part * HEAVY_PART_COLS, hi = lo + HEAVY_PART_COLS;
             for (int j = lane; j < HEAVY_PART_COLS; j += 64) s_acc[j] = 0.0;
             for (int xc = xa; xc < xe; xc += 64) {
-                // 64 A entries (sources) at once: lane q finds where B row k
-                // enters the part and stages its first HEAVY_STAGE entries
-                const int n = min(64, xe - xc);
-                int cb = 0, ce = 0, cnt = 0;
-                bool more = false;
-                double aq = 0.0;  // lane q: a_ik of source q
-                if (lane < n) {
+                // 64 A entries (sources) at once: lane q finds B row k's entries
+                // in the part
+                int b0 = 0, len = 0;
+                double a = 0.0;
+                if (xc + lane < xe) {
                     const int k = Acolx[xc + lane];
-                    aq = Avalx[xc + lane];
-                    ce = Browp[k + 1];
-                    cb = part == p0 ? lower_bound_i(Bcolx, Browp[k], ce, lo) : cur[xc - xa + lane];
-                    int col[HEAVY_STAGE];
-                    double val[HEAVY_STAGE];
-#pragma unroll
-                    for (int j = 0; j < HEAVY_STAGE; j++) {
-                        col[j] = cb + j < ce ? Bcolx[cb + j] : 0x7fffffff;
-                        val[j] = cb + j < ce ? Bvalx[cb + j] : 0.0;
-                    }
-#pragma unroll
-                    for (int j = 0; j < HEAVY_STAGE; j++) {
-                        const bool in = col[j] < hi;  // in-range entries form a prefix
-                        cnt += in;
-                        if (in) {
-                            s_sc[lane * HEAVY_STAGE + j] = col[j];
-                            s_sv[lane * HEAVY_STAGE + j] = val[j];
-                        }
-                    }
-                    more = cnt == HEAVY_STAGE && cb + HEAVY_STAGE < ce;
+                    a = Avalx[xc + lane];
+                    int b1 = Browp[k + 1];
+                    b0 = part == p0 ? Browp[k] : cur[xc - xa + lane];
+                    if (part != p0 && b1 - b0 > HEAVY_PART_COLS) b1 = b0 + HEAVY_PART_COLS;
+                    range_in(Bcolx, b0, b1, part == p0, lo, true, hi);
+                    len = b1 - b0;
+                    if (part + 1 < p1) cur[xc - xa + lane] = b1;
                 }
-                // lane q: staged entries of source q | more may follow << 8;
-                // read by the whole wave with v_readlane, not through LDS
-                const int nq = cnt | (more ? 256 : 0);
-                int next = cb + cnt;  // lane q: where source q's next part starts
-                // only sources with entries in the part take a step
-                unsigned long long act = __ballot(lane < n && cnt > 0);
-                tsg_wave_sync();
-                // the staged data of the next active source is read before this
-                // source's accumulation, which then costs one LDS round trip;
-                // so are the first 256 entries past a source's staged ones
-                // (global loads into registers, one source ahead)
-                auto tail_first = [&](int qq, int snq, int *tc, double *tv) {
+                const int incl = tsg_wave_incl_scan_dpp(len), pre = incl - len, delta = b0 - pre;
+                const int total = __builtin_amdgcn_readlane(incl, 63);
+                int prev = 0;
+                for (int base = 0; base < total; base += HEAVY_BATCH) {
 #pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        tc[u] = 0x7fffffff;
-                        tv[u] = 0.0;
+                    for (int v = 0; v < HEAVY_BATCH / 256; v++) s_mark[64 * v + lane] = 0u;
+                    tsg_wave_sync();
+                    if (len > 0 && pre >= base && pre < base + HEAVY_BATCH) mk[pre - base] = (unsigned char)(lane + 1);
+                    tsg_wave_sync();
+                    int q[HEAVY_ROUNDS], col[HEAVY_ROUNDS];
+                    double b[HEAVY_ROUNDS];
+#pragma unroll
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) {
+                        q[v] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * v + lane]));
+                        prev = __builtin_amdgcn_readlane(q[v], 63);
                     }
-                    if (snq & 256) {
-                        const int e = __builtin_amdgcn_readlane(cb, qq) + HEAVY_STAGE;
-                        const int e1 = __builtin_amdgcn_readlane(ce, qq);
 #pragma unroll
-                        for (int u = 0; u < 4; u++) {
-                            const int ee = e + 64 * u + lane;
-                            if (ee < e1) {
-                                tc[u] = Bcolx[ee];
-                                tv[u] = Bvalx[ee];
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) {  // every lane loads in bounds
+                        const int e = __shfl(delta, q[v] - 1, 64) + min(base + 64 * v + lane, total - 1);
+                        col[v] = Bcolx[e];
+                        b[v] = Bvalx[e];
+                    }
+#pragma unroll
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) {
+                        if (base + 64 * v >= total) break;  // wave-uniform
+                        const bool on = base + 64 * v + lane < total;
+                        const double as = __shfl(a, q[v] - 1, 64);
+                        const int p = col[v] - lo;
+                        const int q0 = __builtin_amdgcn_readlane(q[v], 0), q1 = __builtin_amdgcn_readlane(q[v], 63);
+                        bool clash = false;
+                        if (q0 != q1) {
+                            if (on) s_tag[p] = (unsigned char)lane;
+                            tsg_wave_sync();
+                            clash = __ballot(on && s_tag[p] != (unsigned char)lane) != 0;
+                        }
+                        if (!clash) {
+                            if (on) s_acc[p] = __builtin_fma(as, b[v], s_acc[p]);
+                        } else {
+                            for (int s = q0; s <= q1; s++) {  // sources in ascending k
+                                if (on && q[v] == s) s_acc[p] = __builtin_fma(as, b[v], s_acc[p]);
+                                tsg_wave_sync();
                             }
                         }
-                    }
-                };
-                int q = act ? __ffsll((long long)act) - 1 : 0;
-                int sn = act ? __builtin_amdgcn_readlane(nq, q) : 0, sc = 0;
-                double a = act ? rl_f64(aq, q) : 0.0, sv = 0.0;
-                if (lane < (sn & 255)) {
-                    sc = s_sc[q * HEAVY_STAGE + lane];
-                    sv = s_sv[q * HEAVY_STAGE + lane];
-                }
-                int tc[4];
-                double tv[4];
-                tail_first(q, sn, tc, tv);
-                while (act) {  // ascending k; entries of one k have distinct columns
-                    act &= act - 1;
-                    const int q1 = act ? __ffsll((long long)act) - 1 : 0;
-                    int sn1 = 0, sc1 = 0;
-                    double a1 = 0.0, sv1 = 0.0;
-                    if (act) {
-                        sn1 = __builtin_amdgcn_readlane(nq, q1);
-                        a1 = rl_f64(aq, q1);
-                        if (lane < (sn1 & 255)) {
-                            sc1 = s_sc[q1 * HEAVY_STAGE + lane];
-                            sv1 = s_sv[q1 * HEAVY_STAGE + lane];
-                        }
-                    }
-                    int tc1[4];
-                    double tv1[4];
-                    tail_first(q1, sn1, tc1, tv1);
-                    if (lane < (sn & 255)) s_acc[sc - lo] = __builtin_fma(a, sv, s_acc[sc - lo]);
-                    if (sn & 256) {  // entries past the staged ones, 256 per round trip
-                        int e = __builtin_amdgcn_readlane(cb, q) + HEAVY_STAGE;
-                        const int e1 = __builtin_amdgcn_readlane(ce, q);
-                        bool go;
-                        {  // the first round, loaded one source ahead
-                            int got = 0;
-#pragma unroll
-                            for (int u = 0; u < 4; u++) {
-                                const bool in2 = tc[u] < hi;
-                                if (in2) s_acc[tc[u] - lo] = __builtin_fma(a, tv[u], s_acc[tc[u] - lo]);
-                                got += __popcll(__ballot(in2));
-                            }
-                            e += got;
-                            go = got == 256;  // the part may hold more of this row
-                        }
-                        while (go && e < e1) {
-                            int c[4];
-                            double v[4];
-#pragma unroll
-                            for (int u = 0; u < 4; u++) {
-                                const int ee = e + 64 * u + lane;
-                                c[u] = ee < e1 ? Bcolx[ee] : 0x7fffffff;
-                                v[u] = ee < e1 ? Bvalx[ee] : 0.0;
-                            }
-                            int got = 0;
-#pragma unroll
-                            for (int u = 0; u < 4; u++) {
-                                const bool in2 = c[u] < hi;
-                                if (in2) s_acc[c[u] - lo] = __builtin_fma(a, v[u], s_acc[c[u] - lo]);
-                                got += __popcll(__ballot(in2));
-                            }
-                            e += got;
-                            if (got < 256) break;
-                        }
-                        if (lane == q) next = e;
-                    }
-                    tsg_wave_sync();  // the next k reads what this one wrote
-                    q = q1;
-                    sn = sn1;
-                    sc = sc1;
-                    a = a1;
-                    sv = sv1;
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        tc[u] = tc1[u];
-                        tv[u] = tv1[u];
+                        tsg_wave_sync();
                     }
                 }
-                if (part + 1 < p1 && lane < n) cur[xc - xa + lane] = next;
             }
             // the part's C entries of row i, into their final positions
             const int t0 = lower_bound_i(Ccol, c0, c1, lo >> 4), t1 = lower_bound_i(Ccol, t0, c1, hi >> 4);
@@ -2928,14 +3067,20 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
         if (ev) TSG_HIP(hipEventRecord(ev[1], s));
     }
     if (!P.all && P.s3_unfit && P.s3_elem) {
-        TSG_TRY(launch_segments(s, C, w, 0, G3E_NNZ, w.rowcls));
         const bool rx = op.Arowp != nullptr;
-        hipLaunchKernelGGL(P.s3pk ? (rx ? k_step3_elem<true, true> : k_step3_elem<true, false>)
-                                  : (rx ? k_step3_elem<false, true> : k_step3_elem<false, false>),
-                           dim3((unsigned)w.seg3_cap), dim3(256), 0, s, op, (const int *)B->rowx_ptr,
-                           (const int *)B->rowx_col, (const double *)B->rowx_val, C->m, (const int4 *)w.seg3,
-                           (const int *)(w.segcnt + C->tilem), C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
-                           C->tile_nnz, C->csr_col, C->val, (const unsigned char *)w.hflag);
+        TSG_TRY(launch_segments(s, C, w, 0, rx ? G3F_NNZ : G3E_NNZ, w.rowcls));
+        if (rx)
+            hipLaunchKernelGGL(P.s3span < G3F_SPAN ? k_step3_flat<false> : k_step3_flat<true>, dim3((unsigned)w.seg3_cap), dim3(G3F_THREADS), 0, s, op.Arowp, op.Acolx,
+                               op.Avalx, (const int *)B->rowx_ptr, (const int *)B->rowx_col,
+                               (const double *)B->rowx_val, C->m, (const int4 *)w.seg3,
+                               (const int *)(w.segcnt + C->tilem), C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
+                               C->tile_nnz, C->csr_col, C->val, (const unsigned char *)w.hflag);
+        else
+            hipLaunchKernelGGL(P.s3span < G3E_PK_SPAN ? k_step3_elem<true> : k_step3_elem<false>,
+                               dim3((unsigned)w.seg3_cap), dim3(256), 0, s, op, (const int *)B->rowx_ptr,
+                               (const int *)B->rowx_col, (const double *)B->rowx_val, C->m, (const int4 *)w.seg3,
+                               (const int *)(w.segcnt + C->tilem), C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
+                               C->tile_nnz, C->csr_col, C->val);
         TSG_LAUNCH_CHECK();
         if (w.hflag && w.nitems > 0) {
             hipLaunchKernelGGL(k_step3_heavy, dim3(w.hwaves), dim3(64), 0, s, op.Arowp, op.Acolx, op.Avalx,
@@ -3085,7 +3230,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         const int umax = smax[0], span = smax[1], mspan = smax[2];
         P.s2u = std::max(1, umax);
         P.s2map = umax <= 256 ? mspan : 0;
-        P.s3pk = span < G3E_PK_SPAN ? 1 : 0;
+        P.s3span = span;
         for (int k = 0; k < S2_KINDS; k++) P.n2[k] = smax[3 + k];
         P.s2w = smax[7];
     }

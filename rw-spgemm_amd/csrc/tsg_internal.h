@@ -145,7 +145,7 @@ struct tsg_spgemm_plan {
     int s2map;      // bytes of the step-2 column -> slot map (0: binary search)
     int n2[4];      // step-2 segments per kernel (step2_kind)
     int s2w;        // widest tile-row span of the dense step 2's small blocks
-    int s3pk;       // element step 3 packs hash keys and positions (narrow tile-rows)
+    int s3span;     // widest tile-column span of a tile-row (hash key widths of step 3)
 };
 // symbolic = true runs steps 1-2 and the step-3 plan only (C's values and
 // in-tile columns stay unallocated); stats (when given) then holds C's exact
@@ -301,6 +301,37 @@ __device__ __forceinline__ int emit_window(const unsigned *bm, int nw, int w0, i
         done += tot;
     }
     return done;
+}
+// The 16 row lengths of a tile, one byte each, from its row offsets: next
+// offset minus offset, byte by byte.  Offsets ascend, so no borrow crosses a
+// byte; the last byte's minuend is the entry count (mod 256).
+__device__ __forceinline__ uint4 tile_row_lens(uint4 p, int tnnz) {
+    return make_uint4(((p.x >> 8) | (p.y << 24)) - p.x, ((p.y >> 8) | (p.z << 24)) - p.y,
+                      ((p.z >> 8) | (p.w << 24)) - p.z, ((p.w >> 8) | ((unsigned)tnnz << 24)) - p.w);
+}
+// Bytes as 16-bit pairs: v[2q] = rows 4q and 4q+2, v[2q+1] = rows 4q+1, 4q+3.
+__device__ __forceinline__ void tile_widen_lens(uint4 l, unsigned v[8]) {
+    const unsigned w[4] = {l.x, l.y, l.z, l.w};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        v[2 * q] = w[q] & 0x00ff00ffu;
+        v[2 * q + 1] = (w[q] >> 8) & 0x00ff00ffu;
+    }
+}
+
+// v's entry for row r (0..15)
+__device__ __forceinline__ int tile_row_of(const unsigned v[8], int r) {
+    unsigned x = 0;
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+        if (2 * (r >> 2) + (r & 1) == q) x = v[q];
+    return (int)((r & 2) ? x >> 16 : x & 0xffffu);
+}
+// Bytes of w that are at most j, as 0x80 bits (unsigned, per byte).
+__device__ __forceinline__ unsigned bytes_le(unsigned w, unsigned j) {
+    const unsigned H = 0x80808080u, x = j * 0x01010101u;
+    const unsigned t = (x | H) - (w & ~H);  // per byte, no borrow out
+    return ((x & ~w) | (~(x ^ w) & t)) & H;
 }
 // Value of lane q of this lane's group of 16 lanes (q a constant after
 // unrolling): a DPP row broadcast, a VALU move with no LDS traffic, where
