@@ -13,7 +13,9 @@
 //   the u8 row offsets and tile nnz.  Tile-rows with more C tiles than LDS
 //   holds use k_step2_tiles (one C tile per 16-lane group, pairs from a
 //   sorted-list intersection, 64-bit ballots to keep them in K order).
-// Step 3 (numeric, src/tilespgemm-cuda.h:1505-2608): k_step3_rows, one
+// Step 3 (numeric, src/tilespgemm-cuda.h:1505-2608): k_step3_lines, one block
+//   per C tile-row, adds B rows line by line (both row indices needed);
+//   without them k_step3_rows, one
 //   block per C tile-row, accumulates the row's C values in LDS in their
 //   final order; each C row belongs to one wave, which takes its tasks in
 //   ascending K.  A tile K with several entries has A tile K and B tile-row
@@ -30,6 +32,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "tsg_internal.h"
 
@@ -53,10 +56,11 @@ extern "C" void tsg_tune_default(tsg_tune *t) {
 // every row's room without a scan.  Two launches (graph-capturable, every
 // word of a kept row written once, no memset): k_brow_desc, one lane per
 // tile-row, then k_brow_fill, one lane per B tile, so a hub tile-row's
-// words are spread over as many waves as it has tiles.
+// words are spread over as many waves as it has tiles.  With longest (and B's
+// row pointers), longest[K] = entries of the longest row of tile-row K.
 __global__ void __launch_bounds__(256)
 k_brow_desc(const int *__restrict__ Bptr, const int *__restrict__ Bcol, int tilem, int4 *__restrict__ desc,
-            int *__restrict__ any) {
+            int *__restrict__ any, const int *__restrict__ Browp, int m, int *__restrict__ longest) {
     const int K = blockIdx.x * 256 + threadIdx.x;
     int nw = 0;
     if (K < tilem) {
@@ -68,6 +72,22 @@ k_brow_desc(const int *__restrict__ Bptr, const int *__restrict__ Bcol, int tile
             if (nw > 2 * n + 2) nw = 0;
         }
         desc[K] = make_int4(2 * b0 + 2 * K, F, nw, 0);
+        if (longest) {
+            int p = Browp[16 * K], mx = 0;
+            if (16 * K + 16 <= m) {
+                int q[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++) q[r] = Browp[16 * K + 1 + r];
+#pragma unroll
+                for (int r = 0; r < 16; r++) mx = max(mx, q[r] - (r ? q[r - 1] : p));
+            } else {
+                for (int r = 16 * K + 1; r <= m; r++) {
+                    mx = max(mx, Browp[r] - p);
+                    p = Browp[r];
+                }
+            }
+            longest[K] = mx;
+        }
     }
     // any (may be NULL, zeroed beforehand): set when some row is kept; the
     // same value from every writer, and no store once it reads 1
@@ -2558,30 +2578,300 @@ k_step3_rows(TileOperands op, const int *__restrict__ Cptr, const int *__restric
 }
 #undef SROW
 
+// ------------------------------------------------------------------ step 3, row lines
+// One block per C tile-row with at most LN_UMAX C tiles and LN_NNZ C
+// nonzeros, from A's and B's row index.  A group of G lanes (16, 32 or 64:
+// the first that holds the longest B row the tile-row meets, above 64 in two
+// pieces) owns a C row: it takes the row's A entries k in ascending order, one
+// per step, its lanes the entries of B row k, and adds the products to the
+// row's entries in LDS.  One B row never meets an entry of C twice and groups
+// never share one, so there are no atomics and no checks, and every C entry
+// sums its products in ascending k.
+//   Sources (A entries) are held 16 at a time, one per lane and the same in
+// every 16 lanes of the group, so that a source reaches its group by a DPP row
+// broadcast folded into its use, and the LDS takes only the five accesses
+// below.  B rows are loaded four steps ahead.
+//   Position of a product: the slot of its tile column from a byte map of
+// the columns modulo a power of two (binary search in a tile-row wider than
+// the map whose columns collide there), then one word with the C row's mask
+// and offset in that tile: offset + bits of the mask before the column.
+// Values are summed in final order with a gap after every 16, which moves
+// the equal tiles of a stencil to different LDS banks; the column byte is
+// left beside the sum.  Both are written out as one run, past the L2 (it
+// holds the B rows that the next tile-rows read again: 2.26 -> 2.06 ms).
+//   Four blocks (32 waves) a CU; VALU issue, LDS and L1 accesses are each
+// busy a half to two thirds of the time.  27-point 128^3 periodic 4.00 ms by
+// k_step3_rows -> 2.06 (1.5 G products, 729 a C row), 61x47x53 385 -> 133 us,
+// banded 39989 (half-bandwidth 20) 165 us by k_step3_flat -> 97.  With the
+// sources broadcast by ds_bpermute (four more LDS accesses) 2.65 ms, with 80
+// registers and six waves a SIMD 2.19.
+#define LN_THREADS 512
+#define LN_UMAX 256      // u8 slots
+#define LN_NNZ 4096      // 34 KiB of sums; offsets of a tile row fit 15 bits
+#define LN_MAP 8192      // bytes of the largest column map
+#define LN_MAP_MIN 1024  // any slot byte stays inside LDS behind the mask words
+#define LN_ANNZ 2048     // A entries of the tile-row (one row's are a serial chain)
+#define LN_BROW 128      // entries of a B row: two pieces of 64
+// Lanes idle where the longest B row is far from the mean: k_step3_flat is
+// the better one there.  R-MAT scale 11 A*A^T whole product 388 us with 2 *
+// mean + 16, 401 with 4 *, and 388 without row lines; ER (Poisson rows, means 4
+// to 14) 102..150 us against 137..197 by k_step3_flat.
+#define LN_SKEW 2
+#define LN_SKEW0 16
+#define LN_CLASS 4       // row class LN_CLASS + g: groups of 16 << g lanes
+struct LinesLayout {
+    int nnz, umax, map;
+};
+// LDS (all of it dynamic, so from address 0): the byte of entry p is at base +
+// p, its sum at 8 * ln_pos(base + p): with base a multiple of 16 the sums start
+// at 8.5 * base, behind the bytes, and one register addresses both.  Word 0
+// is the collision flag.
+__host__ __device__ inline int ln_pos(int p) { return p + (p >> 4); }
+__host__ __device__ inline size_t lines_layout(const LinesLayout &L, int *base, size_t off[4]) {
+    *base = ((L.nnz + 8) * 2 / 15 + 16) & ~15;
+    off[0] = 8 * (size_t)ln_pos(*base);                                   // sums
+    off[1] = 8 * (size_t)(ln_pos(*base + L.nnz) + 1);                     // mask and offset words, [row][tile]
+    off[2] = off[1] + 64 * (size_t)L.umax;                                // tile columns
+    off[3] = off[2] + 4 * (size_t)L.umax;                                 // column map
+    return off[3] + (size_t)L.map;
+}
+__global__ void __launch_bounds__(LN_THREADS, 8)
+k_step3_lines(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const double *__restrict__ Avalx,
+              const int *__restrict__ Browp, const int *__restrict__ Bcolx, const double *__restrict__ Bvalx, int m,
+              int tilem, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
+              const unsigned short *__restrict__ Cmask, const unsigned char *__restrict__ Cptr16,
+              const int *__restrict__ Cnnz, const unsigned char *__restrict__ rowcls,
+              unsigned char *__restrict__ Ccol8, double *__restrict__ Cval, LinesLayout L) {
+    extern __shared__ __align__(16) unsigned char s_lds[];
+    typedef __attribute__((address_space(3))) double *lds_f64;
+    typedef __attribute__((address_space(3))) unsigned char *lds_u8;
+    int base;
+    size_t off[4];
+    lines_layout(L, &base, off);
+    int *s_flag = reinterpret_cast<int *>(s_lds);
+    unsigned char *s_byte = s_lds + base;
+    double *s_acc = reinterpret_cast<double *>(s_lds + off[0]);
+    unsigned *s_meta = reinterpret_cast<unsigned *>(s_lds + off[1]);
+    int *s_col = reinterpret_cast<int *>(s_lds + off[2]);
+    unsigned char *s_map = s_lds + off[3];
+    const int I = (int)tsg_xcd_block(blockIdx.x, gridDim.x);
+    if (I >= tilem) return;
+    const int cls = rowcls[I];
+    if (cls < LN_CLASS) return;  // block-uniform
+    const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x;
+    const int gl = 4 + cls - LN_CLASS, G = 1 << gl;
+    const int t = tid & (G - 1), ngrp = nt >> gl;
+    const int c0 = Cptr[I], u = Cptr[I + 1] - c0;
+    const int nbase = Cnnz[c0], nrow = Cnnz[c0 + u] - nbase;
+    const int span = Ccol[c0 + u - 1] - Ccol[c0] + 1;
+    const unsigned mapbits = 31 - __clz(L.map);
+    // sources of the group's row, 16 lanes deep: [b0, last] its B row (a lane
+    // without one: a far b0 and entry 0), k and av those of the next 16
+    int x1 = 0, xk = 0, kk = -1, b0 = 0, last = 0;
+    double a = 0.0, av = 0.0;
+    auto fetch = [&]() {  // A entries xk + lane
+        kk = -1;
+        av = 0.0;
+        if (xk + (lane & 15) < x1) {
+            kk = Acolx[xk + (lane & 15)];
+            av = Avalx[xk + (lane & 15)];
+        }
+        xk += 16;
+    };
+    int p0 = 0, p1 = 0;
+    double an = 0.0;
+    auto bounds = [&]() {  // their B rows
+        p0 = p1 = 0;
+        if (kk >= 0) {
+            p0 = Browp[kk];
+            p1 = Browp[kk + 1];
+        }
+        an = av;
+    };
+    auto take = [&]() {
+        a = an;
+        b0 = p1 > p0 ? p0 : 0x40000000;
+        last = p1 > p0 ? p1 - 1 : 0;
+    };
+    auto start = [&](int r) {
+        const int row = 16 * I + r;
+        xk = x1 = 0;
+        if (r < 16 && row < m) {
+            xk = Arowp[row];
+            x1 = Arowp[row + 1];
+        }
+        fetch();
+    };
+    int r = tid >> gl;
+    start(r);
+    bounds();
+    fetch();
+    if (tid == 0) *s_flag = 0;
+    for (int i = tid; i < ln_pos(nrow) + 1; i += nt) s_acc[i] = 0.0;
+    for (int i = tid; i < u; i += nt) {
+        const long long c = c0 + i;
+        const int J = Ccol[c], at = base + Cnnz[c] - nbase;
+        const uint4 m0 = reinterpret_cast<const uint4 *>(Cmask)[2 * c], m1 = reinterpret_cast<const uint4 *>(Cmask)[2 * c + 1];
+        const uint4 p = reinterpret_cast<const uint4 *>(Cptr16)[c];
+        const unsigned mw[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+        const unsigned pw[4] = {p.x, p.y, p.z, p.w};
+        s_col[i] = J;
+        s_map[(unsigned)J & (L.map - 1)] = (unsigned char)i;
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            // bits 30..15: columns 0..15; bits 14..0: base + offset
+            const unsigned mk = q & 1 ? (mw[q >> 1] >> 1) & 0x7fff8000u : (mw[q >> 1] & 0xffffu) << 15;
+            s_meta[q * L.umax + i] = mk | (unsigned)(at + (int)((pw[q >> 2] >> (8 * (q & 3))) & 255u));
+        }
+    }
+    __syncthreads();
+    // consecutive columns never collide in the map; others are looked at
+    bool direct = span <= L.map;
+    if (!direct) {
+        for (int i = tid; i < u; i += nt)
+            if (s_map[(unsigned)s_col[i] & (L.map - 1)] != i) *s_flag = 1;
+        __syncthreads();
+        direct = *s_flag == 0;
+    }
+    for (; r < 16; r += ngrp) {
+        const unsigned *meta = s_meta + r * L.umax;
+        auto slot_search = [&](int J) -> int {
+            int lo = 0, hi = u - 1;  // J is in the list
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (s_col[mid] < J) lo = mid + 1; else hi = mid;
+            }
+            return lo;
+        };
+        // a lane past its B row may look up any column: every read stays in LDS
+        auto slot_map = [&](int col) -> int { return s_map[__builtin_amdgcn_ubfe((unsigned)col, 4, mapbits)]; };
+        auto place = [&](unsigned w, int col) -> int {
+            return (int)(w & 0x7fffu) + __popc(w >> ((~col & 15) | 16));
+        };
+        auto add = [&](int pos, int col, double as, double b) {
+            lds_f64 p = (lds_f64)(unsigned)(ln_pos(pos) << 3);
+            *p = __builtin_fma(as, b, *p);
+            *(lds_u8)(unsigned)pos = (unsigned char)col;  // low four bits: the column in its tile
+        };
+        for (;;) {
+            take();
+            const unsigned long long has = __ballot(b0 < 0x40000000), cnt = __ballot(x1 > xk - 32 + (lane & 15));
+            if (!__any(x1 > xk - 32)) break;
+            // steps: the longest row of the wave decides
+            unsigned long long fold = cnt | cnt >> 32;
+            fold |= fold >> 16;
+            const int ns = 32 - __clz((int)(fold & 0xffffu));
+            bounds();
+            fetch();
+            // batches of four loads, one batch in flight ahead of the one that is
+            // added: four sources, or two with two pieces each
+            auto batches = [&](auto two) {
+                constexpr int P = decltype(two)::value ? 2 : 1;
+                int col[2][4];
+                bool on[2][4];  // an entry of the B row
+                double b[2][4];
+                auto load = [&](int s, int w) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int e = tsg_row16_bcast(b0, s + i / P) + t + (i % P) * G;
+                        const int ec = min(e, tsg_row16_bcast(last, s + i / P));
+                        on[w][i] = e == ec;
+                        col[w][i] = Bcolx[(unsigned)ec];
+                        b[w][i] = Bvalx[(unsigned)ec];
+                    }
+                };
+                load(0, 0);
+#pragma unroll
+                for (int s = 0; s < 16; s += 4 / P) {
+                    if (s >= ns) break;
+                    const int w = (s * P >> 2) & 1;
+                    if (s + 4 / P < 16 && s + 4 / P < ns) load(s + 4 / P, w ^ 1);
+                    int pos[4];
+                    unsigned mw[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) mw[i] = meta[slot_map(col[w][i])];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        pos[i] = place(mw[i], col[w][i]);
+                        asm("" : "+v"(pos[i]));  // of every lane: not sunk into a branch each
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const double as = tsg_row16_bcast(a, s + i / P);
+                        if (on[w][i]) add(pos[i], col[w][i], as, b[w][i]);
+                        tsg_wave_sync();
+                    }
+                }
+            };
+            if (direct && __any(last - b0 >= G)) {
+                batches(std::true_type{});
+            } else if (direct && has) {
+                batches(std::false_type{});
+            } else {  // columns that collide in the map
+                for (int s = 0; s < ns; s++) {
+                    const int at = (lane & 48) + s;
+                    const int bs = __shfl(b0, at, 64), be = __shfl(last, at, 64);
+                    const double as = __shfl(a, at, 64);
+                    for (int e = bs + t; e <= be; e += G) {
+                        const int c = Bcolx[e];
+                        add(place(meta[slot_search(c >> 4)], c), c, as, Bvalx[e]);
+                    }
+                    tsg_wave_sync();
+                }
+            }
+        }
+        if (r + ngrp < 16) {
+            start(r + ngrp);
+            bounds();
+            fetch();
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < nrow; i += nt) __builtin_nontemporal_store(s_acc[ln_pos(i)], Cval + (long long)nbase + i);
+    // column bytes, by the words of the run
+    const int head = (4 - (nbase & 3)) & 3;  // bytes before the first whole word
+    unsigned char *out = Ccol8 + nbase;
+    const int words = max(0, nrow - head) >> 2;
+    for (int i = tid; i < words; i += nt) {
+        const unsigned *w = reinterpret_cast<const unsigned *>(s_byte) + i;
+        const unsigned v = head ? __builtin_amdgcn_alignbyte(w[1], w[0], head) : w[0];
+        __builtin_nontemporal_store(v & 0x0f0f0f0fu, reinterpret_cast<unsigned *>(out + head) + i);
+    }
+    if (tid < 8) {  // the ragged ends
+        const int i = tid < 4 ? tid : head + 4 * words + tid - 4;
+        if (i < nrow && (tid < 4 ? i < head : true)) out[i] = s_byte[i] & 15;
+    }
+}
+
 // Step-3 class of every C tile-row: 1 = row-wise kernel (its C tiles, C
 // nonzeros, A tiles and B tile-rows are within the G3 caps), 0 = tile-parallel
-// kernel, 2 = nothing to compute.  Per block, part[8 * block + i]: i = 0 the
-// class-0 rows, i = 1..6 the maxima
+// kernel, 2 = nothing to compute, LN_CLASS + g = row lines with groups of 16 <<
+// g lanes (lines set: both operands carry their row index).  Per block,
+// part[CLS_WORDS * block + i]: i = 0 the class-0 rows, i = 1..6 the maxima
 // over class-1 rows of (nonempty C tiles, C nonzeros plus accumulator pads,
 // A tiles, B tiles per B tile-row, B nonzeros per B tile-row, A tile
-// nonzeros) for the LDS layout.
+// nonzeros) for the LDS layout, i = 7..10 those over the row-lines rows of (C
+// nonzeros, C tiles, tile-column span, g + 1).
 // 16 lanes per tile-row (16 tile-rows per block): the lanes walk the row's A
 // tiles and C tiles in strides of 16, so the dependent loads of different A
 // tiles are in flight together.  k_row_class_reduce folds the blocks' partials
-// into out[0] (sum) and out[1..6] (maxima): no atomics, which on one cache
+// into out[0] (sum) and out[1..] (maxima): no atomics, which on one cache
 // line would serialise across the thousands of blocks.
+#define CLS_WORDS 11
 __device__ __forceinline__ int g16_max(int v) {
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 16));
     return v;
 }
 __global__ void __launch_bounds__(256)
-k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tilem,
-            unsigned char *__restrict__ cls, int *__restrict__ part, int none_fit) {
-    __shared__ int s_red[4][7];
+k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict__ Ccol, const int *__restrict__ Cnnz, int tilem,
+            unsigned char *__restrict__ cls, int *__restrict__ part, int none_fit,
+            const int *__restrict__ longest) {
+    __shared__ int s_red[4][CLS_WORDS];
     const int r = threadIdx.x & 15, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int I = blockIdx.x * 16 + (threadIdx.x >> 4);
     int unfit = 0, mu = 0, mn = 0, ml = 0, mq = 0, mb = 0, ma = 0;
+    int ln = 0, lu = 0, ls = 0, lg = 0;
     if (I < tilem) {  // uniform in the 16-lane group
         const int c0 = Cptr[I], c1 = Cptr[I + 1];
         const int nrow = Cnnz[c1] - Cnnz[c0];
@@ -2591,6 +2881,23 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
         } else {
             const int a0 = op.Aptr[I], a1 = op.Aptr[I + 1];
             bool ok = !none_fit && c1 - c0 <= G3_UMAX && nrow <= G3_NNZMAX && a1 - a0 <= G3_LAMAX;
+            if (longest && c1 - c0 <= LN_UMAX && nrow <= LN_NNZ && op.Annz[a1] - op.Annz[a0] <= LN_ANNZ) {  // group-uniform
+                int mx = 0, sum = 0;
+                for (int p = a0 + r; p < a1; p += 16) {
+                    const int K = op.Acol[p];
+                    mx = max(mx, longest[K]);
+                    sum += op.Bnnz[op.Bptr[K + 1]] - op.Bnnz[op.Bptr[K]];
+                }
+                mx = g16_max(mx);
+                const int mean = tsg_group16_sum(sum) / (16 * max(a1 - a0, 1)), g = mx <= 16 ? 0 : mx <= 32 ? 1 : 2;
+                if (mx <= LN_BROW && mx <= LN_SKEW * mean + LN_SKEW0) {
+                    lg = g + 1;
+                    ln = nrow;
+                    lu = c1 - c0;
+                    ls = Ccol[c1 - 1] - Ccol[c0] + 1;
+                    ok = false;
+                }
+            }
             if (ok) {  // group-uniform
                 int bad = 0, lq = 0, lbn = 0, lan = 0, ne = 0;
                 for (int p = a0 + r; p < a1; p += 16) {
@@ -2618,7 +2925,7 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
                     mu = ne; mn = nrow + nbig; ml = a1 - a0; mq = lq; mb = lbn; ma = lan;
                 }
             }
-            k = ok ? 1 : 0;
+            k = lg ? LN_CLASS + lg - 1 : ok ? 1 : 0;
         }
         if (r == 0) cls[I] = k;
         unfit = r == 0 && k == 0;
@@ -2626,50 +2933,49 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
     unfit = tsg_wave_sum(unfit);
     mu = tsg_wave_max(mu); mn = tsg_wave_max(mn); ml = tsg_wave_max(ml);
     mq = tsg_wave_max(mq); mb = tsg_wave_max(mb); ma = tsg_wave_max(ma);
+    ln = tsg_wave_max(ln); lu = tsg_wave_max(lu); ls = tsg_wave_max(ls); lg = tsg_wave_max(lg);
     if (lane == 0) {
         s_red[wave][0] = unfit; s_red[wave][1] = mu; s_red[wave][2] = mn; s_red[wave][3] = ml;
         s_red[wave][4] = mq; s_red[wave][5] = mb; s_red[wave][6] = ma;
+        s_red[wave][7] = ln; s_red[wave][8] = lu; s_red[wave][9] = ls; s_red[wave][10] = lg;
     }
     __syncthreads();
-    if (threadIdx.x < 8) {
+    if (threadIdx.x < CLS_WORDS) {
         const int i = threadIdx.x;
-        int v = 0;
-        if (i < 7) {
-            v = s_red[0][i];
+        int v = s_red[0][i];
 #pragma unroll
-            for (int w = 1; w < 4; w++) v = i == 0 ? v + s_red[w][i] : max(v, s_red[w][i]);
-        }
-        part[8 * (long long)blockIdx.x + i] = v;
+        for (int w = 1; w < 4; w++) v = i == 0 ? v + s_red[w][i] : max(v, s_red[w][i]);
+        part[CLS_WORDS * (long long)blockIdx.x + i] = v;
     }
 }
 
-// out[0] = sum and out[1..6] = maxima of the nb blocks' k_row_class partials
-// (one block of 1024 threads); out[7] = 0.  host (may be NULL): pinned
-// memory that gets the eight words too.
+// out[0] = sum and out[1..] = maxima of the nb blocks' k_row_class partials
+// (one block of 1024 threads).  host (may be NULL): pinned memory that gets
+// the CLS_WORDS words too.
 __global__ void __launch_bounds__(1024)
 k_row_class_reduce(const int *__restrict__ part, int nb, int *__restrict__ out, int *__restrict__ host) {
-    __shared__ int s_r[16][7];
-    int v[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (int b = threadIdx.x; b < nb; b += 1024) {
-        v[0] += part[8 * (long long)b];
+    __shared__ int s_r[16][CLS_WORDS];
+    int v[CLS_WORDS];
 #pragma unroll
-        for (int i = 1; i < 7; i++) v[i] = max(v[i], part[8 * (long long)b + i]);
+    for (int i = 0; i < CLS_WORDS; i++) v[i] = 0;
+    for (int b = threadIdx.x; b < nb; b += 1024) {
+        const int *p = part + CLS_WORDS * (long long)b;
+        v[0] += p[0];
+#pragma unroll
+        for (int i = 1; i < CLS_WORDS; i++) v[i] = max(v[i], p[i]);
     }
     v[0] = tsg_wave_sum(v[0]);
 #pragma unroll
-    for (int i = 1; i < 7; i++) v[i] = tsg_wave_max(v[i]);
+    for (int i = 1; i < CLS_WORDS; i++) v[i] = tsg_wave_max(v[i]);
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
-        for (int i = 0; i < 7; i++) s_r[wave][i] = v[i];
+        for (int i = 0; i < CLS_WORDS; i++) s_r[wave][i] = v[i];
     __syncthreads();
-    if (threadIdx.x < 8) {
+    if (threadIdx.x < CLS_WORDS) {
         const int i = threadIdx.x;
-        int r = 0;
-        if (i < 7) {
-            r = s_r[0][i];
-            for (int w = 1; w < 16; w++) r = i == 0 ? r + s_r[w][i] : max(r, s_r[w][i]);
-        }
+        int r = s_r[0][i];
+        for (int w = 1; w < 16; w++) r = i == 0 ? r + s_r[w][i] : max(r, s_r[w][i]);
         out[i] = r;
         if (host) host[i] = r;
     }
@@ -2843,14 +3149,15 @@ static size_t brow_bits_bytes(const tsg_dtiles *B) {
     return (size_t)B->tilem * 16 + (size_t)words * 4;
 }
 static int launch_brow_bits(hipStream_t s, const tsg_dtiles *B, void *buf, const int4 **desc,
-                            const unsigned **bits, int *any) {
+                            const unsigned **bits, int *any, int *longest) {
     *desc = nullptr;
     *bits = nullptr;
     if (!buf || !brow_bits_bytes(B)) return TSG_OK;
     int4 *d = (int4 *)buf;
     unsigned *w = (unsigned *)((char *)buf + (size_t)B->tilem * 16);
     hipLaunchKernelGGL(k_brow_desc, dim3(tsg_div_up(B->tilem, 256)), dim3(256), 0, s, (const int *)B->tile_ptr,
-                       (const int *)B->tile_colidx, B->tilem, d, any);
+                       (const int *)B->tile_colidx, B->tilem, d, any, (const int *)B->rowx_ptr, B->m,
+                       B->rowx_ptr ? longest : nullptr);
     if (B->numtile > 0)
         hipLaunchKernelGGL(k_brow_fill, dim3(tsg_div_up(B->numtile, 256)), dim3(256), 0, s,
                            (const int *)B->tile_rowidx, (const int *)B->tile_colidx, (long long)B->numtile,
@@ -2903,8 +3210,9 @@ struct SpgemmWork {
     int *segctr;       // S2_KINDS step-2 segment counters
     unsigned char *rowcls;
     int *cls_out;
-    int *cls_part;  // k_row_class partials, 8 ints per block
+    int *cls_part;  // k_row_class partials, CLS_WORDS ints per block
     void *bbits;       // B's tile-row bitmaps for step 1 (may be NULL)
+    int *longest;      // longest row of each B tile-row (enqueue-only pipeline)
     int4 *seg2;        // step-2 segments
     unsigned *bmstore; // step-1 bitmaps kept from the count pass (may be NULL)
     int4 *seg3;        // step-3 element segments
@@ -2927,14 +3235,14 @@ static size_t up16(size_t x) { return (x + 15) & ~(size_t)15; }
 #define WORK_NARR 12
 
 static size_t work_layout(long long tilem, long long numtile, long long nnz, size_t off[WORK_NARR],
-                          int s1w = 256, size_t bbytes = 0) {
+                          int s1w = 256, size_t bbytes = 0, size_t longest_bytes = 0) {
     const size_t sz[WORK_NARR] = {
         8 * (size_t)tsg_scan_partial_count(tilem), 8 * (size_t)tsg_scan_partial_count(numtile),
-        8 * (size_t)tsg_scan_partial_count(tilem), 4 * ((size_t)tilem + 1), (size_t)tilem + 1, 32,
+        8 * (size_t)tsg_scan_partial_count(tilem), 4 * ((size_t)tilem + 1), (size_t)tilem + 1, 4 * CLS_WORDS,
         16 * (size_t)seg2_bound(tilem, numtile),
         keep_bytes(tilem, s1w),  // step-1 bitmaps (enqueue-only pipeline)
-        32 * (size_t)((tilem + 15) / 16 + 1),  // row-class partials, 8 ints per block
-        bbytes,                                // B's tile-row bitmaps (enqueue-only pipeline)
+        4 * CLS_WORDS * (size_t)((tilem + 15) / 16 + 1),  // row-class partials
+        bbytes + longest_bytes,                // B's tile-row bitmaps, longest rows (enqueue-only pipeline)
         4 * S2_KINDS,
         16 * (size_t)(tilem + nnz / (G3E_NNZ - 255) + 2)};
     size_t o = 0;
@@ -2946,9 +3254,9 @@ static size_t work_layout(long long tilem, long long numtile, long long nnz, siz
 }
 
 static SpgemmWork work_at(void *base, long long tilem, long long numtile, long long nnz, void *seg3_base,
-                          int s1w = 256, size_t bbytes = 0) {
+                          int s1w = 256, size_t bbytes = 0, size_t longest_bytes = 0) {
     size_t off[WORK_NARR];
-    work_layout(tilem, numtile, nnz, off, s1w, bbytes);
+    work_layout(tilem, numtile, nnz, off, s1w, bbytes, bbytes ? longest_bytes : 0);
     char *b = (char *)base;
     SpgemmWork w;
     w.part1 = (long long *)(b + off[0]);
@@ -2961,6 +3269,7 @@ static SpgemmWork work_at(void *base, long long tilem, long long numtile, long l
     w.bmstore = keep_bytes(tilem, s1w) ? (unsigned *)(b + off[7]) : nullptr;
     w.cls_part = (int *)(b + off[8]);
     w.bbits = bbytes ? (void *)(b + off[9]) : nullptr;
+    w.longest = bbytes ? (int *)(b + off[9] + bbytes) : nullptr;
     w.segctr = (int *)(b + off[10]);
     w.seg3 = (int4 *)(seg3_base ? (char *)seg3_base : b + off[11]);
     w.seg3_cap = tilem + nnz / (G3E_NNZ - 255) + 2;
@@ -3040,10 +3349,10 @@ static int launch_step2(hipStream_t s, const TileOperands &op, const tsg_dtiles 
 }
 
 static int launch_row_class(hipStream_t s, const TileOperands &op, tsg_dtiles *C, unsigned char *rowcls,
-                            int *cls_part, int *cls_out, int none_fit, int *host = nullptr) {
+                            int *cls_part, int *cls_out, int none_fit, const int *longest, int *host = nullptr) {
     const int nb = (int)tsg_div_up(C->tilem, 16);
-    hipLaunchKernelGGL(k_row_class, dim3(nb), dim3(256), 0, s, op, C->tile_ptr, C->tile_nnz, C->tilem, rowcls,
-                       cls_part, none_fit);
+    hipLaunchKernelGGL(k_row_class, dim3(nb), dim3(256), 0, s, op, C->tile_ptr, C->tile_colidx, C->tile_nnz, C->tilem,
+                       rowcls, cls_part, none_fit, longest);
     TSG_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_row_class_reduce, dim3(1), dim3(1024), 0, s, (const int *)cls_part, nb, cls_out, host);
     TSG_LAUNCH_CHECK();
@@ -3053,19 +3362,31 @@ static int launch_row_class(hipStream_t s, const TileOperands &op, tsg_dtiles *C
 static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles *B, tsg_dtiles *C,
                         const tsg_spgemm_plan &P, const SpgemmWork &w, hipEvent_t *ev = nullptr) {
     if (C->nnz <= 0) return TSG_OK;
+    const bool rows = !P.all && (P.s3_lines || P.s3_rows);
+    if (ev && rows) TSG_HIP(hipEventRecord(ev[0], s));
+    if (!P.all && P.s3_lines) {
+        LinesLayout L;
+        L.nnz = P.ln[0]; L.umax = P.ln[1]; L.map = P.ln[2];
+        int base;
+        size_t off[4];
+        hipLaunchKernelGGL(k_step3_lines, dim3(C->tilem), dim3(P.ln[3]), lines_layout(L, &base, off), s, op.Arowp, op.Acolx,
+                           op.Avalx, (const int *)B->rowx_ptr, (const int *)B->rowx_col, (const double *)B->rowx_val,
+                           C->m, C->tilem, C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr, C->tile_nnz,
+                           (const unsigned char *)w.rowcls, C->csr_col, C->val, L);
+        TSG_LAUNCH_CHECK();
+    }
     if (!P.all && P.s3_rows) {
         G3Layout L;
         L.umax = P.g3[0]; L.nnzmax = P.g3[1]; L.lamax = P.g3[2];
         L.qb = P.g3[3]; L.bnnz = P.g3[4]; L.amax = P.g3[5];
         size_t off[G3_NARR];
         const size_t lds = g3_layout(L, off);
-        if (ev) TSG_HIP(hipEventRecord(ev[0], s));
         hipLaunchKernelGGL(k_step3_rows, dim3(C->tilem), dim3(G3_THREADS), lds, s, op, C->tile_ptr, C->tile_colidx,
                            C->tilem, C->mask, C->csr_ptr, C->tile_nnz, (const unsigned char *)w.rowcls, C->csr_col,
                            C->val, L);
         TSG_LAUNCH_CHECK();
-        if (ev) TSG_HIP(hipEventRecord(ev[1], s));
     }
+    if (ev && rows) TSG_HIP(hipEventRecord(ev[1], s));
     if (!P.all && P.s3_unfit && P.s3_elem) {
         const bool rx = op.Arowp != nullptr;
         TSG_TRY(launch_segments(s, C, w, 0, rx ? G3F_NNZ : G3E_NNZ, w.rowcls));
@@ -3115,14 +3436,14 @@ struct SpgemmTemps {
     unsigned *keep = nullptr;
     void *scr = nullptr, *wbuf = nullptr, *w3buf = nullptr, *bb = nullptr;
     unsigned char *hflag = nullptr;
-    int *hcnt = nullptr, *hinfo = nullptr, *hcur = nullptr, *span = nullptr;
+    int *hcnt = nullptr, *hinfo = nullptr, *hcur = nullptr, *span = nullptr, *longest = nullptr;
     int2 *hitems = nullptr;
     hipEvent_t ev[6] = {};
     int nev = 0;
 };
 
 static void free_temps(tsg_ctx *ctx, SpgemmTemps &t) {
-    void *ps[] = {t.keep, t.scr, t.wbuf, t.w3buf, t.hflag, t.hcnt, t.hinfo, t.hcur, t.hitems, t.span, t.bb};
+    void *ps[] = {t.keep, t.scr, t.wbuf, t.w3buf, t.hflag, t.hcnt, t.hinfo, t.hcur, t.hitems, t.span, t.bb, t.longest};
     for (void *p : ps) tsg_free(ctx, p);
     for (int i = 0; i < t.nev; i++) (void)hipEventDestroy(t.ev[i]);
     t = SpgemmTemps();
@@ -3153,6 +3474,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     // below 2^23 - 1 for the step-2 hash slots
     P.s3_elem = B->rowx_ptr != nullptr && tune.element_mode != 1 && B->n <= (1 << 27) - 32;
     P.elem_all = B->rowx_ptr != nullptr && tune.element_mode == 2;
+    P.lines = A->rowx_ptr && P.s3_elem && !P.elem_all && brow_bits_bytes(B) > 0;
     hipStream_t s = ctx->stream;
 
     hipEvent_t *ev = T.ev;
@@ -3189,7 +3511,8 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     const unsigned *bbits = nullptr;
     if (const size_t bbb = C->tilem > 0 ? brow_bits_bytes(B) : 0) {
         TSG_TRY(tsg_alloc(ctx, &T.bb, bbb));
-        TSG_TRY(launch_brow_bits(s, B, T.bb, &bdesc, &bbits, bany));
+        if (P.lines) TSG_TRY(tsg_alloc_t(ctx, &T.longest, (size_t)B->tilem));
+        TSG_TRY(launch_brow_bits(s, B, T.bb, &bdesc, &bbits, bany, T.longest));
     }
     TSG_TRY(launch_step1(s, A, B, C, false, P.s1w, T.keep, bdesc, bbits, bany, T.span));
     if (C->tilem > 0) {
@@ -3251,13 +3574,13 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     long long *part2 = (long long *)part2v;
     const bool classes = !P.all && numtileC > 0;
     {
-        long long *pin = ctx->pinned;  // [0] the total, [1..4] the eight class words
+        long long *pin = ctx->pinned;  // [0] the total, then the class words
         tsg_scan_publish pub;
         pub.host = pin;
         TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_nnz, C->tile_nnz, numtileC, part2, pub));
         if (timed) TSG_HIP(hipEventRecord(ev[2], s));
         if (classes)
-            TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, (int *)(pin + 1)));
+            TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, T.longest, (int *)(pin + 1)));
         TSG_HIP(hipStreamSynchronize(s));
         nnzC = pin[0];
         if (nnzC > 0x7fffffffLL) {
@@ -3269,6 +3592,11 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
             P.s3_unfit = h[0] > 0;
             P.s3_rows = h[1] > 0;
             for (int i = 0; i < 6; i++) P.g3[i] = std::max(1, h[1 + i]);
+            P.s3_lines = h[10] > 0;
+            P.ln[0] = h[7];
+            P.ln[1] = h[8];
+            for (P.ln[2] = LN_MAP_MIN; P.ln[2] < std::min(h[9], LN_MAP);) P.ln[2] *= 2;
+            P.ln[3] = std::min(LN_THREADS, 16 * (8 << h[10]));
         }
     }
     P.nnzC = nnzC;
@@ -3375,15 +3703,17 @@ extern "C" int tsg_spgemm(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B
 
 size_t tsg_spgemm_work_bytes(const tsg_dtiles *C, const tsg_dtiles *B, int s1w) {
     size_t off[WORK_NARR];
-    return work_layout(C->tilem, C->numtile, C->nnz, off, s1w, brow_bits_bytes(B));
+    const size_t bb = brow_bits_bytes(B);
+    return work_layout(C->tilem, C->numtile, C->nnz, off, s1w, bb, bb ? 4 * (size_t)B->tilem : 0);
 }
 
 int tsg_spgemm_enqueue(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B, tsg_dtiles *C,
                        const tsg_spgemm_plan &P, void *work) {
-    const SpgemmWork w = work_at(work, C->tilem, C->numtile, C->nnz, nullptr, P.s1w, brow_bits_bytes(B));
+    const SpgemmWork w = work_at(work, C->tilem, C->numtile, C->nnz, nullptr, P.s1w, brow_bits_bytes(B),
+                                 4 * (size_t)B->tilem);
     const int4 *bdesc = nullptr;
     const unsigned *bbits = nullptr;
-    if (C->tilem > 0) TSG_TRY(launch_brow_bits(s, B, w.bbits, &bdesc, &bbits, nullptr));
+    if (C->tilem > 0) TSG_TRY(launch_brow_bits(s, B, w.bbits, &bdesc, &bbits, nullptr, w.longest));
     TSG_TRY(launch_step1(s, A, B, C, false, P.s1w, w.bmstore, bdesc, bbits, nullptr, nullptr));
     TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_ptr, C->tile_ptr, C->tilem, w.part1));
     TSG_TRY(launch_step1(s, A, B, C, true, P.s1w, w.bmstore, bdesc, bbits, nullptr, w.segctr));
@@ -3391,7 +3721,7 @@ int tsg_spgemm_enqueue(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B, 
     TSG_TRY(launch_step2(s, op, B, C, P, w));
     TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_nnz, C->tile_nnz, C->numtile, w.part2));
     if (C->nnz > 0) {
-        if (!P.all) TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all));
+        if (!P.all) TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, P.lines ? w.longest : nullptr));
         TSG_TRY(launch_step3(s, op, B, C, P, w));
     }
     return TSG_OK;

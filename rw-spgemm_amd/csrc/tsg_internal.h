@@ -145,6 +145,9 @@ struct tsg_spgemm_plan {
     int s2map;      // bytes of the step-2 column -> slot map (0: binary search)
     int n2[4];      // step-2 segments per kernel (step2_kind)
     int s2w;        // widest tile-row span of the dense step 2's small blocks
+    int lines;      // tile-rows may go by row lines
+    int s3_lines;   // some tile-row does
+    int ln[4];      // row lines: C nonzeros, C tiles, map bytes, threads of a block
     int s3span;     // widest tile-column span of a tile-row (hash key widths of step 3)
 };
 // symbolic = true runs steps 1-2 and the step-3 plan only (C's values and
@@ -336,22 +339,20 @@ __device__ __forceinline__ unsigned bytes_le(unsigned w, unsigned j) {
 // Value of lane q of this lane's group of 16 lanes (q a constant after
 // unrolling): a DPP row broadcast, a VALU move with no LDS traffic, where
 // __shfl would issue a ds_bpermute.  Every lane of the group must be active.
-#define TSG_RB_CASE(Q) case Q: return __builtin_amdgcn_mov_dpp(v, 0x150 + Q, 0xF, 0xF, false);
-__device__ __forceinline__ int tsg_row16_bcast(int v, int q) {
+// (bound_ctrl set, though no lane lacks a source: without it the move is not
+// folded into the instruction that uses it.)
+#define TSG_RB_CASE(Q) case Q: return __builtin_amdgcn_update_dpp((T)0, v, 0x150 + Q, 0xF, 0xF, true);
+template <typename T>
+__device__ __forceinline__ T tsg_row16_bcast(T v, int q) {
     switch (q) {
         TSG_RB_CASE(0) TSG_RB_CASE(1) TSG_RB_CASE(2) TSG_RB_CASE(3)
         TSG_RB_CASE(4) TSG_RB_CASE(5) TSG_RB_CASE(6) TSG_RB_CASE(7)
         TSG_RB_CASE(8) TSG_RB_CASE(9) TSG_RB_CASE(10) TSG_RB_CASE(11)
         TSG_RB_CASE(12) TSG_RB_CASE(13) TSG_RB_CASE(14) default: break;
     }
-    return __builtin_amdgcn_mov_dpp(v, 0x150 + 15, 0xF, 0xF, false);
+    return __builtin_amdgcn_update_dpp((T)0, v, 0x150 + 15, 0xF, 0xF, true);
 }
 #undef TSG_RB_CASE
-__device__ __forceinline__ double tsg_row16_bcast(double v, int q) {
-    const long long b = __double_as_longlong(v);
-    const int lo = tsg_row16_bcast((int)(unsigned)b, q), hi = tsg_row16_bcast((int)(b >> 32), q);
-    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
 template <typename T>
 __device__ __forceinline__ T tsg_group16_sum(T v) {
 #pragma unroll
