@@ -66,6 +66,7 @@ inline bool tsg_arena_owns(const tsg_arena *a, const void *p) {
 }
 
 // ------------------------------------------------------------------ context
+#define TSG_STAGE_WORKERS 4
 struct tsg_ctx {
     int device;
     hipStream_t stream;
@@ -81,6 +82,9 @@ struct tsg_ctx {
     size_t scratch_bytes = 0;
     int num_cu = 0;
     size_t lds_per_block = 0;
+    // pinned slots of large copies to the host, two per worker
+    char *stage = nullptr;
+    hipEvent_t stage_ev[2 * TSG_STAGE_WORKERS] = {};
     // when set, blocks come from this arena (hipMalloc only if it is full)
     tsg_arena *arena = nullptr;
 };
@@ -95,6 +99,15 @@ static inline int tsg_alloc_t(tsg_ctx *ctx, T **p, size_t count) {
 }
 int tsg_scratch(tsg_ctx *ctx, size_t bytes, void **p);
 int tsg_read_scalar_i64(tsg_ctx *ctx, const void *dptr, int is64, long long *out);
+// Device to fresh host memory, all parts, finished on return.
+struct tsg_part {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+int tsg_download_parts(tsg_ctx *ctx, const tsg_part *parts, int n);
+// Host memory for a result (free() it): huge pages asked for when it is large.
+void *tsg_host_alloc(size_t bytes);
 // Bytes the allocator reserved for a live block of ctx (0 if none).
 size_t tsg_alloc_size(const tsg_ctx *ctx, const void *p);
 

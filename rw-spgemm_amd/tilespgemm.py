@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import weakref
 
 import numpy as np
 
@@ -339,18 +340,35 @@ class Csr:
         return Csr(a.shape[0], a.shape[1], a.indptr, a.indices, a.data)
 
 
+def _free_host(address):
+    h = HCsr(0, 0, 0, C.cast(address, C.POINTER(_i)), None, None)
+    lib.tsg_hcsr_free(C.byref(h))
+
+
+def _take_array(p, ctype, dtype, n):
+    """A library-allocated array as numpy: small ones copied, large ones kept where they are (the memory
+    goes back with the last array that uses it) and taken out of the library's hands."""
+    if n * C.sizeof(ctype) < 1 << 20:
+        return np.ctypeslib.as_array(p, shape=(n,)).copy() if n else np.zeros(0, dtype), False
+    address = C.cast(p, C.c_void_p).value
+    buf = (ctype * n).from_address(address)
+    weakref.finalize(buf, _free_host, address).atexit = False
+    return np.frombuffer(buf, dtype=dtype), True
+
+
 def _take_hcsr(h):
-    """Copy a library-allocated HCsr into numpy and free it."""
+    """A library-allocated HCsr as numpy arrays."""
     try:
-        m, n, nnz = h.m, h.n, h.nnz
-        rp = np.ctypeslib.as_array(h.rowptr, shape=(m + 1,)).copy()
-        if nnz:
-            ci = np.ctypeslib.as_array(h.colidx, shape=(nnz,)).copy()
-            va = np.ctypeslib.as_array(h.val, shape=(nnz,)).copy()
-        else:
-            ci = np.zeros(0, np.int32)
-            va = np.zeros(0, np.float64)
-        return Csr(m, n, rp, ci, va)
+        rp, kept = _take_array(h.rowptr, _i, np.int32, h.m + 1)
+        if kept:
+            h.rowptr = None
+        ci, kept = _take_array(h.colidx, _i, np.int32, h.nnz)
+        if kept:
+            h.colidx = None
+        va, kept = _take_array(h.val, _d, np.float64, h.nnz)
+        if kept:
+            h.val = None
+        return Csr(h.m, h.n, rp, ci, va)
     finally:
         lib.tsg_hcsr_free(C.byref(h))
 
