@@ -197,10 +197,12 @@ typedef struct {
                               element-wise segments instead of one wave each
                               (default 0) */
     int heavy_min_products; /* a row with more intermediate products (or more
-                              than 2048 A entries) is heavy (0 = 65536) */
-    int heavy_item_products; /* a heavy row is split into column parts of
-                              4096 columns, handed out in runs of about this
-                              many products (0 = 32768) */
+                              than 2048 A entries) is heavy and spread over one
+                              wave per column part; set, it also lets tile-rows
+                              with many products be taken row by row whatever C's
+                              size (0: reported as heavy from 65536, spread from
+                              a size that C decides) */
+    int heavy_item_products; /* without effect: a column part is one item */
 } tsg_tune;
 void tsg_tune_default(tsg_tune *t);
 
@@ -209,7 +211,7 @@ typedef struct {
     long long numtileC, nnzC;
     long long tiles_sparse_acc, tiles_dense_acc, tiles_empty;
     double t_step3_rows_ms; /* the row-wise numeric kernel's launch alone */
-    long long heavy_rows;   /* rows computed one wave each (k_step3_heavy) */
+    long long heavy_rows;   /* rows with very many products (k_step3_heavy) */
     long long heavy_bytes;  /* transient device bytes of that path */
 } tsg_stats;
 

@@ -1596,6 +1596,28 @@ k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
 }
 
 // ------------------------------------------------------------------ step 3, flat rows
+// One product per lane, in ascending k along the lanes, into sums of which
+// several lanes may share one (a lane's bin decides: equal sums, equal bins).
+// In each round the lowest pending lane of a bin adds, so a shared sum gets
+// its products in lane order.  The winner is the bin's minimum of stamp + lane;
+// stamps descend, so bins need no clearing between rounds.
+__device__ __forceinline__ void add_in_order(double *sum, unsigned *bin, unsigned &stamp, bool on, int lane, double a,
+                                             double b) {
+    for (;;) {
+        stamp -= 64u;
+        const unsigned me = stamp + (unsigned)lane;
+        if (on) atomicMin(bin, me);
+        tsg_wave_sync();
+        const unsigned first = *bin;
+        const double v = *sum;  // with the bin: one LDS round trip a round
+        if (on && first == me) {
+            *sum = __builtin_fma(a, b, v);
+            on = false;
+        }
+        tsg_wave_sync();
+        if (!__ballot(on)) break;
+    }
+}
 // [b0, b1) cut to list's entries in [lo, hi) (list ascending; an end that is
 // not to be cut keeps its place).  Both ends at once and a quarter of the
 // range left per step, six loads in flight: a lane's search is a chain of
@@ -1662,6 +1684,7 @@ __device__ __forceinline__ void range_in(const int *__restrict__ list, int &b0, 
 #define G3F_SLOTS (G3F_NNZ + G3F_NNZ / 2 + 32)
 #define G3F_ROUNDS 4
 #define G3F_BATCH (64 * G3F_ROUNDS)
+#define G3F_BINS 128
 #define G3F_SPAN 65535  // tile columns of a tile-row: offsets + 1 below 2^20
 __device__ __forceinline__ unsigned flat_home(unsigned key, unsigned n) {
     return (unsigned)(((unsigned long long)(key * 2654435761u) * n) >> 32);
@@ -1677,8 +1700,8 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
     __shared__ double s_acc[G3F_NNZ];
     __shared__ unsigned s_key[G3F_SLOTS];
     __shared__ unsigned short s_pos[WIDE ? G3F_SLOTS : 1];
-    __shared__ unsigned char s_tag[G3F_NNZ];
-    __shared__ unsigned s_mark[G3F_WAVES][G3F_BATCH / 4];
+    // marks of a batch, then the bins of its products
+    __shared__ unsigned s_mark[G3F_WAVES][G3F_BINS];
     __shared__ int s_cnt[G3F_WAVES][16], s_rb[17];
     __shared__ unsigned char s_ord[16];
     static_assert(G3F_NNZ <= 4096, "positions take 12 bits of a slot");
@@ -1765,19 +1788,16 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
                     unsigned mr = Cmask[t * 16 + r];
                     const unsigned pw = (r & 8) ? ((r & 4) ? p.w : p.z) : ((r & 4) ? p.y : p.x);
                     int skipn = j - (int)((pw >> (8 * (r & 3))) & 255u);
-                    if (x < total) {
+                    if (x < total && !((skip >> r) & 1u)) {  // (k_step3_heavy writes its rows' columns)
                         // entry j of the tile: the (j - row offset)-th column of row r
-                    for (; skipn > 0; skipn--) mr &= ~(0x80000000u >> __clz((int)mr));
-                        const int c = __clz((int)mr) - 16, pos = start + x;
+                        for (; skipn > 0; skipn--) mr &= ~(0x80000000u >> __clz((int)mr));
+                        const int c = __clz((int)mr) - 16, pos = start + x, rb = s_rb[r];
                         Ccol8[(long long)nbase + pos] = (unsigned char)c;
-                        if (!((skip >> r) & 1u)) {
-                            const int rb = s_rb[r];
-                            const unsigned rs = (unsigned)(s_rb[r + 1] - rb), key = (unsigned)(J * 16 + c - col_lo) + 1u;
-                            unsigned h = flat_home(key, rs);
-                            const unsigned ent = WIDE ? key : key << 12 | (unsigned)pos;
-                            while (atomicCAS(&s_key[rb + h], 0u, ent) != 0u) h = h + 1 == rs ? 0u : h + 1;
-                            if (WIDE) s_pos[rb + h] = (unsigned short)pos;
-                        }
+                        const unsigned rs = (unsigned)(s_rb[r + 1] - rb), key = (unsigned)(J * 16 + c - col_lo) + 1u;
+                        unsigned h = flat_home(key, rs);
+                        const unsigned ent = WIDE ? key : key << 12 | (unsigned)pos;
+                        while (atomicCAS(&s_key[rb + h], 0u, ent) != 0u) h = h + 1 == rs ? 0u : h + 1;
+                        if (WIDE) s_pos[rb + h] = (unsigned short)pos;
                     }
                 }
                 tsg_wave_sync();
@@ -1829,6 +1849,10 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
                 q[i] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * i + lane]));
                 prev = __builtin_amdgcn_readlane(q[i], 63);
             }
+            tsg_wave_sync();
+            for (int j = lane; j < G3F_BINS; j += 64) s_mark[wave][j] = 0xffffffffu;
+            unsigned stamp = 0xffffffc0u;
+            tsg_wave_sync();
 #pragma unroll
             for (int i = 0; i < G3F_ROUNDS; i++) {  // every lane loads in bounds
                 const int e = __shfl(delta, q[i] - 1, 64) + min(base + 64 * i + lane, total - 1);
@@ -1849,21 +1873,12 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
                 while ((ent = key0[h], WIDE ? ent : ent >> 12) != key && ++probe < n_r) h = h + 1 == n_r ? 0u : h + 1;
                 const int pos = WIDE ? (int)s_pos[(rg & 0xffff) + h] : (int)(ent & 4095u);
                 const int q0 = __builtin_amdgcn_readlane(q[i], 0), q1 = __builtin_amdgcn_readlane(q[i], 63);
-                bool clash = false;
-                if (q0 != q1) {
-                    if (on) s_tag[pos] = (unsigned char)lane;
-                    tsg_wave_sync();
-                    clash = __ballot(on && s_tag[pos] != (unsigned char)lane) != 0;
-                }
-                if (!clash) {
+                if (q0 == q1) {
                     if (on) s_acc[pos] = __builtin_fma(as, b[i], s_acc[pos]);
+                    tsg_wave_sync();
                 } else {
-                    for (int s = q0; s <= q1; s++) {
-                        if (on && q[i] == s) s_acc[pos] = __builtin_fma(as, b[i], s_acc[pos]);
-                        tsg_wave_sync();
-                    }
+                    add_in_order(s_acc + pos, s_mark[wave] + (pos & (G3F_BINS - 1)), stamp, on, lane, as, b[i]);
                 }
-                tsg_wave_sync();
             }
         }
     }
@@ -1871,199 +1886,312 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
     for (int i = tid; i < n; i += G3F_THREADS) Cval[(long long)nbase + i] = s_acc[i];
 }
 
-// ------------------------------------------------------------------ step 3, heavy rows
-// Rows with very many intermediate products (hub rows of power-law graphs)
-// would make every C segment of their tile-row re-walk the whole A row.
-// They are computed one wave at a time instead, in column parts of
-// HEAVY_PART_COLS columns whose FP64 accumulators live in the wave's own
-// LDS window: for part [lo, lo + HEAVY_PART_COLS) the wave walks A row i in
-// ascending k, 64 entries (sources) at a time, and adds their products with
-// the B entries in the part as k_step3_flat does (numbered through, 64 per
-// step, source by source where two meet in one column), then copies the
-// part into C's final positions.  A work item is a run of consecutive parts
-// of one row; between parts the wave keeps, per A entry, the position in
-// B row k where the next part starts (a cursor in global scratch), so a
-// search starts there.  Against one source per step (22 of 64 lanes busy on
-// R-MAT scale 16, their first 8 entries staged through LDS): 13.6 -> 6.7 ms
-// there (120 G products/s); parts of 1024 / 2048 / 4096 columns 7.5 / 6.9 /
-// 8.4 ms, 4 / 8 rounds of loads in flight 6.9 / 6.7 ms.
-#define HEAVY_MIN_PRODUCTS 65536
-#ifndef HEAVY_PART_COLS
-#define HEAVY_PART_COLS 2048         // 19 KiB of LDS per wave, eight waves per CU
-#endif
-#define HEAVY_ITEM_PRODUCTS 32768    // products per work item, about
-#define HEAVY_MAX_WAVES 4096
-#define HEAVY_CURSOR_BYTES (512ll << 20)
+// ------------------------------------------------------------------ step 3, heavy and long rows
+// Rows with many products for the tiles of their tile-row (hub rows of
+// power-law graphs, and rows that have a few hubs as sources).  In segments
+// of a tile-row each would walk all its A entries again in every segment
+// and put every entry of C into a hash first (R-MAT scale 16: 68 segments a
+// tile-row, 9,800 VALU instructions each).  Here a wave takes one row and a group
+// of column parts (HEAVY_PART_COLS columns each; a heavy row one part, so that
+// a hub row spreads over many waves, a long row HEAVY_GROUP parts).  It takes
+// as many parts at a time as the row's entries in them fit its sums, writes
+// for each tile the row's mask and its offset among the sums, walks A row i in
+// ascending k, 64 entries (sources) at a time, numbers the products with the B
+// entries in these parts through and adds 64 per step (add_in_order), then
+// copies the sums to C's final positions with their column bytes.
+//   Where B row k's entries of a part start and end is read from a table
+// made once per product (k_heavy_windows), two groups of sources ahead, so no
+// search stands between the loads; blocks go part by part, which keeps the
+// parts' columns of B (and of the table) in the L2.
+//   14 KiB of LDS, eleven waves a CU.  Bound by products behind LDS round
+// trips and fragments of B rows (5.1 of 8.4 ms), scattered 8-byte stores (2)
+// and the walk over tiles (1.4).  R-MAT scale 16 A*A^T, heavy rows with the
+// others by k_step3_flat 13.9 ms -> all by this kernel 7.1.  Parts of 1024 in
+// groups of 4 / 8 / 16 (whole product) 11.0 / 11.7 / 11.9 ms, of 2048 in groups
+// of 2 / 4 / 8 12.1 / 11.8 / 12.0, of 512 in groups of 8 12.1.
+#define HEAVY_MIN_PRODUCTS 65536  // reported as heavy (tsg_stats.heavy_rows)
+#define HEAVY_PART_LOG 10
+#define HEAVY_PART_COLS (1 << HEAVY_PART_LOG)
+#define HEAVY_PART_TILES (1 << (HEAVY_PART_LOG - 4))
+#define HEAVY_GROUP 4
+// A row is split into single parts above C's nonzeros >> 10 products: one
+// wave's share of everything, so that no wave ends long after the others.  R-MAT
+// A*A^T with 16384 / 65536 / 262144: scale 16 (380 M nonzeros) 12.3 / 11.8 /
+// 11.0 ms, scale 14 (30 M) 2.22 / 2.19 / 2.44.
+#define HEAVY_SPLIT_LOG 10
+#define HEAVY_SPLIT_MAX 262144LL
+#define HEAVY_WINDOW_BYTES (512ll << 20)  // largest window table
+// All rows of a tile-row with more products per row than this go here: below,
+// a wave per row walks tiles for few products and k_step3_flat is better.  R-MAT
+// scale 16 A*A^T 10.9 ms with 1024 or 512 and u / 2, 11.2 with 256 and u / 8; ER
+// 30000 (26 per row, 676 products) A^2 0.77 and 1.01 ms, ER 2500 232, 216 and 216 us.
+#define LONG_MIN_PRODUCTS 512
+#define LONG_PER_TILE(u) ((u) / 2)
+// Only in a large product (or when the caller sets heavy_min_products): in a
+// small one the waves of the longest rows end after everything else.  R-MAT
+// A^2 with / without long rows: scale 11 (6 edges a vertex) 410 / 353 us, scale 12
+// 652 / 563, scale 13 (7 M nonzeros) 1210 / 1192; scale 14 A*A^T (30 M) 2.2 / 2.9 ms.
+#define LONG_MIN_NNZ (12LL << 20)
+#define CLS_LONG 3  // row class: heavy and long rows only
 
-// Per C row of an element-wise tile-row: heavy flag and work items (runs of
-// parts); info[0] = longest heavy A row, info[1] = heavy rows.  16 lanes per
-// row, so that a long A row's B row lengths are not one lane's chain of
-// loads (R-MAT scale 16: 665 -> 92 us).
+// Per C row of an element-wise tile-row: 2 heavy (more than min_products
+// products, or more than 2048 A entries), 1 long, 0 neither; cnt[0, m) and cnt[m,
+// 2m) take the heavy and the long rows as counts for the scan that numbers
+// them, info[0] the number of heavy ones.  A tile-row with many products for
+// its tiles has only heavy and long rows and leaves the element-wise class.
+// One block per tile-row, 16 lanes per row, so that a long A row's B row
+// lengths are not one lane's chain of loads (R-MAT scale 16: 665 -> 92 us).
 __global__ void __launch_bounds__(256)
 k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const int *__restrict__ Browp,
-              const unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
-              int m, long long min_products, long long item_products, unsigned char *__restrict__ flag,
-              int *__restrict__ cnt, int *__restrict__ info) {
-    const int i = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15;
-    if (i >= m) return;
-    int h = 0, items = 0;
-    if (rowcls[i >> 4] == 0) {  // uniform in the 16 lanes, as everything below
-        const int x0 = Arowp[i], x1 = Arowp[i + 1];
-        long long p = -1;  // unknown for long A rows
-        if (x1 - x0 > 2048) {
-            h = 1;
-        } else {
-            p = 0;
+              unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, int m, long long min_products,
+              long long count_products, int take_long, unsigned char *__restrict__ flag, int *__restrict__ cnt,
+              int *__restrict__ info) {
+    __shared__ long long s_p[16];
+    const int I = blockIdx.x, r = threadIdx.x >> 4, l = threadIdx.x & 15, i = 16 * I + r;
+    const bool mine = rowcls[I] == 0;  // block-uniform
+    long long p = 0;
+    int x0 = 0, x1 = 0;
+    if (mine && i < m) {
+        x0 = Arowp[i];
+        x1 = Arowp[i + 1];
 #pragma unroll 4
-            for (int x = x0 + l; x < x1; x += 16) {
-                const int k = Acolx[x];
-                p += Browp[k + 1] - Browp[k];
-            }
-            p = tsg_group16_sum(p);
-            h = p > min_products;
+        for (int x = x0 + l; x < x1; x += 16) {
+            const int k = Acolx[x];
+            p += Browp[k + 1] - Browp[k];
         }
-        if (h) {
-            const int I = i >> 4, c0 = Cptr[I], c1 = Cptr[I + 1];
-            const long long span = (long long)(Ccol[c1 - 1] - Ccol[c0] + 1) * 16;
-            const int nparts = (int)((span + HEAVY_PART_COLS - 1) / HEAVY_PART_COLS);
-            items = p < 0 ? nparts
-                          : (int)min<long long>(nparts, max<long long>(1, (p + item_products - 1) / item_products));
-            if (l == 0) {
-                atomicMax(&info[0], x1 - x0);
-                atomicAdd(&info[1], 1);
-            }
-        }
+        p = tsg_group16_sum(p);
     }
-    if (l == 0) {
+    if (l == 0) s_p[r] = p;
+    __syncthreads();
+    long long all = 0;
+    for (int q = 0; q < 16; q++) all += s_p[q];
+    const bool longer = mine && take_long && all > 16 * max((long long)LONG_MIN_PRODUCTS, LONG_PER_TILE(Cptr[I + 1] - Cptr[I]));
+    if (i < m && l == 0) {
+        const int h = !mine ? 0 : x1 - x0 > 2048 || p > min_products ? 2 : longer && p > 0 ? 1 : 0;
         flag[i] = (unsigned char)h;
-        cnt[i] = items;
+        cnt[i] = h == 2;
+        cnt[m + i] = h == 1;
+        if (h == 2) atomicAdd(&info[0], 1);
+        if (mine && (x1 - x0 > 2048 || p > count_products)) atomicAdd(&info[1], 1);
     }
+    if (longer && threadIdx.x == 0) rowcls[I] = CLS_LONG;
 }
 
-// Work items {row, first part | end part << 16}, parts split evenly.
+// rows = the heavy rows, then the long ones
 __global__ void __launch_bounds__(256)
-k_heavy_list(const int *__restrict__ off, const unsigned char *__restrict__ flag, const int *__restrict__ Cptr,
-             const int *__restrict__ Ccol, int m, int2 *__restrict__ items) {
+k_heavy_list(const int *__restrict__ off, const unsigned char *__restrict__ flag, int m, int *__restrict__ rows) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m || !flag[i]) return;
-    const int I = i >> 4, c0 = Cptr[I], c1 = Cptr[I + 1];
-    const long long span = (long long)(Ccol[c1 - 1] - Ccol[c0] + 1) * 16;
-    const int nparts = (int)((span + HEAVY_PART_COLS - 1) / HEAVY_PART_COLS);
-    const int o = off[i], n = off[i + 1] - o;
-    for (int g = 0; g < n; g++) {
-        const int p0 = (int)((long long)nparts * g / n), p1 = (int)((long long)nparts * (g + 1) / n);
-        items[o + g] = make_int2(i, (int)((unsigned)p0 | ((unsigned)p1 << 16)));
-    }
+    if (i < m && flag[i]) rows[off[flag[i] == 2 ? i : m + i]] = i;
 }
 
-#define HEAVY_ROUNDS 8
+// win[w * m + k] = first entry of B row k at or past column w << shift, w = 0
+// .. nw (the last one the row's end).  k along the threads: neighbours search
+// neighbouring rows and write one run.
+__global__ void __launch_bounds__(256)
+k_heavy_windows(const int *__restrict__ Browp, const int *__restrict__ Bcolx, int m, int nw, int shift,
+                int *__restrict__ win) {
+    const int k = blockIdx.x * 256 + threadIdx.x, w = blockIdx.y;
+    if (k >= m) return;
+    const int b0 = Browp[k], b1 = Browp[k + 1];
+    win[(long long)w * m + k] = w == nw ? b1 : w == 0 ? b0 : lower_bound_i(Bcolx, b0, b1, w << shift);
+}
+
+// First of list[lo, hi) (ascending, the same for the whole wave) at or past
+// key: 64 probes a step, two steps for 4096 entries.
+__device__ __forceinline__ int wave_lower_bound(const int *__restrict__ list, int lo, int hi, int key, int lane) {
+    while (lo < hi) {
+        const int step = (hi - lo + 63) >> 6, x = lo + lane * step;
+        const int below = __popcll(__ballot(x < hi && list[min(x, hi - 1)] < key));
+        if (below == 0) return lo;
+        hi = min(hi, lo + below * step);
+        lo += (below - 1) * step + 1;
+    }
+    return lo;
+}
+
+#define HEAVY_ROUNDS 4
+#define HEAVY_BINS 256  // of add_in_order; products of different sums that share one only take a round more
 #define HEAVY_BATCH (64 * HEAVY_ROUNDS)
 __global__ void __launch_bounds__(64)
 k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const double *__restrict__ Avalx,
-              const int *__restrict__ Browp, const int *__restrict__ Bcolx, const double *__restrict__ Bvalx,
-              const int2 *__restrict__ items, const int *__restrict__ nitems, const int *__restrict__ Cptr,
-              const int *__restrict__ Ccol, const unsigned short *__restrict__ Cmask,
-              const unsigned char *__restrict__ Cptr16, const int *__restrict__ Cnnz, double *__restrict__ Cval,
-              int *__restrict__ cursor, long long cur_stride, int *__restrict__ next_item) {
+              const int *__restrict__ win, long long wstride, int nw, int shift, const int *__restrict__ Bcolx,
+              const double *__restrict__ Bvalx, const int *__restrict__ rows, int nheavy, int nlong,
+              long long heavy_blocks, long long first, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
+              const unsigned short *__restrict__ Cmask, const unsigned char *__restrict__ Cptr16,
+              const int *__restrict__ Cnnz, unsigned char *__restrict__ Ccol8, double *__restrict__ Cval) {
     __shared__ double s_acc[HEAVY_PART_COLS];
-    __shared__ unsigned char s_tag[HEAVY_PART_COLS];
+    __shared__ unsigned s_word[HEAVY_GROUP * HEAVY_PART_TILES];  // of a tile: the row's mask, and offset in s_acc
+    __shared__ unsigned s_bin[HEAVY_BINS];
     __shared__ unsigned s_mark[HEAVY_BATCH / 4];
     const int lane = threadIdx.x;
     unsigned char *mk = reinterpret_cast<unsigned char *>(s_mark);
-    int *cur = cursor + (long long)blockIdx.x * cur_stride;
-    const int ni = *nitems;
-    // items are taken from a shared counter, so waves that drew short items
-    // take more (every wave exits once the counter passes ni)
-    for (;;) {
-        int h = 0;
-        if (lane == 0) h = atomicAdd(next_item, 1);
-        h = __shfl(h, 0, 64);
-        if (h >= ni) break;
-        const int2 it = items[h];
-        const int i = it.x, p0 = (int)((unsigned)it.y & 0xffffu), p1 = (int)((unsigned)it.y >> 16);
-        const int I = i >> 4, r = i & 15;
-        const int c0 = Cptr[I], c1 = Cptr[I + 1];
-        const int colbase = Ccol[c0] * 16;
-        const int xa = Arowp[i], xe = Arowp[i + 1];
-        for (int part = p0; part < p1; part++) {
-            const int lo = colbase + part * HEAVY_PART_COLS, hi = lo + HEAVY_PART_COLS;
-            for (int j = lane; j < HEAVY_PART_COLS; j += 64) s_acc[j] = 0.0;
-            for (int xc = xa; xc < xe; xc += 64) {
-                // 64 A entries (sources) at once: lane q finds B row k's entries
-                // in the part
-                int b0 = 0, len = 0;
-                double a = 0.0;
-                if (xc + lane < xe) {
-                    const int k = Acolx[xc + lane];
-                    a = Avalx[xc + lane];
-                    int b1 = Browp[k + 1];
-                    b0 = part == p0 ? Browp[k] : cur[xc - xa + lane];
-                    if (part != p0 && b1 - b0 > HEAVY_PART_COLS) b1 = b0 + HEAVY_PART_COLS;
-                    range_in(Bcolx, b0, b1, part == p0, lo, true, hi);
-                    len = b1 - b0;
-                    if (part + 1 < p1) cur[xc - xa + lane] = b1;
-                }
-                const int incl = tsg_wave_incl_scan_dpp(len), pre = incl - len, delta = b0 - pre;
-                const int total = __builtin_amdgcn_readlane(incl, 63);
-                int prev = 0;
-                for (int base = 0; base < total; base += HEAVY_BATCH) {
+    // blocks: the heavy rows' items, then the long rows'; part by part, 16 rows
+    // of the list on one XCD (blocks go to the 8 XCDs in turn), the next 16 on the
+    // next
+    const long long hb = first + blockIdx.x;
+    const bool heavy = hb < heavy_blocks;
+    const long long h = heavy ? hb : hb - heavy_blocks;
+    const int nrows = heavy ? nheavy : nlong, padded = (nrows + 127) & ~127, group = heavy ? 1 : HEAVY_GROUP;
+    const int p0 = (int)(h / padded) * group, x = (int)(h % padded);
+    int j0 = ((x >> 7) * 8 + (x & 7)) * 16 + ((x >> 3) & 15);
+    if (j0 >= nrows) return;
+    if (!heavy) j0 += nheavy;
+    const int i = rows[j0], I = i >> 4, r = i & 15;
+    const int c0 = Cptr[I], c1 = Cptr[I + 1];
+    const int xa = Arowp[i], xe = Arowp[i + 1];
+    int t = wave_lower_bound(Ccol, c0, c1, p0 * HEAVY_PART_TILES, lane);
+    const int tend = wave_lower_bound(Ccol, t, c1, (p0 + group) * HEAVY_PART_TILES, lane);
+    unsigned stamp = 0u;
+    auto clear_bins = [&]() {
+        for (int j = lane; j < HEAVY_BINS; j += 64) s_bin[j] = 0xffffffffu;
+        stamp = 0xffffffc0u;
+    };
+    while (t < tend) {
+        // a run of parts: as many as their entries of the row fit s_acc (one always does)
+        const int ps = Ccol[t] / HEAVY_PART_TILES, jb = ps * HEAVY_PART_TILES;
+        int pe = p0 + group, te = tend, nn = 0;
+        for (int tb = t; tb < te && nn <= HEAVY_PART_COLS; tb += 256) {
+            int J[4];
+            unsigned cm[4];
 #pragma unroll
-                    for (int v = 0; v < HEAVY_BATCH / 256; v++) s_mark[64 * v + lane] = 0u;
-                    tsg_wave_sync();
-                    if (len > 0 && pre >= base && pre < base + HEAVY_BATCH) mk[pre - base] = (unsigned char)(lane + 1);
-                    tsg_wave_sync();
-                    int q[HEAVY_ROUNDS], col[HEAVY_ROUNDS];
-                    double b[HEAVY_ROUNDS];
+            for (int v = 0; v < 4; v++) {
+                const int tt = tb + 64 * v + lane, ti = min(tt, te - 1);
+                J[v] = Ccol[ti];
+                cm[v] = Cmask[(long long)ti * 16 + r];
+                if (tt >= te) cm[v] = 0u;
+            }
 #pragma unroll
-                    for (int v = 0; v < HEAVY_ROUNDS; v++) {
-                        q[v] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * v + lane]));
-                        prev = __builtin_amdgcn_readlane(q[v], 63);
-                    }
-#pragma unroll
-                    for (int v = 0; v < HEAVY_ROUNDS; v++) {  // every lane loads in bounds
-                        const int e = __shfl(delta, q[v] - 1, 64) + min(base + 64 * v + lane, total - 1);
-                        col[v] = Bcolx[e];
-                        b[v] = Bvalx[e];
-                    }
-#pragma unroll
-                    for (int v = 0; v < HEAVY_ROUNDS; v++) {
-                        if (base + 64 * v >= total) break;  // wave-uniform
-                        const bool on = base + 64 * v + lane < total;
-                        const double as = __shfl(a, q[v] - 1, 64);
-                        const int p = col[v] - lo;
-                        const int q0 = __builtin_amdgcn_readlane(q[v], 0), q1 = __builtin_amdgcn_readlane(q[v], 63);
-                        bool clash = false;
-                        if (q0 != q1) {
-                            if (on) s_tag[p] = (unsigned char)lane;
-                            tsg_wave_sync();
-                            clash = __ballot(on && s_tag[p] != (unsigned char)lane) != 0;
-                        }
-                        if (!clash) {
-                            if (on) s_acc[p] = __builtin_fma(as, b[v], s_acc[p]);
-                        } else {
-                            for (int s = q0; s <= q1; s++) {  // sources in ascending k
-                                if (on && q[v] == s) s_acc[p] = __builtin_fma(as, b[v], s_acc[p]);
-                                tsg_wave_sync();
-                            }
-                        }
-                        tsg_wave_sync();
-                    }
+            for (int v = 0; v < 4; v++) {
+                if (nn > HEAVY_PART_COLS) break;  // wave-uniform
+                const int c = __popc(cm[v]), incl = tsg_wave_incl_scan_dpp(c);
+                if (cm[v]) s_word[J[v] - jb] = cm[v] << 15 | (unsigned)(nn + incl - c);
+                const unsigned long long over = __ballot(nn + incl > HEAVY_PART_COLS);
+                if (over) {  // the run ends before this tile's part
+                    pe = __builtin_amdgcn_readlane(J[v], __ffsll((long long)over) - 1) / HEAVY_PART_TILES;
+                    nn = HEAVY_PART_COLS + 1;
+                } else {
+                    nn += __builtin_amdgcn_readlane(incl, 63);
                 }
             }
-            // the part's C entries of row i, into their final positions
-            const int t0 = lower_bound_i(Ccol, c0, c1, lo >> 4), t1 = lower_bound_i(Ccol, t0, c1, hi >> 4);
-            for (int t = t0 + lane; t < t1; t += 64) {
-                unsigned cm = Cmask[(long long)t * 16 + r];
-                long long pos = (long long)Cnnz[t] + Cptr16[(long long)t * 16 + r];
-                const double *d = s_acc + (Ccol[t] * 16 - lo);
-                while (cm) {
-                    const int bb = 31 - __clz(cm);
-                    cm &= ~(1u << bb);
-                    Cval[pos++] = d[15 - bb];
-                }
-            }
-            tsg_wave_sync();  // the next part clears the window
         }
+        if (nn > HEAVY_PART_COLS) {
+            te = wave_lower_bound(Ccol, t, te, pe * HEAVY_PART_TILES, lane);
+            nn = HEAVY_PART_COLS;
+        }
+        if (nn == 0) {  // other rows' tiles
+            t = te;
+            continue;
+        }
+        const int lo = ps << HEAVY_PART_LOG, hi = pe << HEAVY_PART_LOG;  // columns (n <= 2^27)
+        // sources (A entries) 64 at a time, lane q's B row in the run's windows:
+        // the entries two groups ahead, their windows one group ahead
+        const long long w0 = (long long)(lo >> shift) * wstride;
+        const long long w1 = (long long)min(((hi - 1) >> shift) + 1, nw) * wstride;
+        const int inside = (int)((1u << shift) - 1u);
+        const bool cut_lo = (lo & inside) != 0, cut_hi = (hi & inside) != 0;
+        int k1 = 0, n0 = 0, n1 = 0;
+        double a1 = 0.0, a2 = 0.0;
+        auto fetch = [&](int xc) {
+            k1 = -1;
+            a2 = 0.0;
+            if (xc + lane < xe) {
+                k1 = Acolx[xc + lane];
+                a2 = Avalx[xc + lane];
+            }
+        };
+        auto window = [&]() {
+            n0 = n1 = 0;
+            if (k1 >= 0) {
+                n0 = win[w0 + k1];
+                n1 = win[w1 + k1];
+            }
+            a1 = a2;
+        };
+        fetch(xa);
+        window();
+        fetch(xa + 64);
+        for (int j = lane; j < nn; j += 64) s_acc[j] = 0.0;
+        for (int xc = xa; xc < xe; xc += 64) {
+            int b0 = n0, b1 = n1;
+            const double a = a1;
+            window();
+            fetch(xc + 128);
+            if (cut_lo || cut_hi) range_in(Bcolx, b0, b1, cut_lo, lo, cut_hi, hi);  // windows wider than parts
+            const int len = b1 - b0;
+            const int incl = tsg_wave_incl_scan_dpp(len), pre = incl - len, delta = b0 - pre;
+            const int total = __builtin_amdgcn_readlane(incl, 63);
+            int prev = 0;
+            for (int base = 0; base < total; base += HEAVY_BATCH) {
+#pragma unroll
+                for (int v = 0; v < HEAVY_BATCH / 256; v++) s_mark[64 * v + lane] = 0u;
+                if (stamp < 1u << 20) clear_bins();  // a batch has at most 64 * HEAVY_ROUNDS rounds
+                tsg_wave_sync();
+                if (len > 0 && pre >= base && pre < base + HEAVY_BATCH) mk[pre - base] = (unsigned char)(lane + 1);
+                tsg_wave_sync();
+                int q[HEAVY_ROUNDS], col[HEAVY_ROUNDS];
+                double b[HEAVY_ROUNDS];
+#pragma unroll
+                for (int v = 0; v < HEAVY_ROUNDS; v++) {
+                    q[v] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * v + lane]));
+                    prev = __builtin_amdgcn_readlane(q[v], 63);
+                }
+#pragma unroll
+                for (int v = 0; v < HEAVY_ROUNDS; v++) {  // every lane loads in bounds
+                    const int e = __shfl(delta, q[v] - 1, 64) + min(base + 64 * v + lane, total - 1);
+                    col[v] = Bcolx[e];
+                    b[v] = Bvalx[e];
+                }
+                // all rounds' places before the first sum changes: their reads are in
+                // flight together
+                double as[HEAVY_ROUNDS];
+                unsigned wd[HEAVY_ROUNDS];
+#pragma unroll
+                for (int v = 0; v < HEAVY_ROUNDS; v++) as[v] = __shfl(a, q[v] - 1, 64);
+#pragma unroll
+                for (int v = 0; v < HEAVY_ROUNDS; v++) wd[v] = s_word[(col[v] >> 4) - jb];
+#pragma unroll
+                for (int v = 0; v < HEAVY_ROUNDS; v++) {
+                    if (base + 64 * v >= total) break;  // wave-uniform
+                    const bool on = base + 64 * v + lane < total;
+                    const int p = (int)(wd[v] & 0x7fffu) + __popc(wd[v] >> (31 - (col[v] & 15)));
+                    if (__builtin_amdgcn_readlane(q[v], 0) == __builtin_amdgcn_readlane(q[v], 63)) {  // one source
+                        if (on) s_acc[p] = __builtin_fma(as[v], b[v], s_acc[p]);
+                        tsg_wave_sync();
+                    } else {
+                        add_in_order(s_acc + p, s_bin + (p & (HEAVY_BINS - 1)), stamp, on, lane, as[v], b[v]);
+                    }
+                }
+            }
+        }
+        // the run's entries of row i, into their final positions
+        for (int tb = t; tb < te; tb += 256) {
+            int J[4], at[4];
+            unsigned wd[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int ti = min(tb + 64 * v + lane, te - 1);
+                J[v] = Ccol[ti];
+                wd[v] = Cmask[(long long)ti * 16 + r];
+                at[v] = Cnnz[ti] + Cptr16[(long long)ti * 16 + r];
+                if (tb + 64 * v + lane >= te) wd[v] = 0u;
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                unsigned cm = wd[v] << 16;
+                if (!cm) continue;
+                const double *d = s_acc + (s_word[J[v] - jb] & 0x7fffu);
+                double *o = Cval + at[v];
+                unsigned char *oc = Ccol8 + at[v];
+                while (cm) {
+                    const int c = __clz((int)cm);
+                    cm &= ~(0x80000000u >> c);
+                    *o++ = *d++;
+                    *oc++ = (unsigned char)c;
+                }
+            }
+        }
+        t = te;
+        tsg_wave_sync();  // the next run clears the sums
     }
 }
 
@@ -3219,12 +3347,11 @@ struct SpgemmWork {
     long long seg3_cap;
     // heavy rows (synchronous pipeline only; NULL = none)
     unsigned char *hflag;  // per C row
-    int2 *hitems;          // heavy-row work items
-    int *hcount;           // their number (device)
-    int nheavy, nitems, hwaves;
-    int *cursor;           // hwaves cursor arrays of hstride ints
-    long long hstride;
-    int *hnext;            // work-item counter (zeroed before the launch)
+    int *hrows;            // the heavy rows
+    int nheavy, nlong, ncounted;
+    const int *hwin;       // B rows' window table (k_heavy_windows), its stride and shift
+    long long hstride, hwin_bytes;
+    int hnw, hshift;
 };
 
 static size_t up16(size_t x) { return (x + 15) & ~(size_t)15; }
@@ -3274,12 +3401,10 @@ static SpgemmWork work_at(void *base, long long tilem, long long numtile, long l
     w.seg3 = (int4 *)(seg3_base ? (char *)seg3_base : b + off[11]);
     w.seg3_cap = tilem + nnz / (G3E_NNZ - 255) + 2;
     w.hflag = nullptr;
-    w.hitems = nullptr;
-    w.hcount = nullptr;
-    w.nheavy = w.nitems = w.hwaves = 0;
-    w.cursor = nullptr;
-    w.hstride = 0;
-    w.hnext = nullptr;
+    w.hrows = nullptr;
+    w.nheavy = w.nlong = w.ncounted = w.hnw = w.hshift = 0;
+    w.hwin = nullptr;
+    w.hstride = w.hwin_bytes = 0;
     return w;
 }
 
@@ -3403,12 +3528,18 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
                                (const int *)(w.segcnt + C->tilem), C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
                                C->tile_nnz, C->csr_col, C->val);
         TSG_LAUNCH_CHECK();
-        if (w.hflag && w.nitems > 0) {
-            hipLaunchKernelGGL(k_step3_heavy, dim3(w.hwaves), dim3(64), 0, s, op.Arowp, op.Acolx, op.Avalx,
-                               (const int *)B->rowx_ptr, (const int *)B->rowx_col, (const double *)B->rowx_val,
-                               (const int2 *)w.hitems, (const int *)w.hcount, C->tile_ptr, C->tile_colidx, C->mask,
-                               C->csr_ptr, C->tile_nnz, C->val, w.cursor, w.hstride, w.hnext);
-            TSG_LAUNCH_CHECK();
+        if (w.hflag) {
+            const long long parts = ((long long)B->n + HEAVY_PART_COLS - 1) / HEAVY_PART_COLS;
+            const long long hb = ((w.nheavy + 127LL) & ~127LL) * parts;
+            const long long total = hb + ((w.nlong + 127LL) & ~127LL) * ((parts + HEAVY_GROUP - 1) / HEAVY_GROUP);
+            for (long long at = 0; at < total; at += 1 << 25) {  // a launch takes fewer than 2^32 threads
+                hipLaunchKernelGGL(k_step3_heavy, dim3((unsigned)std::min(total - at, 1LL << 25)), dim3(64), 0, s,
+                                   op.Arowp, op.Acolx, op.Avalx, w.hwin, w.hstride, w.hnw, w.hshift,
+                                   (const int *)B->rowx_col, (const double *)B->rowx_val, (const int *)w.hrows,
+                                   w.nheavy, w.nlong, hb, at, C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
+                                   C->tile_nnz, C->csr_col, C->val);
+                TSG_LAUNCH_CHECK();
+            }
         }
     } else if (P.all || P.s3_unfit) {
         const unsigned nblk = tp_grid(tsg_div_up(C->numtile, S23_WAVES * TILES_PER_WAVE));
@@ -3436,14 +3567,14 @@ struct SpgemmTemps {
     unsigned *keep = nullptr;
     void *scr = nullptr, *wbuf = nullptr, *w3buf = nullptr, *bb = nullptr;
     unsigned char *hflag = nullptr;
-    int *hcnt = nullptr, *hinfo = nullptr, *hcur = nullptr, *span = nullptr, *longest = nullptr;
-    int2 *hitems = nullptr;
+    int *hcnt = nullptr, *hinfo = nullptr, *hwin = nullptr, *span = nullptr, *longest = nullptr;
+    int *hrows = nullptr;
     hipEvent_t ev[6] = {};
     int nev = 0;
 };
 
 static void free_temps(tsg_ctx *ctx, SpgemmTemps &t) {
-    void *ps[] = {t.keep, t.scr, t.wbuf, t.w3buf, t.hflag, t.hcnt, t.hinfo, t.hcur, t.hitems, t.span, t.bb, t.longest};
+    void *ps[] = {t.keep, t.scr, t.wbuf, t.w3buf, t.hflag, t.hcnt, t.hinfo, t.hwin, t.hrows, t.span, t.bb, t.longest};
     for (void *p : ps) tsg_free(ctx, p);
     for (int i = 0; i < t.nev; i++) (void)hipEventDestroy(t.ev[i]);
     t = SpgemmTemps();
@@ -3616,47 +3747,52 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                 // rows with very many products: one wave each (k_step3_heavy)
                 const int m = C->m;
                 TSG_TRY(tsg_alloc_t(ctx, &T.hflag, (size_t)m + 16));
-                TSG_TRY(tsg_alloc_t(ctx, &T.hcnt, (size_t)m + 1));
-                TSG_TRY(tsg_alloc_t(ctx, &T.hinfo, 4));  // {longest heavy A row, heavy rows, item counter, pad}
-                unsigned char *hflag = T.hflag;
-                int *hcnt = T.hcnt, *hinfo = T.hinfo;
-                TSG_HIP(hipMemsetAsync(hinfo, 0, 16, s));
-                hipLaunchKernelGGL(k_heavy_flags, dim3(tsg_div_up(m, 16)), dim3(256), 0, s, op.Arowp, op.Acolx,
-                                   (const int *)B->rowx_ptr, (const unsigned char *)w.rowcls, C->tile_ptr,
-                                   C->tile_colidx, m,
-                                   (long long)(tune.heavy_min_products > 0 ? tune.heavy_min_products
-                                                                           : HEAVY_MIN_PRODUCTS),
-                                   (long long)(tune.heavy_item_products > 0 ? tune.heavy_item_products
-                                                                            : HEAVY_ITEM_PRODUCTS),
-                                   hflag, hcnt, hinfo);
+                TSG_TRY(tsg_alloc_t(ctx, &T.hcnt, 2 * (size_t)m + 1));
+                TSG_TRY(tsg_alloc_t(ctx, &T.hinfo, 4));
+                TSG_HIP(hipMemsetAsync(T.hinfo, 0, 16, s));
+                const long long counted = tune.heavy_min_products > 0 ? tune.heavy_min_products : HEAVY_MIN_PRODUCTS;
+                const bool large = nnzC >= LONG_MIN_NNZ;
+                const long long split = tune.heavy_min_products > 0 || !large
+                                            ? counted
+                                            : std::min(nnzC >> HEAVY_SPLIT_LOG, HEAVY_SPLIT_MAX);
+                hipLaunchKernelGGL(k_heavy_flags, dim3(C->tilem), dim3(256), 0, s, op.Arowp, op.Acolx,
+                                   (const int *)B->rowx_ptr, w.rowcls, C->tile_ptr, m, split, counted,
+                                   large || tune.heavy_min_products > 0 ? 1 : 0, T.hflag, T.hcnt, T.hinfo);
                 TSG_LAUNCH_CHECK();
-                long long ni = 0;
-                TSG_TRY(tsg_scan_i32(ctx, hcnt, hcnt, m, &ni, hinfo, 2));
-                if (ni > 0x7fffffffLL) {
-                    tsg_set_error("spgemm: %lld heavy-row work items exceed the int32 range", ni);
-                    return TSG_ERR_ARG;
-                }
-                if (ni > 0) {
-                    const volatile int *info = (const volatile int *)(ctx->pinned + 1);
-                    const long long maxdeg = info[0], nrows = info[1];
-                    TSG_TRY(tsg_alloc_t(ctx, &T.hitems, (size_t)ni));
-                    int2 *hitems = T.hitems;
-                    hipLaunchKernelGGL(k_heavy_list, dim3(tsg_div_up(m, 256)), dim3(256), 0, s, (const int *)hcnt,
-                                       (const unsigned char *)hflag, C->tile_ptr, C->tile_colidx, m, hitems);
+                long long nh = 0;
+                TSG_TRY(tsg_scan_i32(ctx, T.hcnt, T.hcnt, 2LL * m, &nh, T.hinfo, 2));
+                const volatile int *info = (const volatile int *)(ctx->pinned + 1);
+                const int nheavy = info[0];
+                w.ncounted = info[1];
+                if (nh > 0) {
+                    TSG_TRY(tsg_alloc_t(ctx, &T.hrows, (size_t)nh));
+                    hipLaunchKernelGGL(k_heavy_list, dim3(tsg_div_up(m, 256)), dim3(256), 0, s, (const int *)T.hcnt,
+                                       (const unsigned char *)T.hflag, m, T.hrows);
                     TSG_LAUNCH_CHECK();
-                    // one wave per item up to HEAVY_MAX_WAVES, cursors within HEAVY_CURSOR_BYTES
-                    const long long by_mem = std::max<long long>(256, HEAVY_CURSOR_BYTES / (4 * std::max(1LL, maxdeg)));
-                    w.hwaves = (int)std::min<long long>(ni, std::min<long long>(HEAVY_MAX_WAVES, by_mem));
-                    w.hstride = std::max(1LL, maxdeg);
-                    if (!symbolic) TSG_TRY(tsg_alloc_t(ctx, &T.hcur, (size_t)w.hwaves * (size_t)w.hstride));
-                    int *hcur = T.hcur;
-                    w.hflag = hflag;
-                    w.hitems = hitems;
-                    w.hcount = hcnt + m;
-                    w.nheavy = (int)nrows;
-                    w.nitems = (int)ni;
-                    w.cursor = hcur;
-                    w.hnext = hinfo + 2;
+                    // the narrowest windows whose table is small enough; one window is B's row pointers
+                    int shift = HEAVY_PART_LOG;
+                    long long nw = ((long long)B->n + (1 << shift) - 1) >> shift;
+                    while (nw > 1 && 4 * (nw + 1) * B->m > HEAVY_WINDOW_BYTES) {
+                        shift++;
+                        nw = (nw + 1) >> 1;
+                    }
+                    w.hflag = T.hflag;
+                    w.hrows = T.hrows;
+                    w.nheavy = nheavy;
+                    w.nlong = (int)nh - nheavy;
+                    w.hnw = (int)nw;
+                    w.hshift = nw > 1 ? shift : 31;
+                    w.hstride = nw > 1 ? B->m : 1;
+                    w.hwin_bytes = nw > 1 ? 4 * (nw + 1) * B->m : 0;
+                    w.hwin = B->rowx_ptr;
+                    if (nw > 1 && !symbolic) {
+                        TSG_TRY(tsg_alloc(ctx, (void **)&T.hwin, (size_t)w.hwin_bytes));
+                        hipLaunchKernelGGL(k_heavy_windows, dim3(tsg_div_up(B->m, 256), (unsigned)nw + 1), dim3(256), 0, s,
+                                           (const int *)B->rowx_ptr, (const int *)B->rowx_col, B->m, (int)nw, shift,
+                                           T.hwin);
+                        TSG_LAUNCH_CHECK();
+                        w.hwin = T.hwin;
+                    }
                 }
             }
         }
@@ -3678,8 +3814,8 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         stats->tiles_dense_acc = (long long)hb[2];
         stats->numtileC = numtileC;
         stats->nnzC = nnzC;
-        stats->heavy_rows = w.nheavy;
-        stats->heavy_bytes = (long long)w.hwaves * w.hstride * 4 + (w.nheavy ? 5LL * C->m + 8LL * w.nitems : 0);
+        stats->heavy_rows = w.ncounted;
+        stats->heavy_bytes = w.hwin_bytes + (w.hflag ? 9LL * C->m + 4LL * ((long long)w.nheavy + w.nlong) : 0);
     }
     if (plan_out) *plan_out = P;
     return TSG_OK;
