@@ -1596,27 +1596,28 @@ k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
 }
 
 // ------------------------------------------------------------------ step 3, flat rows
-// One product per lane, in ascending k along the lanes, into sums of which
-// several lanes may share one (a lane's bin decides: equal sums, equal bins).
-// In each round the lowest pending lane of a bin adds, so a shared sum gets
-// its products in lane order.  The winner is the bin's minimum of stamp + lane;
-// stamps descend, so bins need no clearing between rounds.
-__device__ __forceinline__ void add_in_order(double *sum, unsigned *bin, unsigned &stamp, bool on, int lane, double a,
+// One product per lane, of sources q0 (lane 0's) to q1 in ascending k along the
+// lanes, into sums that products of different sources may share: each lane
+// leaves its number at its sum and reads it back, and if some lane finds
+// another's the sources are added one by one.
+__device__ __forceinline__ void add_in_order(double *sum, unsigned char *tag, bool on, int q, int lane, double a,
                                              double b) {
-    for (;;) {
-        stamp -= 64u;
-        const unsigned me = stamp + (unsigned)lane;
-        if (on) atomicMin(bin, me);
+    const int q0 = __builtin_amdgcn_readlane(q, 0), q1 = __builtin_amdgcn_readlane(q, 63);
+    bool clash = false;
+    if (q0 != q1) {
+        if (on) *tag = (unsigned char)lane;
         tsg_wave_sync();
-        const unsigned first = *bin;
-        const double v = *sum;  // with the bin: one LDS round trip a round
-        if (on && first == me) {
-            *sum = __builtin_fma(a, b, v);
-            on = false;
-        }
-        tsg_wave_sync();
-        if (!__ballot(on)) break;
+        clash = __ballot(on && *tag != (unsigned char)lane) != 0;
     }
+    if (!clash) {
+        if (on) *sum = __builtin_fma(a, b, *sum);
+    } else {
+        for (int s = q0; s <= q1; s++) {
+            if (on && q == s) *sum = __builtin_fma(a, b, *sum);
+            tsg_wave_sync();
+        }
+    }
+    tsg_wave_sync();
 }
 // [b0, b1) cut to list's entries in [lo, hi) (list ascending; an end that is
 // not to be cut keeps its place).  Both ends at once and a quarter of the
@@ -1684,7 +1685,6 @@ __device__ __forceinline__ void range_in(const int *__restrict__ list, int &b0, 
 #define G3F_SLOTS (G3F_NNZ + G3F_NNZ / 2 + 32)
 #define G3F_ROUNDS 4
 #define G3F_BATCH (64 * G3F_ROUNDS)
-#define G3F_BINS 128
 #define G3F_SPAN 65535  // tile columns of a tile-row: offsets + 1 below 2^20
 __device__ __forceinline__ unsigned flat_home(unsigned key, unsigned n) {
     return (unsigned)(((unsigned long long)(key * 2654435761u) * n) >> 32);
@@ -1700,8 +1700,8 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
     __shared__ double s_acc[G3F_NNZ];
     __shared__ unsigned s_key[G3F_SLOTS];
     __shared__ unsigned short s_pos[WIDE ? G3F_SLOTS : 1];
-    // marks of a batch, then the bins of its products
-    __shared__ unsigned s_mark[G3F_WAVES][G3F_BINS];
+    __shared__ unsigned char s_tag[G3F_NNZ];
+    __shared__ unsigned s_mark[G3F_WAVES][G3F_BATCH / 4];
     __shared__ int s_cnt[G3F_WAVES][16], s_rb[17];
     __shared__ unsigned char s_ord[16];
     static_assert(G3F_NNZ <= 4096, "positions take 12 bits of a slot");
@@ -1849,10 +1849,6 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
                 q[i] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * i + lane]));
                 prev = __builtin_amdgcn_readlane(q[i], 63);
             }
-            tsg_wave_sync();
-            for (int j = lane; j < G3F_BINS; j += 64) s_mark[wave][j] = 0xffffffffu;
-            unsigned stamp = 0xffffffc0u;
-            tsg_wave_sync();
 #pragma unroll
             for (int i = 0; i < G3F_ROUNDS; i++) {  // every lane loads in bounds
                 const int e = __shfl(delta, q[i] - 1, 64) + min(base + 64 * i + lane, total - 1);
@@ -1872,13 +1868,7 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
                 // (the entry is in C's structure: the probe bound is not reached)
                 while ((ent = key0[h], WIDE ? ent : ent >> 12) != key && ++probe < n_r) h = h + 1 == n_r ? 0u : h + 1;
                 const int pos = WIDE ? (int)s_pos[(rg & 0xffff) + h] : (int)(ent & 4095u);
-                const int q0 = __builtin_amdgcn_readlane(q[i], 0), q1 = __builtin_amdgcn_readlane(q[i], 63);
-                if (q0 == q1) {
-                    if (on) s_acc[pos] = __builtin_fma(as, b[i], s_acc[pos]);
-                    tsg_wave_sync();
-                } else {
-                    add_in_order(s_acc + pos, s_mark[wave] + (pos & (G3F_BINS - 1)), stamp, on, lane, as, b[i]);
-                }
+                add_in_order(s_acc + pos, s_tag + pos, on, q[i], lane, as, b[i]);
             }
         }
     }
@@ -1897,7 +1887,7 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 // as many parts at a time as the row's entries in them fit its sums, writes
 // for each tile the row's mask and its offset among the sums, walks A row i in
 // ascending k, 64 entries (sources) at a time, numbers the products with the B
-// entries in these parts through and adds 64 per step (add_in_order), then
+// entries in these parts through and adds 64 per step (add_in_rounds), then
 // copies the sums to C's final positions with their column bytes.
 //   Where B row k's entries of a part start and end is read from a table
 // made once per product (k_heavy_windows), two groups of sources ahead, so no
@@ -2009,8 +1999,32 @@ __device__ __forceinline__ int wave_lower_bound(const int *__restrict__ list, in
     return lo;
 }
 
+// One product per lane, in ascending k along the lanes, into sums of which
+// several lanes may share one (a lane's bin decides: equal sums, equal bins).
+// In each round the lowest pending lane of a bin adds, so a shared sum gets
+// its products in lane order.  The winner is the bin's minimum of stamp + lane;
+// stamps descend, so bins need no clearing between rounds.  Against
+// add_in_order: R-MAT scale 16 A*A^T 7.65 -> 7.07 ms in k_step3_heavy, whose rows
+// meet many short sources, but scale 13 A^2 344 -> 400 us in k_step3_flat.
+__device__ __forceinline__ void add_in_rounds(double *sum, unsigned *bin, unsigned &stamp, bool on, int lane, double a,
+                                             double b) {
+    for (;;) {
+        stamp -= 64u;
+        const unsigned me = stamp + (unsigned)lane;
+        if (on) atomicMin(bin, me);
+        tsg_wave_sync();
+        const unsigned first = *bin;
+        const double v = *sum;  // with the bin: one LDS round trip a round
+        if (on && first == me) {
+            *sum = __builtin_fma(a, b, v);
+            on = false;
+        }
+        tsg_wave_sync();
+        if (!__ballot(on)) break;
+    }
+}
 #define HEAVY_ROUNDS 4
-#define HEAVY_BINS 256  // of add_in_order; products of different sums that share one only take a round more
+#define HEAVY_BINS 256  // of add_in_rounds; products of different sums that share one only take a round more
 #define HEAVY_BATCH (64 * HEAVY_ROUNDS)
 __global__ void __launch_bounds__(64)
 k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const double *__restrict__ Avalx,
@@ -2158,7 +2172,7 @@ k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
                         if (on) s_acc[p] = __builtin_fma(as[v], b[v], s_acc[p]);
                         tsg_wave_sync();
                     } else {
-                        add_in_order(s_acc + p, s_bin + (p & (HEAVY_BINS - 1)), stamp, on, lane, as[v], b[v]);
+                        add_in_rounds(s_acc + p, s_bin + (p & (HEAVY_BINS - 1)), stamp, on, lane, as[v], b[v]);
                     }
                 }
             }
