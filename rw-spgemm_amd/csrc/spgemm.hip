@@ -58,54 +58,55 @@ extern "C" void tsg_tune_default(tsg_tune *t) {
 // tile-row, then k_brow_fill, one lane per B tile, so a hub tile-row's
 // words are spread over as many waves as it has tiles.  With longest (and B's
 // row pointers), longest[K] = entries of the longest row of tile-row K.
+// Tile-row K's descriptor (and longest[K]); returns whether it is kept.
+__device__ __forceinline__ bool brow_desc(const int *__restrict__ Bptr, const int *__restrict__ Bcol, int K, int4 *desc,
+                                          const int *__restrict__ Browp, int m, int *longest) {
+    const int b0 = Bptr[K], n = Bptr[K + 1] - b0;
+    int F = 0, nw = 0;
+    if (n > 0) {
+        F = Bcol[b0] >> 5;
+        nw = (Bcol[b0 + n - 1] >> 5) - F + 1;
+        if (nw > 2 * n + 2) nw = 0;
+    }
+    desc[K] = make_int4(2 * b0 + 2 * K, F, nw, 0);
+    if (longest) {
+        int p = Browp[16 * K], mx = 0;
+        if (16 * K + 16 <= m) {
+            int q[16];
+#pragma unroll
+            for (int r = 0; r < 16; r++) q[r] = Browp[16 * K + 1 + r];
+#pragma unroll
+            for (int r = 0; r < 16; r++) mx = max(mx, q[r] - (r ? q[r - 1] : p));
+        } else {
+            for (int r = 16 * K + 1; r <= m; r++) {
+                mx = max(mx, Browp[r] - p);
+                p = Browp[r];
+            }
+        }
+        longest[K] = mx;
+    }
+    return nw > 0;
+}
 __global__ void __launch_bounds__(256)
 k_brow_desc(const int *__restrict__ Bptr, const int *__restrict__ Bcol, int tilem, int4 *__restrict__ desc,
             int *__restrict__ any, const int *__restrict__ Browp, int m, int *__restrict__ longest) {
     const int K = blockIdx.x * 256 + threadIdx.x;
-    int nw = 0;
-    if (K < tilem) {
-        const int b0 = Bptr[K], n = Bptr[K + 1] - b0;
-        int F = 0;
-        if (n > 0) {
-            F = Bcol[b0] >> 5;
-            nw = (Bcol[b0 + n - 1] >> 5) - F + 1;
-            if (nw > 2 * n + 2) nw = 0;
-        }
-        desc[K] = make_int4(2 * b0 + 2 * K, F, nw, 0);
-        if (longest) {
-            int p = Browp[16 * K], mx = 0;
-            if (16 * K + 16 <= m) {
-                int q[16];
-#pragma unroll
-                for (int r = 0; r < 16; r++) q[r] = Browp[16 * K + 1 + r];
-#pragma unroll
-                for (int r = 0; r < 16; r++) mx = max(mx, q[r] - (r ? q[r - 1] : p));
-            } else {
-                for (int r = 16 * K + 1; r <= m; r++) {
-                    mx = max(mx, Browp[r] - p);
-                    p = Browp[r];
-                }
-            }
-            longest[K] = mx;
-        }
-    }
+    const bool kept = K < tilem && brow_desc(Bptr, Bcol, K, desc, Browp, m, longest);
     // any (may be NULL, zeroed beforehand): set when some row is kept; the
     // same value from every writer, and no store once it reads 1
-    if (any && __ballot(nw > 0) && (threadIdx.x & 63) == 0 && *(volatile int *)any == 0) *(volatile int *)any = 1;
+    if (any && __ballot(kept) && (threadIdx.x & 63) == 0 && *(volatile int *)any == 0) *(volatile int *)any = 1;
 }
 
 // A run is the tiles of one kept row in one bitmap word (consecutive in the
 // row-major tile order).  Its last tile's lane writes the word (the run's
 // bits OR-ed across lanes, plus the run's tiles before the wave's first,
 // at most 31) and zeroes the empty words up to the row's next run.
-__global__ void __launch_bounds__(256)
-k_brow_fill(const int *__restrict__ Brow, const int *__restrict__ Bcol, long long numtile,
-            const int4 *__restrict__ desc, unsigned *__restrict__ bits, const int *__restrict__ any) {
+// t: the lane's tile, whole waves (desc is not restrict: k_brow_one writes it)
+__device__ __forceinline__ void brow_fill(const int *__restrict__ Brow, const int *__restrict__ Bcol, long long numtile,
+                                          const int4 *desc, unsigned *__restrict__ bits, long long t) {
     const int lane = threadIdx.x & 63;
-    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
     const long long t0 = t - lane;  // the wave's first tile
-    if (t0 >= numtile) return;      // whole waves
-    if (any && *any == 0) return;   // no row kept (k_brow_desc's flag, when given)
+    if (t0 >= numtile) return;
     const bool valid = t < numtile;
     int K = -1, w = -1, col = 0;
     int4 d = make_int4(0, 0, 0, 0);
@@ -150,6 +151,38 @@ k_brow_fill(const int *__restrict__ Brow, const int *__restrict__ Bcol, long lon
         const int wend = Kn == K ? wn : d.z;  // the row's next run, or its end
         for (int g = w + 1; g < wend; g++) row[g] = 0u;
     }
+}
+
+__global__ void __launch_bounds__(256)
+k_brow_fill(const int *__restrict__ Brow, const int *__restrict__ Bcol, long long numtile,
+            const int4 *__restrict__ desc, unsigned *__restrict__ bits, const int *__restrict__ any) {
+    if (any && *any == 0) return;  // no row kept (k_brow_desc's flag, when given)
+    brow_fill(Brow, Bcol, numtile, desc, bits, (long long)blockIdx.x * 256 + threadIdx.x);
+}
+
+// Both for a small B in one block, which also clears the SCR_WORDS words of scr
+// (may be NULL) and sets any: a launch takes about 4 us of a small product, more than
+// its kernels' work.  5-point 64^2 A^2 in 8 launches instead of 13 (this one, k_row_stats_one,
+// the class maxima by k_row_class's last block): 84 -> 77 us.
+// ER 1000 (4 per row, 2,500 tiles) 103 -> 99 us, but with 3,900 tiles 110 -> 114.
+#define BROW_ONE 2560  // tiles of a B that one block takes
+#define BROW_ONE_ROWS 1024  // and tile-rows
+#define SCR_WORDS 32
+__global__ void __launch_bounds__(1024)
+k_brow_one(const int *__restrict__ Bptr, const int *__restrict__ Brow, const int *__restrict__ Bcol, int tilem,
+           int numtile, int4 *desc, unsigned *__restrict__ bits, int *scr, int *any, const int *__restrict__ Browp, int m,
+           int *__restrict__ longest) {
+    __shared__ int s_any;
+    if (threadIdx.x == 0) s_any = 0;
+    if (scr && threadIdx.x < SCR_WORDS && scr + threadIdx.x != any) scr[threadIdx.x] = 0;
+    __syncthreads();
+    bool kept = false;
+    for (int K = threadIdx.x; K < tilem; K += 1024) kept |= brow_desc(Bptr, Bcol, K, desc, Browp, m, longest);
+    if (__ballot(kept) && (threadIdx.x & 63) == 0) s_any = 1;
+    __syncthreads();  // the block's descriptors are written
+    if (any && threadIdx.x == 0) *any = s_any;
+    if (!s_any) return;
+    for (int t = threadIdx.x; t - (int)(threadIdx.x & 63) < numtile; t += 1024) brow_fill(Brow, Bcol, numtile, desc, bits, t);
 }
 
 // ------------------------------------------------------------------ step 1
@@ -634,6 +667,38 @@ k_seg1_fill(const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tile
 // line, serialised) are few.
 #define ROW_STATS_BLOCKS 64
 #define ROW_STATS 8
+__device__ __forceinline__ void row_stats_add(int v[ROW_STATS], int I, int u, const int *__restrict__ span,
+                                              const int *__restrict__ Aptr, const int *__restrict__ Annz, int elem, int all,
+                                              int rx) {
+    if (u <= 0) return;
+    const int s1 = span[I], a0 = Aptr[I], a1 = Aptr[I + 1];
+    const long long ents = (long long)Annz[a1] - Annz[a0];
+    const int kind = step2_kind(u, s1, ents, a1 - a0, elem, all, rx);
+    v[1] = max(v[1], s1);
+    if (kind == 0) {
+        v[0] = max(v[0], min(u, G2_UMAX));
+        if (s1 <= G2_MAP_MAX) v[2] = max(v[2], s1);
+    }
+#pragma unroll
+    for (int k = 0; k < S2_KINDS; k++) v[3 + k] += kind == k ? step2_segments(kind, u, s1, ents) : 0;
+    if (kind == 2) v[7] = max(v[7], s1);
+}
+// The block's (1024 threads) sum or maximum of word i, in the threads i < ROW_STATS.
+__device__ __forceinline__ int row_stats_fold(int v[ROW_STATS], int s_r[16][ROW_STATS]) {
+#pragma unroll
+    for (int i = 0; i < ROW_STATS; i++) {
+        v[i] = i >= 3 && i < 7 ? tsg_wave_sum(v[i]) : tsg_wave_max(v[i]);
+        if ((threadIdx.x & 63) == 0) s_r[threadIdx.x >> 6][i] = v[i];
+    }
+    __syncthreads();
+    int x = 0;
+    if (threadIdx.x < ROW_STATS) {
+        const int i = threadIdx.x;
+        x = s_r[0][i];
+        for (int w = 1; w < 16; w++) x = i >= 3 && i < 7 ? x + s_r[w][i] : max(x, s_r[w][i]);
+    }
+    return x;
+}
 __global__ void __launch_bounds__(1024)
 k_row_stats(const int *__restrict__ cnt, const int *__restrict__ span, const int *__restrict__ Aptr,
             const int *__restrict__ Annz, int tilem, int elem, int all, int rx, int *__restrict__ out) {
@@ -641,34 +706,39 @@ k_row_stats(const int *__restrict__ cnt, const int *__restrict__ span, const int
     int v[ROW_STATS];
 #pragma unroll
     for (int i = 0; i < ROW_STATS; i++) v[i] = 0;
-    for (int I = blockIdx.x * 1024 + threadIdx.x; I < tilem; I += gridDim.x * 1024) {
-        const int u = cnt[I];
-        if (u <= 0) continue;
-        const int s1 = span[I], a0 = Aptr[I], a1 = Aptr[I + 1];
-        const long long ents = (long long)Annz[a1] - Annz[a0];
-        const int kind = step2_kind(u, s1, ents, a1 - a0, elem, all, rx);
-        v[1] = max(v[1], s1);
-        if (kind == 0) {
-            v[0] = max(v[0], min(u, G2_UMAX));
-            if (s1 <= G2_MAP_MAX) v[2] = max(v[2], s1);
-        }
-#pragma unroll
-        for (int k = 0; k < S2_KINDS; k++) v[3 + k] += kind == k ? step2_segments(kind, u, s1, ents) : 0;
-        if (kind == 2) v[7] = max(v[7], s1);
-    }
-#pragma unroll
-    for (int i = 0; i < ROW_STATS; i++) {
-        v[i] = i >= 3 && i < 7 ? tsg_wave_sum(v[i]) : tsg_wave_max(v[i]);
-        if ((threadIdx.x & 63) == 0) s_r[threadIdx.x >> 6][i] = v[i];
-    }
-    __syncthreads();
+    for (int I = blockIdx.x * 1024 + threadIdx.x; I < tilem; I += gridDim.x * 1024)
+        row_stats_add(v, I, cnt[I], span, Aptr, Annz, elem, all, rx);
+    const int x = row_stats_fold(v, s_r);
     if (threadIdx.x < ROW_STATS) {
-        const int i = threadIdx.x;
-        const bool sum = i >= 3 && i < 7;
-        int x = s_r[0][i];
-        for (int w = 1; w < 16; w++) x = sum ? x + s_r[w][i] : max(x, s_r[w][i]);
-        if (sum) atomicAdd(&out[i], x);
-        else atomicMax(&out[i], x);
+        if (threadIdx.x >= 3 && threadIdx.x < 7) atomicAdd(&out[threadIdx.x], x);
+        else atomicMax(&out[threadIdx.x], x);
+    }
+}
+// The same for few tile-rows, one a thread, with the scan of the counts, in
+// place (ptr[tilem] = total); the total and the statistics go to pinned memory.
+// (With four a thread it lost 2 to 10 us against two launches at 3,100 to 3,750
+// tile-rows.)
+#define ROW_STATS_ONE 1024
+__global__ void __launch_bounds__(1024)
+k_row_stats_one(int *ptr, const int *__restrict__ span, const int *__restrict__ Aptr, const int *__restrict__ Annz,
+                int tilem, int elem, int all, int rx, long long *__restrict__ host) {
+    __shared__ int s_r[16][ROW_STATS];
+    __shared__ long long s_w[16];
+    const int I = threadIdx.x, c = I < tilem ? ptr[I] : 0;
+    int v[ROW_STATS];
+#pragma unroll
+    for (int i = 0; i < ROW_STATS; i++) v[i] = 0;
+    row_stats_add(v, I, c, span, Aptr, Annz, elem, all, rx);
+    const long long incl = tsg_wave_incl_scan((long long)c);
+    if ((I & 63) == 63) s_w[I >> 6] = incl;
+    const int x = row_stats_fold(v, s_r);  // (a barrier within)
+    long long at = incl - c;
+    for (int w = 0; w < (I >> 6); w++) at += s_w[w];
+    if (I < ROW_STATS) reinterpret_cast<int *>(host + 1)[I] = x;
+    if (I < tilem) ptr[I] = (int)at;
+    if (I == 1023) {
+        host[0] = at + c;
+        ptr[tilem] = at + c > 0x7fffffffLL ? 0x7fffffff : (int)(at + c);
     }
 }
 
@@ -3007,8 +3077,8 @@ __device__ __forceinline__ int g16_max(int v) {
 }
 __global__ void __launch_bounds__(256)
 k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict__ Ccol, const int *__restrict__ Cnnz, int tilem,
-            unsigned char *__restrict__ cls, int *__restrict__ part, int none_fit,
-            const int *__restrict__ longest) {
+            unsigned char *__restrict__ cls, int *part, int none_fit, const int *__restrict__ longest,
+            int *__restrict__ ticket, int *__restrict__ out, int *__restrict__ host) {
     __shared__ int s_red[4][CLS_WORDS];
     const int r = threadIdx.x & 15, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int I = blockIdx.x * 16 + (threadIdx.x >> 4);
@@ -3088,6 +3158,32 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
 #pragma unroll
         for (int w = 1; w < 4; w++) v = i == 0 ? v + s_red[w][i] : max(v, s_red[w][i]);
         part[CLS_WORDS * (long long)blockIdx.x + i] = v;
+        if (ticket) __threadfence();
+    }
+    if (!ticket) return;
+    // few blocks: the last one to get here folds the partials
+    __shared__ int s_last;
+    __syncthreads();
+    if (threadIdx.x == 0) s_last = atomicAdd(ticket, 1) == (int)gridDim.x - 1;
+    __syncthreads();
+    if (!s_last) return;
+    __threadfence();
+    int v[CLS_WORDS];
+#pragma unroll
+    for (int i = 0; i < CLS_WORDS; i++) v[i] = threadIdx.x < gridDim.x ? part[CLS_WORDS * threadIdx.x + i] : 0;
+#pragma unroll
+    for (int i = 0; i < CLS_WORDS; i++) {
+        v[i] = i == 0 ? tsg_wave_sum(v[i]) : tsg_wave_max(v[i]);
+        if (lane == 0) s_red[wave][i] = v[i];
+    }
+    __syncthreads();
+    if (threadIdx.x < CLS_WORDS) {
+        const int i = threadIdx.x;
+        int x = s_red[0][i];
+#pragma unroll
+        for (int w = 1; w < 4; w++) x = i == 0 ? x + s_red[w][i] : max(x, s_red[w][i]);
+        out[i] = x;
+        if (host) host[i] = x;
     }
 }
 
@@ -3290,20 +3386,29 @@ static size_t brow_bits_bytes(const tsg_dtiles *B) {
     if (words >= 0x7fffffffLL) return 0;
     return (size_t)B->tilem * 16 + (size_t)words * 4;
 }
+// scr: SCR_WORDS words to be cleared, any among them (both may be NULL)
 static int launch_brow_bits(hipStream_t s, const tsg_dtiles *B, void *buf, const int4 **desc,
-                            const unsigned **bits, int *any, int *longest) {
+                            const unsigned **bits, int *scr, int *any, int *longest) {
     *desc = nullptr;
     *bits = nullptr;
-    if (!buf || !brow_bits_bytes(B)) return TSG_OK;
+    const bool make = buf && brow_bits_bytes(B), one = make && B->tilem <= BROW_ONE_ROWS && B->numtile <= BROW_ONE;
+    if (scr && !one) TSG_HIP(hipMemsetAsync(scr, 0, 4 * SCR_WORDS, s));
+    if (!make) return TSG_OK;
     int4 *d = (int4 *)buf;
     unsigned *w = (unsigned *)((char *)buf + (size_t)B->tilem * 16);
-    hipLaunchKernelGGL(k_brow_desc, dim3(tsg_div_up(B->tilem, 256)), dim3(256), 0, s, (const int *)B->tile_ptr,
-                       (const int *)B->tile_colidx, B->tilem, d, any, (const int *)B->rowx_ptr, B->m,
-                       B->rowx_ptr ? longest : nullptr);
-    if (B->numtile > 0)
-        hipLaunchKernelGGL(k_brow_fill, dim3(tsg_div_up(B->numtile, 256)), dim3(256), 0, s,
-                           (const int *)B->tile_rowidx, (const int *)B->tile_colidx, (long long)B->numtile,
-                           (const int4 *)d, w, (const int *)any);
+    const int *browp = B->rowx_ptr;
+    if (!browp) longest = nullptr;
+    if (one) {
+        hipLaunchKernelGGL(k_brow_one, dim3(1), dim3(1024), 0, s, (const int *)B->tile_ptr, (const int *)B->tile_rowidx,
+                           (const int *)B->tile_colidx, B->tilem, B->numtile, d, w, scr, any, browp, B->m, longest);
+    } else {
+        hipLaunchKernelGGL(k_brow_desc, dim3(tsg_div_up(B->tilem, 256)), dim3(256), 0, s, (const int *)B->tile_ptr,
+                           (const int *)B->tile_colidx, B->tilem, d, any, browp, B->m, longest);
+        if (B->numtile > 0)
+            hipLaunchKernelGGL(k_brow_fill, dim3(tsg_div_up(B->numtile, 256)), dim3(256), 0, s,
+                               (const int *)B->tile_rowidx, (const int *)B->tile_colidx, (long long)B->numtile,
+                               (const int4 *)d, w, (const int *)any);
+    }
     TSG_LAUNCH_CHECK();
     *desc = d;
     *bits = w;
@@ -3487,14 +3592,20 @@ static int launch_step2(hipStream_t s, const TileOperands &op, const tsg_dtiles 
     return TSG_OK;
 }
 
+// ticket (may be NULL): a cleared word for k_row_class's last block
+#define CLS_ONE 64
 static int launch_row_class(hipStream_t s, const TileOperands &op, tsg_dtiles *C, unsigned char *rowcls,
-                            int *cls_part, int *cls_out, int none_fit, const int *longest, int *host = nullptr) {
+                            int *cls_part, int *cls_out, int none_fit, const int *longest, int *ticket = nullptr,
+                            int *host = nullptr) {
     const int nb = (int)tsg_div_up(C->tilem, 16);
+    if (nb > CLS_ONE) ticket = nullptr;
     hipLaunchKernelGGL(k_row_class, dim3(nb), dim3(256), 0, s, op, C->tile_ptr, C->tile_colidx, C->tile_nnz, C->tilem,
-                       rowcls, cls_part, none_fit, longest);
+                       rowcls, cls_part, none_fit, longest, ticket, cls_out, host);
     TSG_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_row_class_reduce, dim3(1), dim3(1024), 0, s, (const int *)cls_part, nb, cls_out, host);
-    TSG_LAUNCH_CHECK();
+    if (!ticket) {
+        hipLaunchKernelGGL(k_row_class_reduce, dim3(1), dim3(1024), 0, s, (const int *)cls_part, nb, cls_out, host);
+        TSG_LAUNCH_CHECK();
+    }
     return TSG_OK;
 }
 
@@ -3645,35 +3756,47 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     P.s1w = tsg_s1_words(B, tune);
     const size_t kb = keep_bytes(C->tilem, P.s1w);
     if (kb) TSG_TRY(tsg_alloc(ctx, (void **)&T.keep, kb));
+    static_assert(4 * SCR_WORDS == 128, "bins, flags, row statistics");
     TSG_TRY(tsg_alloc(ctx, &T.scr, 128));
     void *scr = T.scr;
     unsigned long long *bins = (unsigned long long *)scr;
     int *bany = reinterpret_cast<int *>(static_cast<char *>(scr) + 32);  // some B tile-row bitmap kept
     int *st2 = reinterpret_cast<int *>(static_cast<char *>(scr) + 64);   // k_row_stats
-    TSG_HIP(hipMemsetAsync(scr, 0, 128, s));
+    int *ticket = reinterpret_cast<int *>(static_cast<char *>(scr) + 36);  // k_row_class
     TSG_TRY(tsg_alloc_t(ctx, &T.span, (size_t)C->tilem + 1));
     const int4 *bdesc = nullptr;
     const unsigned *bbits = nullptr;
     if (const size_t bbb = C->tilem > 0 ? brow_bits_bytes(B) : 0) {
         TSG_TRY(tsg_alloc(ctx, &T.bb, bbb));
         if (P.lines) TSG_TRY(tsg_alloc_t(ctx, &T.longest, (size_t)B->tilem));
-        TSG_TRY(launch_brow_bits(s, B, T.bb, &bdesc, &bbits, bany, T.longest));
     }
+    TSG_TRY(launch_brow_bits(s, B, T.bb, &bdesc, &bbits, (int *)scr, bany, T.longest));
     TSG_TRY(launch_step1(s, A, B, C, false, P.s1w, T.keep, bdesc, bbits, bany, T.span));
-    if (C->tilem > 0) {
-        hipLaunchKernelGGL(k_row_stats, dim3(std::min<unsigned>(ROW_STATS_BLOCKS, tsg_div_up(C->tilem, 1024))),
-                           dim3(1024), 0, s, (const int *)C->tile_ptr, (const int *)T.span, A->tile_ptr, A->tile_nnz,
-                           C->tilem, P.s3_elem, P.elem_all, A->rowx_ptr ? 1 : 0, st2);
-        TSG_LAUNCH_CHECK();
-    }
     // C's tile-row offsets; their total and the step-2 sizing maxima come
     // back in one read-back
     long long numtileC = 0;
     int smax[ROW_STATS] = {};
-    {
+    const int rx = A->rowx_ptr ? 1 : 0;
+    if (C->tilem > 0 && C->tilem <= ROW_STATS_ONE) {
+        hipLaunchKernelGGL(k_row_stats_one, dim3(1), dim3(1024), 0, s, C->tile_ptr, (const int *)T.span, A->tile_ptr,
+                           A->tile_nnz, C->tilem, P.s3_elem, P.elem_all, rx, ctx->pinned);
+        TSG_LAUNCH_CHECK();
+        TSG_HIP(hipStreamSynchronize(s));
+        numtileC = *(volatile long long *)ctx->pinned;
+        if (numtileC > 0x7fffffffLL) {
+            tsg_set_error("prefix sum total %lld exceeds int32", numtileC);
+            return TSG_ERR_OVERFLOW;
+        }
+    } else {
+        if (C->tilem > 0) {
+            hipLaunchKernelGGL(k_row_stats, dim3(std::min<unsigned>(ROW_STATS_BLOCKS, tsg_div_up(C->tilem, 1024))),
+                               dim3(1024), 0, s, (const int *)C->tile_ptr, (const int *)T.span, A->tile_ptr,
+                               A->tile_nnz, C->tilem, P.s3_elem, P.elem_all, rx, st2);
+            TSG_LAUNCH_CHECK();
+        }
         TSG_TRY(tsg_scan_i32(ctx, C->tile_ptr, C->tile_ptr, C->tilem, &numtileC, st2, ROW_STATS));
-        memcpy(smax, ctx->pinned + 1, sizeof(smax));
     }
+    memcpy(smax, ctx->pinned + 1, sizeof(smax));
     tsg_free(ctx, T.span);
     T.span = nullptr;
     P.numtileC = numtileC;
@@ -3725,7 +3848,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_nnz, C->tile_nnz, numtileC, part2, pub));
         if (timed) TSG_HIP(hipEventRecord(ev[2], s));
         if (classes)
-            TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, T.longest, (int *)(pin + 1)));
+            TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, T.longest, ticket, (int *)(pin + 1)));
         TSG_HIP(hipStreamSynchronize(s));
         nnzC = pin[0];
         if (nnzC > 0x7fffffffLL) {
@@ -3863,7 +3986,7 @@ int tsg_spgemm_enqueue(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B, 
                                  4 * (size_t)B->tilem);
     const int4 *bdesc = nullptr;
     const unsigned *bbits = nullptr;
-    if (C->tilem > 0) TSG_TRY(launch_brow_bits(s, B, w.bbits, &bdesc, &bbits, nullptr, w.longest));
+    if (C->tilem > 0) TSG_TRY(launch_brow_bits(s, B, w.bbits, &bdesc, &bbits, nullptr, nullptr, w.longest));
     TSG_TRY(launch_step1(s, A, B, C, false, P.s1w, w.bmstore, bdesc, bbits, nullptr, nullptr));
     TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_ptr, C->tile_ptr, C->tilem, w.part1));
     TSG_TRY(launch_step1(s, A, B, C, true, P.s1w, w.bmstore, bdesc, bbits, nullptr, w.segctr));
