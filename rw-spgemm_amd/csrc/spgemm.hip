@@ -515,11 +515,16 @@ __device__ __forceinline__ void for_each_pair(const TileOperands &op, int I, int
 // of several.  Tile-pair rows of more than one segment take it too (each
 // pair a loop over 16 rows, the segments a walk each): the 72 hub tile-rows
 // of R-MAT scale 16 A*A^T, 24% of its products, were 5.5 ms of step 2's 17.1;
-// all of it is 2.1 ms now.
+// all of it is 2.1 ms now.  So do those of many A tiles, whose pairs one block
+// visits: above 128 tiles (R-MAT A^2, 6 edges a vertex, scale 12 546 -> 471 us,
+// scale 13 1190 -> 880; scale 13 A*A^T, 14 edges, 2170 -> 1820).  From 65 tiles, a
+// launch more for a part of few tile-rows costs what it saves (R-MAT scale 11, 16
+// edges, 481 -> 538).
 __device__ __forceinline__ int step2_kind(int u, int span, long long ents, int tiles, int elem, int all, int rx) {
     if (!elem) return 0;
     const bool el = all || ents <= 4ll * tiles;
-    if (rx && (el || u > G2_UMAX) && (span <= G2D_WIN ? 2ll * u >= span : 5ll * u >= 3ll * span))
+    const bool many = tiles > 128 && ents <= 64ll * tiles;
+    if (rx && (el || many || u > G2_UMAX) && (span <= G2D_WIN ? 2ll * u >= span : 5ll * u >= 3ll * span))
         return span <= G2D_SMALL ? 2 : 3;
     return el ? 1 : 0;
 }
