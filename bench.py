@@ -605,7 +605,7 @@ def main():
                    "nnzCub": nnzcub, "nnzC": last["nnzC"], "tilesC": last["numtileC"],
                    "tilesC_empty": last["tiles_empty"], "values": "U[-1,1) seed 1",
                    "operand": "resident tiles + CSC tile index" + (" + element row index" if args.rowindex else "")},
-        "roofline": {"bound": "hbm", "kernel": "k_step3_rows (numeric)", "achieved": round(achieved, 1),
+        "roofline": {"bound": "hbm", "kernel": "k_step3_lines (numeric)", "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic, "algorithmic_bytes": s3_bytes, "avg_ms": round(s3_ms, 4)},
         "step_ms": {"step1": round(statistics.mean(s["t_step1_ms"] for s in steps), 4),

@@ -3699,6 +3699,7 @@ struct SpgemmTemps {
     unsigned char *hflag = nullptr;
     int *hcnt = nullptr, *hinfo = nullptr, *hwin = nullptr, *span = nullptr, *longest = nullptr;
     int *hrows = nullptr;
+    tsg_dcsr rowx[2] = {};
     hipEvent_t ev[6] = {};
     int nev = 0;
 };
@@ -3706,8 +3707,37 @@ struct SpgemmTemps {
 static void free_temps(tsg_ctx *ctx, SpgemmTemps &t) {
     void *ps[] = {t.keep, t.scr, t.wbuf, t.w3buf, t.hflag, t.hcnt, t.hinfo, t.hwin, t.hrows, t.span, t.bb, t.longest};
     for (void *p : ps) tsg_free(ctx, p);
+    for (tsg_dcsr &r : t.rowx) tsg_dcsr_free(ctx, &r);
     for (int i = 0; i < t.nev; i++) (void)hipEventDestroy(t.ev[i]);
     t = SpgemmTemps();
+}
+
+// Row indices made for one product whose operands have none: worth it when
+// most tile-rows will go by row lines.  The index costs one pass over an operand.
+// A^2 without / with it: 27-point 128^3 5.54 / 3.91 ms, 61x47x53 605 / 396 us,
+// 36x33x37 (1.1 M entries) 252 / 188, 5-point 700x310 326 / 251, banded 90000
+// (half-bandwidth 6) 283 / 182.  Below a million entries its launches and
+// read-back weigh as much; hypersparse tiles mostly have more C tiles than row
+// lines take; and rows of more than LN_BROW entries would leave dense tiles to
+// k_step3_flat (banded 20000, half-bandwidth 64, 626 / 939 us).
+#define AUTO_INDEX_NNZ (1 << 20)
+#define AUTO_INDEX_TILE 4  // entries per tile
+#define AUTO_INDEX_ROW 96  // entries per row
+static bool auto_index(const tsg_dtiles *t) {
+    return t->nnz >= AUTO_INDEX_NNZ && t->nnz >= AUTO_INDEX_TILE * (long long)t->numtile &&
+           t->nnz <= AUTO_INDEX_ROW * (long long)t->m;
+}
+static int make_index(tsg_ctx *ctx, const tsg_dtiles *t, tsg_dcsr *r, tsg_dtiles *with) {
+    *with = *t;
+    const int st = tsg_tile2csr(ctx, t, r);
+    if (st == TSG_OK) {
+        with->rowx_ptr = r->rowptr;
+        with->rowx_col = r->colidx;
+        with->rowx_val = r->val;
+    } else {
+        tsg_dcsr_free(ctx, r);
+    }
+    return st == TSG_ERR_NOMEM ? TSG_OK : st;  // no room: the tile kernels need none
 }
 
 // symbolic: steps 1 and 2 and the step-3 plan (row classes, element
@@ -3715,7 +3745,7 @@ static void free_temps(tsg_ctx *ctx, SpgemmTemps &t) {
 // neither allocated nor computed.  stats then carries C's exact tile and
 // nonzero counts and the heavy-row scratch the numeric step would add.
 static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, const tsg_tune *tune_in,
-                      tsg_dtiles *C, tsg_stats *stats, tsg_spgemm_plan *plan_out, bool symbolic,
+                      tsg_dtiles *C, tsg_stats *stats, tsg_spgemm_plan *plan_out, bool symbolic, bool may_index,
                       SpgemmTemps &T) {
     if (!A || !B || A->n != B->m) {
         tsg_set_error("tsg_spgemm: inner dimensions differ (%d vs %d)", A ? A->n : -1, B ? B->m : -1);
@@ -3729,13 +3759,6 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
     memset(&P, 0, sizeof(P));
     P.all = tune.force_tile_parallel ? 1 : 0;
     P.dense_min = tune.dense_acc_min_nnz;
-    // element path: B carries its row index, and C's columns fit the
-    // 28-bit entry keys of the element kernel's LDS hash
-    // element-wise keys: (column offset) << 4 in 32 bits, and tile columns
-    // below 2^23 - 1 for the step-2 hash slots
-    P.s3_elem = B->rowx_ptr != nullptr && tune.element_mode != 1 && B->n <= (1 << 27) - 32;
-    P.elem_all = B->rowx_ptr != nullptr && tune.element_mode == 2;
-    P.lines = A->rowx_ptr && P.s3_elem && !P.elem_all && brow_bits_bytes(B) > 0;
     hipStream_t s = ctx->stream;
 
     hipEvent_t *ev = T.ev;
@@ -3747,6 +3770,33 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         TSG_HIP(hipEventRecord(ev[4], s));
         TSG_HIP(hipEventRecord(ev[5], s));
     }
+    tsg_dtiles ax, bx;
+    if (may_index && tune.element_mode == 0 && !P.all && !(A->rowx_ptr && B->rowx_ptr) && auto_index(A) && auto_index(B)) {
+        auto borrow = [](const tsg_dtiles *t, const tsg_dtiles *from, tsg_dtiles *with) {
+            *with = *t;
+            with->rowx_ptr = from->rowx_ptr;
+            with->rowx_col = from->rowx_col;
+            with->rowx_val = from->rowx_val;
+        };
+        const bool same = A->val == B->val && A->tile_ptr == B->tile_ptr;  // one matrix: either's index is the other's
+        if (!A->rowx_ptr) {
+            if (same && B->rowx_ptr) borrow(A, B, &ax);
+            else TSG_TRY(make_index(ctx, A, &T.rowx[0], &ax));
+            A = &ax;
+        }
+        if (!B->rowx_ptr) {
+            if (same) borrow(B, A, &bx);
+            else TSG_TRY(make_index(ctx, B, &T.rowx[1], &bx));
+            B = &bx;
+        }
+    }
+    // element path: B carries its row index, and C's columns fit the
+    // 28-bit entry keys of the element kernel's LDS hash
+    // element-wise keys: (column offset) << 4 in 32 bits, and tile columns
+    // below 2^23 - 1 for the step-2 hash slots
+    P.s3_elem = B->rowx_ptr != nullptr && tune.element_mode != 1 && B->n <= (1 << 27) - 32;
+    P.elem_all = B->rowx_ptr != nullptr && tune.element_mode == 2;
+    P.lines = A->rowx_ptr && P.s3_elem && !P.elem_all && brow_bits_bytes(B) > 0;
     C->m = A->m;
     C->n = B->n;
     C->tilem = A->tilem;
@@ -3964,10 +4014,10 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
 }
 
 int tsg_spgemm_planned(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, const tsg_tune *tune_in,
-                       tsg_dtiles *C, tsg_stats *stats, tsg_spgemm_plan *plan_out, bool symbolic) {
+                       tsg_dtiles *C, tsg_stats *stats, tsg_spgemm_plan *plan_out, bool symbolic, bool may_index) {
     memset(C, 0, sizeof(*C));
     SpgemmTemps T;
-    const int st = spgemm_run(ctx, A, B, tune_in, C, stats, plan_out, symbolic, T);
+    const int st = spgemm_run(ctx, A, B, tune_in, C, stats, plan_out, symbolic, may_index, T);
     free_temps(ctx, T);
     if (st != TSG_OK) tsg_tiles_free(ctx, C);  // a partly built C goes back too
     return st;
@@ -3976,7 +4026,7 @@ int tsg_spgemm_planned(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, c
 
 extern "C" int tsg_spgemm(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, const tsg_tune *tune_in,
                           tsg_dtiles *C, tsg_stats *stats) {
-    return tsg_spgemm_planned(ctx, A, B, tune_in, C, stats, nullptr);
+    return tsg_spgemm_planned(ctx, A, B, tune_in, C, stats, nullptr, false, true);
 }
 
 size_t tsg_spgemm_work_bytes(const tsg_dtiles *C, const tsg_dtiles *B, int s1w) {

@@ -166,10 +166,13 @@ struct tsg_spgemm_plan {
 // symbolic = true runs steps 1-2 and the step-3 plan only (C's values and
 // in-tile columns stay unallocated); stats (when given) then holds C's exact
 // tile and nonzero counts and the numeric step's heavy-row scratch bytes.
+// may_index = true lets it make row indices of its own, for this product, where
+// the operands have none and it pays.
 // On any error every temporary and every array of C allocated so far is
 // freed (C is left zeroed).
 int tsg_spgemm_planned(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, const tsg_tune *tune,
-                       tsg_dtiles *C, tsg_stats *stats, tsg_spgemm_plan *plan_out, bool symbolic = false);
+                       tsg_dtiles *C, tsg_stats *stats, tsg_spgemm_plan *plan_out, bool symbolic = false,
+                       bool may_index = false);
 // tsg_spgemm_tile_rows with the symbolic option above.
 int tsg_spgemm_tile_rows_ex(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, int r0, int r1,
                             const tsg_tune *tune, tsg_dtiles *C, tsg_stats *stats, bool symbolic);
