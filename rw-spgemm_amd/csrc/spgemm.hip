@@ -282,7 +282,7 @@ k_step1(const int *__restrict__ Aptr, const int *__restrict__ Acol, int tilem,
     const bool kept = bmstore != nullptr && jmax >= jmin && jmax - jb < 32 * BMW;
     unsigned *keep = kept ? bmstore + (long long)I * BMW : nullptr;
     constexpr int V = BMW / 64;            // window words per lane: lane + 64 v
-    constexpr int U = BMW == 256 ? 2 : 1;  // kept B tile-rows whose words are loaded together
+    constexpr int U = BMW == 128 ? 8 : BMW == 256 ? 2 : 1;  // kept B tile-rows whose words are loaded together
     for (int w0 = jb; w0 <= jmax; w0 += 32 * BMW) {
         const int wi = (w0 - jb) >> WSH;
         if (wi < 64 && !((wmask >> wi) & 1ull)) continue;  // no candidate in this window
@@ -2002,14 +2002,15 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 // Per C row of an element-wise tile-row: 2 heavy (more than min_products
 // products, or more than 2048 A entries), 1 long, 0 neither; cnt[0, m) and cnt[m,
 // 2m) take the heavy and the long rows as counts for the scan that numbers
-// them, info[0] the number of heavy ones.  A tile-row with many products for
+// them, info[0] the number of heavy ones, info[2..3] the
+// long tile-rows' entries of C.  A tile-row with many products for
 // its tiles has only heavy and long rows and leaves the element-wise class.
 // One block per tile-row, 16 lanes per row, so that a long A row's B row
 // lengths are not one lane's chain of loads (R-MAT scale 16: 665 -> 92 us).
 __global__ void __launch_bounds__(256)
 k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const int *__restrict__ Browp,
-              unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, int m, long long min_products,
-              long long count_products, int take_long, unsigned char *__restrict__ flag, int *__restrict__ cnt,
+              unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int m,
+              long long min_products, long long count_products, int take_long, unsigned char *__restrict__ flag, int *__restrict__ cnt,
               int *__restrict__ info) {
     __shared__ long long s_p[16];
     const int I = blockIdx.x, r = threadIdx.x >> 4, l = threadIdx.x & 15, i = 16 * I + r;
@@ -2039,7 +2040,12 @@ k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
         if (h == 2) atomicAdd(&info[0], 1);
         if (mine && (x1 - x0 > 2048 || p > count_products)) atomicAdd(&info[1], 1);
     }
-    if (longer && threadIdx.x == 0) rowcls[I] = CLS_LONG;
+    if (longer && threadIdx.x == 0) {
+        rowcls[I] = CLS_LONG;
+        // entries that need no segments
+        atomicAdd(reinterpret_cast<unsigned long long *>(info + 2),
+                  (unsigned long long)(Cnnz[Cptr[I + 1]] - Cnnz[Cptr[I]]));
+    }
 }
 
 // rows = the heavy rows, then the long ones
@@ -3363,16 +3369,20 @@ static TileOperands make_operands(const tsg_dtiles *A, const tsg_dtiles *B) {
     return op;
 }
 
-// Step-1 bitmap window in 32-bit words per wave: 256 (8192 tile columns,
-// 8 KiB of LDS per block), 1024 (32768, 16 KiB) or 2048 (65536, 32 KiB).
-// By default B with 8193..32768 tile columns gets the 1024-word window and
-// B with 32769..65536 the 2048-word one, so a row of a product without band
-// structure needs one window, with no more LDS (and, for the kept-row
-// bitmap ORs, registers) than that takes; wider B (banded operands such as
-// stencils) keeps the narrow one.  The count pass's bitmaps are kept for
-// the fill pass up to 1 GiB.
+// Step-1 bitmap window in 32-bit words per wave: 128 (4096 tile columns, 4 KiB
+// of LDS per block with the pair lists), 256 (8192), 1024 (32768, 16 KiB) or
+// 2048 (65536, 32 KiB).  By default B gets the narrowest window that holds all
+// its tile columns up to 65536, so a row of a product without band structure needs
+// one window, with no more LDS (and, for the kept-row bitmap ORs, registers) than
+// that takes; wider B (banded operands such as stencils) keeps 256.  The words a
+// lane does not hold are rows in flight: with 128 words eight kept B tile-rows
+// are loaded together, with 256 two (hub tile-rows are one wave's chain of these
+// loads).  Count pass with 256 / 128 words: R-MAT scale 16 A*A^T 965 / 640 us, ER 65521
+// 143 / 94, ER 20011 77 / 43; twelve and sixteen rows together 627 / 634, 97 / 93,
+// 45 / 43.  The count pass's bitmaps are kept for the fill pass up to 1 GiB.
 int tsg_s1_words(const tsg_dtiles *B, const tsg_tune &t) {
     if (t.s1_window_words == 256 || t.s1_window_words == 1024 || t.s1_window_words == 2048) return t.s1_window_words;
+    if (B->tilen <= 4096) return 128;
     if (B->tilen > 8192 && B->tilen <= 32768) return 1024;
     return B->tilen > 32768 && B->tilen <= 65536 ? 2048 : 256;
 }
@@ -3420,35 +3430,28 @@ static int launch_brow_bits(hipStream_t s, const tsg_dtiles *B, void *buf, const
     return TSG_OK;
 }
 
+template <int BMW>
+static void launch_step1_w(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B, tsg_dtiles *C, bool fill,
+                           unsigned *bmstore, const int4 *bdesc, const unsigned *bbits, const int *bany, int *rowspan) {
+    const dim3 g(tsg_div_up(C->tilem, S1_WAVES)), blk(64 * S1_WAVES);
+    if (fill)
+        hipLaunchKernelGGL((k_step1<true, BMW>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
+                           B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, C->tile_colidx, C->tile_rowidx, bmstore,
+                           rowspan);
+    else
+        hipLaunchKernelGGL((k_step1<false, BMW>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
+                           B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, (int *)nullptr, (int *)nullptr, bmstore,
+                           rowspan);
+}
 static int launch_step1(hipStream_t s, const tsg_dtiles *A, const tsg_dtiles *B, tsg_dtiles *C, bool fill,
                         int words, unsigned *bmstore, const int4 *bdesc, const unsigned *bbits,
                         const int *bany, int *rowspan) {
     if (C->tilem <= 0) return TSG_OK;
-    const dim3 g(tsg_div_up(C->tilem, S1_WAVES)), blk(64 * S1_WAVES);
-    const bool wide = words == 2048;
-    if (words == 1024) {
-        if (!fill)
-            hipLaunchKernelGGL((k_step1<false, 1024>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem,
-                               B->tile_ptr, B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, (int *)nullptr,
-                               (int *)nullptr, bmstore, rowspan);
-        else
-            hipLaunchKernelGGL((k_step1<true, 1024>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem,
-                               B->tile_ptr, B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, C->tile_colidx,
-                               C->tile_rowidx, bmstore, rowspan);
-    } else if (!fill && !wide)
-        hipLaunchKernelGGL((k_step1<false, 256>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
-                           B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, (int *)nullptr, (int *)nullptr, bmstore, rowspan);
-    else if (!fill)
-        hipLaunchKernelGGL((k_step1<false, 2048>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
-                           B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, (int *)nullptr, (int *)nullptr, bmstore, rowspan);
-    else if (!wide)
-        hipLaunchKernelGGL((k_step1<true, 256>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
-                           B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, C->tile_colidx, C->tile_rowidx, bmstore,
-                           rowspan);
-    else
-        hipLaunchKernelGGL((k_step1<true, 2048>), g, blk, 0, s, A->tile_ptr, A->tile_colidx, A->tilem, B->tile_ptr,
-                           B->tile_colidx, bdesc, bbits, bany, C->tile_ptr, C->tile_colidx, C->tile_rowidx, bmstore,
-                           rowspan);
+    auto launch = words == 128    ? launch_step1_w<128>
+                  : words == 1024 ? launch_step1_w<1024>
+                  : words == 2048 ? launch_step1_w<2048>
+                                  : launch_step1_w<256>;
+    launch(s, A, B, C, fill, bmstore, bdesc, bbits, bany, rowspan);
     TSG_LAUNCH_CHECK();
     return TSG_OK;
 }
@@ -3948,14 +3951,17 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                                             ? counted
                                             : std::min(nnzC >> HEAVY_SPLIT_LOG, HEAVY_SPLIT_MAX);
                 hipLaunchKernelGGL(k_heavy_flags, dim3(C->tilem), dim3(256), 0, s, op.Arowp, op.Acolx,
-                                   (const int *)B->rowx_ptr, w.rowcls, C->tile_ptr, m, split, counted,
+                                   (const int *)B->rowx_ptr, w.rowcls, C->tile_ptr, C->tile_nnz, m, split,
+                                   counted,
                                    large || tune.heavy_min_products > 0 ? 1 : 0, T.hflag, T.hcnt, T.hinfo);
                 TSG_LAUNCH_CHECK();
                 long long nh = 0;
-                TSG_TRY(tsg_scan_i32(ctx, T.hcnt, T.hcnt, 2LL * m, &nh, T.hinfo, 2));
+                TSG_TRY(tsg_scan_i32(ctx, T.hcnt, T.hcnt, 2LL * m, &nh, T.hinfo, 4));
                 const volatile int *info = (const volatile int *)(ctx->pinned + 1);
                 const int nheavy = info[0];
                 w.ncounted = info[1];
+                const long long done = (unsigned)info[2] | (long long)info[3] << 32;
+                w.seg3_cap = C->tilem + (nnzC - done) / (G3E_NNZ - 255) + 2;  // blocks: those past the segments only end
                 if (nh > 0) {
                     TSG_TRY(tsg_alloc_t(ctx, &T.hrows, (size_t)nh));
                     hipLaunchKernelGGL(k_heavy_list, dim3(tsg_div_up(m, 256)), dim3(256), 0, s, (const int *)T.hcnt,
