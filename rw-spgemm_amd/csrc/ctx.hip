@@ -339,8 +339,15 @@ void *tsg_host_alloc(size_t bytes) {
 
 static int stage_ready(tsg_ctx *c) {
     if (c->stage) return TSG_OK;
+    // events belong to the stream's device; the caller's current device stays
+    int cur = c->device;
+    TSG_HIP(hipGetDevice(&cur));
+    if (cur != c->device) TSG_HIP(hipSetDevice(c->device));
+    hipError_t err = hipSuccess;
     for (hipEvent_t &e : c->stage_ev)
-        if (!e) TSG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        if (!e && err == hipSuccess) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+    if (cur != c->device) (void)hipSetDevice(cur);
+    TSG_HIP(err);
     TSG_HIP(hipHostMalloc((void **)&c->stage, STAGE_SLOT * 2 * TSG_STAGE_WORKERS, hipHostMallocDefault));
     return TSG_OK;
 }
@@ -362,7 +369,7 @@ int tsg_download_parts(tsg_ctx *c, const tsg_part *parts, int n) {
     std::atomic<size_t> next{0};
     std::atomic<int> failed{0};
     auto work = [&](int w) {
-        if (hipSetDevice(c->device) != hipSuccess) { failed = 1; return; }
+        if (w > 0 && hipSetDevice(c->device) != hipSuccess) { failed = 1; return; }
         char *slot[2] = {c->stage + STAGE_SLOT * (2 * w), c->stage + STAGE_SLOT * (2 * w + 1)};
         char *dst[2] = {nullptr, nullptr};
         size_t len[2] = {0, 0};
