@@ -3729,8 +3729,12 @@ static void free_temps(tsg_ctx *ctx, SpgemmTemps &t) {
 #define AUTO_INDEX_NNZ (1 << 20)
 #define AUTO_INDEX_TILE 4  // entries per tile
 #define AUTO_INDEX_ROW 96  // entries per row
+// The index is read off the tiles' entries, in-tile columns among them, which
+// steps 1 to 3 do without: an operand may come without csr_col (the drop-in
+// entry point's, and tsg_tiles_from_csc_order's of one that has none) and then
+// stays on the tile kernels.
 static bool auto_index(const tsg_dtiles *t) {
-    return t->nnz >= AUTO_INDEX_NNZ && t->nnz >= AUTO_INDEX_TILE * (long long)t->numtile &&
+    return t->csr_col && t->nnz >= AUTO_INDEX_NNZ && t->nnz >= AUTO_INDEX_TILE * (long long)t->numtile &&
            t->nnz <= AUTO_INDEX_ROW * (long long)t->m;
 }
 static int make_index(tsg_ctx *ctx, const tsg_dtiles *t, tsg_dcsr *r, tsg_dtiles *with) {
