@@ -3788,7 +3788,12 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
             with->rowx_col = from->rowx_col;
             with->rowx_val = from->rowx_val;
         };
-        const bool same = A->val == B->val && A->tile_ptr == B->tile_ptr;  // one matrix: either's index is the other's
+        // one matrix: either's index is the other's.  Every array it is read from
+        // and every size counts: A may be B's leading tile-rows (the same arrays,
+        // fewer rows), or share all but one of them
+        const bool same = A->m == B->m && A->n == B->n && A->numtile == B->numtile && A->nnz == B->nnz &&
+                          A->tile_ptr == B->tile_ptr && A->tile_colidx == B->tile_colidx && A->tile_nnz == B->tile_nnz &&
+                          A->csr_ptr == B->csr_ptr && A->csr_col == B->csr_col && A->val == B->val;
         if (!A->rowx_ptr) {
             if (same && B->rowx_ptr) borrow(A, B, &ax);
             else TSG_TRY(make_index(ctx, A, &T.rowx[0], &ax));

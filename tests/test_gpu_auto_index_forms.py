@@ -93,3 +93,63 @@ def test_drop_in_operands_without_csr(csr_a, csr_b):
     libc.free.argtypes = [C.c_void_p]
     for p in (Cm.rowpointer, Cm.columnindex, Cm.value):
         libc.free(C.cast(p, C.c_void_p))
+
+
+@pytest.mark.parametrize("index_a,index_b", [(False, False), (True, False), (False, True)])
+def test_leading_tile_rows_of_b(ctx, index_a, index_b):
+    """A = B's first tile-rows: B's arrays with smaller sizes."""
+    a = mesh()
+    d = ctx.upload(a)
+    tb = ctx.csr2tile(d)
+    ctx.build_csc(tb)
+    host = ctx.download_tiles(tb)
+    want = tile_parallel(ctx, tb, tb)
+    ta = ts.DTiles.from_buffer_copy(tb)
+    ta.tilem = 2700
+    ta.m = 16 * ta.tilem
+    ta.numtile = int(host["tile_ptr"][ta.tilem])
+    ta.nnz = int(host["tile_nnz"][ta.numtile])
+    assert ta.m < tb.m and ta.nnz >= 1 << 20
+    log(f"[auto index] {ta.tilem} of {tb.tilem} tile-rows, index {index_a} {index_b}")
+    ta.csc_ptr = ta.csc_rowidx = ta.csc_tileid = None
+    if index_a:
+        ctx.build_rowindex(ta)
+    if index_b:
+        ctx.build_rowindex(tb)
+    nt = int(want["tile_ptr"][ta.tilem])
+    nz = int(want["tile_nnz"][nt])
+    cut = {"tile_ptr": ta.tilem + 1, "tile_colidx": nt, "tile_rowidx": nt, "tile_nnz": nt + 1, "csr_ptr": 16 * nt,
+           "csr_col": nz, "mask": 16 * nt, "val": nz}
+    for _ in range(2):
+        c, _ = ctx.spgemm(ta, tb)
+        got = ctx.download_tiles(c)
+        for k in KEYS:
+            assert np.array_equal(got[k], want[k][:cut[k]]), k
+        ctx.free(c)
+    if index_a:
+        for p in (ta.rowx_ptr, ta.rowx_col, ta.rowx_val):
+            ctx.dfree(p)
+    ctx.free(tb)
+    ctx.free(d)
+
+
+def test_operands_that_share_values_only(ctx):
+    """B = A one tile column to the right: every array A's but the tile columns."""
+    a = mesh()
+    d = ctx.upload(a)
+    ta = ctx.csr2tile(d)
+    ctx.build_csc(ta)
+    host = ctx.download_tiles(ta)
+    tb = ts.DTiles.from_buffer_copy(ta)
+    tb.n, tb.tilen = ta.n + 16, ta.tilen + 1
+    tb.csc_ptr = tb.csc_rowidx = tb.csc_tileid = None
+    tb.tile_colidx = ctx.dev_ints(host["tile_colidx"] + 1)
+    ctx.build_csc(tb)
+    want = tile_parallel(ctx, ta, tb)
+    c, _ = ctx.spgemm(ta, tb)
+    same_tiles(ctx.download_tiles(c), want)
+    ctx.free(c)
+    for p in (tb.tile_colidx, tb.csc_ptr, tb.csc_rowidx, tb.csc_tileid):
+        ctx.dfree(p)
+    ctx.free(ta)
+    ctx.free(d)
