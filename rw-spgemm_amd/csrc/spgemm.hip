@@ -1989,6 +1989,7 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 #define HEAVY_SPLIT_LOG 10
 #define HEAVY_SPLIT_MAX 262144LL
 #define HEAVY_WINDOW_BYTES (512ll << 20)  // largest window table
+#define HEAVY_WINDOWS_MAX 65535  // k_heavy_windows has one per grid row (reached with few rows of B and 2^26 columns)
 // All rows of a tile-row with more products per row than this go here: below,
 // a wave per row walks tiles for few products and k_step3_flat is better.  R-MAT
 // scale 16 A*A^T 10.9 ms with 1024 or 512 and u / 2, 11.2 with 256 and u / 8; ER
@@ -3982,7 +3983,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                     // the narrowest windows whose table is small enough; one window is B's row pointers
                     int shift = HEAVY_PART_LOG;
                     long long nw = ((long long)B->n + (1 << shift) - 1) >> shift;
-                    while (nw > 1 && 4 * (nw + 1) * B->m > HEAVY_WINDOW_BYTES) {
+                    while (nw > 1 && (nw + 1 > HEAVY_WINDOWS_MAX || 4 * (nw + 1) * B->m > HEAVY_WINDOW_BYTES)) {
                         shift++;
                         nw = (nw + 1) >> 1;
                     }
