@@ -194,8 +194,8 @@ template <bool FILL>
 __global__ void __launch_bounds__(256)
 k_union_rows(int m, const int *__restrict__ ap, const int *__restrict__ ac, const int *__restrict__ tp,
              const int *__restrict__ tc, int *__restrict__ cnt_or_ptr, int *__restrict__ gc) {
-    const int i = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15, gb = threadIdx.x & 48;
-    if (i >= m) return;  // whole groups
+    const unsigned i = tsg_block() * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15, gb = threadIdx.x & 48;
+    if (i >= (unsigned)m) return;  // whole groups
     const int a0 = ap[i], a1 = ap[i + 1], b0 = tp[i], b1 = tp[i + 1];
     const int out = FILL ? cnt_or_ptr[i] : 0;
     int both = 0;  // entries of both rows so far
@@ -240,9 +240,9 @@ extern "C" int tsg_dcsr_symmetrize(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dcsr *g)
     TSG_TRY(tsg_dcsr_transpose(ctx, a, &at));
     g->m = g->n = a->m;
     TSG_TRY(tsg_alloc_t(ctx, &g->rowptr, (size_t)a->m + 1));
-    const unsigned gr = tsg_div_up(a->m, 16);
+    const dim3 gr = tsg_grid(tsg_div_up(a->m, 16), 256);
     if (a->m > 0) {
-        hipLaunchKernelGGL(k_union_rows<false>, dim3(gr), dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
+        hipLaunchKernelGGL(k_union_rows<false>, gr, dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
                            at.rowptr, at.colidx, g->rowptr, (int *)nullptr);
         TSG_LAUNCH_CHECK();
     }
@@ -252,7 +252,7 @@ extern "C" int tsg_dcsr_symmetrize(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dcsr *g)
     TSG_TRY(tsg_alloc_t(ctx, &g->colidx, (size_t)nnz + 1));
     TSG_TRY(tsg_alloc_t(ctx, &g->val, (size_t)nnz + 1));
     if (a->m > 0 && nnz > 0) {
-        hipLaunchKernelGGL(k_union_rows<true>, dim3(gr), dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
+        hipLaunchKernelGGL(k_union_rows<true>, gr, dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
                            at.rowptr, at.colidx, g->rowptr, g->colidx);
         hipLaunchKernelGGL(k_fill_f64, dim3(tsg_div_up(nnz, 256)), dim3(256), 0, ctx->stream, g->val, nnz, 1.0);
         TSG_LAUNCH_CHECK();
@@ -306,8 +306,8 @@ __device__ __forceinline__ int cc_root(const int *parent, int x) {
 template <bool FIRST>
 __global__ void __launch_bounds__(256)
 k_cc_hook(const int *__restrict__ gp, const int *__restrict__ gc, int n, const int *__restrict__ id, int *parent) {
-    const int v = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VERT_LANES), l = threadIdx.x % VERT_LANES;
-    if (v >= n) return;
+    const unsigned v = tsg_block() * (256 / VERT_LANES) + threadIdx.x / VERT_LANES, l = threadIdx.x % VERT_LANES;
+    if (v >= (unsigned)n) return;
     const int iv = id[v], e1 = gp[v + 1];
     int mn = iv;
     for (int e = gp[v] + l; e < e1; e += VERT_LANES) mn = min(mn, id[gc[e]]);
@@ -329,8 +329,8 @@ k_cc_label(const int *__restrict__ rank, int n, int *parent, int *__restrict__ l
 }
 __global__ void __launch_bounds__(256)
 k_cc_link(const int *__restrict__ gp, const int *__restrict__ gc, int n, const int *__restrict__ label, int *parent) {
-    const int v = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VERT_LANES), l = threadIdx.x % VERT_LANES;
-    if (v >= n) return;
+    const unsigned v = tsg_block() * (256 / VERT_LANES) + threadIdx.x / VERT_LANES, l = threadIdx.x % VERT_LANES;
+    if (v >= (unsigned)n) return;
     const int lv = label[v], e1 = gp[v + 1];
     for (int e = gp[v] + l; e < e1; e += VERT_LANES) {
         const int lu = label[gc[e]];
@@ -497,8 +497,8 @@ k_list_children(const int *__restrict__ gp, const int *__restrict__ gc, const in
                 const int *__restrict__ visited, const int *__restrict__ claim, const int *__restrict__ deg,
                 const int *__restrict__ off, unsigned long long *__restrict__ key, int *__restrict__ par) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int q = blockIdx.x * 4 + wave;
-    if (q >= nf) return;
+    const unsigned q = tsg_block() * 4 + wave;
+    if (q >= (unsigned)nf) return;
     const int p = front[q], e1 = gp[p + 1];
     int k = off[q];
     for (int e0 = gp[p]; e0 < e1; e0 += 64) {
@@ -507,13 +507,13 @@ k_list_children(const int *__restrict__ gp, const int *__restrict__ gc, const in
         bool mine = false;
         if (e < e1) {
             u = gc[e];
-            mine = !visited[u] && claim[u] == q;
+            mine = !visited[u] && claim[u] == (int)q;
         }
         const unsigned long long b = __ballot(mine);
         if (mine) {
             const int at = k + __popcll(b & ((1ull << lane) - 1ull));
             key[at] = ((unsigned long long)(unsigned)deg[u] << 32) | (unsigned)u;
-            par[at] = q;
+            par[at] = (int)q;
         }
         k += __popcll(b);
     }
@@ -564,14 +564,14 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     TSG_TRY(sort_ids_by_degree(ctx, deg, n, 0, order));  // ascending (degree, id)
     // connected components: label = lowest rank in the component (parents in
     // claim, which is set up for the traversal below)
-    const unsigned gv = tsg_div_up((long long)n * VERT_LANES, 256);
+    const dim3 gv = tsg_grid(tsg_div_up(n, 256 / VERT_LANES), 256);
     hipLaunchKernelGGL(k_scatter_rank, dim3(gn), dim3(256), 0, s, order, n, rank);
     for (int round = 0; round < CC_ROUNDS; round++) {
-        hipLaunchKernelGGL(round == 0 ? k_cc_hook<true> : k_cc_hook<false>, dim3(gv), dim3(256), 0, s, g.rowptr,
+        hipLaunchKernelGGL(round == 0 ? k_cc_hook<true> : k_cc_hook<false>, gv, dim3(256), 0, s, g.rowptr,
                            g.colidx, n, (const int *)(round == 0 ? rank : label), claim);
         hipLaunchKernelGGL(k_cc_label, dim3(gn), dim3(256), 0, s, (const int *)rank, n, claim, label);
     }
-    hipLaunchKernelGGL(k_cc_link, dim3(gv), dim3(256), 0, s, g.rowptr, g.colidx, n, (const int *)label, claim);
+    hipLaunchKernelGGL(k_cc_link, gv, dim3(256), 0, s, g.rowptr, g.colidx, n, (const int *)label, claim);
     hipLaunchKernelGGL(k_cc_label, dim3(gn), dim3(256), 0, s, (const int *)rank, n, claim, label);
     TSG_LAUNCH_CHECK();
     // level 0: all component seeds, in rank order
@@ -643,9 +643,9 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
         ahead = 2;
         // a parent with many children: the level's by sorting
         const int *front = seq + fstart;
-        const unsigned gl = tsg_div_up(nf, 4);
+        const dim3 gl = tsg_grid(tsg_div_up(nf, 4), 256);
         {
-            hipLaunchKernelGGL(k_list_children, dim3(gl), dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
+            hipLaunchKernelGGL(k_list_children, gl, dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
                                claim, deg, cnt, key, par);
             TSG_LAUNCH_CHECK();
             const unsigned gc2 = tsg_div_up(nc, 256);
@@ -714,8 +714,8 @@ k_perm_rows(const int *__restrict__ rowptr, const int *__restrict__ col, const d
             const int *__restrict__ row_old, const int *__restrict__ col_new, int m, const int *__restrict__ optr,
             int *__restrict__ ocol, double *__restrict__ oval) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + wave;
-    if (r >= m) return;
+    const unsigned r = tsg_block() * 4 + wave;
+    if (r >= (unsigned)m) return;
     const int e0 = rowptr[row_old[r]], o0 = optr[r], n = optr[r + 1] - o0;
     if (n == 0 || n > PERM_WAVE) return;  // wave-uniform
     int c = 0x7fffffff;
@@ -733,10 +733,11 @@ k_perm_rows(const int *__restrict__ rowptr, const int *__restrict__ col, const d
 }
 __global__ void __launch_bounds__(256)
 k_perm_rows_block(const int *__restrict__ rowptr, const int *__restrict__ col, const double *__restrict__ val,
-                  const int *__restrict__ row_old, const int *__restrict__ col_new, const int *__restrict__ optr,
+                  const int *__restrict__ row_old, const int *__restrict__ col_new, int m, const int *__restrict__ optr,
                   int *__restrict__ ocol, double *__restrict__ oval) {
     __shared__ unsigned long long s_key[PERM_BLOCK];
-    const int r = blockIdx.x, tid = threadIdx.x;
+    const unsigned r = tsg_block(), tid = threadIdx.x;
+    if (r >= (unsigned)m) return;
     const int e0 = rowptr[row_old[r]], o0 = optr[r], n = optr[r + 1] - o0;
     if (n <= PERM_WAVE) return;  // block-uniform
     int p2 = 2 * PERM_WAVE;
@@ -767,8 +768,9 @@ k_perm_rows_block(const int *__restrict__ rowptr, const int *__restrict__ col, c
 __global__ void k_perm_emit(const int *__restrict__ rowptr, const int *__restrict__ col, const int *__restrict__ row_old,
                             const int *__restrict__ col_new, int m, int n, const int *__restrict__ optr,
                             unsigned long long *__restrict__ key, int *__restrict__ src) {
-    const int r = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15;  // 16 lanes per row
-    if (r >= m) return;
+    const unsigned r = tsg_block() * 16 + (threadIdx.x >> 4);  // 16 lanes per row
+    const int l = threadIdx.x & 15;
+    if (r >= (unsigned)m) return;
     const int e0 = rowptr[row_old[r]], w0 = optr[r], len = optr[r + 1] - w0;
     for (int j = l; j < len; j += 16) {
         key[w0 + j] = (unsigned long long)r * (unsigned long long)n + (unsigned)col_new[col[e0 + j]];
@@ -812,18 +814,18 @@ extern "C" int tsg_dcsr_permute(tsg_ctx *ctx, const tsg_dcsr *a, const int *d_ro
     const int longest = ((volatile int *)(ctx->pinned + 1))[0];
     if (tot != nnz) { tsg_set_error("permute: row permutation is not a bijection"); return TSG_ERR_ARG; }
     if (nnz > 0 && longest <= PERM_BLOCK) {
-        hipLaunchKernelGGL(k_perm_rows, dim3(tsg_div_up(m, 4)), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, a->val,
+        hipLaunchKernelGGL(k_perm_rows, tsg_grid(tsg_div_up(m, 4), 256), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, a->val,
                            d_row_old, d_col_new, m, out->rowptr, out->colidx, out->val);
         if (longest > PERM_WAVE)
-            hipLaunchKernelGGL(k_perm_rows_block, dim3((unsigned)m), dim3(256), 0, ctx->stream, a->rowptr, a->colidx,
-                               a->val, d_row_old, d_col_new, out->rowptr, out->colidx, out->val);
+            hipLaunchKernelGGL(k_perm_rows_block, tsg_grid(m, 256), dim3(256), 0, ctx->stream, a->rowptr, a->colidx,
+                               a->val, d_row_old, d_col_new, m, out->rowptr, out->colidx, out->val);
         TSG_LAUNCH_CHECK();
     } else if (nnz > 0) {
         unsigned long long *key;
         int *src;
         TSG_TRY(tsg_alloc_t(ctx, &key, (size_t)nnz));
         TSG_TRY(tsg_alloc_t(ctx, &src, (size_t)nnz));
-        hipLaunchKernelGGL(k_perm_emit, dim3(tsg_div_up(m, 16)), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, d_row_old, d_col_new,
+        hipLaunchKernelGGL(k_perm_emit, tsg_grid(tsg_div_up(m, 16), 256), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, d_row_old, d_col_new,
                            m, n, out->rowptr, key, src);
         TSG_LAUNCH_CHECK();
         TSG_TRY(tsg_sort_pairs_u64(ctx, key, src, nnz, bits_of((long long)m * n)));

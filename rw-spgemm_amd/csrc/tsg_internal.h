@@ -389,6 +389,14 @@ __device__ __forceinline__ unsigned tsg_xcd_block(unsigned bid, unsigned nblocks
 }
 
 static inline unsigned tsg_div_up(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
+// Grid of `blocks` blocks of `threads`: a launch takes fewer than 2^32 threads
+// along x, so more go in rows of 2^31 along y.  Blocks are numbered by
+// tsg_block(); the last row may have some past the end.
+static inline dim3 tsg_grid(long long blocks, int threads) {
+    const long long row = (1LL << 31) / threads;
+    return blocks <= row ? dim3((unsigned)blocks) : dim3((unsigned)row, (unsigned)((blocks + row - 1) / row));
+}
+__device__ __forceinline__ unsigned tsg_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
 int tsg_validate_csr(tsg_ctx *ctx, const tsg_dcsr *a);
 // sorted = 0: row pointers and column range only (repeated or unsorted
 // columns allowed, as mmio_allinone leaves them).
