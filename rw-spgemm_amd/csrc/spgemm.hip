@@ -1789,8 +1789,9 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
     // the grid is an upper bound: the first *nseg blocks (spread evenly over
     // the XCDs) take the segments, each XCD a contiguous range
     const int ns = *nseg;
-    if ((int)blockIdx.x >= ns) return;  // block-uniform
-    const int4 sg = segs[tsg_xcd_block(blockIdx.x, (unsigned)ns)];
+    const unsigned blk = tsg_block();
+    if (blk >= (unsigned)ns) return;  // block-uniform
+    const int4 sg = segs[tsg_xcd_block(blk, (unsigned)ns)];
     const int I = sg.x, cend = Cptr[I + 1];
     const int c0 = Cptr[I] + sg.y, u = sg.z - sg.y;
     const int nbase = Cnnz[c0], n = Cnnz[c0 + u] - nbase;
@@ -2013,11 +2014,12 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 // lengths are not one lane's chain of loads (R-MAT scale 16: 665 -> 92 us).
 __global__ void __launch_bounds__(256)
 k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const int *__restrict__ Browp,
-              unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int m,
+              unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tilem, int m,
               long long min_products, long long count_products, int take_long, unsigned char *__restrict__ flag, int *__restrict__ cnt,
               int *__restrict__ info) {
     __shared__ long long s_p[16];
-    const int I = blockIdx.x, r = threadIdx.x >> 4, l = threadIdx.x & 15, i = 16 * I + r;
+    const int I = (int)tsg_block(), r = threadIdx.x >> 4, l = threadIdx.x & 15, i = 16 * I + r;
+    if (I >= tilem) return;  // block-uniform
     const bool mine = rowcls[I] == 0;  // block-uniform
     long long p = 0;
     int x0 = 0, x1 = 0;
@@ -2881,8 +2883,9 @@ k_step3_lines(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
     unsigned *s_meta = reinterpret_cast<unsigned *>(s_lds + off[1]);
     int *s_col = reinterpret_cast<int *>(s_lds + off[2]);
     unsigned char *s_map = s_lds + off[3];
-    const int I = (int)tsg_xcd_block(blockIdx.x, gridDim.x);
-    if (I >= tilem) return;
+    const unsigned blk = tsg_block();
+    if (blk >= (unsigned)tilem) return;
+    const int I = (int)tsg_xcd_block(blk, (unsigned)tilem);
     const int cls = rowcls[I];
     if (cls < LN_CLASS) return;  // block-uniform
     const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x;
@@ -3631,7 +3634,7 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
         L.nnz = P.ln[0]; L.umax = P.ln[1]; L.map = P.ln[2];
         int base;
         size_t off[4];
-        hipLaunchKernelGGL(k_step3_lines, dim3(C->tilem), dim3(P.ln[3]), lines_layout(L, &base, off), s, op.Arowp, op.Acolx,
+        hipLaunchKernelGGL(k_step3_lines, tsg_grid(C->tilem, P.ln[3]), dim3(P.ln[3]), lines_layout(L, &base, off), s, op.Arowp, op.Acolx,
                            op.Avalx, (const int *)B->rowx_ptr, (const int *)B->rowx_col, (const double *)B->rowx_val,
                            C->m, C->tilem, C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr, C->tile_nnz,
                            (const unsigned char *)w.rowcls, C->csr_col, C->val, L);
@@ -3653,7 +3656,7 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
         const bool rx = op.Arowp != nullptr;
         TSG_TRY(launch_segments(s, C, w, 0, rx ? G3F_NNZ : G3E_NNZ, w.rowcls));
         if (rx)
-            hipLaunchKernelGGL(P.s3span < G3F_SPAN ? k_step3_flat<false> : k_step3_flat<true>, dim3((unsigned)w.seg3_cap), dim3(G3F_THREADS), 0, s, op.Arowp, op.Acolx,
+            hipLaunchKernelGGL(P.s3span < G3F_SPAN ? k_step3_flat<false> : k_step3_flat<true>, tsg_grid(w.seg3_cap, G3F_THREADS), dim3(G3F_THREADS), 0, s, op.Arowp, op.Acolx,
                                op.Avalx, (const int *)B->rowx_ptr, (const int *)B->rowx_col,
                                (const double *)B->rowx_val, C->m, (const int4 *)w.seg3,
                                (const int *)(w.segcnt + C->tilem), C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
@@ -3963,8 +3966,8 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                 const long long split = tune.heavy_min_products > 0 || !large
                                             ? counted
                                             : std::min(nnzC >> HEAVY_SPLIT_LOG, HEAVY_SPLIT_MAX);
-                hipLaunchKernelGGL(k_heavy_flags, dim3(C->tilem), dim3(256), 0, s, op.Arowp, op.Acolx,
-                                   (const int *)B->rowx_ptr, w.rowcls, C->tile_ptr, C->tile_nnz, m, split,
+                hipLaunchKernelGGL(k_heavy_flags, tsg_grid(C->tilem, 256), dim3(256), 0, s, op.Arowp, op.Acolx,
+                                   (const int *)B->rowx_ptr, w.rowcls, C->tile_ptr, C->tile_nnz, C->tilem, m, split,
                                    counted,
                                    large || tune.heavy_min_products > 0 ? 1 : 0, T.hflag, T.hcnt, T.hinfo);
                 TSG_LAUNCH_CHECK();

@@ -83,3 +83,51 @@ def test_rcm_and_permute(ctx):
     ref = oracle.permute_csr(small, want.astype(np.int32), inv)
     assert np.array_equal(got.rowptr[:k + 1], ref[0]) and np.all(got.rowptr[k:] == a.nnz)
     assert np.array_equal(got.colidx, ref[1]) and np.array_equal(got.val, ref[2])
+
+
+@pytest.mark.parametrize("mode,heavy", [(0, 0), (0, 2000), (2, 0)])
+def test_product(ctx, mode, heavy):
+    """2^23 tile-rows and more, of which some dozens have entries: some for row lines, some element-wise, some
+    with heavy rows.  C is the C of those tile-rows alone."""
+    rng = np.random.default_rng(11)
+    n, tilem = 4000, (1 << 23) + 5
+    m = 16 * tilem - 3
+    b = ts.gen_er(n, 20.0, seed=4)
+    at = np.unique(np.r_[0, 1, tilem // 2, tilem - 1, rng.integers(0, tilem, 40)])  # tile-rows with entries
+    counts = rng.integers(0, 4, 16 * len(at)).astype(np.int32)
+    counts[16 * 3:16 * 6] = 40  # their C rows are long
+    counts[16 * 9 + 2] = 600
+    counts[-3:] = 0  # past the last row
+    cols = np.concatenate([np.sort(rng.choice(n, c, replace=False)) for c in counts])
+    val = rng.uniform(-1, 1, len(cols))
+    rows = (16 * at[:, None] + np.arange(16)[None, :]).ravel()
+    tall = ts.Csr(m, n, rowptr_of(m, rows[:-3], counts[:-3]), cols, val)
+    small = ts.Csr(16 * len(at), n, np.r_[0, np.cumsum(counts)], cols, val)
+    log(f"[tall] product, {tilem} tile-rows, mode {mode}, heavy from {heavy}")
+    db = ctx.upload(b)
+    tb = ctx.csr2tile(db)
+    ctx.build_csc(tb)
+    ctx.build_rowindex(tb)
+    tune = ts.default_tune()
+    tune.element_mode = mode
+    tune.heavy_min_products = heavy
+    out = []
+    for a in (small, tall):
+        da = ctx.upload(a)
+        ta = ctx.csr2tile(da)
+        ctx.build_rowindex(ta)
+        c, st = ctx.spgemm(ta, tb, tune)
+        out.append((ctx.download_tiles(c), st.heavy_rows))
+        for x in (c, ta, da):
+            ctx.free(x)
+    ctx.free(tb)
+    ctx.free(db)
+    ctx.trim()
+    (want, hw), (got, hg) = out
+    assert hw == hg and (heavy == 0 or hg > 0)
+    ptr = np.zeros(tilem + 1, np.int32)
+    ptr[at + 1] = np.diff(want["tile_ptr"])
+    assert np.array_equal(got["tile_ptr"], np.cumsum(ptr))
+    assert np.array_equal(got["tile_rowidx"], at[want["tile_rowidx"]])
+    for k in ("tile_colidx", "tile_nnz", "csr_ptr", "csr_col", "mask", "val"):
+        assert np.array_equal(got[k], want[k]), k
