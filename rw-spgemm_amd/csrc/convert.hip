@@ -887,13 +887,8 @@ extern "C" int tsg_tile2csr(tsg_ctx *ctx, const tsg_dtiles *t, tsg_dcsr *out) {
     return tsg_tile2csr_view(ctx, t, 0, out);
 }
 
-// t may be a view of a tile-row range of a larger tile matrix (tile_ptr
-// pointing into the parent's, every other array the parent's, indices
-// absolute); output columns are taken relative to tile column jbase.
-int tsg_tile2csr_view(tsg_ctx *ctx, const tsg_dtiles *t, int jbase, tsg_dcsr *out) {
-    memset(out, 0, sizeof(*out));
-    out->m = t->m;
-    out->n = t->n;
+// buf: the further runs' count, then the runs (the caller frees it)
+static int tile2csr_run(tsg_ctx *ctx, const tsg_dtiles *t, int jbase, tsg_dcsr *out, char **buf) {
     TSG_TRY(tsg_alloc_t(ctx, &out->rowptr, (size_t)t->m + 1));
     if (t->m <= 0) {
         TSG_HIP(hipMemsetAsync(out->rowptr, 0, 4, ctx->stream));
@@ -903,14 +898,13 @@ int tsg_tile2csr_view(tsg_ctx *ctx, const tsg_dtiles *t, int jbase, tsg_dcsr *ou
     }
     const int tilem = (int)tsg_div_up(t->m, 16);
     const unsigned nb = tsg_div_up(tilem, CV_WAVES);
-    char *buf = nullptr;  // the item count, then the items
     long long maxitems = 0, nnz = 0;
     for (long long tiles = std::max(t->numtile, 0);;) {
         maxitems = tiles / CV_SEG + 1;  // further runs: at most one per CV_SEG tiles
-        TSG_TRY(tsg_alloc(ctx, (void **)&buf, 64 + (size_t)maxitems * sizeof(T2cItem)));
-        TSG_HIP(hipMemsetAsync(buf, 0, 4, ctx->stream));
+        TSG_TRY(tsg_alloc(ctx, (void **)buf, 64 + (size_t)maxitems * sizeof(T2cItem)));
+        TSG_HIP(hipMemsetAsync(*buf, 0, 4, ctx->stream));
         hipLaunchKernelGGL(k_t2c_rowptr, dim3(nb), dim3(64 * CV_WAVES), 0, ctx->stream, t->m, tilem, t->tile_ptr,
-                           t->tile_nnz, t->csr_ptr, out->rowptr, (T2cItem *)(buf + 64), (int *)buf, (int)maxitems,
+                           t->tile_nnz, t->csr_ptr, out->rowptr, (T2cItem *)(*buf + 64), (int *)*buf, (int)maxitems,
                            ctx->pinned);
         TSG_LAUNCH_CHECK();
         TSG_HIP(hipStreamSynchronize(ctx->stream));
@@ -918,10 +912,11 @@ int tsg_tile2csr_view(tsg_ctx *ctx, const tsg_dtiles *t, int jbase, tsg_dcsr *ou
         const long long have = ((volatile long long *)ctx->pinned)[1];
         if (have <= tiles) break;
         tiles = have;  // a view whose numtile is not its own: once more, with room for every run
-        tsg_free(ctx, buf);
+        tsg_free(ctx, *buf);
+        *buf = nullptr;
     }
-    const T2cItem *items = (const T2cItem *)(buf + 64);
-    const int *nitems = (const int *)buf;
+    const T2cItem *items = (const T2cItem *)(*buf + 64);
+    const int *nitems = (const int *)*buf;
     out->nnz = (int)nnz;
     TSG_TRY(tsg_alloc_t(ctx, &out->colidx, (size_t)nnz + 1));
     TSG_TRY(tsg_alloc_t(ctx, &out->val, (size_t)nnz + 1));
@@ -932,8 +927,21 @@ int tsg_tile2csr_view(tsg_ctx *ctx, const tsg_dtiles *t, int jbase, tsg_dcsr *ou
                            (int)nb, jbase, out->colidx, out->val);
         TSG_LAUNCH_CHECK();
     }
-    tsg_free(ctx, buf);
     return TSG_OK;
+}
+
+// t may be a view of a tile-row range of a larger tile matrix (tile_ptr
+// pointing into the parent's, every other array the parent's, indices
+// absolute); output columns are taken relative to tile column jbase.
+int tsg_tile2csr_view(tsg_ctx *ctx, const tsg_dtiles *t, int jbase, tsg_dcsr *out) {
+    memset(out, 0, sizeof(*out));
+    out->m = t->m;
+    out->n = t->n;
+    char *buf = nullptr;
+    const int st = tile2csr_run(ctx, t, jbase, out, &buf);
+    tsg_free(ctx, buf);
+    if (st != TSG_OK) tsg_dcsr_free(ctx, out);  // what it got before the error
+    return st;
 }
 
 // ------------------------------------------------------------------ checksums, sampled rows

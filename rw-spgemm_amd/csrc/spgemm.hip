@@ -3748,8 +3748,6 @@ static int make_index(tsg_ctx *ctx, const tsg_dtiles *t, tsg_dcsr *r, tsg_dtiles
         with->rowx_ptr = r->rowptr;
         with->rowx_col = r->colidx;
         with->rowx_val = r->val;
-    } else {
-        tsg_dcsr_free(ctx, r);
     }
     return st == TSG_ERR_NOMEM ? TSG_OK : st;  // no room: the tile kernels need none
 }
