@@ -4037,9 +4037,15 @@ int tsg_spgemm_planned(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, c
                        tsg_dtiles *C, tsg_stats *stats, tsg_spgemm_plan *plan_out, bool symbolic, bool may_index) {
     memset(C, 0, sizeof(*C));
     SpgemmTemps T;
-    const int st = spgemm_run(ctx, A, B, tune_in, C, stats, plan_out, symbolic, may_index, T);
+    int st = spgemm_run(ctx, A, B, tune_in, C, stats, plan_out, symbolic, may_index, T);
+    const bool indexed = T.rowx[0].rowptr || T.rowx[1].rowptr;
     free_temps(ctx, T);
     if (st != TSG_OK) tsg_tiles_free(ctx, C);  // a partly built C goes back too
+    if (st == TSG_ERR_NOMEM && indexed) {  // the indices made for this product may be what it lacked
+        st = spgemm_run(ctx, A, B, tune_in, C, stats, plan_out, symbolic, false, T);
+        free_temps(ctx, T);
+        if (st != TSG_OK) tsg_tiles_free(ctx, C);
+    }
     return st;
 }
 

@@ -35,3 +35,51 @@ for room in [0, 1 << 10] + [x << 20 for x in (1, 2, 4, 6, 8, 10, 12, 14, 16, 20,
 log("failed", failed)
 assert failed > 4 and t.rowx_ptr
 """)
+
+
+@pytest.mark.parametrize("apart", [False, True])
+def test_products_index_themselves_only_if_there_is_room(tmp_path, apart):
+    """Wherever the product fits without indices of its own it is computed; what does not fit leaves nothing."""
+    run_limited(tmp_path, f"apart = {apart}" + """
+ctx = ts.Context(0)
+a = ts.gen_stencil27(36, 33, 37, valmode=ts.VAL_UNIFORM_PM1, seed=3)
+d = ctx.upload(a)
+ta = ctx.csr2tile(d)
+tb = ctx.csr2tile(d) if apart else ta
+ctx.build_csc(tb)
+plain = ts.default_tune()
+plain.element_mode = 1  # no element kernels, so no indices
+
+def product(tune):
+    c, _ = ctx.spgemm(ta, tb, tune)
+    out = ctx.download_tiles(c)
+    ctx.free(c)
+    return out
+
+peak = []
+for tune in (plain, None):
+    for _ in range(2):  # the second time the context's scratch is there
+        ctx.trim()
+        limit.limit_peak(1)
+        want = product(tune)
+    peak.append(limit.limit_peak(0))
+ctx.trim()
+base, before = limit.limit_live(), ctx.bytes_in_use()
+log("base", base, "peak without / with indices", peak)
+assert peak[1] > peak[0] + 8 * a.nnz
+done, refused = [], 0
+for room in sorted(set(np.linspace(base, peak[1] + (1 << 20), 24).astype(int)) | {peak[0]}):
+    limit.limit_set(int(room))
+    ctx.trim()
+    try:
+        got = product(None)
+        for k in ("tile_ptr", "tile_colidx", "tile_nnz", "csr_ptr", "csr_col", "mask", "val"):
+            assert np.array_equal(got[k], want[k]), (room, k)
+        done.append(room)
+    except ts.TsgError as e:
+        assert e.status == -4, e
+        refused += 1
+    assert ctx.bytes_in_use() == before, room
+log("done from", min(done), "refused", refused)
+assert min(done) <= peak[0] and refused > 0
+""")
