@@ -749,7 +749,7 @@ k_row_stats_one(int *ptr, const int *__restrict__ span, const int *__restrict__ 
 
 static_assert(G2_PCHUNK == G2_THREADS, "one A tile of a chunk per thread");
 __global__ void __launch_bounds__(G2_THREADS)
-k_step2_rows(TileOperands op, const int4 *__restrict__ segs, const int *__restrict__ Cptr, const int *__restrict__ Ccol, unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16,
+k_step2_rows(TileOperands op, const int4 *__restrict__ segs, int nseg, const int *__restrict__ Cptr, const int *__restrict__ Ccol, unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16,
              int *__restrict__ Cnnz, int umax, int mapbytes) {
     // dynamic LDS, sized by the largest segment: the segment's C tile masks
     // (two 16-bit rows per word, even row high; G2_MSTRIDE words per tile so
@@ -776,7 +776,9 @@ k_step2_rows(TileOperands op, const int4 *__restrict__ segs, const int *__restri
     const int tid = threadIdx.x;
     // one block per segment, each XCD a contiguous range; without a list
     // (segs NULL) every tile-row is one segment
-    const int w = (int)tsg_xcd_block(blockIdx.x, gridDim.x);
+    const unsigned blk = tsg_block();
+    if (blk >= (unsigned)nseg) return;  // block-uniform
+    const int w = (int)tsg_xcd_block(blk, (unsigned)nseg);
     int4 sg = make_int4(w, 0, 0, 0);
     if (segs) {
         sg = segs[w];
@@ -967,7 +969,7 @@ __device__ __forceinline__ unsigned col_hash10(int J) { return ((unsigned)J * 26
 
 __global__ void __launch_bounds__(G2_THREADS)
 k_step2_elem(TileOperands op, const int *__restrict__ Browp, const int *__restrict__ Bcolx,
-             const int4 *__restrict__ segs, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
+             const int4 *__restrict__ segs, int nseg, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
              unsigned short *__restrict__ Cmask, unsigned char *__restrict__ Cptr16, int *__restrict__ Cnnz) {
     __shared__ unsigned s_m[G2_UMAX * 8];  // two 16-bit rows per word, even row high
     // hash of the segment's tile columns: slot (J - jlo + 1) << 9 | C tile
@@ -975,7 +977,9 @@ k_step2_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
     // kernel runs, index < G2_UMAX = 512); 0 = empty
     __shared__ unsigned s_hkey[G2E_HASH];
     const int tid = threadIdx.x;
-    const int4 sg = segs[tsg_xcd_block(blockIdx.x, gridDim.x)];
+    const unsigned blk = tsg_block();
+    if (blk >= (unsigned)nseg) return;  // block-uniform
+    const int4 sg = segs[tsg_xcd_block(blk, (unsigned)nseg)];
     const int I = sg.x;
     const int c0 = Cptr[I] + sg.y, u = sg.z - sg.y;
     for (int i = tid; i < u * 8; i += G2_THREADS) s_m[i] = 0u;
@@ -1523,8 +1527,9 @@ k_step3_elem(TileOperands op, const int *__restrict__ Browp, const int *__restri
     // the grid is an upper bound: the first *nseg blocks (spread evenly over
     // the XCDs) take the segments, each XCD a contiguous range
     const int ns = *nseg;
-    if ((int)blockIdx.x >= ns) return;  // block-uniform
-    const int w = (int)tsg_xcd_block(blockIdx.x, (unsigned)ns);
+    const unsigned blk = tsg_block();
+    if (blk >= (unsigned)ns) return;  // block-uniform
+    const int w = (int)tsg_xcd_block(blk, (unsigned)ns);
     const int4 sg = segs[w];
     const int I = sg.x;
     const int c0 = Cptr[I] + sg.y, u = sg.z - sg.y;
@@ -2547,8 +2552,10 @@ k_step3_rows(TileOperands op, const int *__restrict__ Cptr, const int *__restric
     static_assert(G3_UMAX <= G3_THREADS, "one C tile per thread in the setup");
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
-    const int I = (int)tsg_xcd_block(blockIdx.x, gridDim.x);
-    if (I >= tilem || rowcls[I] != 1) return;  // block-uniform
+    const unsigned blk = tsg_block();
+    if (blk >= (unsigned)tilem) return;
+    const int I = (int)tsg_xcd_block(blk, (unsigned)tilem);
+    if (rowcls[I] != 1) return;  // block-uniform
     const int c0 = Cptr[I], u = Cptr[I + 1] - c0;
     const int nbase = Cnnz[c0], nrow = Cnnz[c0 + u] - nbase;
     const int a0 = op.Aptr[I], la = op.Aptr[I + 1] - a0;
@@ -3580,14 +3587,15 @@ static int launch_step2(hipStream_t s, const TileOperands &op, const tsg_dtiles 
     if (n2[0] > 0) {
         const int s2u = P.s2u > 0 ? P.s2u : G2_UMAX;
         const size_t lds2 = (4 * G2_MSTRIDE + 4) * (size_t)s2u + (((size_t)P.s2map + 15) & ~(size_t)15);
-        hipLaunchKernelGGL(k_step2_rows, dim3((unsigned)(list ? n2[0] : C->tilem)), dim3(G2_THREADS), lds2, s, op,
-                           list ? (const int4 *)w.seg2 : (const int4 *)nullptr, C->tile_ptr, C->tile_colidx, C->mask,
+        const int nseg = list ? n2[0] : C->tilem;
+        hipLaunchKernelGGL(k_step2_rows, tsg_grid(nseg, G2_THREADS), dim3(G2_THREADS), lds2, s, op,
+                           list ? (const int4 *)w.seg2 : (const int4 *)nullptr, nseg, C->tile_ptr, C->tile_colidx, C->mask,
                            C->csr_ptr, C->tile_nnz, s2u, P.s2map);
         TSG_LAUNCH_CHECK();
     }
     if (n2[1] > 0) {
-        hipLaunchKernelGGL(k_step2_elem, dim3((unsigned)n2[1]), dim3(G2_THREADS), 0, s, op, (const int *)B->rowx_ptr,
-                           (const int *)B->rowx_col, (const int4 *)(w.seg2 + base.y), C->tile_ptr, C->tile_colidx,
+        hipLaunchKernelGGL(k_step2_elem, tsg_grid(n2[1], G2_THREADS), dim3(G2_THREADS), 0, s, op, (const int *)B->rowx_ptr,
+                           (const int *)B->rowx_col, (const int4 *)(w.seg2 + base.y), n2[1], C->tile_ptr, C->tile_colidx,
                            C->mask, C->csr_ptr, C->tile_nnz);
         TSG_LAUNCH_CHECK();
     }
@@ -3597,7 +3605,7 @@ static int launch_step2(hipStream_t s, const TileOperands &op, const tsg_dtiles 
         const int threads = k == 2 ? 256 : 1024;
         const size_t lds = g2d_lds(width, threads);
         // kind 3: a few blocks per CU take the windows in turn (one at a time fits)
-        const unsigned grid = k == 2 ? (unsigned)n2[k] : (unsigned)std::min(n2[k], 4096);
+        const unsigned grid = (unsigned)std::min(n2[k], k == 2 ? 1 << 23 : 4096);
         hipLaunchKernelGGL(k_step2_dense, dim3(grid), dim3(threads), lds, s, op.Arowp, op.Acolx, C->m,
                            (const int *)B->rowx_ptr, (const int *)B->rowx_col,
                            (const int4 *)(w.seg2 + (k == 2 ? base.z : base.w)), n2[k], C->tile_ptr, C->tile_colidx,
@@ -3646,7 +3654,7 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
         L.qb = P.g3[3]; L.bnnz = P.g3[4]; L.amax = P.g3[5];
         size_t off[G3_NARR];
         const size_t lds = g3_layout(L, off);
-        hipLaunchKernelGGL(k_step3_rows, dim3(C->tilem), dim3(G3_THREADS), lds, s, op, C->tile_ptr, C->tile_colidx,
+        hipLaunchKernelGGL(k_step3_rows, tsg_grid(C->tilem, G3_THREADS), dim3(G3_THREADS), lds, s, op, C->tile_ptr, C->tile_colidx,
                            C->tilem, C->mask, C->csr_ptr, C->tile_nnz, (const unsigned char *)w.rowcls, C->csr_col,
                            C->val, L);
         TSG_LAUNCH_CHECK();
@@ -3663,7 +3671,7 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
                                C->tile_nnz, C->csr_col, C->val, (const unsigned char *)w.hflag);
         else
             hipLaunchKernelGGL(P.s3span < G3E_PK_SPAN ? k_step3_elem<true> : k_step3_elem<false>,
-                               dim3((unsigned)w.seg3_cap), dim3(256), 0, s, op, (const int *)B->rowx_ptr,
+                               tsg_grid(w.seg3_cap, 256), dim3(256), 0, s, op, (const int *)B->rowx_ptr,
                                (const int *)B->rowx_col, (const double *)B->rowx_val, C->m, (const int4 *)w.seg3,
                                (const int *)(w.segcnt + C->tilem), C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
                                C->tile_nnz, C->csr_col, C->val);

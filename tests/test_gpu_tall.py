@@ -85,12 +85,13 @@ def test_rcm_and_permute(ctx):
     assert np.array_equal(got.colidx, ref[1]) and np.array_equal(got.val, ref[2])
 
 
-@pytest.mark.parametrize("mode,heavy", [(0, 0), (0, 2000), (2, 0)])
-def test_product(ctx, mode, heavy):
-    """2^23 tile-rows and more, of which some dozens have entries: some for row lines, some element-wise, some
-    with heavy rows.  C is the C of those tile-rows alone."""
+@pytest.mark.parametrize("log_rows", [23, 24])
+@pytest.mark.parametrize("mode,heavy", [(0, 0), (0, 2000), (2, 0), (None, 0)])
+def test_product(ctx, log_rows, mode, heavy):
+    """2^23 and 2^24 tile-rows, of which some dozens have entries: some for row lines, some element-wise, some
+    with heavy rows; mode None without A's row index.  C is the C of those tile-rows alone."""
     rng = np.random.default_rng(11)
-    n, tilem = 4000, (1 << 23) + 5
+    n, tilem = 4000, (1 << log_rows) + 5
     m = 16 * tilem - 3
     b = ts.gen_er(n, 20.0, seed=4)
     at = np.unique(np.r_[0, 1, tilem // 2, tilem - 1, rng.integers(0, tilem, 40)])  # tile-rows with entries
@@ -109,13 +110,14 @@ def test_product(ctx, mode, heavy):
     ctx.build_csc(tb)
     ctx.build_rowindex(tb)
     tune = ts.default_tune()
-    tune.element_mode = mode
+    tune.element_mode = mode or 0
     tune.heavy_min_products = heavy
     out = []
-    for a in (small, tall):
+    for a in (tall, small):  # in this order: C of the first is not left where the second's goes
         da = ctx.upload(a)
         ta = ctx.csr2tile(da)
-        ctx.build_rowindex(ta)
+        if mode is not None:
+            ctx.build_rowindex(ta)
         c, st = ctx.spgemm(ta, tb, tune)
         out.append((ctx.download_tiles(c), st.heavy_rows))
         for x in (c, ta, da):
@@ -123,7 +125,7 @@ def test_product(ctx, mode, heavy):
     ctx.free(tb)
     ctx.free(db)
     ctx.trim()
-    (want, hw), (got, hg) = out
+    (got, hg), (want, hw) = out
     assert hw == hg and (heavy == 0 or hg > 0)
     ptr = np.zeros(tilem + 1, np.int32)
     ptr[at + 1] = np.diff(want["tile_ptr"])
