@@ -358,14 +358,18 @@ int tsg_download_parts(tsg_ctx *c, const tsg_part *parts, int n) {
         total += parts[i].bytes;
         pieces += (parts[i].bytes + STAGE_SLOT - 1) / STAGE_SLOT;
     }
-    if (total < STAGE_MIN) {
+    bool staged = total >= STAGE_MIN;
+    if (staged && stage_ready(c) != TSG_OK) {  // no pinned memory to be had: the runtime's copy needs none of ours
+        (void)hipGetLastError();
+        staged = false;
+    }
+    if (!staged) {
         for (int i = 0; i < n; i++)
             if (parts[i].bytes)
                 TSG_HIP(hipMemcpyAsync(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDeviceToHost, c->stream));
         TSG_HIP(hipStreamSynchronize(c->stream));
         return TSG_OK;
     }
-    TSG_TRY(stage_ready(c));
     std::atomic<size_t> next{0};
     std::atomic<int> failed{0};
     auto work = [&](int w) {

@@ -83,3 +83,17 @@ for room in sorted(set(np.linspace(base, peak[1] + (1 << 20), 24).astype(int)) |
 log("done from", min(done), "refused", refused)
 assert min(done) <= peak[0] and refused > 0
 """)
+
+
+def test_large_results_without_pinned_memory(tmp_path):
+    run_limited(tmp_path, """
+ctx = ts.Context(0)
+n = 3000001
+a = ts.Csr(1, n, np.array([0, n], np.int32), np.arange(n, dtype=np.int32), np.arange(n) * 0.5)
+d = ctx.upload(a)
+for off in (1, 0, 1):
+    limit.limit_no_pinned(off)
+    h = ctx.download(d)
+    assert np.array_equal(h.rowptr, a.rowptr) and np.array_equal(h.colidx, a.colidx) and np.array_equal(h.val, a.val)
+    ctx.trim()
+""")
