@@ -3996,6 +3996,13 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                         shift++;
                         nw = (nw + 1) >> 1;
                     }
+                    while (nw > 1 && !symbolic) {  // wider ones where that much is not to be had
+                        const int st = tsg_alloc(ctx, (void **)&T.hwin, (size_t)(4 * (nw + 1) * B->m));
+                        if (st == TSG_OK) break;
+                        if (st != TSG_ERR_NOMEM) return st;
+                        shift++;
+                        nw = (nw + 1) >> 1;
+                    }
                     w.hflag = T.hflag;
                     w.hrows = T.hrows;
                     w.nheavy = nheavy;
@@ -4006,7 +4013,6 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                     w.hwin_bytes = nw > 1 ? 4 * (nw + 1) * B->m : 0;
                     w.hwin = B->rowx_ptr;
                     if (nw > 1 && !symbolic) {
-                        TSG_TRY(tsg_alloc(ctx, (void **)&T.hwin, (size_t)w.hwin_bytes));
                         hipLaunchKernelGGL(k_heavy_windows, dim3(tsg_div_up(B->m, 256), (unsigned)nw + 1), dim3(256), 0, s,
                                            (const int *)B->rowx_ptr, (const int *)B->rowx_col, B->m, (int)nw, shift,
                                            T.hwin);

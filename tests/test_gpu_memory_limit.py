@@ -97,3 +97,48 @@ for off in (1, 0, 1):
     assert np.array_equal(h.rowptr, a.rowptr) and np.array_equal(h.colidx, a.colidx) and np.array_equal(h.val, a.val)
     ctx.trim()
 """)
+
+
+def test_heavy_rows_with_less_room_than_their_windows(tmp_path):
+    """The window table of heavy rows (68 MB here) shrinks to what memory there is."""
+    run_limited(tmp_path, """
+ctx = ts.Context(0)
+rng = np.random.default_rng(1)
+rows, n = 260, (1 << 26) - 2048  # 65534 windows, one fewer than the most
+def csr(m, n, cols):
+    ptr = np.r_[0, np.cumsum([len(c) for c in cols])]
+    return ts.Csr(m, n, ptr, np.concatenate(cols), rng.uniform(-1, 1, int(ptr[-1])))
+b = csr(rows, n, [np.unique(np.r_[0, n - 1, rng.integers(0, n, 40), rng.integers(0, 3000, 60)]) for _ in range(rows)])
+a = csr(5, rows, [np.sort(rng.choice(rows, k, replace=False)) for k in (200, 250, 1, 150, 3)])
+da, db = ctx.upload(a), ctx.upload(b)
+ta, tb = ctx.csr2tile(da), ctx.csr2tile(db)
+ctx.build_csc(tb)
+ctx.build_rowindex(ta)
+ctx.build_rowindex(tb)
+tune = ts.default_tune()
+tune.heavy_min_products = 5000
+def product():
+    c, st = ctx.spgemm(ta, tb, tune)
+    assert st.heavy_rows == 3
+    out = ctx.download_tiles(c)
+    ctx.free(c)
+    return out, st.heavy_bytes
+want, table = product()
+ctx.trim()
+limit.limit_peak(1)
+product()
+peak = limit.limit_peak(0)
+log("peak", peak, "heavy rows' bytes", table)
+assert table > 60 << 20
+before, least = ctx.bytes_in_use(), table
+for less in range(0, int(table * 0.95), 8 << 20):
+    ctx.trim()
+    limit.limit_set(int(peak - less))
+    got, used = product()
+    for k in ("tile_ptr", "tile_colidx", "tile_nnz", "csr_ptr", "csr_col", "mask", "val"):
+        assert np.array_equal(got[k], want[k]), (less, k)
+    assert ctx.bytes_in_use() == before
+    least = min(least, used)
+log("least", least)
+assert least < table / 7  # halved three times, plus the rows' lists
+""")
