@@ -1961,7 +1961,7 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 }
 
 // ------------------------------------------------------------------ step 3, heavy and long rows
-// Rows with many products for the tiles of their tile-row (hub rows of
+// Rows with many products for the columns of their tile-row (hub rows of
 // power-law graphs, and rows that have a few hubs as sources).  In segments
 // of a tile-row each would walk all its A entries again in every segment
 // and put every entry of C into a hash first (R-MAT scale 16: 68 segments a
@@ -1996,12 +1996,19 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 #define HEAVY_SPLIT_MAX 262144LL
 #define HEAVY_WINDOW_BYTES (512ll << 20)  // largest window table
 #define HEAVY_WINDOWS_MAX 65535  // k_heavy_windows has one per grid row (reached with few rows of B and 2^26 columns)
-// All rows of a tile-row with more products per row than this go here: below,
-// a wave per row walks tiles for few products and k_step3_flat is better.  R-MAT
-// scale 16 A*A^T 10.9 ms with 1024 or 512 and u / 2, 11.2 with 256 and u / 8; ER
-// 30000 (26 per row, 676 products) A^2 0.77 and 1.01 ms, ER 2500 232, 216 and 216 us.
+// All rows of a tile-row with more products per row than LONG_MIN_PRODUCTS, and
+// than LONG_PER_GROUP for every group of parts that its columns span, go here:
+// below, a wave per row and group walks the row's sources and tiles for few
+// products and k_step3_flat is better.  What counts is the products a wave gets,
+// not the row's against its tiles (more than half as many products as tiles):
+// random tiles of 48 entries, 8 a tile-row, 575 products a row, over 12 groups
+// 1.16 ms, over 24 groups (96000 rows) 3.76, by k_step3_flat 0.56 and 0.97;
+// 24 tiles of 24 entries, 1290 products over 24 groups 5.10 / 2.63 ms; over 8
+// groups, 164 a wave, 0.86 / 0.90.  With 100 / 160 / 220 / 320: random tiles (8
+// of 64 entries, 116 a wave) 0.81 / 0.58 / 0.58 / 0.58 ms, ER 30000 (40 per row,
+// 218 a wave) 1.27 / 1.26 / 1.41 / 1.47, R-MAT scale 16 A*A^T 11.1 / 10.9 / 10.9 / 11.2.
 #define LONG_MIN_PRODUCTS 512
-#define LONG_PER_TILE(u) ((u) / 2)
+#define LONG_PER_GROUP 160
 // Only in a large product (or when the caller sets heavy_min_products): in a
 // small one the waves of the longest rows end after everything else.  R-MAT
 // A^2 with / without long rows: scale 11 (6 edges a vertex) 410 / 353 us, scale 12
@@ -2014,12 +2021,13 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 // 2m) take the heavy and the long rows as counts for the scan that numbers
 // them, info[0] the number of heavy ones, info[2..3] the
 // long tile-rows' entries of C.  A tile-row with many products for
-// its tiles has only heavy and long rows and leaves the element-wise class.
+// its columns has only heavy and long rows and leaves the element-wise class.
 // One block per tile-row, 16 lanes per row, so that a long A row's B row
 // lengths are not one lane's chain of loads (R-MAT scale 16: 665 -> 92 us).
 __global__ void __launch_bounds__(256)
 k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const int *__restrict__ Browp,
-              unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, const int *__restrict__ Cnnz, int tilem, int m,
+              unsigned char *__restrict__ rowcls, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
+              const int *__restrict__ Cnnz, int tilem, int m,
               long long min_products, long long count_products, int take_long, unsigned char *__restrict__ flag, int *__restrict__ cnt,
               int *__restrict__ info) {
     __shared__ long long s_p[16];
@@ -2042,7 +2050,11 @@ k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
     __syncthreads();
     long long all = 0;
     for (int q = 0; q < 16; q++) all += s_p[q];
-    const bool longer = mine && take_long && all > 16 * max((long long)LONG_MIN_PRODUCTS, LONG_PER_TILE(Cptr[I + 1] - Cptr[I]));
+    bool longer = mine && take_long && all > 16 * LONG_MIN_PRODUCTS;
+    if (longer) {
+        const int span = Ccol[Cptr[I + 1] - 1] - Ccol[Cptr[I]] + 1;  // tile columns
+        longer = all * (HEAVY_GROUP * HEAVY_PART_TILES) > 16LL * LONG_PER_GROUP * span;
+    }
     if (i < m && l == 0) {
         const int h = !mine ? 0 : x1 - x0 > 2048 || p > min_products ? 2 : longer && p > 0 ? 1 : 0;
         flag[i] = (unsigned char)h;
@@ -3973,7 +3985,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                                             ? counted
                                             : std::min(nnzC >> HEAVY_SPLIT_LOG, HEAVY_SPLIT_MAX);
                 hipLaunchKernelGGL(k_heavy_flags, tsg_grid(C->tilem, 256), dim3(256), 0, s, op.Arowp, op.Acolx,
-                                   (const int *)B->rowx_ptr, w.rowcls, C->tile_ptr, C->tile_nnz, C->tilem, m, split,
+                                   (const int *)B->rowx_ptr, w.rowcls, C->tile_ptr, C->tile_colidx, C->tile_nnz, C->tilem, m, split,
                                    counted,
                                    large || tune.heavy_min_products > 0 ? 1 : 0, T.hflag, T.hcnt, T.hinfo);
                 TSG_LAUNCH_CHECK();
