@@ -3100,13 +3100,14 @@ k_step3_lines(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
 // over class-1 rows of (nonempty C tiles, C nonzeros plus accumulator pads,
 // A tiles, B tiles per B tile-row, B nonzeros per B tile-row, A tile
 // nonzeros) for the LDS layout, i = 7..10 those over the row-lines rows of (C
-// nonzeros, C tiles, tile-column span, g + 1).
+// nonzeros, C tiles, tile-column span, g + 1), i = 11 the rows of classes 0 and 1.
 // 16 lanes per tile-row (16 tile-rows per block): the lanes walk the row's A
 // tiles and C tiles in strides of 16, so the dependent loads of different A
 // tiles are in flight together.  k_row_class_reduce folds the blocks' partials
-// into out[0] (sum) and out[1..] (maxima): no atomics, which on one cache
+// into out (sums and maxima): no atomics, which on one cache
 // line would serialise across the thousands of blocks.
-#define CLS_WORDS 11
+#define CLS_WORDS 12
+__device__ __forceinline__ bool cls_sums(int i) { return i == 0 || i == 11; }
 __device__ __forceinline__ int g16_max(int v) {
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 16));
@@ -3120,7 +3121,7 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
     const int r = threadIdx.x & 15, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int I = blockIdx.x * 16 + (threadIdx.x >> 4);
     int unfit = 0, mu = 0, mn = 0, ml = 0, mq = 0, mb = 0, ma = 0;
-    int ln = 0, lu = 0, ls = 0, lg = 0;
+    int ln = 0, lu = 0, ls = 0, lg = 0, other = 0;
     if (I < tilem) {  // uniform in the 16-lane group
         const int c0 = Cptr[I], c1 = Cptr[I + 1];
         const int nrow = Cnnz[c1] - Cnnz[c0];
@@ -3178,8 +3179,10 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
         }
         if (r == 0) cls[I] = k;
         unfit = r == 0 && k == 0;
+        other = r == 0 && k <= 1;
     }
     unfit = tsg_wave_sum(unfit);
+    other = tsg_wave_sum(other);
     mu = tsg_wave_max(mu); mn = tsg_wave_max(mn); ml = tsg_wave_max(ml);
     mq = tsg_wave_max(mq); mb = tsg_wave_max(mb); ma = tsg_wave_max(ma);
     ln = tsg_wave_max(ln); lu = tsg_wave_max(lu); ls = tsg_wave_max(ls); lg = tsg_wave_max(lg);
@@ -3187,13 +3190,14 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
         s_red[wave][0] = unfit; s_red[wave][1] = mu; s_red[wave][2] = mn; s_red[wave][3] = ml;
         s_red[wave][4] = mq; s_red[wave][5] = mb; s_red[wave][6] = ma;
         s_red[wave][7] = ln; s_red[wave][8] = lu; s_red[wave][9] = ls; s_red[wave][10] = lg;
+        s_red[wave][11] = other;
     }
     __syncthreads();
     if (threadIdx.x < CLS_WORDS) {
         const int i = threadIdx.x;
         int v = s_red[0][i];
 #pragma unroll
-        for (int w = 1; w < 4; w++) v = i == 0 ? v + s_red[w][i] : max(v, s_red[w][i]);
+        for (int w = 1; w < 4; w++) v = cls_sums(i) ? v + s_red[w][i] : max(v, s_red[w][i]);
         part[CLS_WORDS * (long long)blockIdx.x + i] = v;
         if (ticket) __threadfence();
     }
@@ -3210,7 +3214,7 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
     for (int i = 0; i < CLS_WORDS; i++) v[i] = threadIdx.x < gridDim.x ? part[CLS_WORDS * threadIdx.x + i] : 0;
 #pragma unroll
     for (int i = 0; i < CLS_WORDS; i++) {
-        v[i] = i == 0 ? tsg_wave_sum(v[i]) : tsg_wave_max(v[i]);
+        v[i] = cls_sums(i) ? tsg_wave_sum(v[i]) : tsg_wave_max(v[i]);
         if (lane == 0) s_red[wave][i] = v[i];
     }
     __syncthreads();
@@ -3218,13 +3222,13 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
         const int i = threadIdx.x;
         int x = s_red[0][i];
 #pragma unroll
-        for (int w = 1; w < 4; w++) x = i == 0 ? x + s_red[w][i] : max(x, s_red[w][i]);
+        for (int w = 1; w < 4; w++) x = cls_sums(i) ? x + s_red[w][i] : max(x, s_red[w][i]);
         out[i] = x;
         if (host) host[i] = x;
     }
 }
 
-// out[0] = sum and out[1..] = maxima of the nb blocks' k_row_class partials
+// out = sums (words 0 and 11) and maxima of the nb blocks' k_row_class partials
 // (one block of 1024 threads).  host (may be NULL): pinned memory that gets
 // the CLS_WORDS words too.
 __global__ void __launch_bounds__(1024)
@@ -3235,13 +3239,11 @@ k_row_class_reduce(const int *__restrict__ part, int nb, int *__restrict__ out, 
     for (int i = 0; i < CLS_WORDS; i++) v[i] = 0;
     for (int b = threadIdx.x; b < nb; b += 1024) {
         const int *p = part + CLS_WORDS * (long long)b;
-        v[0] += p[0];
 #pragma unroll
-        for (int i = 1; i < CLS_WORDS; i++) v[i] = max(v[i], p[i]);
+        for (int i = 0; i < CLS_WORDS; i++) v[i] = cls_sums(i) ? v[i] + p[i] : max(v[i], p[i]);
     }
-    v[0] = tsg_wave_sum(v[0]);
 #pragma unroll
-    for (int i = 1; i < CLS_WORDS; i++) v[i] = tsg_wave_max(v[i]);
+    for (int i = 0; i < CLS_WORDS; i++) v[i] = cls_sums(i) ? tsg_wave_sum(v[i]) : tsg_wave_max(v[i]);
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -3250,7 +3252,7 @@ k_row_class_reduce(const int *__restrict__ part, int nb, int *__restrict__ out, 
     if (threadIdx.x < CLS_WORDS) {
         const int i = threadIdx.x;
         int r = s_r[0][i];
-        for (int w = 1; w < 16; w++) r = i == 0 ? r + s_r[w][i] : max(r, s_r[w][i]);
+        for (int w = 1; w < 16; w++) r = cls_sums(i) ? r + s_r[w][i] : max(r, s_r[w][i]);
         out[i] = r;
         if (host) host[i] = r;
     }
@@ -3757,9 +3759,38 @@ static void free_temps(tsg_ctx *ctx, SpgemmTemps &t) {
 // steps 1 to 3 do without: an operand may come without csr_col (the drop-in
 // entry point's, and tsg_tiles_from_csc_order's of one that has none) and then
 // stays on the tile kernels.
+#define ELEM_MAX_N ((1 << 27) - 32)  // columns of a B that the element kernels take
 static bool auto_index(const tsg_dtiles *t) {
     return t->csr_col && t->nnz >= AUTO_INDEX_NNZ && t->nnz >= AUTO_INDEX_TILE * (long long)t->numtile &&
            t->nnz <= AUTO_INDEX_ROW * (long long)t->m;
+}
+// Tiles dense enough, and few enough to a tile-row of A and a tile column of B,
+// for the tile kernels: what row lines do not take is better off there than
+// element by element (tiles of 28 entries and more, which meet in some 50
+// products), and the lines have to pay for the index alone.  Then it is made
+// after step 2, and only if nearly every tile-row would use it: beside a
+// tile kernel that runs anyway the lines' rows cost more than they save.
+// Index before step 1 and the rest element-wise / by tiles / this rule, A^2:
+// random tiles, 8 of 48 entries a tile-row, 0.63 / 0.37 / 0.35 ms, 12 of 40 0.77 / 0.53 /
+// 0.50; bands of half-width 20 (70% of the rows) and 100 1.14 / 1.23 / 1.12; of
+// half-width 40, all by lines, 0.40 / 0.40 / 0.41, without an index 0.48.  Random
+// tiles, 16 of 24 entries (not dense) element-wise 0.65, by tiles 0.78.
+#define AUTO_DENSE_TILE 28  // entries per tile, geometric mean of A and B
+#define AUTO_DENSE_LIST 16  // tiles per tile-row of A and per tile column of B
+#define AUTO_LINES(other, tilem) (32LL * (other) <= (tilem))
+static bool auto_dense(const tsg_dtiles *A, const tsg_dtiles *B) {
+    return (double)A->nnz * B->nnz >= (double)(AUTO_DENSE_TILE * AUTO_DENSE_TILE) * A->numtile * B->numtile &&
+           A->numtile <= AUTO_DENSE_LIST * (long long)A->tilem && B->numtile <= AUTO_DENSE_LIST * (long long)B->tilen;
+}
+// longest[K] = entries of the longest row of B's tile-row K, from its masks: 16 lanes a tile-row, a row each.
+__global__ void __launch_bounds__(256)
+k_longest_rows(const int *__restrict__ Bptr, const unsigned short *__restrict__ Bmask, int tilem, int *__restrict__ longest) {
+    const int K = blockIdx.x * 16 + (threadIdx.x >> 4), r = threadIdx.x & 15;
+    if (K >= tilem) return;
+    int c = 0;
+    for (int t = Bptr[K]; t < Bptr[K + 1]; t++) c += __popc((unsigned)Bmask[(long long)t * 16 + r]);
+    c = g16_max(c);
+    if (r == 0) longest[K] = c;
 }
 static int make_index(tsg_ctx *ctx, const tsg_dtiles *t, tsg_dcsr *r, tsg_dtiles *with) {
     *with = *t;
@@ -3803,7 +3834,9 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         TSG_HIP(hipEventRecord(ev[5], s));
     }
     tsg_dtiles ax, bx;
-    if (may_index && tune.element_mode == 0 && !P.all && !(A->rowx_ptr && B->rowx_ptr) && auto_index(A) && auto_index(B)) {
+    may_index = may_index && tune.element_mode == 0 && !P.all && B->n <= ELEM_MAX_N && !(A->rowx_ptr && B->rowx_ptr) &&
+                auto_index(A) && auto_index(B);
+    auto index_operands = [&]() -> int {
         auto borrow = [](const tsg_dtiles *t, const tsg_dtiles *from, tsg_dtiles *with) {
             *with = *t;
             with->rowx_ptr = from->rowx_ptr;
@@ -3826,12 +3859,15 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
             else TSG_TRY(make_index(ctx, B, &T.rowx[1], &bx));
             B = &bx;
         }
-    }
+        return TSG_OK;
+    };
+    const bool index_later = may_index && auto_dense(A, B);
+    if (may_index && !index_later) TSG_TRY(index_operands());
     // element path: B carries its row index, and C's columns fit the
     // 28-bit entry keys of the element kernel's LDS hash
     // element-wise keys: (column offset) << 4 in 32 bits, and tile columns
     // below 2^23 - 1 for the step-2 hash slots
-    P.s3_elem = B->rowx_ptr != nullptr && tune.element_mode != 1 && B->n <= (1 << 27) - 32;
+    P.s3_elem = B->rowx_ptr != nullptr && tune.element_mode != 1 && B->n <= ELEM_MAX_N;
     P.elem_all = B->rowx_ptr != nullptr && tune.element_mode == 2;
     P.lines = A->rowx_ptr && P.s3_elem && !P.elem_all && brow_bits_bytes(B) > 0;
     C->m = A->m;
@@ -3918,7 +3954,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         P.s2w = smax[7];
     }
     // ---- step 2
-    const TileOperands op = make_operands(A, B);
+    TileOperands op = make_operands(A, B);
     TSG_TRY(launch_step2(s, op, B, C, P, w));
     if (timed && numtileC > 0) {
         hipLaunchKernelGGL(k_bins, dim3(std::min<unsigned>(2048, tsg_div_up(numtileC, 256))), dim3(256), 0, s,
@@ -3939,23 +3975,44 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         pub.host = pin;
         TSG_TRY(tsg_scan_i32_enqueue(s, C->tile_nnz, C->tile_nnz, numtileC, part2, pub));
         if (timed) TSG_HIP(hipEventRecord(ev[2], s));
-        if (classes)
-            TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, T.longest, ticket, (int *)(pin + 1)));
-        TSG_HIP(hipStreamSynchronize(s));
-        nnzC = pin[0];
+        if (classes && index_later) {
+            TSG_TRY(tsg_alloc_t(ctx, &T.longest, (size_t)B->tilem));
+            hipLaunchKernelGGL(k_longest_rows, dim3(tsg_div_up(B->tilem, 16)), dim3(256), 0, s, (const int *)B->tile_ptr,
+                               (const unsigned short *)B->mask, B->tilem, T.longest);
+            TSG_LAUNCH_CHECK();
+        }
+        const volatile int *h = reinterpret_cast<const int *>(pin + 1);
+        auto classify = [&](const int *longest, int *cls_ticket) -> int {
+            TSG_TRY(launch_row_class(s, op, C, w.rowcls, w.cls_part, w.cls_out, P.elem_all, longest, cls_ticket, (int *)(pin + 1)));
+            TSG_HIP(hipStreamSynchronize(s));
+            return TSG_OK;
+        };
+        if (classes) TSG_TRY(classify(T.longest, ticket));
+        else TSG_HIP(hipStreamSynchronize(s));
+        nnzC = *(volatile long long *)pin;
         if (nnzC > 0x7fffffffLL) {
             tsg_set_error("prefix sum total %lld exceeds int32", nnzC);
             return TSG_ERR_OVERFLOW;
         }
+        if (classes && index_later && h[10] > 0) {  // some tile-rows would go by row lines
+            int cls[CLS_WORDS];
+            for (int i = 0; i < CLS_WORDS; i++) cls[i] = h[i];
+            if (AUTO_LINES(cls[11], C->tilem)) TSG_TRY(index_operands());
+            if (A->rowx_ptr && B->rowx_ptr) {
+                op = make_operands(A, B);
+                for (int i = 0; i < CLS_WORDS; i++) ((int *)(pin + 1))[i] = cls[i];  // (making the index read back there)
+            } else {
+                TSG_TRY(classify(nullptr, nullptr));
+            }
+        }
         if (classes) {
-            const int *h = reinterpret_cast<const int *>(pin + 1);
             P.s3_unfit = h[0] > 0;
             P.s3_rows = h[1] > 0;
-            for (int i = 0; i < 6; i++) P.g3[i] = std::max(1, h[1 + i]);
+            for (int i = 0; i < 6; i++) P.g3[i] = std::max(1, (int)h[1 + i]);
             P.s3_lines = h[10] > 0;
             P.ln[0] = h[7];
             P.ln[1] = h[8];
-            for (P.ln[2] = LN_MAP_MIN; P.ln[2] < std::min(h[9], LN_MAP);) P.ln[2] *= 2;
+            for (P.ln[2] = LN_MAP_MIN; P.ln[2] < std::min((int)h[9], LN_MAP);) P.ln[2] *= 2;
             P.ln[3] = std::min(LN_THREADS, 16 * (8 << h[10]));
         }
     }

@@ -2,6 +2,7 @@
 not whole tile matrices with every array: without in-tile columns (the drop-in
 entry point uploads none), and one operand a part of the other."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -152,4 +153,89 @@ def test_operands_that_share_values_only(ctx):
     for p in (tb.tile_colidx, tb.csc_ptr, tb.csc_rowidx, tb.csc_tileid):
         ctx.dfree(p)
     ctx.free(ta)
+    ctx.free(d)
+
+
+def bands(n, widths, ends):
+    """Rows up to ends[i] hold every column within widths[i]."""
+    half = np.zeros(n, np.int64)
+    for w, lo, hi in zip(widths, [0] + ends[:-1], ends):
+        half[lo:hi] = w
+    i = np.arange(n)
+    first, last = np.maximum(i - half, 0), np.minimum(i + half, n - 1)
+    ptr = np.r_[0, np.cumsum(np.maximum(last - first + 1, 0))]
+    col = np.arange(ptr[-1]) - np.repeat(ptr[:-1], np.diff(ptr)) + np.repeat(first, np.diff(ptr))
+    return ts.Csr(n, n, ptr, col, np.random.default_rng(n).uniform(-1, 1, len(col)))
+
+
+def dense_tiles(tile_rows, tiles, entries, seed=0):
+    """`tiles` tiles of `entries` entries in each tile-row, anywhere."""
+    rng = np.random.default_rng(seed)
+    n = 16 * tile_rows
+    key = np.unique(np.repeat(np.arange(tile_rows), tiles) * tile_rows + rng.integers(0, tile_rows, tile_rows * tiles))
+    at = np.argsort(rng.random((len(key), 256)), axis=1)[:, :entries]
+    key = np.sort(((key[:, None] // tile_rows * 16 + at // 16) * n + key[:, None] % tile_rows * 16 + at % 16).ravel())
+    return ts.Csr(n, n, np.r_[0, np.cumsum(np.bincount(key // n, minlength=n))], key % n, rng.uniform(-1, 1, len(key)))
+
+
+DENSE = {
+    "all_by_lines": lambda: bands(30000, [40], [30000]),
+    "few_not": lambda: bands(30000, [20, 100, 20], [10000, 10300, 30000]),
+    "half_not": lambda: bands(30000, [10, 64], [15000, 30000]),
+    "none": lambda: dense_tiles(3000, 8, 48),
+    "none_long_lists": lambda: dense_tiles(1500, 24, 32),
+    "some_empty_rows": lambda: bands(60000, [40, -1, 6], [20000, 40000, 60000]),
+}
+
+
+@pytest.mark.parametrize("index_a,index_b", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("name", list(DENSE))
+def test_dense_tiles(ctx, name, index_a, index_b):
+    """Tiles that meet in dozens of products: the index is made only where nearly all of C goes by row lines."""
+    a = DENSE[name]()
+    assert a.nnz >= 1 << 20 and a.nnz <= 96 * a.m
+    log(f"[auto index] dense, {name}: nnz {a.nnz} index {index_a} {index_b}")
+    b = ts.Csr(a.m, a.n, a.rowptr, a.colidx, np.random.default_rng(2).uniform(-1, 1, a.nnz))
+    da, db = ctx.upload(a), ctx.upload(b)
+    ta, tb = ctx.csr2tile(da), ctx.csr2tile(db)
+    ctx.build_csc(tb)
+    want = tile_parallel(ctx, ta, tb)
+    if index_a:
+        ctx.build_rowindex(ta)
+    if index_b:
+        ctx.build_rowindex(tb)
+    before = ctx.bytes_in_use()
+    for _ in range(2):
+        c, _ = ctx.spgemm(ta, tb)
+        same_tiles(ctx.download_tiles(c), want)
+        ctx.free(c)
+        assert ctx.bytes_in_use() == before
+    for x in (ta, tb, da, db):
+        ctx.free(x)
+
+
+def best_ms(ctx, t, tune):
+    best = 1e9
+    for _ in range(8):
+        ctx.sync()
+        t0 = time.perf_counter()
+        c, _ = ctx.spgemm(t, t, tune, timed=False)
+        ctx.sync()
+        best = min(best, time.perf_counter() - t0)
+        ctx.free(c)
+    return best * 1e3
+
+
+@pytest.mark.parametrize("name,least", [("none", 1.5), ("half_not", 1.5)])
+def test_index_is_no_loss_on_dense_tiles(ctx, name, least):
+    """Against the product that may make none: element by element the first took 1.8 times as long."""
+    d = ctx.upload(DENSE[name]())
+    t = ctx.csr2tile(d)
+    ctx.build_csc(t)
+    without = ts.default_tune()
+    without.element_mode = 1
+    w, m = best_ms(ctx, t, without), best_ms(ctx, t, None)
+    log(f"[auto index] {name}: {m:.3f} ms, without an index {w:.3f}")
+    assert m <= least * w
+    ctx.free(t)
     ctx.free(d)

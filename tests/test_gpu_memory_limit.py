@@ -37,12 +37,13 @@ assert failed > 4 and t.rowx_ptr
 """)
 
 
+@pytest.mark.parametrize("matrix", ["ts.gen_stencil27(36, 33, 37, valmode=ts.VAL_UNIFORM_PM1, seed=3)",
+                                    "ts.gen_banded(30000, 40, seed=3)"], ids=["mesh", "band"])
 @pytest.mark.parametrize("apart", [False, True])
-def test_products_index_themselves_only_if_there_is_room(tmp_path, apart):
+def test_products_index_themselves_only_if_there_is_room(tmp_path, apart, matrix):
     """Wherever the product fits without indices of its own it is computed; what does not fit leaves nothing."""
-    run_limited(tmp_path, f"apart = {apart}" + """
+    run_limited(tmp_path, f"apart, a = {apart}, {matrix}" + """
 ctx = ts.Context(0)
-a = ts.gen_stencil27(36, 33, 37, valmode=ts.VAL_UNIFORM_PM1, seed=3)
 d = ctx.upload(a)
 ta = ctx.csr2tile(d)
 tb = ctx.csr2tile(d) if apart else ta
