@@ -111,9 +111,10 @@ static int max_of(tsg_ctx *ctx, const int *v, int n, int *out) {
 }
 
 // ids sorted by degree (ascending or descending), ties by ascending id
-static int sort_ids_by_degree(tsg_ctx *ctx, const int *deg, int n, int descending, int *ids) {
+static int sort_ids_by_degree(tsg_ctx *ctx, const int *deg, int n, int descending, int *ids, int *most = nullptr) {
     int maxdeg = 0;
     TSG_TRY(max_of(ctx, deg, n, &maxdeg));
+    if (most) *most = maxdeg;
     unsigned *key;
     TSG_TRY(tsg_alloc_t(ctx, &key, (size_t)n + 1));
     if (n > 0) {
@@ -187,19 +188,21 @@ __device__ __forceinline__ int lower_bound_r(const int *__restrict__ list, int l
     return lo;
 }
 
-// Union of two sorted rows, 16 lanes per row: an entry's place is its index
+// Union of two sorted rows, L lanes per row: an entry's place is its index
 // plus the other row's smaller entries, less those of both rows before it.
-// (One thread merging a row: 27-point mesh of 230k rows 357 -> 87 us.)
-template <bool FILL>
+// (One thread merging a row: 27-point mesh of 230k rows 357 -> 87 us with 16.
+// Rows of one entry, 4,000,000 of them: 16 lanes 433 us, 4 lanes 150.)
+template <bool FILL, int L>
 __global__ void __launch_bounds__(256)
 k_union_rows(int m, const int *__restrict__ ap, const int *__restrict__ ac, const int *__restrict__ tp,
              const int *__restrict__ tc, int *__restrict__ cnt_or_ptr, int *__restrict__ gc) {
-    const unsigned i = tsg_block() * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15, gb = threadIdx.x & 48;
+    const unsigned i = tsg_block() * (256 / L) + threadIdx.x / L, l = threadIdx.x % L, gb = (threadIdx.x & 63) / L * L;
     if (i >= (unsigned)m) return;  // whole groups
+    const unsigned lanes = (1u << L) - 1u;
     const int a0 = ap[i], a1 = ap[i + 1], b0 = tp[i], b1 = tp[i + 1];
     const int out = FILL ? cnt_or_ptr[i] : 0;
     int both = 0;  // entries of both rows so far
-    for (int e0 = a0; e0 < a1; e0 += 16) {
+    for (int e0 = a0; e0 < a1; e0 += L) {
         const int e = e0 + l;
         bool dup = false;
         int x = 0, at = 0;
@@ -208,7 +211,7 @@ k_union_rows(int m, const int *__restrict__ ap, const int *__restrict__ ac, cons
             at = lower_bound_r(tc, b0, b1, x);
             dup = at < b1 && tc[at] == x;
         }
-        const unsigned d = (unsigned)(__ballot(dup) >> gb) & 0xffffu;
+        const unsigned d = (unsigned)(__ballot(dup) >> gb) & lanes;
         if (FILL && e < a1) gc[out + (e - a0) + (at - b0) - both - __popc(d & ((1u << l) - 1u))] = x;
         both += __popc(d);
     }
@@ -217,7 +220,7 @@ k_union_rows(int m, const int *__restrict__ ap, const int *__restrict__ ac, cons
         return;
     }
     both = 0;
-    for (int e0 = b0; e0 < b1; e0 += 16) {  // entries of the second row alone
+    for (int e0 = b0; e0 < b1; e0 += L) {  // entries of the second row alone
         const int e = e0 + l;
         bool dup = false;
         int x = 0, at = 0;
@@ -226,10 +229,30 @@ k_union_rows(int m, const int *__restrict__ ap, const int *__restrict__ ac, cons
             at = lower_bound_r(ac, a0, a1, x);
             dup = at < a1 && ac[at] == x;
         }
-        const unsigned d = (unsigned)(__ballot(dup) >> gb) & 0xffffu;
+        const unsigned d = (unsigned)(__ballot(dup) >> gb) & lanes;
         if (e < b1 && !dup) gc[out + (e - b0) + (at - a0) - both - __popc(d & ((1u << l) - 1u))] = x;
         both += __popc(d);
     }
+}
+// Whether four lanes per row are enough: entries few on the whole and in every
+// row (asked of large matrices only: it costs a launch and a wait).
+#define UNION_LOW_ROWS (1 << 18)
+#define UNION_LOW_MEAN 4  // entries of A per row
+#define UNION_LOW_MAX 64  // of a row of A and of A^T together
+__global__ void __launch_bounds__(256)
+k_both_lengths(int m, const int *__restrict__ ap, const int *__restrict__ tp, int *__restrict__ len) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i < (unsigned)m) len[i] = ap[i + 1] - ap[i] + (tp[i + 1] - tp[i]);
+}
+static int union_is_low(tsg_ctx *ctx, const tsg_dcsr *a, const tsg_dcsr *at, int *len, bool *low) {
+    *low = false;
+    if (a->m < UNION_LOW_ROWS || a->nnz > UNION_LOW_MEAN * (long long)a->m) return TSG_OK;
+    hipLaunchKernelGGL(k_both_lengths, dim3(tsg_div_up(a->m, 256)), dim3(256), 0, ctx->stream, a->m, a->rowptr, at->rowptr, len);
+    TSG_LAUNCH_CHECK();
+    int most = 0;
+    TSG_TRY(max_of(ctx, len, a->m, &most));
+    *low = most <= UNION_LOW_MAX;
+    return TSG_OK;
 }
 
 // pattern(A + A^T), sorted rows, self loops kept
@@ -240,9 +263,11 @@ extern "C" int tsg_dcsr_symmetrize(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dcsr *g)
     TSG_TRY(tsg_dcsr_transpose(ctx, a, &at));
     g->m = g->n = a->m;
     TSG_TRY(tsg_alloc_t(ctx, &g->rowptr, (size_t)a->m + 1));
-    const dim3 gr = tsg_grid(tsg_div_up(a->m, 16), 256);
+    bool low;
+    TSG_TRY(union_is_low(ctx, a, &at, g->rowptr, &low));
+    const dim3 gr = tsg_grid(tsg_div_up(a->m, low ? 64 : 16), 256);
     if (a->m > 0) {
-        hipLaunchKernelGGL(k_union_rows<false>, gr, dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
+        hipLaunchKernelGGL((low ? k_union_rows<false, 4> : k_union_rows<false, 16>), gr, dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
                            at.rowptr, at.colidx, g->rowptr, (int *)nullptr);
         TSG_LAUNCH_CHECK();
     }
@@ -252,7 +277,7 @@ extern "C" int tsg_dcsr_symmetrize(tsg_ctx *ctx, const tsg_dcsr *a, tsg_dcsr *g)
     TSG_TRY(tsg_alloc_t(ctx, &g->colidx, (size_t)nnz + 1));
     TSG_TRY(tsg_alloc_t(ctx, &g->val, (size_t)nnz + 1));
     if (a->m > 0 && nnz > 0) {
-        hipLaunchKernelGGL(k_union_rows<true>, gr, dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
+        hipLaunchKernelGGL((low ? k_union_rows<true, 4> : k_union_rows<true, 16>), gr, dim3(256), 0, ctx->stream, a->m, a->rowptr, a->colidx,
                            at.rowptr, at.colidx, g->rowptr, g->colidx);
         hipLaunchKernelGGL(k_fill_f64, dim3(tsg_div_up(nnz, 256)), dim3(256), 0, ctx->stream, g->val, nnz, 1.0);
         TSG_LAUNCH_CHECK();
@@ -299,20 +324,27 @@ __device__ __forceinline__ int cc_root(const int *parent, int x) {
     }
     return x;
 }
-#define VERT_LANES 16  // lanes per vertex of the kernels that walk adjacency lists
+// Lanes per vertex of the kernels that walk adjacency lists: VERT_LANES, and a
+// wave where children are put in order; VERT_LANES_LOW and VERT_LANES where every
+// list is short and most are shorter than a line (RCM of 2,000,000 pairs 7.3 -> 3.1
+// ms with the scan by runs below, of ER 1,000,000, two a row, 4.0 -> 2.5).
+#define VERT_LANES 16
+#define VERT_LANES_LOW 4
+#define VERT_LOW_MAX 64   // longest list
+#define VERT_LOW_MEAN 8
 // FIRST: parent of each vertex = the lowest rank among itself and its
 // neighbours.  Else: the parent of its tree's root, label[v], lowered to the
 // lowest label next to it.
-template <bool FIRST>
+template <bool FIRST, int VL>
 __global__ void __launch_bounds__(256)
 k_cc_hook(const int *__restrict__ gp, const int *__restrict__ gc, int n, const int *__restrict__ id, int *parent) {
-    const unsigned v = tsg_block() * (256 / VERT_LANES) + threadIdx.x / VERT_LANES, l = threadIdx.x % VERT_LANES;
+    const unsigned v = tsg_block() * (256 / VL) + threadIdx.x / VL, l = threadIdx.x % VL;
     if (v >= (unsigned)n) return;
     const int iv = id[v], e1 = gp[v + 1];
     int mn = iv;
-    for (int e = gp[v] + l; e < e1; e += VERT_LANES) mn = min(mn, id[gc[e]]);
+    for (int e = gp[v] + l; e < e1; e += VL) mn = min(mn, id[gc[e]]);
 #pragma unroll
-    for (int o = VERT_LANES / 2; o > 0; o >>= 1) mn = min(mn, __shfl_xor(mn, o, VERT_LANES));
+    for (int o = VL / 2; o > 0; o >>= 1) mn = min(mn, __shfl_xor(mn, o, VL));
     if (l == 0) {
         if (FIRST) parent[iv] = mn;
         else if (mn < iv && mn < cc_load(&parent[iv])) atomicMin(&parent[iv], mn);  // few trees: one address for many
@@ -327,12 +359,13 @@ k_cc_label(const int *__restrict__ rank, int n, int *parent, int *__restrict__ l
     label[v] = t;
     if (t != r) __hip_atomic_store(&parent[r], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+template <int VL>
 __global__ void __launch_bounds__(256)
 k_cc_link(const int *__restrict__ gp, const int *__restrict__ gc, int n, const int *__restrict__ label, int *parent) {
-    const unsigned v = tsg_block() * (256 / VERT_LANES) + threadIdx.x / VERT_LANES, l = threadIdx.x % VERT_LANES;
+    const unsigned v = tsg_block() * (256 / VL) + threadIdx.x / VL, l = threadIdx.x % VL;
     if (v >= (unsigned)n) return;
     const int lv = label[v], e1 = gp[v + 1];
-    for (int e = gp[v] + l; e < e1; e += VERT_LANES) {
+    for (int e = gp[v] + l; e < e1; e += VL) {
         const int lu = label[gc[e]];
         if (lu >= lv) continue;  // one tree, or the edge's other end takes it (the pattern is symmetric)
         int a = cc_root(parent, lv), b = cc_root(parent, lu);
@@ -359,14 +392,30 @@ __global__ void k_seed_compact(const int *__restrict__ order, const int *__restr
 }
 // One BFS level: every unvisited neighbour is claimed by its first parent in
 // level order (its position q), the claimed ones are counted per parent, and
-// put in (degree, id) order behind one another.  VERT_LANES lanes per parent
-// for the first two, a wave for the last, which sorts a parent's children by
+// put in (degree, id) order behind one another.  VL lanes per parent
+// for the first two, EL for the last, which sorts a parent's children by
 // counting the smaller keys; a level with more than RCM_KIDS children of one
 // parent (word[0] then) goes through the radix sort instead.  Against sorting
 // every level (62 of a 27-point 61x64x59 mesh, some 40 launches each, 18 ms for
 // the call): 4 launches, 1.9 ms.
+//   A block counts the parents of one run of positions and leaves each its
+// children's place within the run; the runs' totals (at most RCM_BLOCKS) are all
+// that is left to scan, whatever the level's size (scanning every count in
+// one block took 1.3 ms of a level of 2,000,000).
 #define RCM_KIDS 64
 #define RCM_AHEAD 8  // levels enqueued behind one another
+#define RCM_BLOCKS 1024
+// Positions per block of a level of nf: whole steps of `step` parents.
+__device__ __forceinline__ int rcm_run(int nf, int blocks, int step) {
+    const int per = (int)(((unsigned)nf + (unsigned)blocks - 1u) / (unsigned)blocks);
+    return (per + step - 1) / step * step;
+}
+// Where parent q's children go in the level's (q < nf), from k_count_children's
+// places and k_level_scan's totals.
+__device__ __forceinline__ int rcm_place(const int *__restrict__ cnt, const int *__restrict__ first, int run, int q) {
+    return first[q / run] + cnt[q];
+}
+template <int VL>
 __global__ void __launch_bounds__(256)
 k_claim(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ seq, int2 *__restrict__ level,
         int2 given, const int *__restrict__ visited, int *__restrict__ claim, int *__restrict__ word) {
@@ -375,117 +424,120 @@ k_claim(const int *__restrict__ gp, const int *__restrict__ gc, const int *__res
         word[0] = 0;
         if (given.y > 0) *level = given;
     }
-    const int l = threadIdx.x % VERT_LANES;
-    for (int q = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VERT_LANES); q < lv.y;
-         q += (int)(gridDim.x * (256 / VERT_LANES))) {
+    const int l = threadIdx.x % VL;
+    for (int q = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / VL); q < lv.y; q += (int)(gridDim.x * (256 / VL))) {
         const int p = seq[lv.x + q], e1 = gp[p + 1];
-        for (int e = gp[p] + l; e < e1; e += VERT_LANES) {
+        for (int e = gp[p] + l; e < e1; e += VL) {
             const int u = gc[e];
             if (!visited[u]) atomicMin(&claim[u], q);
         }
     }
 }
+template <int VL>
 __global__ void __launch_bounds__(256)
 k_count_children(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ seq,
                  const int2 *__restrict__ level, const int *__restrict__ visited, const int *__restrict__ claim,
-                 int *__restrict__ cnt, int *__restrict__ word) {
+                 int *__restrict__ cnt, int *__restrict__ total, int *__restrict__ word) {
+    __shared__ int s_w[2][4];
     const int2 lv = *level;
-    const int l = threadIdx.x % VERT_LANES;
-    for (int b = blockIdx.x * (256 / VERT_LANES); b < lv.y; b += gridDim.x * (256 / VERT_LANES)) {  // block-uniform
-        const int q = b + threadIdx.x / VERT_LANES;
+    if (lv.y == 0) return;  // (an empty level leaves the places of the one before)
+    constexpr int STEP = 256 / VL;
+    const int l = threadIdx.x % VL, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int run = rcm_run(lv.y, gridDim.x, STEP);
+    const long long q0 = (long long)blockIdx.x * run, q1 = min((long long)lv.y, q0 + run);
+    int before = 0, k = 0;
+    for (long long b = q0; b < q1; b += STEP, k ^= 1) {  // block-uniform
+        const int q = (int)b + threadIdx.x / VL;
         int c = 0;
-        if (q < lv.y) {
+        if (q < q1) {
             const int p = seq[lv.x + q], e1 = gp[p + 1];
-            for (int e = gp[p] + l; e < e1; e += VERT_LANES) {
+            for (int e = gp[p] + l; e < e1; e += VL) {
                 const int u = gc[e];
                 c += !visited[u] && claim[u] == q;
             }
         }
-        c = tsg_group16_sum(c);
-        if (q < lv.y && l == 0) cnt[q] = c;
+#pragma unroll
+        for (int o = VL / 2; o > 0; o >>= 1) c += __shfl_xor(c, o, VL);
         const int mx = tsg_wave_max(c);
-        if ((threadIdx.x & 63) == 0 && mx > RCM_KIDS) atomicMax(&word[0], mx);
+        if (lane == 0 && mx > RCM_KIDS) atomicMax(&word[0], mx);
+        const int mine = l == 0 ? c : 0, incl = tsg_wave_incl_scan_dpp(mine);
+        if (lane == 63) s_w[k][wave] = incl;
+        __syncthreads();
+        int at = before + incl - mine;
+        for (int w = 0; w < 4; w++) {
+            if (w < wave) at += s_w[k][w];
+            before += s_w[k][w];
+        }
+        if (q < q1 && l == 0) cnt[q] = at;
     }
+    if (threadIdx.x == 0) total[blockIdx.x] = before;
 }
 
-// One block: cnt's exclusive scan in place (cnt[nf] = total), the next level
+// One block: the runs' totals to their first places, the next level
 // behind this one (empty when a parent has too many children for
 // k_emit_children), {children, most of one parent beyond RCM_KIDS} to the host.
-__global__ void __launch_bounds__(1024)
-k_level_scan(int *cnt, int2 *level, const int *__restrict__ word, int *__restrict__ host) {
-    __shared__ int s_w[16], s_carry;
+__global__ void __launch_bounds__(RCM_BLOCKS)
+k_level_scan(int *total, int blocks, int2 *level, const int *__restrict__ word, int *__restrict__ host) {
+    __shared__ int s_w[RCM_BLOCKS / 64];
     const int2 lv = level[0];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    if (tid == 0) s_carry = 0;
-    __syncthreads();
-    for (int b = 0; b < lv.y; b += 4096) {
-        int c[4], sum = 0;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int x = b + 4 * tid + v;
-            c[v] = x < lv.y ? cnt[x] : 0;
-            sum += c[v];
+    if (lv.y == 0) {  // block-uniform
+        if (tid == 0) {
+            level[1] = make_int2(0, 0);
+            host[0] = host[1] = 0;
         }
-        const int incl = tsg_wave_incl_scan(sum);
-        if (lane == 63) s_w[wave] = incl;
-        __syncthreads();
-        int at = s_carry + incl - sum;
-        for (int w = 0; w < wave; w++) at += s_w[w];
-        __syncthreads();
-        if (tid == 1023) s_carry = at + sum;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int x = b + 4 * tid + v;
-            if (x < lv.y) cnt[x] = at;
-            at += c[v];
-        }
-        __syncthreads();
+        return;
     }
-    if (tid == 0) {
-        const int total = s_carry, most = lv.y > 0 ? word[0] : 0;
-        if (lv.y > 0) cnt[lv.y] = total;
-        level[1] = most > RCM_KIDS ? make_int2(0, 0) : make_int2(lv.x + lv.y, total);
-        host[0] = total;
+    const int c = tid < blocks ? total[tid] : 0, incl = tsg_wave_incl_scan_dpp(c);
+    if (lane == 63) s_w[wave] = incl;
+    __syncthreads();
+    int at = incl - c;
+    for (int w = 0; w < wave; w++) at += s_w[w];
+    if (tid < blocks) total[tid] = at;
+    if (tid == RCM_BLOCKS - 1) {
+        const int all = at + c, most = word[0];
+        level[1] = most > RCM_KIDS ? make_int2(0, 0) : make_int2(lv.x + lv.y, all);
+        host[0] = all;
         host[1] = most;
     }
 }
-// Children of a wave's parent q into out[off[q]..), marked visited (only q's
+// Children of parent q, EL lanes', into their places, marked visited (only q's
 // own claims are, so the other parents' tests do not change).
+template <int EL>
 __global__ void __launch_bounds__(256)
 k_emit_children(const int *__restrict__ gp, const int *__restrict__ gc, const int2 *__restrict__ level, const int *__restrict__ word,
                 int *__restrict__ visited, const int *__restrict__ claim, const int *__restrict__ deg,
-                const int *__restrict__ off, int *__restrict__ seq) {
-    __shared__ unsigned long long s_key[4][RCM_KIDS];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+                const int *__restrict__ cnt, const int *__restrict__ first, int blocks, int step, int *__restrict__ seq) {
+    __shared__ unsigned long long s_key[256 / EL][RCM_KIDS];
+    const int g = threadIdx.x / EL, l = threadIdx.x % EL, gb = (threadIdx.x & 63) / EL * EL;
+    const unsigned long long mask = EL == 64 ? ~0ull : (1ull << (EL & 63)) - 1ull;
     const int2 lv = *level;
     if (lv.y == 0 || *word > RCM_KIDS) return;
+    const int run = rcm_run(lv.y, blocks, step);
     int *out = seq + lv.x + lv.y;
-    for (int q = blockIdx.x * 4 + wave; q < lv.y; q += gridDim.x * 4) {
-        const int n = off[q + 1] - off[q];  // at most RCM_KIDS
-        if (n == 0) continue;
-        const int p = seq[lv.x + q], e1 = gp[p + 1];
-        int have = 0;
-        for (int e0 = gp[p]; e0 < e1; e0 += 64) {
-            const int e = e0 + lane;
+    for (int q = blockIdx.x * (256 / EL) + g; q < lv.y; q += gridDim.x * (256 / EL)) {
+        const int p = seq[lv.x + q], e0 = gp[p], e1 = gp[p + 1];
+        int n = 0;  // at most RCM_KIDS
+        for (int eb = e0; eb < e1; eb += EL) {
+            const int e = eb + l;
             int u = 0;
             bool mine = false;
             if (e < e1) {
                 u = gc[e];
                 mine = !visited[u] && claim[u] == q;
             }
-            const unsigned long long b = __ballot(mine);
-            if (mine)
-                s_key[wave][have + __popcll(b & ((1ull << lane) - 1ull))] =
-                    ((unsigned long long)(unsigned)deg[u] << 32) | (unsigned)u;
-            have += __popcll(b);
+            const unsigned long long b = (__ballot(mine) >> gb) & mask;
+            if (mine) s_key[g][n + __popcll(b & ((1ull << l) - 1ull))] = ((unsigned long long)(unsigned)deg[u] << 32) | (unsigned)u;
+            n += __popcll(b);
         }
         tsg_wave_sync();
-        if (lane < n) {
-            const unsigned long long key = s_key[wave][lane];
+        const int at = n > 0 ? rcm_place(cnt, first, run, q) : 0;
+        for (int i = l; i < n; i += EL) {
+            const unsigned long long key = s_key[g][i];
             int r = 0;
-            for (int j = 0; j < n; j++) r += s_key[wave][j] < key;  // ids differ, so keys do
+            for (int j = 0; j < n; j++) r += s_key[g][j] < key;  // ids differ, so keys do
             const int u = (int)(key & 0xffffffffu);
-            out[off[q] + r] = u;
+            out[at + r] = u;
             visited[u] = 1;
         }
         tsg_wave_sync();  // the next parent rewrites the keys
@@ -495,12 +547,13 @@ k_emit_children(const int *__restrict__ gp, const int *__restrict__ gc, const in
 __global__ void __launch_bounds__(256)
 k_list_children(const int *__restrict__ gp, const int *__restrict__ gc, const int *__restrict__ front, int nf,
                 const int *__restrict__ visited, const int *__restrict__ claim, const int *__restrict__ deg,
-                const int *__restrict__ off, unsigned long long *__restrict__ key, int *__restrict__ par) {
+                const int *__restrict__ cnt, const int *__restrict__ first, int blocks, int step,
+                unsigned long long *__restrict__ key, int *__restrict__ par) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned q = tsg_block() * 4 + wave;
     if (q >= (unsigned)nf) return;
     const int p = front[q], e1 = gp[p + 1];
-    int k = off[q];
+    int k = rcm_place(cnt, first, rcm_run(nf, blocks, step), (int)q);
     for (int e0 = gp[p]; e0 < e1; e0 += 64) {
         const int e = e0 + lane;
         int u = 0;
@@ -546,8 +599,9 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     if (n == 0) return TSG_OK;
     tsg_dcsr g;
     TSG_TRY(tsg_dcsr_symmetrize(ctx, a, &g));
-    int *deg, *order, *rank, *label, *visited, *claim, *seq, *flag, *pos, *word;
+    int *deg, *order, *rank, *label, *visited, *claim, *seq, *flag, *pos, *word, *first;
     TSG_TRY(tsg_alloc_t(ctx, &word, RCM_AHEAD));
+    TSG_TRY(tsg_alloc_t(ctx, &first, RCM_BLOCKS));
     TSG_TRY(tsg_alloc_t(ctx, &deg, (size_t)n + 1));
     TSG_TRY(tsg_alloc_t(ctx, &order, (size_t)n + 1));
     TSG_TRY(tsg_alloc_t(ctx, &rank, (size_t)n + 1));
@@ -561,17 +615,21 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     const unsigned gn = tsg_div_up(n, 256);
     hipLaunchKernelGGL(k_rcm_deg, dim3(gn), dim3(256), 0, s, g.rowptr, g.colidx, n, deg);
     TSG_LAUNCH_CHECK();
-    TSG_TRY(sort_ids_by_degree(ctx, deg, n, 0, order));  // ascending (degree, id)
+    int longest = 0;
+    TSG_TRY(sort_ids_by_degree(ctx, deg, n, 0, order, &longest));  // ascending (degree, id)
+    const bool low = longest <= VERT_LOW_MAX && g.nnz <= VERT_LOW_MEAN * (long long)n;
+    const int vl = low ? VERT_LANES_LOW : VERT_LANES, el = low ? VERT_LANES : 64, step = 256 / vl;
     // connected components: label = lowest rank in the component (parents in
     // claim, which is set up for the traversal below)
-    const dim3 gv = tsg_grid(tsg_div_up(n, 256 / VERT_LANES), 256);
+    const dim3 gv = tsg_grid(tsg_div_up(n, 256 / vl), 256);
     hipLaunchKernelGGL(k_scatter_rank, dim3(gn), dim3(256), 0, s, order, n, rank);
     for (int round = 0; round < CC_ROUNDS; round++) {
-        hipLaunchKernelGGL(round == 0 ? k_cc_hook<true> : k_cc_hook<false>, gv, dim3(256), 0, s, g.rowptr,
-                           g.colidx, n, (const int *)(round == 0 ? rank : label), claim);
+        auto hook = low ? (round == 0 ? k_cc_hook<true, VERT_LANES_LOW> : k_cc_hook<false, VERT_LANES_LOW>)
+                        : (round == 0 ? k_cc_hook<true, VERT_LANES> : k_cc_hook<false, VERT_LANES>);
+        hipLaunchKernelGGL(hook, gv, dim3(256), 0, s, g.rowptr, g.colidx, n, (const int *)(round == 0 ? rank : label), claim);
         hipLaunchKernelGGL(k_cc_label, dim3(gn), dim3(256), 0, s, (const int *)rank, n, claim, label);
     }
-    hipLaunchKernelGGL(k_cc_link, gv, dim3(256), 0, s, g.rowptr, g.colidx, n, (const int *)label, claim);
+    hipLaunchKernelGGL(low ? k_cc_link<VERT_LANES_LOW> : k_cc_link<VERT_LANES>, gv, dim3(256), 0, s, g.rowptr, g.colidx, n, (const int *)label, claim);
     hipLaunchKernelGGL(k_cc_label, dim3(gn), dim3(256), 0, s, (const int *)rank, n, claim, label);
     TSG_LAUNCH_CHECK();
     // level 0: all component seeds, in rank order
@@ -606,16 +664,20 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     static_assert(2 * RCM_AHEAD <= 128, "the pinned words hold every level's");
     double growth = 1.0;  // of the last level against the one before
     for (int ahead = 2; nf > 0 && done < n;) {
-        const unsigned gf = std::min(1024u, std::max(64u, tsg_div_up(2 * nf * VERT_LANES, 256)));
-        const unsigned gw = std::min(2048u, std::max(64u, tsg_div_up(2 * nf, 4)));
+        const unsigned gf = std::min<unsigned>(RCM_BLOCKS, std::max(64u, tsg_div_up(2 * nf * vl, 256)));
+        const unsigned gw = std::min(2048u, std::max(64u, tsg_div_up(2 * nf * el, 256)));
         for (int i = 0; i < ahead; i++) {
-            hipLaunchKernelGGL(k_claim, dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx, (const int *)seq, lvl + i,
-                               i ? make_int2(0, 0) : make_int2((int)fstart, (int)nf), visited, claim, word + i);
-            hipLaunchKernelGGL(k_count_children, dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx, (const int *)seq,
-                               (const int2 *)(lvl + i), visited, claim, cnt, word + i);
-            hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(1024), 0, s, cnt, lvl + i, (const int *)(word + i), host + 2 * i);
-            hipLaunchKernelGGL(k_emit_children, dim3(gw), dim3(256), 0, s, g.rowptr, g.colidx, (const int2 *)(lvl + i),
-                               (const int *)(word + i), visited, claim, deg, cnt, seq);
+            hipLaunchKernelGGL(low ? k_claim<VERT_LANES_LOW> : k_claim<VERT_LANES>, dim3(gf), dim3(256), 0, s, g.rowptr, g.colidx,
+                               (const int *)seq, lvl + i, i ? make_int2(0, 0) : make_int2((int)fstart, (int)nf), visited, claim,
+                               word + i);
+            hipLaunchKernelGGL(low ? k_count_children<VERT_LANES_LOW> : k_count_children<VERT_LANES>, dim3(gf), dim3(256), 0, s,
+                               g.rowptr, g.colidx, (const int *)seq, (const int2 *)(lvl + i), visited, claim, cnt, first,
+                               word + i);
+            hipLaunchKernelGGL(k_level_scan, dim3(1), dim3(RCM_BLOCKS), 0, s, first, (int)gf, lvl + i, (const int *)(word + i),
+                               host + 2 * i);
+            hipLaunchKernelGGL(low ? k_emit_children<VERT_LANES> : k_emit_children<64>, dim3(gw), dim3(256), 0, s, g.rowptr,
+                               g.colidx, (const int2 *)(lvl + i), (const int *)(word + i), visited, claim, deg,
+                               (const int *)cnt, (const int *)first, (int)gf, step, seq);
             TSG_LAUNCH_CHECK();
         }
         TSG_HIP(hipStreamSynchronize(s));
@@ -646,7 +708,7 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
         const dim3 gl = tsg_grid(tsg_div_up(nf, 4), 256);
         {
             hipLaunchKernelGGL(k_list_children, gl, dim3(256), 0, s, g.rowptr, g.colidx, front, (int)nf, visited,
-                               claim, deg, cnt, key, par);
+                               claim, deg, (const int *)cnt, (const int *)first, (int)gf, step, key, par);
             TSG_LAUNCH_CHECK();
             const unsigned gc2 = tsg_div_up(nc, 256);
             hipLaunchKernelGGL(k_mark_children, dim3(gc2), dim3(256), 0, s, key, (int)nc, visited);
@@ -680,7 +742,7 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
     hipLaunchKernelGGL(k_reverse_gather, dim3(gn), dim3(256), 0, s, seq, idx, n, d_old_id);
     TSG_LAUNCH_CHECK();
     if (levels_out) *levels_out = levels;
-    void *ps[] = {deg, order, rank, label, visited, claim, seq, flag, pos, word, key, par, cnt, idx, k2, ck, lvl};
+    void *ps[] = {deg, order, rank, label, visited, claim, seq, flag, pos, word, first, key, par, cnt, idx, k2, ck, lvl};
     for (void *p : ps) tsg_free(ctx, p);
     tsg_dcsr_free(ctx, &g);
     return TSG_OK;
