@@ -752,21 +752,36 @@ extern "C" int tsg_order_rcm(tsg_ctx *ctx, const tsg_dcsr *a, int *d_old_id, int
 #define PERM_WAVE 64
 #define PERM_BLOCK 4096
 // Row lengths of the result; word[0] (zeroed beforehand) = the longest over
-// PERM_WAVE, if any (an atomic per wave on one address is 43 us of its own).
+// PERM_WAVE, if any, word[1] = the number of such rows, listed in rows (in no
+// order).  (An atomic per wave on one address is 43 us of its own.)
 __global__ void __launch_bounds__(256)
 k_perm_counts(const int *__restrict__ rowptr, const int *__restrict__ row_old, int m, int *__restrict__ cnt,
-              int *__restrict__ word) {
+              int *__restrict__ word, int *__restrict__ rows) {
+    const int lane = threadIdx.x & 63;
     int mx = 0;
-    for (int r = blockIdx.x * 256 + threadIdx.x; r < m; r += gridDim.x * 256) {
-        const int c = rowptr[row_old[r] + 1] - rowptr[row_old[r]];
-        cnt[r] = c;
+    for (unsigned r0 = blockIdx.x * 256; r0 < (unsigned)m; r0 += gridDim.x * 256) {  // block-uniform
+        const unsigned r = r0 + threadIdx.x;
+        int c = 0;
+        if (r < (unsigned)m) {
+            c = rowptr[row_old[r] + 1] - rowptr[row_old[r]];
+            cnt[r] = c;
+        }
         mx = max(mx, c);
+        const unsigned long long b = __ballot(c > PERM_WAVE);
+        if (!b) continue;
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&word[1], __popcll(b));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (c > PERM_WAVE) rows[at + __popcll(b & ((1ull << lane) - 1ull))] = (int)r;
     }
     mx = tsg_wave_max(mx);
-    if ((threadIdx.x & 63) == 0 && mx > PERM_WAVE) atomicMax(&word[0], mx);
+    if (lane == 0 && mx > PERM_WAVE) atomicMax(&word[0], mx);
 }
-// Rows of at most PERM_WAVE entries: one wave per row, each entry's place by
-// counting the smaller columns.  Up to PERM_BLOCK: one block per row, bitonic
+// Rows of at most PERM_WAVE entries: each entry's place by counting the
+// smaller columns, one wave per row, or 16 lanes where rows have at most 16
+// entries on average (4,000,000 rows of one entry 2.43 -> 1.74 ms for the call,
+// 5-point 1500x1000 1.02 -> 0.77).  Longer ones, up to PERM_BLOCK: one block per
+// listed row (a block for every row: 3.51 / 1.74 ms with one row of 100), bitonic
 // sort in LDS.  A matrix with a longer row has all its entries sorted by
 // (row, column) with the radix sort (two words an entry, five passes and
 // more): 27-point 61x64x59 (5.9M entries) some 0.9 ms of kernels
@@ -794,37 +809,82 @@ k_perm_rows(const int *__restrict__ rowptr, const int *__restrict__ col, const d
     }
 }
 __global__ void __launch_bounds__(256)
+k_perm_rows16(const int *__restrict__ rowptr, const int *__restrict__ col, const double *__restrict__ val,
+              const int *__restrict__ row_old, const int *__restrict__ col_new, int m, const int *__restrict__ optr,
+              int *__restrict__ ocol, double *__restrict__ oval) {
+    constexpr int Q = PERM_WAVE / 16;  // entries of a lane
+    const unsigned r = tsg_block() * 16 + (threadIdx.x >> 4);
+    const int l = threadIdx.x & 15;
+    int e0 = 0, o0 = 0, n = 0;
+    if (r < (unsigned)m) {
+        e0 = rowptr[row_old[r]];
+        o0 = optr[r];
+        n = optr[r + 1] - o0;
+        if (n > PERM_WAVE) n = 0;
+    }
+    int c[Q], at[Q];
+    double v[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        c[q] = 0x7fffffff;
+        at[q] = 0;
+        v[q] = 0.0;
+        if (l + 16 * q < n) {
+            c[q] = col_new[col[e0 + l + 16 * q]];
+            v[q] = val[e0 + l + 16 * q];
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < Q; s++) {
+        if (!__any(n > 16 * s)) break;  // wave-uniform; every lane is active in the broadcasts
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const int x = tsg_row16_bcast(c[s], j);
+#pragma unroll
+            for (int q = 0; q < Q; q++) at[q] += x < c[q];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+        if (l + 16 * q < n) {
+            ocol[o0 + at[q]] = c[q];
+            oval[o0 + at[q]] = v[q];
+        }
+}
+__global__ void __launch_bounds__(256)
 k_perm_rows_block(const int *__restrict__ rowptr, const int *__restrict__ col, const double *__restrict__ val,
-                  const int *__restrict__ row_old, const int *__restrict__ col_new, int m, const int *__restrict__ optr,
-                  int *__restrict__ ocol, double *__restrict__ oval) {
+                  const int *__restrict__ row_old, const int *__restrict__ col_new, const int *__restrict__ rows, int nrows,
+                  const int *__restrict__ optr, int *__restrict__ ocol, double *__restrict__ oval) {
     __shared__ unsigned long long s_key[PERM_BLOCK];
-    const unsigned r = tsg_block(), tid = threadIdx.x;
-    if (r >= (unsigned)m) return;
-    const int e0 = rowptr[row_old[r]], o0 = optr[r], n = optr[r + 1] - o0;
-    if (n <= PERM_WAVE) return;  // block-uniform
-    int p2 = 2 * PERM_WAVE;
-    while (p2 < n) p2 <<= 1;
-    for (int i = tid; i < p2; i += 256)
-        s_key[i] = i < n ? ((unsigned long long)(unsigned)col_new[col[e0 + i]] << 32) | (unsigned)i : ~0ull;
-    __syncthreads();
-    for (int k = 2; k <= p2; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = tid; i < p2; i += 256) {
-                const int x = i ^ j;
-                if (x > i) {
-                    const unsigned long long a = s_key[i], b = s_key[x];
-                    if ((a > b) == ((i & k) == 0)) {
-                        s_key[i] = b;
-                        s_key[x] = a;
+    const int tid = threadIdx.x;
+    for (int w = blockIdx.x; w < nrows; w += gridDim.x) {
+        const int r = rows[w];
+        const int e0 = rowptr[row_old[r]], o0 = optr[r], n = optr[r + 1] - o0;
+        int p2 = 2 * PERM_WAVE;
+        while (p2 < n) p2 <<= 1;
+        for (int i = tid; i < p2; i += 256)
+            s_key[i] = i < n ? ((unsigned long long)(unsigned)col_new[col[e0 + i]] << 32) | (unsigned)i : ~0ull;
+        __syncthreads();
+        for (int k = 2; k <= p2; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int i = tid; i < p2; i += 256) {
+                    const int x = i ^ j;
+                    if (x > i) {
+                        const unsigned long long a = s_key[i], b = s_key[x];
+                        if ((a > b) == ((i & k) == 0)) {
+                            s_key[i] = b;
+                            s_key[x] = a;
+                        }
                     }
                 }
+                __syncthreads();
             }
-            __syncthreads();
+        for (int i = tid; i < n; i += 256) {
+            const unsigned long long key = s_key[i];
+            ocol[o0 + i] = (int)(key >> 32);
+            oval[o0 + i] = val[e0 + (int)(key & 0xffffffffu)];
         }
-    for (int i = tid; i < n; i += 256) {
-        const unsigned long long key = s_key[i];
-        ocol[o0 + i] = (int)(key >> 32);
-        oval[o0 + i] = val[e0 + (int)(key & 0xffffffffu)];
+        __syncthreads();  // the next row rewrites the keys
     }
 }
 __global__ void k_perm_emit(const int *__restrict__ rowptr, const int *__restrict__ col, const int *__restrict__ row_old,
@@ -861,26 +921,33 @@ extern "C" int tsg_dcsr_permute(tsg_ctx *ctx, const tsg_dcsr *a, const int *d_ro
     TSG_TRY(tsg_alloc_t(ctx, &out->rowptr, (size_t)m + 1));
     TSG_TRY(tsg_alloc_t(ctx, &out->colidx, (size_t)nnz + 1));
     TSG_TRY(tsg_alloc_t(ctx, &out->val, (size_t)nnz + 1));
-    int *word;
+    int *word, *rows;  // {longest row, rows of more than PERM_WAVE entries}, those rows
     TSG_TRY(tsg_alloc_t(ctx, &word, 4));
-    TSG_HIP(hipMemsetAsync(word, 0, 4, ctx->stream));
+    TSG_TRY(tsg_alloc_t(ctx, &rows, (size_t)nnz / (PERM_WAVE + 1) + 1));
+    TSG_HIP(hipMemsetAsync(word, 0, 8, ctx->stream));
     if (m > 0) {
         hipLaunchKernelGGL(k_perm_counts, dim3(std::min<unsigned>(1024, tsg_div_up(m, 256))), dim3(256), 0, ctx->stream,
-                           a->rowptr, d_row_old, m, out->rowptr, word);
+                           a->rowptr, d_row_old, m, out->rowptr, word, rows);
         TSG_LAUNCH_CHECK();
     }
     long long tot = 0;
-    const int sc = tsg_scan_i32(ctx, out->rowptr, out->rowptr, m, &tot, word, 1);
+    const int sc = tsg_scan_i32(ctx, out->rowptr, out->rowptr, m, &tot, word, 2);
+    const int longest = ((volatile int *)(ctx->pinned + 1))[0], nlong = ((volatile int *)(ctx->pinned + 1))[1];
     tsg_free(ctx, word);
+    tsg_free(ctx, rows);  // (what frees and allocates later is behind these kernels on the stream)
     TSG_TRY(sc);
-    const int longest = ((volatile int *)(ctx->pinned + 1))[0];
     if (tot != nnz) { tsg_set_error("permute: row permutation is not a bijection"); return TSG_ERR_ARG; }
     if (nnz > 0 && longest <= PERM_BLOCK) {
-        hipLaunchKernelGGL(k_perm_rows, tsg_grid(tsg_div_up(m, 4), 256), dim3(256), 0, ctx->stream, a->rowptr, a->colidx, a->val,
-                           d_row_old, d_col_new, m, out->rowptr, out->colidx, out->val);
-        if (longest > PERM_WAVE)
-            hipLaunchKernelGGL(k_perm_rows_block, tsg_grid(m, 256), dim3(256), 0, ctx->stream, a->rowptr, a->colidx,
+        if (nlong < m && nnz <= 16LL * m)
+            hipLaunchKernelGGL(k_perm_rows16, tsg_grid(tsg_div_up(m, 16), 256), dim3(256), 0, ctx->stream, a->rowptr, a->colidx,
                                a->val, d_row_old, d_col_new, m, out->rowptr, out->colidx, out->val);
+        else if (nlong < m)
+            hipLaunchKernelGGL(k_perm_rows, tsg_grid(tsg_div_up(m, 4), 256), dim3(256), 0, ctx->stream, a->rowptr, a->colidx,
+                               a->val, d_row_old, d_col_new, m, out->rowptr, out->colidx, out->val);
+        if (nlong > 0)
+            hipLaunchKernelGGL(k_perm_rows_block, dim3((unsigned)std::min(nlong, 1 << 16)), dim3(256), 0, ctx->stream,
+                               a->rowptr, a->colidx, a->val, d_row_old, d_col_new, (const int *)rows, nlong, out->rowptr,
+                               out->colidx, out->val);
         TSG_LAUNCH_CHECK();
     } else if (nnz > 0) {
         unsigned long long *key;

@@ -1,6 +1,7 @@
 """RCM of large sparse graphs whose lists are all short (few lanes a vertex):
 many components, chains, lists of the longest length that still counts as
-short and one more, vertices alone; against the oracle."""
+short and one more, vertices alone; permutation of matrices with 16 entries a
+row or fewer on average; against the oracle."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -65,4 +66,31 @@ def test_rcm_short_lists(ctx, name):
     order, _ = ctx.order_rcm(d)
     assert np.array_equal(order, oracle.rcm(a))
     ctx.free(g)
+    ctx.free(d)
+
+
+@pytest.mark.parametrize("longest,some", [(0, 0), (1, 1), (15, 3), (16, 9), (17, 9), (32, 40), (33, 40), (48, 7), (49, 7), (63, 5),
+                                          (64, 200), (65, 1), (65, 200), (4096, 3), (4097, 2)])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 700])
+def test_permute_short_rows(ctx, rows, longest, some):
+    """`some` rows of `longest` entries among rows of 0 to 6, a last row of any length among them."""
+    rng = np.random.default_rng(longest * 1000 + rows)
+    n = 4500
+    cnt = rng.integers(0, 7, rows)
+    cnt[rng.choice(rows, min(some, rows), replace=False)] = longest
+    cols = [np.sort(rng.choice(n, c, replace=False)) for c in cnt]
+    if longest:
+        for c in cols[-1:]:
+            c[-1:] = n - 1
+    a = ts.Csr(rows, n, np.r_[0, np.cumsum(cnt)], np.concatenate(cols), rng.uniform(-1, 1, int(cnt.sum())))
+    log(f"[permute] {rows} rows, nnz {a.nnz}, longest {cnt.max()}")
+    old, new = rng.permutation(rows).astype(np.int32), rng.permutation(n).astype(np.int32)
+    d = ctx.upload(a)
+    before = ctx.bytes_in_use()
+    p = ctx.permute(d, old, new)
+    got = ctx.download(p)
+    ref = oracle.permute_csr(a, old, new)
+    assert np.array_equal(got.rowptr, ref[0]) and np.array_equal(got.colidx, ref[1]) and np.array_equal(got.val, ref[2])
+    ctx.free(p)
+    assert ctx.bytes_in_use() == before
     ctx.free(d)
