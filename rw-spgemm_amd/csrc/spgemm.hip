@@ -1416,7 +1416,7 @@ __device__ __forceinline__ void step3_tile_body(const TileOperands &op, const in
     if (t >= numtileC) return;
     const int coff = Cnnz[t], cn = Cnnz[t + 1] - coff;
     if (cn == 0) return;  // structurally empty tile (step-1 phantom)
-    if (!all_rows && rowcls[Crow[t]] == 1) return;  // done by k_step3_rows
+    if (!all_rows && rowcls[Crow[t]] != 0) return;  // done by k_step3_rows or k_step3_lines
     const unsigned cm = Cmask[t * 16 + r];
     const int cp = Cptr16[t * 16 + r];
     const int rowlen = __popc(cm);
@@ -3105,14 +3105,15 @@ k_step3_lines(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
 // over class-1 rows of (nonempty C tiles, C nonzeros plus accumulator pads,
 // A tiles, B tiles per B tile-row, B nonzeros per B tile-row, A tile
 // nonzeros) for the LDS layout, i = 7..10 those over the row-lines rows of (C
-// nonzeros, C tiles, tile-column span, g + 1), i = 11 the rows of classes 0 and 1.
+// nonzeros, C tiles, tile-column span, g + 1), i = 11 the rows of classes 0 and
+// 1, i = 12 the element segments of the class-0 rows, at most.
 // 16 lanes per tile-row (16 tile-rows per block): the lanes walk the row's A
 // tiles and C tiles in strides of 16, so the dependent loads of different A
 // tiles are in flight together.  k_row_class_reduce folds the blocks' partials
 // into out (sums and maxima): no atomics, which on one cache
 // line would serialise across the thousands of blocks.
-#define CLS_WORDS 12
-__device__ __forceinline__ bool cls_sums(int i) { return i == 0 || i == 11; }
+#define CLS_WORDS 13
+__device__ __forceinline__ bool cls_sums(int i) { return i == 0 || i >= 11; }
 __device__ __forceinline__ int g16_max(int v) {
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 16));
@@ -3126,7 +3127,7 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
     const int r = threadIdx.x & 15, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int I = blockIdx.x * 16 + (threadIdx.x >> 4);
     int unfit = 0, mu = 0, mn = 0, ml = 0, mq = 0, mb = 0, ma = 0;
-    int ln = 0, lu = 0, ls = 0, lg = 0, other = 0;
+    int ln = 0, lu = 0, ls = 0, lg = 0, other = 0, segs = 0;
     if (I < tilem) {  // uniform in the 16-lane group
         const int c0 = Cptr[I], c1 = Cptr[I + 1];
         const int nrow = Cnnz[c1] - Cnnz[c0];
@@ -3185,9 +3186,11 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
         if (r == 0) cls[I] = k;
         unfit = r == 0 && k == 0;
         other = r == 0 && k <= 1;
+        segs = unfit ? nrow / (G3F_NNZ - 255) + 1 : 0;
     }
     unfit = tsg_wave_sum(unfit);
     other = tsg_wave_sum(other);
+    segs = tsg_wave_sum(segs);
     mu = tsg_wave_max(mu); mn = tsg_wave_max(mn); ml = tsg_wave_max(ml);
     mq = tsg_wave_max(mq); mb = tsg_wave_max(mb); ma = tsg_wave_max(ma);
     ln = tsg_wave_max(ln); lu = tsg_wave_max(lu); ls = tsg_wave_max(ls); lg = tsg_wave_max(lg);
@@ -3195,7 +3198,7 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
         s_red[wave][0] = unfit; s_red[wave][1] = mu; s_red[wave][2] = mn; s_red[wave][3] = ml;
         s_red[wave][4] = mq; s_red[wave][5] = mb; s_red[wave][6] = ma;
         s_red[wave][7] = ln; s_red[wave][8] = lu; s_red[wave][9] = ls; s_red[wave][10] = lg;
-        s_red[wave][11] = other;
+        s_red[wave][11] = other; s_red[wave][12] = segs;
     }
     __syncthreads();
     if (threadIdx.x < CLS_WORDS) {
@@ -3233,7 +3236,7 @@ k_row_class(TileOperands op, const int *__restrict__ Cptr, const int *__restrict
     }
 }
 
-// out = sums (words 0 and 11) and maxima of the nb blocks' k_row_class partials
+// out = sums (words 0, 11, 12) and maxima of the nb blocks' k_row_class partials
 // (one block of 1024 threads).  host (may be NULL): pinned memory that gets
 // the CLS_WORDS words too.
 __global__ void __launch_bounds__(1024)
@@ -3769,20 +3772,24 @@ static bool auto_index(const tsg_dtiles *t) {
     return t->csr_col && t->nnz >= AUTO_INDEX_NNZ && t->nnz >= AUTO_INDEX_TILE * (long long)t->numtile &&
            t->nnz <= AUTO_INDEX_ROW * (long long)t->m;
 }
-// Tiles dense enough, and few enough to a tile-row of A and a tile column of B,
-// for the tile kernels: what row lines do not take is better off there than
-// element by element (tiles of 28 entries and more, which meet in some 50
-// products), and the lines have to pay for the index alone.  Then it is made
-// after step 2, and only if nearly every tile-row would use it: beside a
-// tile kernel that runs anyway the lines' rows cost more than they save.
-// Index before step 1 and the rest element-wise / by tiles / this rule, A^2:
-// random tiles, 8 of 48 entries a tile-row, 0.63 / 0.37 / 0.35 ms, 12 of 40 0.77 / 0.53 /
-// 0.50; bands of half-width 20 (70% of the rows) and 100 1.14 / 1.23 / 1.12; of
-// half-width 40, all by lines, 0.40 / 0.40 / 0.41, without an index 0.48.  Random
-// tiles, 16 of 24 entries (not dense) element-wise 0.65, by tiles 0.78.
+// Tiles dense enough (28 entries and more, which meet in some 50 products), and
+// few enough to a tile-row of A and a tile column of B, that k_step3 is the
+// better one for many tile-rows that row lines do not take.  Then the index is
+// made after step 2, when the classes of the tile-rows are known: where at
+// least half go by lines and the rest is few enough to run at once as segments of
+// k_step3_flat (if C's tiles have several pairs: one of k_step3 is a chain of
+// them), or where seven in eight go by lines (and the rest by k_step3); else not at all.  A^2, index before
+// step 1 with the rest in segments / index after step 2 with the rest by k_step3 /
+// no index: bands of half-width 10 and 64, 20% of the rows wide (375 tile-rows,
+// 750 segments) 0.50 / 0.67 / 0.74 ms, 50% (1870 segments) 0.86 / 0.80 / 0.79; 12 and 70,
+// 60000 rows, 10% wide 0.61 / 0.91 / 1.06; 20 and 100, 30% wide (1690) 1.10 / 1.25 /
+// 1.11; random tiles, 8 of 48 entries a tile-row, none by lines, 0.63 / - / 0.35, within
+// 8 of the diagonal (1.9 pairs), most by lines, 0.37 / 0.29 / 0.38; 5 of 200 there (1.3
+// pairs) 0.40 / 0.39 / 0.33.
 #define AUTO_DENSE_TILE 28  // entries per tile, geometric mean of A and B
 #define AUTO_DENSE_LIST 16  // tiles per tile-row of A and per tile column of B
-#define AUTO_LINES(other, tilem) (32LL * (other) <= (tilem))
+#define AUTO_SEGMENTS 1536  // four blocks of k_step3_flat fit a CU
+#define AUTO_PAIRS 1.6      // per tile of C
 static bool auto_dense(const tsg_dtiles *A, const tsg_dtiles *B) {
     return (double)A->nnz * B->nnz >= (double)(AUTO_DENSE_TILE * AUTO_DENSE_TILE) * A->numtile * B->numtile &&
            A->numtile <= AUTO_DENSE_LIST * (long long)A->tilem && B->numtile <= AUTO_DENSE_LIST * (long long)B->tilen;
@@ -3866,7 +3873,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         }
         return TSG_OK;
     };
-    const bool index_later = may_index && auto_dense(A, B);
+    const bool index_later = may_index && !B->rowx_ptr && auto_dense(A, B);
     if (may_index && !index_later) TSG_TRY(index_operands());
     // element path: B carries its row index, and C's columns fit the
     // 28-bit entry keys of the element kernel's LDS hash
@@ -4002,9 +4009,12 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         if (classes && index_later && h[10] > 0) {  // some tile-rows would go by row lines
             int cls[CLS_WORDS];
             for (int i = 0; i < CLS_WORDS; i++) cls[i] = h[i];
-            if (AUTO_LINES(cls[11], C->tilem)) TSG_TRY(index_operands());
+            const double pairs = (double)A->numtile * B->numtile / std::max(1, B->tilen);
+            const bool few = 2LL * cls[11] <= C->tilem && cls[12] <= AUTO_SEGMENTS && pairs >= AUTO_PAIRS * numtileC;
+            if (few || 8LL * cls[11] <= C->tilem) TSG_TRY(index_operands());
             if (A->rowx_ptr && B->rowx_ptr) {
                 op = make_operands(A, B);
+                P.s3_elem = few;
                 for (int i = 0; i < CLS_WORDS; i++) ((int *)(pin + 1))[i] = cls[i];  // (making the index read back there)
             } else {
                 TSG_TRY(classify(nullptr, nullptr));

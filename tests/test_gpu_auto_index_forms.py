@@ -180,7 +180,8 @@ def dense_tiles(tile_rows, tiles, entries, seed=0):
 
 DENSE = {
     "all_by_lines": lambda: bands(30000, [40], [30000]),
-    "few_not": lambda: bands(30000, [20, 100, 20], [10000, 10300, 30000]),
+    "few_not": lambda: bands(30000, [20, 100, 20], [10000, 10300, 30000]),  # those as segments
+    "one_in_ten_not": lambda: bands(200000, [5, 70, 5], [50000, 70000, 200000]),  # those by tiles, beside the lines
     "half_not": lambda: bands(30000, [10, 64], [15000, 30000]),
     "none": lambda: dense_tiles(3000, 8, 48),
     "none_long_lists": lambda: dense_tiles(1500, 24, 32),
@@ -191,7 +192,7 @@ DENSE = {
 @pytest.mark.parametrize("index_a,index_b", [(False, False), (True, False), (False, True)])
 @pytest.mark.parametrize("name", list(DENSE))
 def test_dense_tiles(ctx, name, index_a, index_b):
-    """Tiles that meet in dozens of products: the index is made only where nearly all of C goes by row lines."""
+    """Tiles that meet in dozens of products: the index is made after step 2, or not, by what goes by row lines."""
     a = DENSE[name]()
     assert a.nnz >= 1 << 20 and a.nnz <= 96 * a.m
     log(f"[auto index] dense, {name}: nnz {a.nnz} index {index_a} {index_b}")
