@@ -52,11 +52,6 @@ extern "C" int tsg_ctx_create(int device, tsg_ctx **out) {
         delete c;
         return TSG_ERR_HIP;
     }
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
-        c->num_cu = prop.multiProcessorCount;
-        c->lds_per_block = prop.sharedMemPerBlock;
-    }
     *out = c;
     return TSG_OK;
 }

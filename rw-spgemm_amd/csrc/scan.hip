@@ -12,9 +12,8 @@
 // words of an earlier kernel's) in pinned host memory, so a read-back is a
 // stream wait with no copy behind the scan.  Against four launches (reduce,
 // partials, down, total) plus copies, whole products: 5-point 64^2 A^2 169
-// -> 108 us, 27d 61x47x53 651 -> 621 us, ER 65521 1.96 -> 1.92 ms; RCM of 27d
-// 61x64x59 (80 scans a BFS level) 22.2 -> 17.9 ms.  The two-launch form
-// re-reads at most 32 KB of partials per block from L2.
+// -> 108 us, 27d 61x47x53 651 -> 621 us, ER 65521 1.96 -> 1.92 ms.  The
+// two-launch form re-reads at most 32 KB of partials per block from L2.
 #include "tsg_internal.h"
 
 #define SCAN_THREADS 256
@@ -236,28 +235,5 @@ extern "C" int tsg_copy_kernel(tsg_ctx *ctx, void *dst, const void *src, size_t 
                            ctx->stream, (const uint4 *)src, (uint4 *)dst, n16);
         TSG_LAUNCH_CHECK();
     }
-    return TSG_OK;
-}
-
-__global__ void __launch_bounds__(256)
-k_reduce_u64(const unsigned long long *__restrict__ in, long long n, unsigned long long *out) {
-    unsigned long long s = 0;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) s += in[i];
-    s = tsg_wave_sum(s);
-    if ((threadIdx.x & 63) == 0) atomicAdd(out, s);
-}
-
-int tsg_reduce_u64(tsg_ctx *ctx, const unsigned long long *in, long long n, unsigned long long *out) {
-    void *scr;
-    TSG_TRY(tsg_scratch(ctx, 64, &scr));
-    TSG_HIP(hipMemsetAsync(scr, 0, 8, ctx->stream));
-    if (n > 0) {
-        unsigned nb = (unsigned)std::min<long long>((n + 255) / 256, 4096);
-        hipLaunchKernelGGL(k_reduce_u64, dim3(nb), dim3(256), 0, ctx->stream, in, n, (unsigned long long *)scr);
-        TSG_LAUNCH_CHECK();
-    }
-    long long t;
-    TSG_TRY(tsg_read_scalar_i64(ctx, scr, 1, &t));
-    *out = (unsigned long long)t;
     return TSG_OK;
 }

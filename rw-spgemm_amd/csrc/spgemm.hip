@@ -10,22 +10,25 @@
 //   k_step2_rows, one block per C tile-row, visits every (A tile, B tile)
 //   pair of the row once (no intersection search) and ORs the pair's
 //   boolean product rows into the C tile masks held in LDS; popcounts give
-//   the u8 row offsets and tile nnz.  Tile-rows with more C tiles than LDS
-//   holds use k_step2_tiles (one C tile per 16-lane group, pairs from a
-//   sorted-list intersection, 64-bit ballots to keep them in K order).
+//   the u8 row offsets and tile nnz; a tile-row with more C tiles than LDS
+//   holds is cut into segments.  With row indices, hypersparse and hub
+//   tile-rows go entry by entry instead (k_step2_elem, C tiles in a hash;
+//   k_step2_dense, the tile-row's columns as bits).  k_step2_tiles (one C tile
+//   per 16-lane group, pairs from a sorted-list intersection, 64-bit ballots
+//   to keep them in K order) takes all of C on request (force_tile_parallel).
 // Step 3 (numeric, src/tilespgemm-cuda.h:1505-2608): k_step3_lines, one block
 //   per C tile-row, adds B rows line by line (both row indices needed);
-//   without them k_step3_rows, one
-//   block per C tile-row, accumulates the row's C values in LDS in their
-//   final order; each C row belongs to one wave, which takes its tasks in
+//   tile-rows it does not take, and all without them, go by k_step3_rows if
+//   they fit it: one block per C tile-row accumulates the row's C values in
+//   LDS in their final order; each C row belongs to one wave, which takes its tasks in
 //   ascending K.  A tile K with several entries has A tile K and B tile-row
 //   K staged into LDS (software pipelined) and the (B tile, A row) tasks
 //   that meet nonempty B rows run compacted per wave; a single-entry A tile
-//   is handled by its row's wave from registers.  Hypersparse and hub rows
-//   use k_step3_elem / k_step3_heavy (B's row index); larger tile-rows
-//   otherwise use k_step3 (one C tile per
+//   is handled by its row's wave from registers.  The rest, hypersparse and
+//   hub rows mostly: k_step3_flat and k_step3_heavy with both row indices,
+//   k_step3_elem with B's alone, else k_step3 (one C tile per
 //   16-lane group, lane r owns tile row r, dense or compact LDS row
-//   accumulator).  No atomics anywhere: every C entry receives its
+//   accumulator).  No floating-point atomics: every C entry receives its
 //   products in ascending inner index k, the order of the serial SPA
 //   reference, so results are deterministic and bit-identical to it.  (The
 //   reference uses FP64 atomicAdd, src/tilespgemm-cuda.h:1670.)
@@ -1258,8 +1261,8 @@ k_step2_dense(const int *__restrict__ Arowp, const int *__restrict__ Acolx, int 
     }
 }
 
-// Tile-parallel step 2 for tile-rows with more than G2_UMAX C tiles: one C
-// tile per 16-lane group, pairs from the sorted-list intersection.
+// Tile-parallel step 2 (force_tile_parallel): one C tile per 16-lane group,
+// pairs from the sorted-list intersection.
 // Tile-parallel grids cover 16 work-items per C tile, which exceeds the
 // 2^32 work-items of a launch beyond 2^28 tiles: such kernels run at most
 // TP_MAX_BLOCKS blocks, each looping over virtual blocks.
@@ -1269,39 +1272,37 @@ static inline unsigned tp_grid(long long vblocks) {
     return (unsigned)std::min<long long>(std::max<long long>(vblocks, 1), TP_MAX_BLOCKS);
 }
 
-__device__ __forceinline__ void step2_tile_body(const TileOperands &op, const int *__restrict__ Cptr,
-                                                const int *__restrict__ Crow, const int *__restrict__ Ccol,
+__device__ __forceinline__ void step2_tile_body(const TileOperands &op, const int *__restrict__ Crow,
+                                                const int *__restrict__ Ccol,
                                                 int numtileC, unsigned short *__restrict__ Cmask,
                                                 unsigned char *__restrict__ Cptr16, int *__restrict__ Cnnz,
-                                                int all_rows, long long vblk, unsigned short *s_bm,
+                                                long long vblk, unsigned short *s_bm,
                                                 int (*s_la)[PAIR_LDS_MAX], int (*s_lb)[PAIR_LDS_MAX]);
 
 __global__ void __launch_bounds__(64 * S23_WAVES)
-k_step2_tiles(TileOperands op, const int *__restrict__ Cptr, const int *__restrict__ Crow,
-              const int *__restrict__ Ccol, int numtileC, unsigned short *__restrict__ Cmask,
-              unsigned char *__restrict__ Cptr16, int *__restrict__ Cnnz, int all_rows) {
+k_step2_tiles(TileOperands op, const int *__restrict__ Crow, const int *__restrict__ Ccol, int numtileC, unsigned short *__restrict__ Cmask,
+              unsigned char *__restrict__ Cptr16, int *__restrict__ Cnnz) {
     __shared__ unsigned short s_bm[S23_WAVES][64];
     __shared__ int s_la[S23_WAVES][TILES_PER_WAVE][PAIR_LDS_MAX];
     __shared__ int s_lb[S23_WAVES][TILES_PER_WAVE][PAIR_LDS_MAX];
     const int wave = threadIdx.x >> 6;
     const long long nvb = ((long long)numtileC + S23_WAVES * TILES_PER_WAVE - 1) / (S23_WAVES * TILES_PER_WAVE);
     for (long long vb = tsg_xcd_block(blockIdx.x, gridDim.x); vb < nvb; vb += gridDim.x)
-        step2_tile_body(op, Cptr, Crow, Ccol, numtileC, Cmask, Cptr16, Cnnz, all_rows, vb, s_bm[wave], s_la[wave],
+        step2_tile_body(op, Crow, Ccol, numtileC, Cmask, Cptr16, Cnnz, vb, s_bm[wave], s_la[wave],
                         s_lb[wave]);
 }
 
-__device__ __forceinline__ void step2_tile_body(const TileOperands &op, const int *__restrict__ Cptr,
-                                                const int *__restrict__ Crow, const int *__restrict__ Ccol,
+__device__ __forceinline__ void step2_tile_body(const TileOperands &op, const int *__restrict__ Crow,
+                                                const int *__restrict__ Ccol,
                                                 int numtileC, unsigned short *__restrict__ Cmask,
                                                 unsigned char *__restrict__ Cptr16, int *__restrict__ Cnnz,
-                                                int all_rows, long long vblk, unsigned short *s_bmw,
+                                                long long vblk, unsigned short *s_bmw,
                                                 int (*s_law)[PAIR_LDS_MAX], int (*s_lbw)[PAIR_LDS_MAX]) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = lane >> 4, r = lane & 15;
     const long long t = (vblk * S23_WAVES + wave) * TILES_PER_WAVE + g;
     if (t >= numtileC) return;  // whole groups exit together
     const int I = Crow[t], J = Ccol[t];
-    if (!all_rows && Cptr[I + 1] - Cptr[I] <= G2_UMAX) return;  // done by k_step2_rows
     unsigned short *bmg = &s_bmw[g * 16];
     unsigned orow = 0;
     for_each_pair(op, I, J, g, r, s_law[g], s_lbw[g], [&](int ta, int tb) {
@@ -1346,17 +1347,6 @@ k_bins(const int *__restrict__ cnt, long long n, int dense_min, unsigned long lo
     }
     __syncthreads();
     if (threadIdx.x < 3) atomicAdd(&bins[threadIdx.x], (unsigned long long)s[threadIdx.x]);
-}
-
-__global__ void __launch_bounds__(256)
-k_max_rowlen(const int *__restrict__ ptr, int n, int *__restrict__ out) {
-    int m = 0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) m = max(m, ptr[i + 1] - ptr[i]);
-    m = tsg_wave_max(m);
-    __shared__ int s[4];
-    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicMax(out, max(max(s[0], s[1]), max(s[2], s[3])));
 }
 
 // ------------------------------------------------------------------ step 3
@@ -3592,8 +3582,8 @@ static int launch_step2(hipStream_t s, const TileOperands &op, const tsg_dtiles 
     if (C->numtile <= 0) return TSG_OK;
     if (P.all) {
         const unsigned nblk = tp_grid(tsg_div_up(C->numtile, S23_WAVES * TILES_PER_WAVE));
-        hipLaunchKernelGGL(k_step2_tiles, dim3(nblk), dim3(64 * S23_WAVES), 0, s, op, C->tile_ptr, C->tile_rowidx,
-                           C->tile_colidx, C->numtile, C->mask, C->csr_ptr, C->tile_nnz, 1);
+        hipLaunchKernelGGL(k_step2_tiles, dim3(nblk), dim3(64 * S23_WAVES), 0, s, op, C->tile_rowidx, C->tile_colidx, C->numtile,
+                           C->mask, C->csr_ptr, C->tile_nnz);
         TSG_LAUNCH_CHECK();
         return TSG_OK;
     }

@@ -80,8 +80,6 @@ struct tsg_ctx {
     // persistent small device scratch (scan partials, counters)
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
-    int num_cu = 0;
-    size_t lds_per_block = 0;
     // pinned slots of large copies to the host, two per worker
     char *stage = nullptr;
     hipEvent_t stage_ev[2 * TSG_STAGE_WORKERS] = {};
@@ -131,10 +129,6 @@ struct tsg_scan_publish {
 long long tsg_scan_partial_count(long long n);
 int tsg_scan_i32_enqueue(hipStream_t stream, const int *in, int *out, long long n, long long *partial,
                          tsg_scan_publish pub = {});
-// Same for unsigned-char counts of 16-row tiles is done inside the kernels.
-// Sum of n int64 values (device) -> host.
-int tsg_reduce_u64(tsg_ctx *ctx, const unsigned long long *in, long long n,
-                   unsigned long long *out);
 
 // ------------------------------------------------------------------ spgemm
 // Decisions of one SpGEMM that depend only on the operand patterns (sizes
