@@ -1966,7 +1966,12 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 //   Where B row k's entries of a part start and end is read from a table
 // made once per product (k_heavy_windows), two groups of sources ahead, so no
 // search stands between the loads; blocks go part by part, which keeps the
-// parts' columns of B (and of the table) in the L2.
+// parts' columns of B (and of the table) in the L2.  A row's parts are those from
+// the first to the last that its tile-row reaches, and it has as many blocks as
+// twice the mean asks for, each taking its parts in strides of that: over all parts of
+// B a random band (1,000,000 rows, half-width 2000, 24 per row) had 244 million
+// blocks for 2.6 million with work, 118.5 ms, now 22.0; 128 diagonal blocks of ER
+// 8000 (24 per row) 125 -> 25.6, R-MAT scale 16 10.76 -> 10.78.
 //   14 KiB of LDS, eleven waves a CU.  Bound by products behind LDS round
 // trips and fragments of B rows (5.1 of 8.4 ms), scattered 8-byte stores (2)
 // and the walk over tiles (1.4).  R-MAT scale 16 A*A^T, heavy rows with the
@@ -2009,9 +2014,11 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 // Per C row of an element-wise tile-row: 2 heavy (more than min_products
 // products, or more than 2048 A entries), 1 long, 0 neither; cnt[0, m) and cnt[m,
 // 2m) take the heavy and the long rows as counts for the scan that numbers
-// them, info[0] the number of heavy ones, info[2..3] the
-// long tile-rows' entries of C.  A tile-row with many products for
-// its columns has only heavy and long rows and leaves the element-wise class.
+// them, info[0] the number of heavy ones, info[2] and [3] the long tile-rows'
+// entries of C and their number, info[4..5] the sum of the groups of parts they
+// reach, info[6..7] that of the parts which the heavy rows reach.  A tile-row
+// with many products for its columns has only heavy and long rows and leaves
+// the element-wise class.
 // One block per tile-row, 16 lanes per row, so that a long A row's B row
 // lengths are not one lane's chain of loads (R-MAT scale 16: 665 -> 92 us).
 __global__ void __launch_bounds__(256)
@@ -2050,22 +2057,32 @@ k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
         flag[i] = (unsigned char)h;
         cnt[i] = h == 2;
         cnt[m + i] = h == 1;
-        if (h == 2) atomicAdd(&info[0], 1);
+        if (h == 2) {
+            atomicAdd(&info[0], 1);
+            const int parts = Ccol[Cptr[I + 1] - 1] / HEAVY_PART_TILES - Ccol[Cptr[I]] / HEAVY_PART_TILES + 1;
+            atomicAdd(reinterpret_cast<unsigned long long *>(info + 6), (unsigned long long)parts);
+        }
         if (mine && (x1 - x0 > 2048 || p > count_products)) atomicAdd(&info[1], 1);
     }
     if (longer && threadIdx.x == 0) {
         rowcls[I] = CLS_LONG;
         // entries that need no segments
         atomicAdd(reinterpret_cast<unsigned long long *>(info + 2),
-                  (unsigned long long)(Cnnz[Cptr[I + 1]] - Cnnz[Cptr[I]]));
+                  1ULL << 32 | (unsigned)(Cnnz[Cptr[I + 1]] - Cnnz[Cptr[I]]));
+        const int parts = Ccol[Cptr[I + 1] - 1] / HEAVY_PART_TILES - Ccol[Cptr[I]] / HEAVY_PART_TILES + 1;
+        atomicAdd(reinterpret_cast<unsigned long long *>(info + 4), (unsigned long long)((parts + HEAVY_GROUP - 1) / HEAVY_GROUP));
     }
 }
 
-// rows = the heavy rows, then the long ones
+// rows = the heavy rows, then the long ones, each with the parts [y, z) that its
+// tile-row reaches
 __global__ void __launch_bounds__(256)
-k_heavy_list(const int *__restrict__ off, const unsigned char *__restrict__ flag, int m, int *__restrict__ rows) {
+k_heavy_list(const int *__restrict__ off, const unsigned char *__restrict__ flag, int m, const int *__restrict__ Cptr,
+             const int *__restrict__ Ccol, int4 *__restrict__ rows) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < m && flag[i]) rows[off[flag[i] == 2 ? i : m + i]] = i;
+    if (i >= m || !flag[i]) return;
+    rows[off[flag[i] == 2 ? i : m + i]] =
+        make_int4(i, Ccol[Cptr[i >> 4]] / HEAVY_PART_TILES, Ccol[Cptr[(i >> 4) + 1] - 1] / HEAVY_PART_TILES + 1, 0);
 }
 
 // win[w * m + k] = first entry of B row k at or past column w << shift, w = 0
@@ -2122,14 +2139,19 @@ __device__ __forceinline__ void add_in_rounds(double *sum, unsigned *bin, unsign
 // XCD some 40 ns (1,000,000 diagonal entries and one row of 3000, whose row alone
 // comes here, 977 parts: A^2 8.09 ms in 125,000 blocks, 7.54 in 977).
 __host__ __device__ inline int heavy_padded(int nrows) { return nrows < 128 ? nrows : (nrows + 127) & ~127; }
+// Long rows taken part by part together: all of them where they reach most of
+// B's parts, else this many (then neighbouring rows share B rows, not parts).
+// All / 1024: R-MAT scale 16 11.06 / 11.40 ms, block-diagonal ER (24 of 20000, 32 per
+// row) 21.1 / 19.2, random band (300,000 rows, half-width 4000, 64 per row) 14.6 / 14.5.
+#define LONG_CHUNK 1024
 #define HEAVY_ROUNDS 4
 #define HEAVY_BINS 256  // of add_in_rounds; products of different sums that share one only take a round more
 #define HEAVY_BATCH (64 * HEAVY_ROUNDS)
 __global__ void __launch_bounds__(64)
 k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const double *__restrict__ Avalx,
               const int *__restrict__ win, long long wstride, int nw, int shift, const int *__restrict__ Bcolx,
-              const double *__restrict__ Bvalx, const int *__restrict__ rows, int nheavy, int nlong,
-              long long heavy_blocks, long long first, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
+              const double *__restrict__ Bvalx, const int4 *__restrict__ rows, int nheavy, int nlong,
+              int hstep, int lstep, int lchunk, long long first, const int *__restrict__ Cptr, const int *__restrict__ Ccol,
               const unsigned short *__restrict__ Cmask, const unsigned char *__restrict__ Cptr16,
               const int *__restrict__ Cnnz, unsigned char *__restrict__ Ccol8, double *__restrict__ Cval) {
     __shared__ double s_acc[HEAVY_PART_COLS];
@@ -2138,173 +2160,183 @@ k_step3_heavy(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
     __shared__ unsigned s_mark[HEAVY_BATCH / 4];
     const int lane = threadIdx.x;
     unsigned char *mk = reinterpret_cast<unsigned char *>(s_mark);
-    // blocks: the heavy rows' items, then the long rows'; part by part, 16 rows
-    // of the list on one XCD (blocks go to the 8 XCDs in turn), the next 16 on the
-    // next
-    const long long hb = first + blockIdx.x;
+    // blocks: the heavy rows' items, part by part of each row's own, then the long
+    // rows', lchunk rows after the others; 16 rows of the list on one XCD (blocks go
+    // to the 8 XCDs in turn), the next 16 on the next
+    const long long hb = first + blockIdx.x, heavy_blocks = heavy_padded(nheavy) * (long long)hstep;
     const bool heavy = hb < heavy_blocks;
     const long long h = heavy ? hb : hb - heavy_blocks;
     const int nrows = heavy ? nheavy : nlong, padded = heavy_padded(nrows), group = heavy ? 1 : HEAVY_GROUP;
-    const int p0 = (int)(h / padded) * group, x = (int)(h % padded);
+    const int step = heavy ? hstep : lstep;
+    int chunk = 0, in_chunk = padded;
+    if (!heavy && lchunk < padded) {
+        chunk = (int)(h / ((long long)lchunk * step)) * lchunk;
+        in_chunk = min(lchunk, padded - chunk);
+    }
+    const long long at = h - (long long)chunk * step, g = at / in_chunk;
+    const int x = chunk + (int)(at - g * in_chunk);
     int j0 = nrows < 128 ? x : ((x >> 7) * 8 + (x & 7)) * 16 + ((x >> 3) & 15);
     if (j0 >= nrows) return;
     if (!heavy) j0 += nheavy;
-    const int i = rows[j0], I = i >> 4, r = i & 15;
-    const int c0 = Cptr[I], c1 = Cptr[I + 1];
+    const int4 row = rows[j0];
+    const int i = row.x, I = i >> 4, r = i & 15;
+    const int c1 = Cptr[I + 1];
     const int xa = Arowp[i], xe = Arowp[i + 1];
-    int t = wave_lower_bound(Ccol, c0, c1, p0 * HEAVY_PART_TILES, lane);
-    const int tend = wave_lower_bound(Ccol, t, c1, (p0 + group) * HEAVY_PART_TILES, lane);
     unsigned stamp = 0u;
     auto clear_bins = [&]() {
         for (int j = lane; j < HEAVY_BINS; j += 64) s_bin[j] = 0xffffffffu;
         stamp = 0xffffffc0u;
     };
-    while (t < tend) {
-        // a run of parts: as many as their entries of the row fit s_acc (one always does)
-        const int ps = Ccol[t] / HEAVY_PART_TILES, jb = ps * HEAVY_PART_TILES;
-        int pe = p0 + group, te = tend, nn = 0;
-        for (int tb = t; tb < te && nn <= HEAVY_PART_COLS; tb += 256) {
-            int J[4];
-            unsigned cm[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int tt = tb + 64 * v + lane, ti = min(tt, te - 1);
-                J[v] = Ccol[ti];
-                cm[v] = Cmask[(long long)ti * 16 + r];
-                if (tt >= te) cm[v] = 0u;
-            }
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if (nn > HEAVY_PART_COLS) break;  // wave-uniform
-                const int c = __popc(cm[v]), incl = tsg_wave_incl_scan_dpp(c);
-                if (cm[v]) s_word[J[v] - jb] = cm[v] << 15 | (unsigned)(nn + incl - c);
-                const unsigned long long over = __ballot(nn + incl > HEAVY_PART_COLS);
-                if (over) {  // the run ends before this tile's part
-                    pe = __builtin_amdgcn_readlane(J[v], __ffsll((long long)over) - 1) / HEAVY_PART_TILES;
-                    nn = HEAVY_PART_COLS + 1;
-                } else {
-                    nn += __builtin_amdgcn_readlane(incl, 63);
+    for (int p0 = row.y + (int)g * group, tend = Cptr[I]; p0 < row.z; p0 += step * group) {
+        int t = wave_lower_bound(Ccol, tend, c1, p0 * HEAVY_PART_TILES, lane);
+        tend = wave_lower_bound(Ccol, t, c1, (p0 + group) * HEAVY_PART_TILES, lane);
+        while (t < tend) {
+            // a run of parts: as many as their entries of the row fit s_acc (one always does)
+            const int ps = Ccol[t] / HEAVY_PART_TILES, jb = ps * HEAVY_PART_TILES;
+            int pe = p0 + group, te = tend, nn = 0;
+            for (int tb = t; tb < te && nn <= HEAVY_PART_COLS; tb += 256) {
+                int J[4];
+                unsigned cm[4];
+    #pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int tt = tb + 64 * v + lane, ti = min(tt, te - 1);
+                    J[v] = Ccol[ti];
+                    cm[v] = Cmask[(long long)ti * 16 + r];
+                    if (tt >= te) cm[v] = 0u;
                 }
-            }
-        }
-        if (nn > HEAVY_PART_COLS) {
-            te = wave_lower_bound(Ccol, t, te, pe * HEAVY_PART_TILES, lane);
-            nn = HEAVY_PART_COLS;
-        }
-        if (nn == 0) {  // other rows' tiles
-            t = te;
-            continue;
-        }
-        const int lo = ps << HEAVY_PART_LOG, hi = pe << HEAVY_PART_LOG;  // columns (n <= 2^27)
-        // sources (A entries) 64 at a time, lane q's B row in the run's windows:
-        // the entries two groups ahead, their windows one group ahead
-        const long long w0 = (long long)(lo >> shift) * wstride;
-        const long long w1 = (long long)min(((hi - 1) >> shift) + 1, nw) * wstride;
-        const int inside = (int)((1u << shift) - 1u);
-        const bool cut_lo = (lo & inside) != 0, cut_hi = (hi & inside) != 0;
-        int k1 = 0, n0 = 0, n1 = 0;
-        double a1 = 0.0, a2 = 0.0;
-        auto fetch = [&](int xc) {
-            k1 = -1;
-            a2 = 0.0;
-            if (xc + lane < xe) {
-                k1 = Acolx[xc + lane];
-                a2 = Avalx[xc + lane];
-            }
-        };
-        auto window = [&]() {
-            n0 = n1 = 0;
-            if (k1 >= 0) {
-                n0 = win[w0 + k1];
-                n1 = win[w1 + k1];
-            }
-            a1 = a2;
-        };
-        fetch(xa);
-        window();
-        fetch(xa + 64);
-        for (int j = lane; j < nn; j += 64) s_acc[j] = 0.0;
-        for (int xc = xa; xc < xe; xc += 64) {
-            int b0 = n0, b1 = n1;
-            const double a = a1;
-            window();
-            fetch(xc + 128);
-            if (cut_lo || cut_hi) range_in(Bcolx, b0, b1, cut_lo, lo, cut_hi, hi);  // windows wider than parts
-            const int len = b1 - b0;
-            const int incl = tsg_wave_incl_scan_dpp(len), pre = incl - len, delta = b0 - pre;
-            const int total = __builtin_amdgcn_readlane(incl, 63);
-            int prev = 0;
-            for (int base = 0; base < total; base += HEAVY_BATCH) {
-#pragma unroll
-                for (int v = 0; v < HEAVY_BATCH / 256; v++) s_mark[64 * v + lane] = 0u;
-                if (stamp < 1u << 20) clear_bins();  // a batch has at most 64 * HEAVY_ROUNDS rounds
-                tsg_wave_sync();
-                if (len > 0 && pre >= base && pre < base + HEAVY_BATCH) mk[pre - base] = (unsigned char)(lane + 1);
-                tsg_wave_sync();
-                int q[HEAVY_ROUNDS], col[HEAVY_ROUNDS];
-                double b[HEAVY_ROUNDS];
-#pragma unroll
-                for (int v = 0; v < HEAVY_ROUNDS; v++) {
-                    q[v] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * v + lane]));
-                    prev = __builtin_amdgcn_readlane(q[v], 63);
-                }
-#pragma unroll
-                for (int v = 0; v < HEAVY_ROUNDS; v++) {  // every lane loads in bounds
-                    const int e = __shfl(delta, q[v] - 1, 64) + min(base + 64 * v + lane, total - 1);
-                    col[v] = Bcolx[e];
-                    b[v] = Bvalx[e];
-                }
-                // all rounds' places before the first sum changes: their reads are in
-                // flight together
-                double as[HEAVY_ROUNDS];
-                unsigned wd[HEAVY_ROUNDS];
-#pragma unroll
-                for (int v = 0; v < HEAVY_ROUNDS; v++) as[v] = __shfl(a, q[v] - 1, 64);
-#pragma unroll
-                for (int v = 0; v < HEAVY_ROUNDS; v++) wd[v] = s_word[(col[v] >> 4) - jb];
-#pragma unroll
-                for (int v = 0; v < HEAVY_ROUNDS; v++) {
-                    if (base + 64 * v >= total) break;  // wave-uniform
-                    const bool on = base + 64 * v + lane < total;
-                    const int p = (int)(wd[v] & 0x7fffu) + __popc(wd[v] >> (31 - (col[v] & 15)));
-                    if (__builtin_amdgcn_readlane(q[v], 0) == __builtin_amdgcn_readlane(q[v], 63)) {  // one source
-                        if (on) s_acc[p] = __builtin_fma(as[v], b[v], s_acc[p]);
-                        tsg_wave_sync();
+    #pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    if (nn > HEAVY_PART_COLS) break;  // wave-uniform
+                    const int c = __popc(cm[v]), incl = tsg_wave_incl_scan_dpp(c);
+                    if (cm[v]) s_word[J[v] - jb] = cm[v] << 15 | (unsigned)(nn + incl - c);
+                    const unsigned long long over = __ballot(nn + incl > HEAVY_PART_COLS);
+                    if (over) {  // the run ends before this tile's part
+                        pe = __builtin_amdgcn_readlane(J[v], __ffsll((long long)over) - 1) / HEAVY_PART_TILES;
+                        nn = HEAVY_PART_COLS + 1;
                     } else {
-                        add_in_rounds(s_acc + p, s_bin + (p & (HEAVY_BINS - 1)), stamp, on, lane, as[v], b[v]);
+                        nn += __builtin_amdgcn_readlane(incl, 63);
                     }
                 }
             }
-        }
-        // the run's entries of row i, into their final positions
-        for (int tb = t; tb < te; tb += 256) {
-            int J[4], at[4];
-            unsigned wd[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int ti = min(tb + 64 * v + lane, te - 1);
-                J[v] = Ccol[ti];
-                wd[v] = Cmask[(long long)ti * 16 + r];
-                at[v] = Cnnz[ti] + Cptr16[(long long)ti * 16 + r];
-                if (tb + 64 * v + lane >= te) wd[v] = 0u;
+            if (nn > HEAVY_PART_COLS) {
+                te = wave_lower_bound(Ccol, t, te, pe * HEAVY_PART_TILES, lane);
+                nn = HEAVY_PART_COLS;
             }
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                unsigned cm = wd[v] << 16;
-                if (!cm) continue;
-                const double *d = s_acc + (s_word[J[v] - jb] & 0x7fffu);
-                double *o = Cval + at[v];
-                unsigned char *oc = Ccol8 + at[v];
-                while (cm) {
-                    const int c = __clz((int)cm);
-                    cm &= ~(0x80000000u >> c);
-                    *o++ = *d++;
-                    *oc++ = (unsigned char)c;
+            if (nn == 0) {  // other rows' tiles
+                t = te;
+                continue;
+            }
+            const int lo = ps << HEAVY_PART_LOG, hi = pe << HEAVY_PART_LOG;  // columns (n <= 2^27)
+            // sources (A entries) 64 at a time, lane q's B row in the run's windows:
+            // the entries two groups ahead, their windows one group ahead
+            const long long w0 = (long long)(lo >> shift) * wstride;
+            const long long w1 = (long long)min(((hi - 1) >> shift) + 1, nw) * wstride;
+            const int inside = (int)((1u << shift) - 1u);
+            const bool cut_lo = (lo & inside) != 0, cut_hi = (hi & inside) != 0;
+            int k1 = 0, n0 = 0, n1 = 0;
+            double a1 = 0.0, a2 = 0.0;
+            auto fetch = [&](int xc) {
+                k1 = -1;
+                a2 = 0.0;
+                if (xc + lane < xe) {
+                    k1 = Acolx[xc + lane];
+                    a2 = Avalx[xc + lane];
+                }
+            };
+            auto window = [&]() {
+                n0 = n1 = 0;
+                if (k1 >= 0) {
+                    n0 = win[w0 + k1];
+                    n1 = win[w1 + k1];
+                }
+                a1 = a2;
+            };
+            fetch(xa);
+            window();
+            fetch(xa + 64);
+            for (int j = lane; j < nn; j += 64) s_acc[j] = 0.0;
+            for (int xc = xa; xc < xe; xc += 64) {
+                int b0 = n0, b1 = n1;
+                const double a = a1;
+                window();
+                fetch(xc + 128);
+                if (cut_lo || cut_hi) range_in(Bcolx, b0, b1, cut_lo, lo, cut_hi, hi);  // windows wider than parts
+                const int len = b1 - b0;
+                const int incl = tsg_wave_incl_scan_dpp(len), pre = incl - len, delta = b0 - pre;
+                const int total = __builtin_amdgcn_readlane(incl, 63);
+                int prev = 0;
+                for (int base = 0; base < total; base += HEAVY_BATCH) {
+    #pragma unroll
+                    for (int v = 0; v < HEAVY_BATCH / 256; v++) s_mark[64 * v + lane] = 0u;
+                    if (stamp < 1u << 20) clear_bins();  // a batch has at most 64 * HEAVY_ROUNDS rounds
+                    tsg_wave_sync();
+                    if (len > 0 && pre >= base && pre < base + HEAVY_BATCH) mk[pre - base] = (unsigned char)(lane + 1);
+                    tsg_wave_sync();
+                    int q[HEAVY_ROUNDS], col[HEAVY_ROUNDS];
+                    double b[HEAVY_ROUNDS];
+    #pragma unroll
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) {
+                        q[v] = max(prev, tsg_wave_incl_max_dpp((int)mk[64 * v + lane]));
+                        prev = __builtin_amdgcn_readlane(q[v], 63);
+                    }
+    #pragma unroll
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) {  // every lane loads in bounds
+                        const int e = __shfl(delta, q[v] - 1, 64) + min(base + 64 * v + lane, total - 1);
+                        col[v] = Bcolx[e];
+                        b[v] = Bvalx[e];
+                    }
+                    // all rounds' places before the first sum changes: their reads are in
+                    // flight together
+                    double as[HEAVY_ROUNDS];
+                    unsigned wd[HEAVY_ROUNDS];
+    #pragma unroll
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) as[v] = __shfl(a, q[v] - 1, 64);
+    #pragma unroll
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) wd[v] = s_word[(col[v] >> 4) - jb];
+    #pragma unroll
+                    for (int v = 0; v < HEAVY_ROUNDS; v++) {
+                        if (base + 64 * v >= total) break;  // wave-uniform
+                        const bool on = base + 64 * v + lane < total;
+                        const int p = (int)(wd[v] & 0x7fffu) + __popc(wd[v] >> (31 - (col[v] & 15)));
+                        if (__builtin_amdgcn_readlane(q[v], 0) == __builtin_amdgcn_readlane(q[v], 63)) {  // one source
+                            if (on) s_acc[p] = __builtin_fma(as[v], b[v], s_acc[p]);
+                            tsg_wave_sync();
+                        } else {
+                            add_in_rounds(s_acc + p, s_bin + (p & (HEAVY_BINS - 1)), stamp, on, lane, as[v], b[v]);
+                        }
+                    }
                 }
             }
+            // the run's entries of row i, into their final positions
+            for (int tb = t; tb < te; tb += 256) {
+                int J[4], at[4];
+                unsigned wd[4];
+    #pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int ti = min(tb + 64 * v + lane, te - 1);
+                    J[v] = Ccol[ti];
+                    wd[v] = Cmask[(long long)ti * 16 + r];
+                    at[v] = Cnnz[ti] + Cptr16[(long long)ti * 16 + r];
+                    if (tb + 64 * v + lane >= te) wd[v] = 0u;
+                }
+    #pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    unsigned cm = wd[v] << 16;
+                    if (!cm) continue;
+                    const double *d = s_acc + (s_word[J[v] - jb] & 0x7fffu);
+                    double *o = Cval + at[v];
+                    unsigned char *oc = Ccol8 + at[v];
+                    while (cm) {
+                        const int c = __clz((int)cm);
+                        cm &= ~(0x80000000u >> c);
+                        *o++ = *d++;
+                        *oc++ = (unsigned char)c;
+                    }
+                }
+            }
+            t = te;
+            tsg_wave_sync();  // the next run clears the sums
         }
-        t = te;
-        tsg_wave_sync();  // the next run clears the sums
     }
 }
 
@@ -3497,8 +3529,10 @@ struct SpgemmWork {
     long long seg3_cap;
     // heavy rows (synchronous pipeline only; NULL = none)
     unsigned char *hflag;  // per C row
-    int *hrows;            // the heavy rows
+    int4 *hrows;           // the heavy rows, the long ones
     int nheavy, nlong, ncounted;
+    int hstep, lstep;      // blocks of a heavy row, of a long one
+    int lchunk;            // long rows taken part by part together
     const int *hwin;       // B rows' window table (k_heavy_windows), its stride and shift
     long long hstride, hwin_bytes;
     int hnw, hshift;
@@ -3552,7 +3586,7 @@ static SpgemmWork work_at(void *base, long long tilem, long long numtile, long l
     w.seg3_cap = tilem + nnz / (G3E_NNZ - 255) + 2;
     w.hflag = nullptr;
     w.hrows = nullptr;
-    w.nheavy = w.nlong = w.ncounted = w.hnw = w.hshift = 0;
+    w.nheavy = w.nlong = w.ncounted = w.hstep = w.lstep = w.lchunk = w.hnw = w.hshift = 0;
     w.hwin = nullptr;
     w.hstride = w.hwin_bytes = 0;
     return w;
@@ -3687,14 +3721,12 @@ static int launch_step3(hipStream_t s, const TileOperands &op, const tsg_dtiles 
                                C->tile_nnz, C->csr_col, C->val);
         TSG_LAUNCH_CHECK();
         if (w.hflag) {
-            const long long parts = ((long long)B->n + HEAVY_PART_COLS - 1) / HEAVY_PART_COLS;
-            const long long hb = heavy_padded(w.nheavy) * parts;
-            const long long total = hb + heavy_padded(w.nlong) * ((parts + HEAVY_GROUP - 1) / HEAVY_GROUP);
+            const long long total = heavy_padded(w.nheavy) * (long long)w.hstep + heavy_padded(w.nlong) * (long long)w.lstep;
             for (long long at = 0; at < total; at += 1 << 25) {  // a launch takes fewer than 2^32 threads
                 hipLaunchKernelGGL(k_step3_heavy, dim3((unsigned)std::min(total - at, 1LL << 25)), dim3(64), 0, s,
                                    op.Arowp, op.Acolx, op.Avalx, w.hwin, w.hstride, w.hnw, w.hshift,
-                                   (const int *)B->rowx_col, (const double *)B->rowx_val, (const int *)w.hrows,
-                                   w.nheavy, w.nlong, hb, at, C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
+                                   (const int *)B->rowx_col, (const double *)B->rowx_val, (const int4 *)w.hrows,
+                                   w.nheavy, w.nlong, w.hstep, w.lstep, w.lchunk, at, C->tile_ptr, C->tile_colidx, C->mask, C->csr_ptr,
                                    C->tile_nnz, C->csr_col, C->val);
                 TSG_LAUNCH_CHECK();
             }
@@ -3726,7 +3758,7 @@ struct SpgemmTemps {
     void *scr = nullptr, *wbuf = nullptr, *w3buf = nullptr, *bb = nullptr;
     unsigned char *hflag = nullptr;
     int *hcnt = nullptr, *hinfo = nullptr, *hwin = nullptr, *span = nullptr, *longest = nullptr;
-    int *hrows = nullptr;
+    int4 *hrows = nullptr;
     tsg_dcsr rowx[2] = {};
     hipEvent_t ev[6] = {};
     int nev = 0;
@@ -4037,8 +4069,8 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                 const int m = C->m;
                 TSG_TRY(tsg_alloc_t(ctx, &T.hflag, (size_t)m + 16));
                 TSG_TRY(tsg_alloc_t(ctx, &T.hcnt, 2 * (size_t)m + 1));
-                TSG_TRY(tsg_alloc_t(ctx, &T.hinfo, 4));
-                TSG_HIP(hipMemsetAsync(T.hinfo, 0, 16, s));
+                TSG_TRY(tsg_alloc_t(ctx, &T.hinfo, 8));
+                TSG_HIP(hipMemsetAsync(T.hinfo, 0, 32, s));
                 const long long counted = tune.heavy_min_products > 0 ? tune.heavy_min_products : HEAVY_MIN_PRODUCTS;
                 const bool large = nnzC >= LONG_MIN_NNZ;
                 const long long split = tune.heavy_min_products > 0 || !large
@@ -4050,16 +4082,18 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                                    large || tune.heavy_min_products > 0 ? 1 : 0, T.hflag, T.hcnt, T.hinfo);
                 TSG_LAUNCH_CHECK();
                 long long nh = 0;
-                TSG_TRY(tsg_scan_i32(ctx, T.hcnt, T.hcnt, 2LL * m, &nh, T.hinfo, 4));
+                TSG_TRY(tsg_scan_i32(ctx, T.hcnt, T.hcnt, 2LL * m, &nh, T.hinfo, 8));
                 const volatile int *info = (const volatile int *)(ctx->pinned + 1);
                 const int nheavy = info[0];
                 w.ncounted = info[1];
-                const long long done = (unsigned)info[2] | (long long)info[3] << 32;
+                const long long done = (unsigned)info[2], ntl = info[3];
+                const long long groups = (unsigned)info[4] | (long long)info[5] << 32;
+                const long long parts = (unsigned)info[6] | (long long)info[7] << 32;
                 w.seg3_cap = C->tilem + (nnzC - done) / (G3E_NNZ - 255) + 2;  // blocks: those past the segments only end
                 if (nh > 0) {
                     TSG_TRY(tsg_alloc_t(ctx, &T.hrows, (size_t)nh));
                     hipLaunchKernelGGL(k_heavy_list, dim3(tsg_div_up(m, 256)), dim3(256), 0, s, (const int *)T.hcnt,
-                                       (const unsigned char *)T.hflag, m, T.hrows);
+                                       (const unsigned char *)T.hflag, m, C->tile_ptr, C->tile_colidx, T.hrows);
                     TSG_LAUNCH_CHECK();
                     // the narrowest windows whose table is small enough; one window is B's row pointers
                     int shift = HEAVY_PART_LOG;
@@ -4079,6 +4113,11 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
                     w.hrows = T.hrows;
                     w.nheavy = nheavy;
                     w.nlong = (int)nh - nheavy;
+                    // twice the mean; a row with more takes several a block
+                    const long long most = ((long long)B->n + HEAVY_PART_COLS - 1) / HEAVY_PART_COLS;
+                    w.hstep = (int)std::min(most, 2 * (parts / std::max(nheavy, 1) + 1));
+                    w.lstep = (int)std::min((most + HEAVY_GROUP - 1) / HEAVY_GROUP, 2 * (groups / std::max(ntl, 1LL) + 1));
+                    w.lchunk = w.lstep * HEAVY_GROUP >= most ? heavy_padded(w.nlong) : LONG_CHUNK;
                     w.hnw = (int)nw;
                     w.hshift = nw > 1 ? shift : 31;
                     w.hstride = nw > 1 ? B->m : 1;
@@ -4113,7 +4152,7 @@ static int spgemm_run(tsg_ctx *ctx, const tsg_dtiles *A, const tsg_dtiles *B, co
         stats->numtileC = numtileC;
         stats->nnzC = nnzC;
         stats->heavy_rows = w.ncounted;
-        stats->heavy_bytes = w.hwin_bytes + (w.hflag ? 9LL * C->m + 4LL * ((long long)w.nheavy + w.nlong) : 0);
+        stats->heavy_bytes = w.hwin_bytes + (w.hflag ? 9LL * C->m + 16LL * ((long long)w.nheavy + w.nlong) : 0);
     }
     if (plan_out) *plan_out = P;
     return TSG_OK;
