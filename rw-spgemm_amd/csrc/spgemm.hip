@@ -2052,26 +2052,31 @@ k_heavy_flags(const int *__restrict__ Arowp, const int *__restrict__ Acolx, cons
         const int span = Ccol[Cptr[I + 1] - 1] - Ccol[Cptr[I]] + 1;  // tile columns
         longer = all * (HEAVY_GROUP * HEAVY_PART_TILES) > 16LL * LONG_PER_GROUP * span;
     }
+    const int h = !mine ? 0 : x1 - x0 > 2048 || p > min_products ? 2 : longer && p > 0 ? 1 : 0;
     if (i < m && l == 0) {
-        const int h = !mine ? 0 : x1 - x0 > 2048 || p > min_products ? 2 : longer && p > 0 ? 1 : 0;
         flag[i] = (unsigned char)h;
         cnt[i] = h == 2;
         cnt[m + i] = h == 1;
-        if (h == 2) {
-            atomicAdd(&info[0], 1);
-            const int parts = Ccol[Cptr[I + 1] - 1] / HEAVY_PART_TILES - Ccol[Cptr[I]] / HEAVY_PART_TILES + 1;
-            atomicAdd(reinterpret_cast<unsigned long long *>(info + 6), (unsigned long long)parts);
-        }
-        if (mine && (x1 - x0 > 2048 || p > count_products)) atomicAdd(&info[1], 1);
     }
-    if (longer && threadIdx.x == 0) {
-        rowcls[I] = CLS_LONG;
-        // entries that need no segments
-        atomicAdd(reinterpret_cast<unsigned long long *>(info + 2),
-                  1ULL << 32 | (unsigned)(Cnnz[Cptr[I + 1]] - Cnnz[Cptr[I]]));
+    if (!mine) return;  // block-uniform
+    // the block's share of info, which every block adds to: one atomic a word
+    const int heavy = __syncthreads_count(l == 0 && h == 2);
+    const int counted = __syncthreads_count(l == 0 && (x1 - x0 > 2048 || p > count_products));
+    if (threadIdx.x == 0 && (heavy || longer)) {
         const int parts = Ccol[Cptr[I + 1] - 1] / HEAVY_PART_TILES - Ccol[Cptr[I]] / HEAVY_PART_TILES + 1;
-        atomicAdd(reinterpret_cast<unsigned long long *>(info + 4), (unsigned long long)((parts + HEAVY_GROUP - 1) / HEAVY_GROUP));
+        unsigned long long *sums = reinterpret_cast<unsigned long long *>(info + 2);
+        if (longer) {
+            rowcls[I] = CLS_LONG;
+            // entries that need no segments
+            atomicAdd(sums, 1ULL << 32 | (unsigned)(Cnnz[Cptr[I + 1]] - Cnnz[Cptr[I]]));
+            atomicAdd(sums + 1, (unsigned long long)((parts + HEAVY_GROUP - 1) / HEAVY_GROUP));
+        }
+        if (heavy) {
+            atomicAdd(&info[0], heavy);
+            atomicAdd(sums + 2, (unsigned long long)heavy * parts);
+        }
     }
+    if (threadIdx.x == 0 && counted) atomicAdd(&info[1], counted);
 }
 
 // rows = the heavy rows, then the long ones, each with the parts [y, z) that its
