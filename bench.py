@@ -24,18 +24,17 @@ METRIC = "SpGEMM GFLOPS (A², 27-pt 128³); batched/served solves/s + p99 latenc
 HBM_PEAK_GBS = 8000.0
 
 
-def step3_algorithmic_bytes(ta, tc_numtile, tc_nnz, tilen):
-    """Compulsory bytes of one numeric-step launch (the dominant kernel):
-    read A once and B once in tile format (B aliases A for A^2 but is
-    counted again), read the CSC tile index, read C's step-2 outputs
-    (row/col tile index, tile offsets, u8 row offsets, masks), write C's
-    values and in-tile columns."""
-    T, nnz, tilem = ta.numtile, ta.nnz, ta.tilem
-    a_bytes = 4 * (tilem + 1) + 4 * T + 4 * (T + 1) + 8 * nnz + 16 * T + 32 * T
-    b_bytes = a_bytes + 4 * (tilen + 1) + 4 * T + 4 * T
-    c_meta = 4 * tc_numtile * 2 + 4 * (tc_numtile + 1) + 16 * tc_numtile + 32 * tc_numtile
-    c_write = 9 * tc_nnz
-    return a_bytes + b_bytes + c_meta + c_write
+def step3_algorithmic_bytes(a, b_rows, tilem, numtile_c, nnz_c):
+    """Compulsory bytes of one launch of the numeric kernel of the headline
+    product (k_step3_lines, every tile-row): the row indices of A and of B
+    (row pointers, column and value of every entry; B is A for A^2 but is
+    counted again), C's step-2 outputs (row pointer and a class byte per
+    tile-row; tile column, tile offset, row offsets, masks per tile), C's
+    values and in-tile columns written."""
+    row_index = 12 * a.nnz
+    operands = 4 * (a.m + 1) + row_index + 4 * (b_rows + 1) + row_index
+    c_meta = 4 * (tilem + 1) + tilem + 4 * (numtile_c + 1) + (4 + 16 + 32) * numtile_c
+    return operands + c_meta + 9 * nnz_c
 
 
 def cpu_model():
@@ -162,7 +161,7 @@ def batch_leg(ts, ctx, count=512, seed=2, nmin=1000, nmax=65536, steps=5, autotu
     seq_s = seq_std_s = float("nan")
     if sequential:
         # the same calls on operands with the standard preparation only (tiles
-        # + CSC, no element row index): what plain tsg_spgemm calls get
+        # + CSC, no element row index): the larger ones make it for the call
         std = []
         for d, op in zip(dps, ops):
             ta = ctx.csr2tile(d)
@@ -544,8 +543,8 @@ def main():
         ctx.copy_kernel_run(args.copy_calibration)
     da = ctx.upload(a)
     # operand preparation outside the timed region: tiles and the CSC tile
-    # index (every tile-row of this product fits the row-wise kernels, which
-    # do not read B's element row index)
+    # index.  Without --rowindex every product makes the row indices of its
+    # operands itself, inside the timed region
     ta = ctx.csr2tile(da)
     ctx.build_csc(ta)
     if args.rowindex:
@@ -580,7 +579,7 @@ def main():
     ev_s3 = [s["t_step3_rows_ms"] for s in steps]
     last = steps[-1]
     gflops = 2.0 * nnzcub / (ms_per_step * 1e6)
-    s3_bytes = step3_algorithmic_bytes(ta, last["numtileC"], last["nnzC"], ta.tilen)
+    s3_bytes = step3_algorithmic_bytes(a, a.n, ta.tilem, last["numtileC"], last["nnzC"])
     s3_ms = statistics.mean(ev_s3)
     achieved = s3_bytes / (s3_ms * 1e-3) / 1e9
     traffic = None

@@ -210,7 +210,7 @@ typedef struct {
     double t_step1_ms, t_step2_ms, t_step3_ms, t_alloc_ms, t_total_ms;
     long long numtileC, nnzC;
     long long tiles_sparse_acc, tiles_dense_acc, tiles_empty;
-    double t_step3_rows_ms; /* the row-wise numeric kernel's launch alone */
+    double t_step3_rows_ms; /* the row-wise numeric kernels alone (row lines and tile-rows) */
     long long heavy_rows;   /* rows with very many products (k_step3_heavy) */
     long long heavy_bytes;  /* transient device bytes of that path */
 } tsg_stats;
