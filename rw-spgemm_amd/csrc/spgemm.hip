@@ -1130,9 +1130,10 @@ __device__ __forceinline__ void step2_store(const unsigned mk[8], long long t, u
 // the window are taken by the whole wave one after another; the products of
 // the others are numbered through and taken one per lane, the entry of each
 // found from a mark at its first product (running maximum over the lanes).
-// Bound by the block's chain of loads and its 52 bytes of output per tile
-// for short rows (one block of 131 KiB fits a CU at a time), by LDS and
-// VALU issue for hub rows.  Against the hash kernel (a probe chain per
+// Bound by HBM for short rows (ER 65521 A^2 1.17 GB in 0.285 ms, three quarters
+// of it the 52 bytes per tile written), for hub rows by VALU (busy half of the
+// time) and LDS (a third) behind the block's chain of loads, with the last
+// blocks alone on the chip (R-MAT scale 16: CUs busy 62%).  Against the hash kernel (a probe chain per
 // product, the tile-row cut every 512 tiles) and tile pairs: ER 65521 A^2 0.53
 // -> 0.285 ms, R-MAT scale 16 A*A^T 17.1 -> 2.15 ms (580 G products/s).  Without
 // the read before the atomic, the long rows' own path and the split of hub
@@ -1746,7 +1747,7 @@ __device__ __forceinline__ void range_in(const int *__restrict__ list, int &b0, 
 //   is added source by source.  So every C entry still sums its products in
 //   ascending k, without atomics.
 // Four blocks (32 waves) fit a CU; it is bound by the latency of each block's
-// phases and half by VALU issue.  Against 16 lanes per C row taking one
+// phases (waves wait 72% of their cycles) and by VALU (busy 59%, ER 65521).  Against 16 lanes per C row taking one
 // source at a time (4.5 entries of a source in a segment of ER 65521), a
 // search per source and segment of 1536: ER 65521 A^2 0.62 -> 0.545 ms, banded
 // 39989 (half-bandwidth 20) 0.29 -> 0.167, R-MAT scale 16 A*A^T 12.9 -> 7.7.
@@ -1974,7 +1975,8 @@ k_step3_flat(const int *__restrict__ Arowp, const int *__restrict__ Acolx, const
 // 8000 (24 per row) 125 -> 25.6, R-MAT scale 16 10.76 -> 10.78.
 //   14 KiB of LDS, eleven waves a CU.  Bound by products behind LDS round
 // trips and fragments of B rows (5.1 of 8.4 ms), scattered 8-byte stores (2)
-// and the walk over tiles (1.4).  R-MAT scale 16 A*A^T, heavy rows with the
+// and the walk over tiles (1.4): L1 taken in 54% of its cycles, VALU busy 36%, LDS
+// 31%, 2.6 TB/s of HBM.  R-MAT scale 16 A*A^T, heavy rows with the
 // others by k_step3_flat 13.9 ms -> all by this kernel 7.1.  Parts of 1024 in
 // groups of 4 / 8 / 16 (whole product) 11.0 / 11.7 / 11.9 ms, of 2048 in groups
 // of 2 / 4 / 8 12.1 / 11.8 / 12.0, of 512 in groups of 8 12.1.
@@ -2879,8 +2881,9 @@ k_step3_rows(TileOperands op, const int *__restrict__ Cptr, const int *__restric
 // the equal tiles of a stencil to different LDS banks; the column byte is
 // left beside the sum.  Both are written out as one run, past the L2 (it
 // holds the B rows that the next tile-rows read again: 2.26 -> 2.06 ms).
-//   Four blocks (32 waves) a CU; VALU issue, LDS and L1 accesses are each
-// busy a half to two thirds of the time.  27-point 128^3 periodic 4.00 ms by
+//   Four blocks (32 waves) a CU; the L1 is taken in four of five of its cycles,
+// VALU and LDS are busy in two of three (half of the LDS's are bank conflicts),
+// HBM carries 2.6 TB/s.  27-point 128^3 periodic 4.00 ms by
 // k_step3_rows -> 2.06 (1.5 G products, 729 a C row), 61x47x53 385 -> 133 us,
 // banded 39989 (half-bandwidth 20) 165 us by k_step3_flat -> 97.  With the
 // sources broadcast by ds_bpermute (four more LDS accesses) 2.65 ms, with 80
